@@ -161,11 +161,13 @@ size_t ttt_mlp_bwd_workspace_bytes(int32_t B, int32_t NH, int32_t checkpoint_gro
 /* Byte offset of that status word (an int) inside the workspace; 0 when the mode does not apply. */
 size_t ttt_mlp_bwd_status_offset(int32_t B, int32_t NH);
 
-/* The forward with two workgroups per (batch, head), under the same conditions and with the same
+/* The forward with two roles per (batch, head), under the same conditions and with the same
  * conventions (launches, workspace, status word at int index n*32, TTT_MLP_ERR_NO_ROOM, bit-identical
- * results): one workgroup carries the state through the mini-batches and leaves every new state
- * in the workspace as bf16 operands, the other computes Out from them, 8 mini-batches behind
- * (32 when NC >= 512).
+ * results): one carries the state through the mini-batches and leaves every new state
+ * in the workspace as bf16 operands, the other computes Out from them.  With few pairs the first role takes two
+ * workgroups, which hold half of the hidden columns each and exchange partial sums, and the second one or two: three
+ * per pair where ceil(n/8)*3 fits an eighth of the CUs, four where ceil(n/8)*4 does (80 and 64 pairs on 256 CUs).
+ * Otherwise each role is one workgroup, the second 8 mini-batches behind (32 when NC >= 512).
  * Pairs are covered as in the backward: full rounds of the device with one workgroup per pair, then the
  * remaining n pairs with two each if 2*n fits the CUs.
  * No counterpart in the reference launcher (kernels/ttt/ttt.cu:594-721). */
@@ -228,7 +230,7 @@ const char* ttt_mlp_error_string(int code);
 /* How an overlapped launch of `pairs` = B*NH (batch, head) pairs is laid out on a device with
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
  * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  which = 0
- * forward (1 or 2 per pair), 1 backward (1 to 5: one or two that replay the checkpoint groups, one that walks
+ * forward (1 or 2 roles per pair; see ttt_mlp_fwd_workspace_bytes for what a role takes), 1 backward (1 to 5: one or two that replay the checkpoint groups, one that walks
  * them backwards, one for grad_L_XK / grad_L_XV, one that fetches the walk's operands into the L2 ahead of it). */
 int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long* one_workgroup_pairs,
                         long long* other_pairs, int* workgroups_per_other_pair);

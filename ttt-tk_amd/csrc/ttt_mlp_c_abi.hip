@@ -296,18 +296,31 @@ struct BwdWorkspace {
 
 // Workspace of the forward's two-workgroup mode: synchronisation words, then per (batch, head) a ring of
 // 2 * FWD_RING_MAX slots of state images and of bias vectors.
+// With the recurrence on two workgroups (n_out > 0) the ring has FWD_WIDE_RING slots, and the exchange follows.
 struct FwdWorkspace {
-  size_t off[3];
+  size_t off[4];
   size_t total;
-  explicit FwdWorkspace(long long n) {
-    const size_t slots = (size_t)n * 2 * ttt::FWD_RING_MAX;
-    const size_t bytes[3] = {ttt::bwd_sync_ints(n) * sizeof(int), slots * ttt::FWD_IMG_BYTES,
-                             slots * ttt::FWD_BIAS_FLOATS * sizeof(float)};
+  FwdWorkspace(long long n, int n_out) {
+    const size_t slots = (size_t)n * (n_out > 0 ? ttt::FWD_WIDE_RING : 2 * ttt::FWD_RING_MAX);
+    const size_t bytes[4] = {ttt::bwd_sync_ints(n) * sizeof(int), slots * ttt::FWD_IMG_BYTES,
+                             slots * ttt::FWD_BIAS_FLOATS * sizeof(float),
+                             n_out > 0 ? (size_t)n * ttt::FWD_XCHG_WORDS * 8 : 0};
     size_t o = 0;
-    for (int i = 0; i < 3; i++) { off[i] = o; o += (bytes[i] + 255) & ~(size_t)255; }
+    for (int i = 0; i < 4; i++) { off[i] = o; o += (bytes[i] + 255) & ~(size_t)255; }
     total = o;
   }
 };
+
+// Output workgroups per pair when the recurrence of each of the n pairs of a several-workgroup launch runs on two CUs of one
+// XCD, 0 if it does not: the workgroups of a pair share an XCD and wait for each other, so those of ceil(n / 8) pairs
+// must fit its CUs (an eighth of the device's).  One output workgroup keeps up with the recurrence only just; two where they fit.
+int fwd_wide_outputs(long long n, int cus) {
+#ifdef TTT_STAGE_CLOCKS   // the stage clocks are those of the one- and two-workgroup kernels
+  return 0;
+#endif
+  const long long per_xcd = (n + 7) / 8;
+  return n <= 0 ? 0 : 4 * per_xcd <= cus / 8 ? 2 : 3 * per_xcd <= cus / 8 ? 1 : 0;
+}
 
 int check_workspace(const void* workspace) {
   if (workspace == nullptr) return TTT_MLP_ERR_BAD_ARG;
@@ -433,7 +446,7 @@ extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
 extern "C" size_t ttt_mlp_fwd_workspace_bytes(int B, int NH) {
   if (B <= 0 || NH <= 0) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, false);
-  return pl.rest_split ? FwdWorkspace(pl.n_rest).total : 0;
+  return pl.rest_split ? FwdWorkspace(pl.n_rest, fwd_wide_outputs(pl.n_rest, device_cus())).total : 0;
 }
 
 extern "C" size_t ttt_mlp_fwd_status_offset(int B, int NH) {
@@ -448,7 +461,8 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, false);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const FwdWorkspace w(pl.n_rest);
+  const int n_out = fwd_wide_outputs(pl.n_rest, device_cus());
+  const FwdWorkspace w(pl.n_rest, n_out);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   {
@@ -476,6 +490,13 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
   p.wait_limit = g_wait_limit;
+  if (n_out > 0) {
+    p.n_out = n_out;
+    p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * ttt::FWD_WIDE_RING * (ttt::FWD_IMG_BYTES / 2);
+    p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
+    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
+    return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
+  }
   p.ring_log2 = p.NC >= 512 ? 5 : 3;   // 32 or 8 mini-batches per hand-over
   p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * 2 * ttt::FWD_RING_MAX * (ttt::FWD_IMG_BYTES / 2);
   p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * 2 * ttt::FWD_RING_MAX * ttt::FWD_BIAS_FLOATS;
@@ -538,7 +559,7 @@ extern "C" int ttt_mlp_fwd_launch_static(const ttt_mlp_fwd_args* a, int* sticky_
   if (pairs > STATIC_MAX_PAIRS) return TTT_MLP_ERR_SCRATCH;
   const LaunchPlan pl = plan_launches(pairs, false);
   if (!pl.rest_split || pl.n_single != 0) return TTT_MLP_ERR_NO_ROOM;
-  const FwdWorkspace w(pl.n_rest);
+  const FwdWorkspace w(pl.n_rest, fwd_wide_outputs(pl.n_rest, device_cus()));
   static_assert(static_scratch_bytes() % 256 == 0, "scratch parts are 256-byte aligned");
   if (w.total > static_scratch_bytes()) return TTT_MLP_ERR_SCRATCH;
   void* ws = nullptr;

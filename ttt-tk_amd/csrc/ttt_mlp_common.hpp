@@ -50,7 +50,9 @@ TTT_DEV bf16x8 pack8(const f32x16& x, int t) {
 // Two values at a time: one packed conversion for the high-order terms, a shift and a mask to read them back as
 // fp32, two subtractions, one packed conversion for the low-order terms (6 instructions per pair).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+// (No contraction of the subtraction with a product that formed a or b: the kernels that share a computation agree to the bit.)
 TTT_DEV void split2(float a, float b, bf16x2& hi, bf16x2& lo) {
+#pragma clang fp contract(off)
   const f32x2 ab = {a, b};
   hi = __builtin_convertvector(ab, bf16x2);
   const uint32_t hp = __builtin_bit_cast(uint32_t, hi);
@@ -138,6 +140,7 @@ TTT_DEV float half_sum2(float s01, float s23) {
 // 16 (one rotation), then the four rows, two values per swap: in the end row r of one register holds the total of
 // x[r], of the other that of x[4 + r], and lanes 0..7 of every row store their two totals.  Fixed order, fp32.
 TTT_DEV void ln_token_sum_store(float* vec, const float (&x)[8], int lane, int f0) {
+#pragma clang fp contract(off)   // not with the product that formed x: see split2
   float y[8];
 #pragma unroll
   for (int e = 0; e < 8; e++)

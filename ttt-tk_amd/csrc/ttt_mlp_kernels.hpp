@@ -24,6 +24,10 @@ struct FwdParams {
   int* sync;
   int* status;    // the status word behind the synchronisation words
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
+  // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2048 fp32],
+  // and the output workgroups per pair (1 or 2); the ring then has FWD_WIDE_RING slots.
+  unsigned long long* xchg;
+  int n_out;
   int bh0, nbh;   // this launch covers (batch, head) pairs bh0 .. bh0 + nbh - 1
   // One workgroup per pair, sequence cut into segments (seg_len > 0, a multiple of cgs): workgroup i of the launch
   // runs job job0 + i, job q = segment q / (B*NH) of pair q % (B*NH); a segment starts from the checkpoint that the
@@ -34,6 +38,8 @@ struct FwdParams {
 #endif
 };
 constexpr int FWD_RING_MAX = 32;               // most mini-batches per hand-over (8 or 32 are compiled)
+constexpr int FWD_WIDE_RING = 8;               // ring slots with the recurrence on two workgroups
+constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 1024;  // 8-byte words of a pair's exchange: 64 KiB
 constexpr int FWD_IMG_BYTES = 64 * 256 * 2 * 2;  // W1 and W2 as bf16 operands
 constexpr int FWD_BIAS_FLOATS = 256 + 64;
 
@@ -165,6 +171,8 @@ extern "C" void ttt_mlp_set_stage_clocks(unsigned* forward, unsigned* backward);
 
 // p.sync == nullptr: one workgroup per (batch, head); otherwise two (state recurrence / output branch).
 hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, hipStream_t stream);
+// The recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
+hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream);
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
 // p.sync == nullptr: one workgroup per (batch, head); otherwise two (replay / reverse walk).
 hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream);

@@ -184,17 +184,19 @@ TTT_DEV void ln_load_f32(float (&x)[8], const float* p) {
 #pragma unroll
   for (int e = 0; e < 4; e++) { x[e] = a[e]; x[4 + e] = b[e]; }
 }
-// Sum of the four pair sums of this lane's token / features.  `row` points at this token's row of the
-// first pair's region; the regions of successive pairs are 2 regions apart.
+// Sum of the four pair sums of this lane's token / features, (P0 + P1) + (P2 + P3): the order in which two CUs that hold two
+// pairs each form it.  `row` points at this token's row of the first pair's region; the regions of successive pairs are
+// 2 regions apart.
 TTT_DEV void ln_gather(float (&z)[8], const float* row) {
-  f32x4 a = *reinterpret_cast<const f32x4*>(row), b = *reinterpret_cast<const f32x4*>(row + 4);
 #pragma unroll
-  for (int pp = 1; pp < 4; pp++) {
-    a += *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN);
-    b += *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN + 4);
+  for (int q = 0; q < 2; q++) {
+    f32x4 a[4];
+#pragma unroll
+    for (int pp = 0; pp < 4; pp++) a[pp] = *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN + 4 * q);
+    const f32x4 t = (a[0] + a[1]) + (a[2] + a[3]);
+#pragma unroll
+    for (int e = 0; e < 4; e++) z[4 * q + e] = t[e];
   }
-#pragma unroll
-  for (int e = 0; e < 4; e++) { z[e] = a[e]; z[4 + e] = b[e]; }
 }
 TTT_DEV float sum8(const float (&x)[8]) {
   float s = 0.f;
@@ -221,11 +223,45 @@ TTT_DEV float ln_normalize(float (&z)[8], float* std_out) {
   *std_out = v * rstd;  // sqrt(v)
   return rstd;
 }
+// Second-order pass through the fused LayerNorm loss for the 8 features of this lane's token.  gg: the sum over the hidden
+// dimension of what the weight step backwards gives (gradient wrt dl/dZ2 before the bias term and -eta); gb: gradient
+// wrt b2; xh, go, gz: x_hat, grad_output and dl/dZ2 of the loss.  Out: gy (gradient wrt y), dg (norm-weight gradient
+// terms), dz = dZ2; returns sum_F gz * gb, the bias part of d eta.
+TTT_DEV float walk_layernorm(float (&gg)[8], const float (&gb)[8], float neg_eta, const float (&xh)[8], const float (&go)[8],
+                             const float (&gz)[8], const float (&gam)[8], float sdf, float (&gy)[8], float (&dg)[8], float (&dz)[8]) {
+#pragma clang fp contract(off)   // which product of a sum of two is fused is written out: every launch shape gives the same bits
+#pragma unroll
+  for (int e = 0; e < 8; e++) gg[e] = (gg[e] + gb[e]) * neg_eta;   // grad wrt dl/dZ2
+  const float rsd = 1.f / sdf;
+  const float eta_bias = oct_sum(dot8(gz, gb));
+  const float s0 = oct_sum(sum8(gg)), a = oct_sum(dot8(gg, xh));
+  float bb = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) bb = __builtin_fmaf(go[e] * gam[e], xh[e], bb);
+  bb = oct_sum(bb);
+  const float inv = rsd * (1.f / FD);
+  float sg = 0.f, sx = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const float ggx = __builtin_fmaf(-__builtin_fmaf(xh[e], a, s0), 1.f / FD, gg[e]) * rsd;
+    gy[e] = gam[e] * ggx;
+    dg[e] = __builtin_fmaf(go[e], ggx, gy[e] * xh[e]);
+    dz[e] = __builtin_fmaf(-__builtin_fmaf(go[e] * gam[e], a, gg[e] * bb), inv, gy[e] * gam[e]);
+    sg = __builtin_fmaf(-__builtin_fmaf(dz[e], xh[e], gg[e] * gz[e]), rsd, sg);
+    sx += dz[e];
+  }
+  sg = oct_sum(sg);
+  sx = oct_sum(sx);
+#pragma unroll
+  for (int e = 0; e < 8; e++) dz[e] = __builtin_fmaf(__builtin_fmaf(sg, xh[e], -sx * rsd), 1.f / FD, dz[e] * rsd);
+  return eta_bias;
+}
 // acc[f0 + e] += sum over this wave's tokens of x[e]   (wave-private LDS vector).  The 8 tokens sit in the lanes
 // that share lane % 8: lanes 8 apart inside a row of 16 (one rotation), then the four rows, two values per swap
 // (row_pair_sum2, half_sum2): in the end row r of one register holds the total of x[r], of the other that of
 // x[4 + r], and lanes 0..7 of every row add their two totals to the vector.
 TTT_DEV void ln_token_sum_add(float* s_acc, const float (&x)[8], int lane, int f0) {
+#pragma clang fp contract(off)   // not with the products that formed x: every launch shape gives the same bits
   float y[8];
 #pragma unroll
   for (int e = 0; e < 8; e++)
@@ -394,7 +430,8 @@ constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK wo
 // FIN: grad_L_XK is a leaf of the walk - it needs the running gradients, but nothing needs it.  With a
 // fourth workgroup the walk hands over the operands of its two products (gW1, G1, dZ1 as register images)
 // and g_y, and that workgroup (bwd_finish_dxk) forms the products, their pair sum and the final sum.
-template <int ROLE, bool IMG, bool FIN>
+// WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
+template <int ROLE, bool IMG, bool FIN, bool WIDE = false>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; the other roles take
 // the whole sequence, K - 1 .. 0).
 TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int turn, const int k_hi, const int k_lo) {
@@ -534,41 +571,30 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     acc_load_rows(gW2s, gbuf((seg_first ? p.grad_L_W2_last : p.grad_L_W2_init) + (size_t)bh * HID * FD), 0, FD, hid0, 0, c, h);
   }
   int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;   // + 0, + 8: groups replayed by workgroup 0 / 1
-  int* const w_walked = w_sync + 16;
+  int* const w_walked = w_sync + (WIDE ? BWW_WALKED : 16);
   int* const w_finished = w_sync + 24;
-  const int n_replay = ROLE == 0 ? 1 : p.n_replay, n_sets = 2 * n_replay;
+  const int n_replay = ROLE == 0 ? 1 : p.n_replay, n_sets = WIDE ? p.n_sets : 2 * n_replay;
   int* const w_status = p.status;
   int* const s_flag = reinterpret_cast<int*>(smem + SB_FLAG);
 
-  // The replay's share of the norm gradients is kept as two sums, of the even and of the odd groups (counted
-  // from the end of the sequence), whoever replays them; the walk's share is a third.  A workgroup that adds
-  // to more than one of them keeps the others parked in HBM, 4 KiB each: one workgroup per (batch, head) in
-  // two slots of the caller's x_hat_ln_group, a single replaying workgroup in the workspace.
+  // The replay's share of the norm gradients is formed group by group and added to a running sum in the groups' order, so it
+  // does not depend on who replays them.  The running sum sits in HBM (slot 0 of the park, 4 KiB): with one workgroup per
+  // (batch, head) in the caller's x_hat_ln_group, where the walk's sum waits behind it (slot 1) while the LDS accumulators
+  // serve a replay, otherwise in the workspace, added to by the walk (by the grad_L_XK workgroup where there is one).
   const gptr_t gPark = ROLE == 0 ? gbuf(p.x_hat_ln_group + (size_t)bh * cgs * (CS * FD))
                                  : gbuf(p.norm_park + (size_t)bh * (BW_NWAVE * 2 * FD));
   constexpr unsigned PARK_BYTES = BW_NWAVE * 2 * FD * 4;
-  if (ROLE == 0 ? seg_first : (ROLE == 1 && n_replay == 1)) {   // parked sums start at zero
+  if (ROLE == 0 ? seg_first : (ROLE == 2 && !FIN)) {   // the running sum starts at zero
     g_stf(gPark, np_off, 0, 0.f);
     g_stf(gPark, np_off, FD * 4, 0.f);
-    if constexpr (ROLE == 0) {
-      g_stf(gPark, np_off, PARK_BYTES, 0.f);
-      g_stf(gPark, np_off, PARK_BYTES + FD * 4, 0.f);
-    }
   }
-  if (ROLE == 0 && !seg_first) {   // the walk's sum as the segment before this one left it (a third slot of the park)
-    s_dgw[lane] = g_ldf(gPark, np_off, 2 * PARK_BYTES);
-    s_dbw[lane] = g_ldf(gPark, np_off, 2 * PARK_BYTES + FD * 4);
+  if (ROLE == 0 && !seg_first) {   // the walk's sum as the segment before this one left it
+    s_dgw[lane] = g_ldf(gPark, np_off, PARK_BYTES);
+    s_dbw[lane] = g_ldf(gPark, np_off, PARK_BYTES + FD * 4);
   }
-  // Exchanges the wave's LDS accumulators with a parked sum (every lane owns two words of both).
-  auto norm_swap = [&](unsigned slot) {
-    WAVE_SYNC();
-    const float a0 = s_dgw[lane], a1 = s_dbw[lane];
-    const float p0 = g_ldf(gPark, np_off, slot * PARK_BYTES), p1 = g_ldf(gPark, np_off, slot * PARK_BYTES + FD * 4);
-    s_dgw[lane] = p0;
-    s_dbw[lane] = p1;
-    g_stf(gPark, np_off, slot * PARK_BYTES, a0);
-    g_stf(gPark, np_off, slot * PARK_BYTES + FD * 4, a1);
-    WAVE_SYNC();
+  auto add_to_running_sum = [&](float a0, float a1) {
+    g_stf(gPark, np_off, 0, g_ldf(gPark, np_off, 0) + a0);
+    g_stf(gPark, np_off, FD * 4, g_ldf(gPark, np_off, FD * 4) + a1);
   };
 
   TTT_STAGES_BEGIN();
@@ -577,7 +603,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     const int done = p.K - 1 - k;                    // number of this group, counted from the end of the sequence
     if (ROLE == 1 && done % n_replay != turn) continue;
     const int set = ROLE == 0 ? 0 : done % n_sets;
-    int* const w_replayed = w_sync + 8 * (done % n_replay);
+    int* const w_replayed = w_sync + (WIDE ? 1 : 8) * (done % n_replay);
     REFRESH_OFFSETS();
     const size_t slot = (size_t)bh * p.K + k;
     const unsigned ckW = static_cast<unsigned>(k) * (FD * HID * 4u);   // byte offset of this group's checkpoint in bCW1 / bCW2
@@ -585,18 +611,23 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     if constexpr (ROLE != 2) {
       if constexpr (ROLE == 1) {   // the set is free once the reverse walk is done with the group that used it last
         if (done >= n_sets && !wait_at_least(w_walked, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
+        if (WIDE && done >= n_sets && !wait_at_least(w_walked + 4, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
         if constexpr (FIN) {   // ... and so is the workgroup that reads the before-state images for grad_L_XK
           if (done >= n_sets && !wait_at_least(w_finished, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
         }
-        // a single replaying workgroup adds to the sum of this group's parity: the groups alternate, so from
-        // the second group on the live sum and the parked one change places
-        if (n_replay == 1 && done > 0) norm_swap(0);
+        WAVE_SYNC();
+        s_dgw[lane] = 0.f;   // (every lane its own words)
+        s_dbw[lane] = 0.f;
       }
       // park the running gradients while the forward state needs the registers
       if constexpr (ROLE == 0) {
         acc_store_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_store_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
-        norm_swap(done & 1);   // the walk's sum out, the replay's sum of this parity in
+        WAVE_SYNC();
+        g_stf(gPark, np_off, PARK_BYTES, s_dgw[lane]);   // the walk's sum out
+        g_stf(gPark, np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
+        s_dgw[lane] = 0.f;
+        s_dbw[lane] = 0.f;
       }
       AccT<2, 1> W1s;
       AccT<1, 2> W2s;
@@ -1038,23 +1069,20 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         TTT_STAGE(BS_R_OUT_BACKWARD);
       }
       if constexpr (ROLE == 1) {
-        if (done + n_replay >= p.K) {   // this workgroup's last group: hand its norm-gradient sums to the walk
-          WAVE_SYNC();
-          float* np = p.norm_partial + ((size_t)bh * 2 + (done & 1)) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
-          np[lane] = s_dgw[lane];
-          np[FD + lane] = s_dbw[lane];
-          if (n_replay == 1) {   // and the sum of the other parity (zero if there was one group only)
-            float* no = p.norm_partial + ((size_t)bh * 2 + (1 - (done & 1))) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
-            no[lane] = g_ldf(gPark, np_off, 0);
-            no[FD + lane] = g_ldf(gPark, np_off, FD * 4);
-          }
-        }
+        WAVE_SYNC();   // this group's norm-gradient sums go with it
+        float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
+        np[lane] = s_dgw[lane];
+        np[FD + lane] = s_dbw[lane];
       }
       // running gradients back into registers
       if constexpr (ROLE == 0) {
         acc_load_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_load_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
-        norm_swap(done & 1);
+        WAVE_SYNC();
+        add_to_running_sum(s_dgw[lane], s_dbw[lane]);
+        s_dgw[lane] = g_ldf(gPark, np_off, PARK_BYTES);
+        s_dbw[lane] = g_ldf(gPark, np_off, PARK_BYTES + FD * 4);
+        WAVE_SYNC();
       }
       if constexpr (ROLE == 1) publish(w_replayed, done / n_replay + 1);
       TTT_STAGE(BS_PUBLISH);
@@ -1068,6 +1096,9 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       if (!wait_at_least(w_replayed, done / n_replay + 1, w_status, s_flag, p.wait_limit)) return;
       if constexpr (FIN) {   // the hand-over set of this group's parity is free once the group before last is finished
         if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return;
+      } else {
+        const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
+        add_to_running_sum(np[lane], np[FD + lane]);
       }
     }
     // hand-over buffers of this group for the grad_L_XK workgroup (set = parity of the group)
@@ -1284,49 +1315,26 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         const float sdf = sdf_n;
         ln_gather(gg, s_lnrow);
         ln_load_f32(gb, s_gb2 + f0);
-        const float neg_eta = -s_eta[tok];
-#pragma unroll
-        for (int e = 0; e < 8; e++) gg[e] = (gg[e] + gb[e]) * neg_eta;   // grad wrt dl/dZ2
         ln_cvt8(xh, xhf);
         ln_cvt8(go, gof);
         ln_load(gz, s_gz2 + tok * LDX + f0);
         ln_load_f32(gam, s_gam + f0);
-        const float rsd = 1.f / sdf;
+        float gx[8], dg[8];
+        float tot = walk_layernorm(gg, gb, -s_eta[tok], xh, go, gz, gam, sdf, gy, dg, gx);
         // dEta: -(sum_F gZ2*(X2 gW2 + gb2) + sum_H gZ1*(XK gW1 + gb1))
         {
           LANE_VARS;
-          float tot = oct_sum(dot8(gz, gb));
+          float d[BW_NWAVE];
 #pragma unroll
-          for (int u = 0; u < BW_NWAVE; u++) tot += s_deta[u * CS + tok];
+          for (int u = 0; u < BW_NWAVE; u++) d[u] = s_deta[u * CS + tok];
+          tot += ((d[0] + d[4]) + (d[1] + d[5])) + ((d[2] + d[6]) + (d[3] + d[7]));
           if ((lane & 7) == 0) g_sth(bDETA, 2 * tok, mb * (CS * 2), (bf16)((float)deta_old - tot));
         }
-        const float s0 = oct_sum(sum8(gg)), a = oct_sum(dot8(gg, xh));
-        float bb = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) bb = __builtin_fmaf(go[e] * gam[e], xh[e], bb);
-        bb = oct_sum(bb);
-        float gx[8], dg[8];
-        const float inv = rsd * (1.f / FD);
-        float sg = 0.f, sx = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const float ggx = (gg[e] - (s0 + xh[e] * a) * (1.f / FD)) * rsd;
-          gy[e] = gam[e] * ggx;
-          dg[e] = go[e] * ggx + gy[e] * xh[e];
-          gx[e] = gy[e] * gam[e] - (go[e] * gam[e] * a + gg[e] * bb) * inv;
-          sg += (-gx[e] * xh[e] - gg[e] * gz[e]) * rsd;
-          sx += gx[e];
-        }
-        sg = oct_sum(sg);
-        sx = oct_sum(sx);
         if constexpr (!FIN) {   // with a grad_L_XK workgroup these token sums and grad_L_XV are formed there, from g_y and dg
           ln_token_sum_add(s_dgw, dg, lane, f0);
           ln_token_sum_add(s_dbw, gy, lane, f0);
-        }
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          gx[e] = gx[e] * rsd + (sg * xh[e] - sx * rsd) * (1.f / FD);   // dZ2
-          if constexpr (!FIN) dxv_old[e] = (bf16)((float)dxv_old[e] - gy[e]);   // dXV accumulates -g_y
+          for (int e = 0; e < 8; e++) dxv_old[e] = (bf16)((float)dxv_old[e] - gy[e]);   // dXV accumulates -g_y
         }
         // g_y is needed again for dXK: park it (the XQ / E2 tiles are dead by now), or hand it over
         {
@@ -1486,28 +1494,23 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   if (tid < HID) p.grad_L_b1_init[(size_t)bh * HID + tid] = s_gb1[tid];
   if (tid < FD) p.grad_L_b2_init[(size_t)bh * FD + tid] = s_gb2[tid];
   // norm-weight / norm-bias gradients: sum the per-wave LDS accumulators
-  // The replay's two sums: parked in HBM by this workgroup, or handed over by the replaying workgroups, whose
-  // last counts this workgroup has acquired (a second replaying workgroup has nothing to hand over if there is
-  // one group only).
   if constexpr (FIN) return;   // with a grad_L_XK workgroup the walk holds no share of these sums: they are written there
-  if (ROLE == 0 && !seg_last) {   // the next segment goes on with the walk's sum (the replay's two are parked already)
-    g_stf(gPark, np_off, 2 * PARK_BYTES, s_dgw[lane]);
-    g_stf(gPark, np_off, 2 * PARK_BYTES + FD * 4, s_dbw[lane]);
+  if (ROLE == 0 && !seg_last) {   // the next segment goes on with the walk's sum (the replay's is in place already)
+    g_stf(gPark, np_off, PARK_BYTES, s_dgw[lane]);
+    g_stf(gPark, np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
     return;
   }
   if (tid < 2 * FD) {
     const int which = tid / FD, f = tid % FD;
     const float* rp = ROLE == 0 ? reinterpret_cast<const float*>(p.x_hat_ln_group + (size_t)bh * cgs * (CS * FD))
-                                : p.norm_partial + (size_t)bh * 2 * (BW_NWAVE * 2 * FD);
-    const bool have_odd = ROLE == 0 || p.K > 1 || n_replay == 1;
-    float s = 0.f, sr0 = 0.f, sr1 = 0.f;
+                                : p.norm_park + (size_t)bh * (BW_NWAVE * 2 * FD);
+    float s = 0.f, sr = 0.f;
 #pragma unroll
     for (int u = 0; u < BW_NWAVE; u++) {
       s += s_red[(u * 2 + which) * FD + f];
-      sr0 += rp[(u * 2 + which) * FD + f];
-      if (have_odd) sr1 += rp[BW_NWAVE * 2 * FD + (u * 2 + which) * FD + f];
+      sr += rp[(u * 2 + which) * FD + f];   // the other waves' stores: before the barrier above
     }
-    (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = (sr0 + sr1) + s;
+    (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = sr + s;
   }
 }
 #undef REFRESH_OFFSETS
@@ -1539,6 +1542,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #undef bDXV
 #undef bDETA
 
+#ifndef TTT_BWD_ROLES_ONLY   // ttt_mlp_bwd_wide.hip takes the roles above and below without these kernels
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   int bh = p.bh0 + blockIdx.x, k_hi = p.K - 1, k_lo = 0;
@@ -1550,11 +1554,13 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_kernel(const BwdParams
   }
   bwd_body<0, false, false>(p, smem, bh, 0, k_hi, k_lo);
 }
+#endif
 
 // grad_L_XK on a workgroup of its own: for every mini-batch of every group, as soon as the walk is done with the
 // group, dk = gW1 G1^T + W1 dZ1^T (W1 before the step: from the replay's image, or the checkpoint), its sum over
 // the hidden dimension, + g_y, accumulated into grad_L_XK.  Same wave / lane roles and the same order of every
 // sum as in the walk, so the result is the same to the bit.
+template <bool IMG, bool WIDE>
 TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int bh) {
   float* s_P = reinterpret_cast<float*>(smem + SB_P);
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
@@ -1566,7 +1572,7 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
   float* s_own = s_P + (pp * 2 + r) * RGN;
   float* s_partner = s_P + (pp * 2 + (1 - r)) * RGN;
   const float* s_lnrow = s_P + (1 - r) * RGN + (tok & 31) * LDR + f0;
-  const int cgs = p.cgs, n_sets = 2 * p.n_replay;
+  const int cgs = p.cgs, n_sets = WIDE ? p.n_sets : 2 * p.n_replay;
   const unsigned t16 = 16 * tid, vln = (tok * FD + f0) * 2;
   int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   int* const w_walked = w_sync + 16;
@@ -1592,26 +1598,109 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
   float* s_dgw = s_red + (v * 2 + 0) * FD;
   float* s_dbw = s_red + (v * 2 + 1) * FD;
   if (lane < FD) { s_dgw[lane] = 0.f; s_dbw[lane] = 0.f; }
+  int n_step = 0, n_seen = 0;
+  int lane_v = lane;
+#define FIN_LANE                                                                                  \
+  asm volatile("" : "+v"(lane_v));                                                                \
+  const int lane = lane_v, h = lane >> 5, c = lane & 31, tid = (v << 6) | lane;                   \
+  const int tok = 8 * v + (lane >> 3), f0 = 8 * (lane & 7);                                       \
+  const unsigned t16 = 16 * tid, vln = (tok * FD + f0) * 2;                                       \
+  const float* s_lnrow = s_P + (1 - r) * RGN + (tok & 31) * LDR + f0;                             \
+  (void)h; (void)c; (void)t16; (void)vln; (void)s_lnrow
+  float nr0 = 0.f, nr1 = 0.f;   // the replay's share: this lane's two words of the wave's running sum
   TTT_STAGES_BEGIN();
   for (int k = p.K - 1; k >= 0; k--) {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k, set = done % n_sets;
     // the walk hands over whole groups, except the last one it walks (k = 0): that one in chunks of FIN_CHUNK mini-batches
-    if (k > 0 && !wait_at_least(w_walked, done + 1, p.status, s_flag, p.wait_limit)) return;
+    // (WIDE: every mini-batch is announced by both halves of the walk)
+    if (!WIDE && k > 0 && !wait_at_least(w_walked, done + 1, p.status, s_flag, p.wait_limit)) return;
     TTT_STAGE(BS_X_GROUP);
     const size_t ofin = uni64(((size_t)bh * 2 + (done & 1)) * cgs);
     const size_t o_img = uni64((size_t)bh * cgs * (CS * HID)), o_tile = uni64((size_t)bh * cgs * (CS * FD));
     const gptr_t gIMG2 = gbuf((set ? p.alt_grad_l_wrt_Z1_group[set - 1] : p.grad_l_wrt_Z1_group) + o_img);   // W2 after each step
     const gptr_t gGZ2 = gbuf((set ? p.alt_grad_l_wrt_Z2_group[set - 1] : p.grad_l_wrt_Z2_group) + o_tile);   // dl/dZ2
-    const gptr_t gDD = gbuf((set ? p.alt_W1_init_group[set - 1] : p.W1_init_group) + uni64((size_t)bh * cgs * (FD * HID)));   // gelu'(Z1) images
+    // gelu'(Z1) images, or (without IMG) the images of Z1
+    const gptr_t gDD = IMG ? gbuf((set ? p.alt_W1_init_group[set - 1] : p.W1_init_group) + uni64((size_t)bh * cgs * (FD * HID)))
+                           : gbuf((set ? p.alt_Z1_group[set - 1] : p.Z1_group) + o_img);
     const gptr_t gGZ1B = gbuf((set ? p.alt_Z1_bar_group[set - 1] : p.Z1_bar_group) + uni64((size_t)bh * cgs * (CS * HID)));
     const gptr_t gDZ = gbuf(p.fin_dz + ofin * (CS * HID)), gGY = gbuf(p.fin_gy + ofin * (2 * CS * FD));
     const gptr_t gIMG1 = gbuf((set ? p.alt_X2_group[set - 1] : p.X2_group) + uni64((size_t)bh * cgs * (CS * HID)));
     const unsigned ckW = static_cast<unsigned>(k) * (FD * HID * 4u);
+    // What a mini-batch takes from the replay's images and the inputs is asked for during the mini-batch before it, each operand
+    // as soon as its registers are free (the first mini-batch of a group: here): fetched where it is used, this workgroup
+    // spent 18 k of its 22 k clocks per mini-batch waiting, and the walk on two CUs is faster than that.
+    u32x4 xq, xk, gz;
+    bf16 eta_n[2];
+    bf16x8 g1b[4];   // gZ1_bar^T of the output branch: lane = hid, contraction = tok
+    bf16x8 w2bf[4];  // W2 before the step: lane = hid, contraction = F
+    bf16x8 d1[2][2], w1b[2][2];
+    auto ask_tiles = [&](int jn) {
+      FIN_LANE;
+      const unsigned xo = (k * cgs + jn) * TILE_BYTES;
+      xq = g_ld_stream<u32x4>(gXQ, t16, xo);
+      xk = g_ld_stream<u32x4>(gXK, t16, xo);
+      gz = g_ld_stream<u32x4>(gGZ2, t16, jn * TILE_BYTES);
+      eta_n[0] = g_ldh(gETA, 2 * c, (k * cgs + jn) * (CS * 2) + 64 * tb[0]);
+      eta_n[1] = g_ldh(gETA, 2 * c, (k * cgs + jn) * (CS * 2) + 64 * tb[1]);
+    };
+    auto ask_g1b = [&](int jn) {
+      FIN_LANE;
+#pragma unroll
+      for (int s = 0; s < 4; s++) g1b[s] = image_load<true>(gGZ1B, jn * IMG_BYTES, s, t16);
+    };
+    auto ask_w2 = [&](int jn) {
+      FIN_LANE;
+      if (jn > 0) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) w2bf[s] = image_load<true>(gIMG2, (jn - 1) * IMG_BYTES, s, t16);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; s++) w2bf[s] = piece_from_f32(gCW2, ckW, FD, hid0, 0, s, c, h);
+      }
+    };
+    auto ask_d1 = [&](int jn) {   // gelu'(Z1)
+      FIN_LANE;
+#pragma unroll
+      for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) d1[a][t] = image_load<true>(gDD, jn * (IMG ? 2 * IMG_BYTES : IMG_BYTES), 2 * tb[a] + t, t16);
+    };
+    auto ask_w1 = [&](int jn) {   // W1 before the step
+      FIN_LANE;
+      if (jn > 0) {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) w1b[a][t] = image_load<true>(gIMG1, (jn - 1) * IMG_BYTES, 2 * a + t, t16);
+      } else {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) w1b[a][t] = piece_from_f32(gCW1, ckW, HID, 32 * a, hid0, t, c, h);
+      }
+    };
     for (int j = n_mb - 1; j >= 0; j--) {
-      if (k == 0 && (j == n_mb - 1 || (j & (FIN_CHUNK - 1)) == FIN_CHUNK - 1)) {
+      const int jn = j > 0 ? j - 1 : 0;
+      FIN_LANE;
+      if constexpr (WIDE) {
+        if (++n_step > n_seen) {
+          n_seen = wait_for_both(w_sync + BWW_GIVEN, w_sync + BWW_GIVEN + 4, n_step, p.status, s_flag, p.wait_limit);
+          if (n_seen < 0) return;
+        }
+      } else if (k == 0 && (j == n_mb - 1 || (j & (FIN_CHUNK - 1)) == FIN_CHUNK - 1)) {
         if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return;
         TTT_STAGE(BS_X_GROUP);
+      }
+      if (j == n_mb - 1) {   // the group's norm-gradient sums: published with it, and the walk has acquired it
+        const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
+        nr0 += np[lane];
+        nr1 += np[FD + lane];
+        ask_tiles(j);
+        ask_g1b(j);
+        ask_w2(j);
+        ask_d1(j);
+        ask_w1(j);
       }
       const unsigned xo = (k * cgs + j) * TILE_BYTES, so = j * TILE_BYTES, ho = j * IMG_BYTES;
       const bf16x8 dxk_ld = g_ld_stream<bf16x8>(p.overwrite ? gbuf(zero_tile) : gDXK, vln, p.overwrite ? 0u : xo);
@@ -1619,39 +1708,31 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
       const f32x4 gy_lo = g_ld_stream<f32x4>(gGY, 2 * vln, 4 * so), gy_hi = g_ld_stream<f32x4>(gGY, 2 * vln + 16, 4 * so);
       const f32x4 dg_lo = g_ld_stream<f32x4>(gGY, 2 * vln, 4 * so + 2 * TILE_BYTES);
       const f32x4 dg_hi = g_ld_stream<f32x4>(gGY, 2 * vln + 16, 4 * so + 2 * TILE_BYTES);
-      // everything this workgroup reads it reads once: streaming loads, so that the lines fetched ahead of the walk
-      // on the same XCD stay in the L2 (c4 backward -0.35 ms)
-      const u32x4 xq = g_ld_stream<u32x4>(gXQ, t16, xo), xk = g_ld_stream<u32x4>(gXK, t16, xo);
-      const u32x4 gz = g_ld_stream<u32x4>(gGZ2, t16, so);
-      const float eta_i[2] = {bf2f(g_ldh(gETA, 2 * c, (k * cgs + j) * (CS * 2) + 64 * tb[0])),
-                              bf2f(g_ldh(gETA, 2 * c, (k * cgs + j) * (CS * 2) + 64 * tb[1]))};
-      bf16x8 g1b[4];   // gZ1_bar^T of the output branch: lane = hid, contraction = tok
-      bf16x8 w2bf[4];  // W2 before the step: lane = hid, contraction = F
-#pragma unroll
-      for (int s = 0; s < 4; s++) {
-        g1b[s] = image_load<true>(gGZ1B, ho, s, t16);
-        w2bf[s] = w2_before<true>(gIMG2, gCW2, ckW, j, s, hid0, c, h, t16);
-      }
-      bf16x8 g1[2][2], dz[2][2], w1b[2][2], d1[2][2];
+      bf16x8 g1[2][2], dz[2][2];
 #pragma unroll
       for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-          d1[a][t] = image_load<true>(gDD, j * (2 * IMG_BYTES), 2 * tb[a] + t, t16);   // gelu'(Z1)
-          dz[a][t] = image_load<true>(gDZ, ho, 2 * tb[a] + t, t16);
-          w1b[a][t] = w1_before<true>(gIMG1, gCW1, ckW, j, a, t, hid0, c, h, t16);
-        }
+        for (int t = 0; t < 2; t++) dz[a][t] = image_load<true>(gDZ, ho, 2 * tb[a] + t, t16);
+      const float eta_i[2] = {bf2f(eta_n[0]), bf2f(eta_n[1])};
       lds_put16x(s_xq, tid, xq);
       lds_put16x(s_xk, tid, xk);
       lds_put16(s_gz2, tid, gz);
+      ask_tiles(jn);
       __syncthreads();
+      {
+      FIN_LANE;
       mma_jit<4>(gW1s, [&](int fb, int s) { return xpiece_tr(s_xq, fb, s, lane); },         // + XQ^T gZ1_bar
                  [&](int, int s) { return g1b[s]; });
+      ask_g1b(jn);
+      }
+      AccT<2, 2> dk;
+      {
+      FIN_LANE;
       store_state_rows<LDF>(T2, gW1s, c, h);                                                  // gW1 rows [hid][F]
 #pragma unroll
       for (int s = 0; s < 4; s++) store_piece_rows<LDF>(T1, 0, s, c, h, w2bf[s]);            // W2 before the step, rows [hid][F]
+      ask_w2(jn);
       WAVE_SYNC();
-      AccT<2, 2> dk;
       acc_zero(dk);
 #pragma unroll
       for (int i = 0; i < 2; i++) {
@@ -1664,7 +1745,12 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
         for (int t = 0; t < 2; t++) {
 #pragma unroll
           for (int jj = 0; jj < 8; jj++) {
-            const float a = (float)d1[i][t][jj];
+            float a = (float)d1[i][t][jj];
+            if constexpr (!IMG) {
+              float g, b;
+              gelu_fdd(a, g, a, b);
+              a = (float)(bf16)a;
+            }
             const float gz1 = R.b[0][0][8 * t + jj] * a;
             g1[i][t][jj] = (bf16)(-eta_i[i] * gz1);
           }
@@ -1672,6 +1758,10 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
           for (int rb = 0; rb < 2; rb++) dk.b[rb][i] = MFMA(piece_tr<LDF>(T2, rb, t, lane), g1[i][t], dk.b[rb][i]);
         }
       }
+      ask_d1(jn);
+      }
+      {
+      FIN_LANE;
       WAVE_SYNC();   // the readers of T1 (W2 rows) are done
 #pragma unroll
       for (int i = 0; i < 2; i++)
@@ -1679,11 +1769,13 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
         for (int t = 0; t < 2; t++) store_piece_rows<LDH>(T1, tb[i], t, c, h, dz[i][t]);     // dZ1 rows [tok][hid]
       WAVE_SYNC();
       mma_jit<2>(dk, [&](int rb, int s) { return w1b[rb][s]; }, [&](int i, int s) { return dz[i][s]; });
+      ask_w1(jn);
       mma_jit<4>(gW1s, [&](int fb, int s) { return xpiece_tr(s_xk, fb, s, lane); },         // + XK^T dZ1
                  [&](int, int s) { return piece_tr<LDH>(T1, 0, s, lane); });
       WAVE_SYNC();   // this wave's readers of T1 / T2 are done
       TTT_STAGE(BS_X_PRODUCTS);
       pair_sum(s_own, s_partner, dk, c, h);
+      }
       float z[8];
       ln_gather(z, s_lnrow);
       const float gyv[8] = {gy_lo[0], gy_lo[1], gy_lo[2], gy_lo[3], gy_hi[0], gy_hi[1], gy_hi[2], gy_hi[3]};
@@ -1705,24 +1797,25 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
     TTT_STAGE(BS_PUBLISH);
   }
   TTT_STAGES_END(p.stage_clocks == nullptr ? nullptr : p.stage_clocks + ((size_t)bh * 4 + 3) * (BW_NWAVE * STAGE_SLOTS));
-  // norm-weight / norm-bias gradients: the replaying workgroups' two sums (handed over before their last counts,
-  // which the walk had acquired before its own last count) + the walk's, in the order of the other launch shapes
+  // norm-weight / norm-bias gradients: the replay's sum + the walk's, in the order of the other launch shapes
+  __syncthreads();
+  s_P[v * 2 * FD + lane] = nr0;
+  s_P[v * 2 * FD + FD + lane] = nr1;
   __syncthreads();
   if (tid < 2 * FD) {
     const int which = tid / FD, f = tid % FD;
-    const float* rp = p.norm_partial + (size_t)bh * 2 * (BW_NWAVE * 2 * FD);
-    const bool have_odd = p.K > 1 || p.n_replay == 1;
-    float s = 0.f, sr0 = 0.f, sr1 = 0.f;
+    float s = 0.f, sr = 0.f;
 #pragma unroll
     for (int u = 0; u < BW_NWAVE; u++) {
       s += s_red[(u * 2 + which) * FD + f];
-      sr0 += rp[(u * 2 + which) * FD + f];
-      if (have_odd) sr1 += rp[BW_NWAVE * 2 * FD + (u * 2 + which) * FD + f];
+      sr += s_P[(u * 2 + which) * FD + f];
     }
-    (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = (sr0 + sr1) + s;
+    (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = sr + s;
   }
 }
+#undef FIN_LANE
 
+#ifndef TTT_BWD_ROLES_ONLY
 // ------------------------------------------------------------------ the workgroup that fetches ahead of the walk
 // The walk asks per mini-batch for 240 KiB that a replaying workgroup wrote a checkpoint group earlier (six register
 // images, four tiles) or that the caller passed in (two tiles): none of it is in the L2 by then, and one CU cannot
@@ -1801,7 +1894,7 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_split_kernel(const Bwd
   if (role < NREPLAY) bwd_body<1, IMG, FINISH>(p, smem, bh, role, p.K - 1, 0);
   else if (role == NREPLAY) bwd_body<2, IMG, FINISH>(p, smem, bh, 0, p.K - 1, 0);
   else if constexpr (FINISH) {
-    if (role == NREPLAY + 1) bwd_finish_dxk(p, smem, bh);
+    if (role == NREPLAY + 1) bwd_finish_dxk<true, false>(p, smem, bh);
     else bwd_prefetch(p, smem, bh);
   }
 }
@@ -1838,3 +1931,6 @@ hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
   if (p.n_replay == 2) return launch(ttt::ttt_mlp_bwd_split_kernel<2, false>);
   return launch(ttt::ttt_mlp_bwd_split_kernel<1, false>);
 }
+#else
+}  // namespace ttt
+#endif

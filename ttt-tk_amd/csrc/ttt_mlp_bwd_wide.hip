@@ -1,0 +1,726 @@
+// Remat backward with the reverse walk of one (batch, head) spread over two CUs (few pairs: the walk's chain is the bound).
+//
+// The walk on one CU spends 28 k clocks on a mini-batch.  Here two workgroups of one XCD hold 128 hidden columns each
+// (two of the four wave pairs of ttt_mlp_bwd.hip), with two kinds of waves as in ttt_mlp_fwd_wide.hip:
+//   waves 0-3 (one per SIMD)  32 hidden columns each: every matrix product and the running gradients
+//   waves 4-7                 sums over the hidden dimension, their exchange with the other CU, the LayerNorm lanes, the
+//                             gradient wrt b2, and everything that comes from HBM ahead of time: the next mini-batch's
+//                             tiles through their registers into LDS, and one load per cache line of the operand images of
+//                             the mini-batch after it, which the compute waves then find in the L2
+// The sum that crosses (the gradient wrt dl/dZ2, one fp32 tile per mini-batch and direction) is taken in two blocks of 32
+// tokens: block 0's travels while block 1 is computed, block 1's while the products that do not wait for it run.
+// Two to four further workgroups per pair replay checkpoint groups in turn (bwd_body<1>), one forms grad_L_XK / grad_L_XV and
+// the norm gradients (bwd_finish_dxk).  Every sum has the order of the one-workgroup kernel: same results to the bit.
+#define TTT_BWD_ROLES_ONLY
+#include "ttt_mlp_bwd.hip"
+#include "ttt_mlp_exchange.hpp"
+
+namespace ttt {
+
+// LDS carve-up of a workgroup of the walk (bytes)
+constexpr int BWW_XQ = 0;
+constexpr int BWW_GZB = BWW_XQ + SB_TILE;                 // gZ2_bar
+constexpr int BWW_XK = BWW_GZB + SB_TILE;                 // two buffers, alternating per mini-batch
+constexpr int BWW_GZ2 = BWW_XK + 2 * SB_TILE;             // dl/dZ2, two buffers
+constexpr int BWW_DZ2 = BWW_GZ2 + 2 * SB_TILE;
+constexpr int BWW_T12 = BWW_DZ2 + SB_TILE;                // per compute wave: T1, T2
+constexpr int BWW_T0 = BWW_T12 + 4 * SB_REGION;           // per compute wave: X2 rows
+constexpr int BWW_P = BWW_T0 + 4 * SB_WTILE;              // per compute wave: its partial sum of one token block, [32 tok][F] fp32
+constexpr int BWW_PTILE = 32 * LDR * 4;
+constexpr int BWW_GB1 = BWW_P + 4 * BWW_PTILE;            // gradient wrt b1, 32 per compute wave
+constexpr int BWW_GB2 = BWW_GB1 + 4 * BW_NS * 4;
+constexpr int BWW_GAM = BWW_GB2 + FD * 4;
+constexpr int BWW_DETA = BWW_GAM + FD * 4;                // [4 compute waves][64 tokens]
+constexpr int BWW_ETA = BWW_DETA + 4 * CS * 4;            // fp32, two buffers
+constexpr int BWW_FLAG = BWW_ETA + 2 * CS * 4;            // [0] a wait gave up, [1] gathers of block 0 done
+constexpr int BWW_BYTES = BWW_FLAG + 16;
+static_assert(BWW_BYTES <= SM_BWD_BYTES, "the launch asks for SM_BWD_BYTES (the replay's carve-up)");
+
+template <bool IMG>
+TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh, const int half) {
+  typedef __attribute__((address_space(3))) int* lint_t;
+  const lint_t s_flag = (lint_t)reinterpret_cast<int*>(smem + BWW_FLAG);
+  auto flag = [&](int i) { return __hip_atomic_load(s_flag + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int u = w & 3;                                   // number among its kind
+  const int v = 2 * half + (u & 1) + 4 * (u >> 1);       // compute wave u: hidden block, = wave of the one-workgroup kernel
+  const int head = bh % p.NH, hid0 = BW_NS * v;
+  const int cgs = p.cgs, n_sets = p.n_sets, n_replay = p.n_replay;
+  bf16* const s_xq = reinterpret_cast<bf16*>(smem + BWW_XQ);
+  bf16* const s_gzb = reinterpret_cast<bf16*>(smem + BWW_GZB);
+  bf16* const s_dz2 = reinterpret_cast<bf16*>(smem + BWW_DZ2);
+  float* const s_gb2 = reinterpret_cast<float*>(smem + BWW_GB2);
+  float* const s_gam = reinterpret_cast<float*>(smem + BWW_GAM);
+  float* const s_deta = reinterpret_cast<float*>(smem + BWW_DETA);
+  int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; j++) ones[j] = (bf16)1.0f;
+  if (tid == 0) say_xcd(words + BWW_XCD + half);
+  if (tid < 2) s_flag[tid] = 0;
+  if (tid < FD) {
+    s_gam[tid] = p.ttt_norm_weight[head * FD + tid];
+    s_gb2[tid] = p.grad_L_b2_last[(size_t)bh * FD + tid];
+  }
+  // this (batch, head)'s part of each class of tensor (elements), and the per-group tensors of set `set`
+  const size_t ox = uni64((size_t)bh * p.NC * (CS * FD)), oe = uni64((size_t)bh * p.NC * CS);
+  const size_t of = uni64((size_t)bh * cgs * (CS * FD)), oh = uni64((size_t)bh * cgs * (CS * HID));
+  const size_t ot = uni64((size_t)bh * cgs * CS), ock = uni64((size_t)bh * p.K * (FD * HID));
+  // The pointers are read from the kernel-argument segment where they are used (see bwd_body).
+  typedef const __attribute__((address_space(4))) BwdParams* KernArgs;
+  KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+#define WGRP(name) (set ? ka->alt_##name[set - 1] : ka->name)
+  int lane_v = lane;
+#define WW_LANE                                                        \
+  asm volatile("" : "+v"(lane_v));                                     \
+  const int lane = lane_v, h = lane >> 5, c = lane & 31;               \
+  const unsigned t16 = 16 * ((v << 6) | lane);                         \
+  (void)h; (void)c; (void)t16
+
+  if (w < 4) {
+    // ================================================================ compute waves
+    bf16* const T1 = reinterpret_cast<bf16*>(smem + BWW_T12 + u * SB_REGION);
+    bf16* const T2 = T1 + 64 * LDH;
+    bf16* const T0 = reinterpret_cast<bf16*>(smem + BWW_T0 + u * SB_WTILE);
+    float* const s_Pw = reinterpret_cast<float*>(smem + BWW_P + u * BWW_PTILE);
+    float* const s_gb1w = reinterpret_cast<float*>(smem + BWW_GB1) + u * BW_NS;
+    AccT<2, 1> gW1s;
+    AccT<1, 2> gW2s;
+    acc_load_rows(gW1s, gbuf(p.grad_L_W1_last + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
+    acc_load_rows(gW2s, gbuf(p.grad_L_W2_last + (size_t)bh * HID * FD), 0, FD, hid0, 0, c, h);
+    if (lane < BW_NS) s_gb1w[lane] = p.grad_L_b1_last[(size_t)bh * HID + hid0 + lane];
+    __syncthreads();   // flags
+    __syncthreads();   // placement known, the first group is there, its last mini-batch's tiles too
+    if (flag(0) != 0) return;
+    bf16x8 x2b[4], g1b[4];   // what the output branch adds (lane = hid, contraction = tok), asked for a mini-batch ahead
+    bf16x8 w2bf[4];          // W2 before the step, and gelu, gelu', gelu'' of Z1 by token block
+    bf16x8 gq[2][2], aq[2][2], bq[2][2];
+    gptr_t gX2B, gGZ1B, gI2, gZ, gD;
+    auto group_images = [&](int set) {
+      gX2B = gbuf(WGRP(X2_bar_group) + oh);
+      gGZ1B = gbuf(WGRP(Z1_bar_group) + oh);
+      gI2 = gbuf(WGRP(grad_l_wrt_Z1_group) + oh);
+      gZ = gbuf(WGRP(Z1_group) + oh);
+      gD = gbuf(WGRP(W1_init_group) + oh);
+    };
+    const gptr_t gCk = gbuf(ka->W2_ck + ock);
+    auto ask_gelu = [&](int i, int j) {
+      WW_LANE;
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        gq[i][t] = image_load<IMG>(gZ, j * IMG_BYTES, 2 * i + t, t16);
+        if constexpr (IMG) {
+          aq[i][t] = image_load<false>(gD, 2 * j * IMG_BYTES, 2 * i + t, t16);
+          bq[i][t] = image_load<true>(gD, 2 * j * IMG_BYTES + IMG_BYTES, 2 * i + t, t16);
+        }
+      }
+    };
+    // Operands are asked for one to two stages ahead.  One CU cannot keep enough requests in flight to hide the way to HBM (80 KiB
+    // asked for in a row take 9 k clocks to issue), so another workgroup brings the lines into the L2 before (bwd_wide_prefetch);
+    // what the grad_L_XK workgroup reads next is left there.
+    auto ask_bar = [&](int j) {
+      WW_LANE;
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        x2b[s] = image_load<true>(gX2B, j * IMG_BYTES, s, t16);
+        g1b[s] = image_load<false>(gGZ1B, j * IMG_BYTES, s, t16);
+      }
+    };
+    auto ask_step = [&](int k, int j) {
+      WW_LANE;
+      if (j > 0) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) w2bf[s] = image_load<false>(gI2, (j - 1) * IMG_BYTES, s, t16);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; s++) w2bf[s] = piece_from_f32(gCk, static_cast<unsigned>(k) * (FD * HID * 4u), FD, hid0, 0, s, c, h);
+      }
+      ask_gelu(0, j);
+    };
+    // One wave per SIMD: the latency of an LDS read is hidden only by what is put between it and its use, so operands are read a
+    // product or more ahead, and the fences keep the scheduler from sinking the reads again.
+#define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+    // row sums of a 32-row operand of four pieces on the matrix cores (as lds_rowsum_add_jit), and their addition to gb1
+    auto rowsum4 = [&](bf16x8 a, bf16x8 b, bf16x8 c4, bf16x8 d) {
+      f32x16 t;
+#pragma unroll
+      for (int i = 0; i < 16; i++) t[i] = 0.f;
+      t = MFMA(a, ones, t);
+      t = MFMA(b, ones, t);
+      t = MFMA(c4, ones, t);
+      return MFMA(d, ones, t);
+    };
+    auto add_gb1 = [&](const f32x16& t) {
+      WW_LANE;
+      f32x4 old[4];
+#pragma unroll
+      for (int g = 0; g < 4; g++) old[g] = *reinterpret_cast<const f32x4*>(s_gb1w + 8 * g + 4 * h);
+      if (c == 0) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) old[g][e] += t[4 * g + e];
+          *reinterpret_cast<f32x4*>(s_gb1w + 8 * g + 4 * h) = old[g];
+        }
+      }
+      WAVE_SYNC();
+    };
+    int n = 0;   // mini-batches walked
+    group_images(0);
+    ask_bar(min(cgs, p.NC - (p.K - 1) * cgs) - 1);
+    ask_step(p.K - 1, min(cgs, p.NC - (p.K - 1) * cgs) - 1);
+    for (int k = p.K - 1; k >= 0; k--) {
+      const int n_mb = min(cgs, p.NC - k * cgs);
+      const int done = p.K - 1 - k;
+      const gptr_t gDZ = gbuf(ka->fin_dz + uni64(((size_t)bh * 2 + (done & 1)) * cgs) * (CS * HID));
+      for (int j = n_mb - 1; j >= 0; j--, n++) {
+        const unsigned ho = j * IMG_BYTES;
+        const bf16* const s_xk = reinterpret_cast<const bf16*>(smem + BWW_XK + (n & 1) * SB_TILE);
+        const bf16* const s_gz2 = reinterpret_cast<const bf16*>(smem + BWW_GZ2 + (n & 1) * SB_TILE);
+        const float* const s_eta = reinterpret_cast<const float*>(smem + BWW_ETA) + (n & 1) * CS;
+        // ---- what the output branch adds to the running gradients
+        {
+          WW_LANE;
+          bf16x8 zb[4][2], xq[4][2];
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) zb[s][fb] = piece_tr<LDX>(s_gzb, fb, s, lane);
+          SCHED_FENCE();
+          f32x16 t = rowsum4(g1b[0], g1b[1], g1b[2], g1b[3]);
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gW2s.b[0][fb] = MFMA(x2b[s], zb[s][fb], gW2s.b[0][fb]);
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) xq[s][fb] = xpiece_tr(s_xq, fb, s, lane);
+            SCHED_FENCE();
+          }
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gW1s.b[fb][0] = MFMA(xq[s][fb], g1b[s], gW1s.b[fb][0]);
+          add_gb1(t);
+        }
+        ask_gelu(1, j);
+        // ---- the weight step, backwards (state BEFORE this mini-batch), one token block at a time
+        bf16x8 t2p[2][2], uhp[2][2], d1p[2][2];   // d1p: gelu'(Z1)
+        float eta_i[2];
+        {
+          WW_LANE;
+#pragma unroll
+          for (int s = 0; s < 4; s++) store_piece_rows<LDF>(T1, 0, s, c, h, w2bf[s]);   // W2 before the step, rows [hid][F]
+          store_state_rows<LDF>(T2, gW1s, c, h);                                         // gW1 rows [hid][F]
+          WAVE_SYNC();
+        }
+        auto step_back = [&](int i) {
+          WW_LANE;
+          eta_i[i] = s_eta[32 * i + c];
+          AccT<1, 1> R, S;   // R = gZ2 W2^T, S = XK gW1 + gb1   (rows hid, lane = tok)
+          acc_zero(R);
+          acc_init_rows_lds(S, s_gb1w, h);
+          bf16x8 w2r[4], w1r[4], gz[4], xk[4];
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            w2r[s] = piece_rows<LDF>(T1, 0, s, c, h);
+            gz[s] = piece_rows<LDX>(s_gz2, i, s, c, h);
+            w1r[s] = piece_rows<LDF>(T2, 0, s, c, h);
+            xk[s] = xpiece_rows(s_xk, i, s, c, h);
+          }
+          SCHED_FENCE();
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            R.b[0][0] = MFMA(w2r[s], gz[s], R.b[0][0]);
+            S.b[0][0] = MFMA(w1r[s], xk[s], S.b[0][0]);
+          }
+          AccT<2, 1> pz;
+          acc_zero(pz);
+          float de = 0.f;
+          bf16x8 x2c[2], uc[2];
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            if constexpr (!IMG) {
+              const bf16x8 zc = gq[i][t];
+#pragma unroll
+              for (int jj = 0; jj < 8; jj++) {
+                float g, a, b;
+                gelu_fdd((float)zc[jj], g, a, b);
+                x2c[t][jj] = (bf16)g;
+                aq[i][t][jj] = (bf16)a;
+                bq[i][t][jj] = (bf16)b;
+              }
+              asm volatile("" : "+v"(x2c[t]), "+v"(aq[i][t]), "+v"(bq[i][t]));   // finished here (see the replay's gelu')
+            } else {
+              x2c[t] = gq[i][t];
+            }
+#pragma unroll
+            for (int jj = 0; jj < 8; jj++) {
+              const float a = (float)aq[i][t][jj], b = (float)bq[i][t][jj];
+              const float r0 = R.b[0][0][8 * t + jj], sv = S.b[0][0][8 * t + jj];
+              const float gz1 = r0 * a;                                   // dl/dZ1
+              de = __builtin_fmaf(gz1, sv, de);
+              uc[t][jj] = (bf16)(sv * a);
+              uhp[i][t][jj] = (bf16)(-eta_i[i] * sv * a);
+              t2p[i][t][jj] = (bf16)(-eta_i[i] * r0 * sv * b);
+            }
+            d1p[i][t] = aq[i][t];
+            store_piece_rows<LDH>(T0, i, t, c, h, x2c[t]);                // X2 rows [tok][hid]
+          }
+          bf16x8 gzv[4], w2t[2][2];
+#pragma unroll
+          for (int s = 0; s < 2; s++) gzv[s] = piece_rows<LDX>(s_gz2, i, s, c, h);
+          SCHED_FENCE();
+          // pz = gW2^T X2^T ; d eta partial ; + W2^T u^T
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) pz.b[rb][0] = MFMA(piece_state(gW2s, rb, t), x2c[t], pz.b[rb][0]);
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+#pragma unroll
+            for (int jj = 0; jj < 8; jj++) de = __builtin_fmaf((float)gzv[s][jj],  pz.b[s >> 1][0][8 * (s & 1) + jj], de);
+            if (s == 1) {
+              SCHED_FENCE();
+              gzv[2] = piece_rows<LDX>(s_gz2, i, 2, c, h);
+              gzv[3] = piece_rows<LDX>(s_gz2, i, 3, c, h);
+#pragma unroll
+              for (int q = 0; q < 4; q++) w2t[q >> 1][q & 1] = piece_tr<LDF>(T1, q & 1, q >> 1, lane);
+              SCHED_FENCE();
+            }
+          }
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) pz.b[rb][0] = MFMA(w2t[t][rb], uc[t], pz.b[rb][0]);
+          const float a = half_sum_valu(de);
+          if (i == 1) {   // block 0's sums have been gathered (long since)
+            while (flag(1) < 4 * (n + 1)) __builtin_amdgcn_s_sleep(1);
+          }
+          if (h == 0) s_deta[u * CS + 32 * i + c] = a;
+#pragma unroll
+          for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+              const f32x16& x = pz.b[rb][0];
+              f32x4 q = {x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]};
+              *reinterpret_cast<f32x4*>(s_Pw + c * LDR + 32 * rb + 8 * g + 4 * h) = q;
+            }
+        };
+        step_back(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // dZ1 of the last mini-batch is out (and everything asked for is here)
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                    // B1: block 0's sums
+        __builtin_amdgcn_sched_barrier(0);
+        step_back(1);
+        // ---- inner MLP backwards and the updates of the running gradients, token block i
+        f32x16 dx2[2], gb1_t;                               // gradient wrt X2; row sums of dZ1
+        auto mlp_back = [&](int i) {
+          WW_LANE;
+          bf16x8 w2r[4], dr[4], dt[2][2], x2[2], xkt[2][2], dz1[2];
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            w2r[s] = piece_rows<LDF>(T1, 0, s, c, h);
+            dr[s] = piece_rows<LDX>(s_dz2, i, s, c, h);
+          }
+          SCHED_FENCE();
+          f32x16 q = dx2[i];
+#pragma unroll
+          for (int s = 0; s < 4; s++) q = MFMA(w2r[s], dr[s], q);                              // + dZ2 W2^T
+          SCHED_FENCE();
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            x2[t] = piece_tr<LDH>(T0, 0, 2 * i + t, lane);
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) dt[t][fb] = piece_tr<LDX>(s_dz2, fb, 2 * i + t, lane);
+          }
+          SCHED_FENCE();
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gW2s.b[0][fb] = MFMA(x2[t], dt[t][fb], gW2s.b[0][fb]);   // + X2^T dZ2
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            bf16x8 dz;
+#pragma unroll
+            for (int jj = 0; jj < 8; jj++) dz[jj] = (bf16)__builtin_fmaf(q[8 * t + jj], (float)d1p[i][t][jj], (float)t2p[i][t][jj]);   // dZ1
+            image_store<true>(gDZ, ho, 2 * i + t, t16, dz);                                    // for the grad_L_XK workgroup
+            store_piece_rows<LDH>(T2, i, t, c, h, dz);                                         // rows [tok][hid]
+          }
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) xkt[t][fb] = xpiece_tr(s_xk, fb, 2 * i + t, lane);
+          WAVE_SYNC();
+#pragma unroll
+          for (int t = 0; t < 2; t++) dz1[t] = piece_tr<LDH>(T2, 0, 2 * i + t, lane);
+          if (i == 0) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) gb1_t[e] = 0.f;
+          }
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gW1s.b[fb][0] = MFMA(xkt[t][fb], dz1[t], gW1s.b[fb][0]);   // + XK^T dZ1
+            gb1_t = MFMA(dz1[t], ones, gb1_t);
+          }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                    // B2: block 1's sums; dZ2 of block 0
+        __builtin_amdgcn_sched_barrier(0);
+        if (j == 0) group_images((done + 1) % n_sets);
+        const int kn = j > 0 || k == 0 ? k : k - 1, jn = j > 0 ? j - 1 : cgs - 1;   // (behind the last mini-batch: dropped)
+        // ---- while block 1's sums cross: the products of the inner MLP backwards that do not need them
+        {
+          WW_LANE;
+          store_state_rows<LDH>(T2, gW2s, c, h);            // gW2 rows [F][hid] (transposed read gives lane = hid)
+          bf16x8 gz[2][4], gw[4];
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) gz[i][s] = piece_rows<LDX>(s_gz2, i, s, c, h);
+          WAVE_SYNC();
+#pragma unroll
+          for (int s = 0; s < 4; s++) gw[s] = piece_tr<LDH>(T2, 0, s, lane);
+          SCHED_FENCE();
+          f32x16 q[2];
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) q[i][e] = 0.f;
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) q[i] = MFMA(gw[s], gz[i][s], q[i]);                  // P2 = gZ2 gW2^T
+          WAVE_SYNC();
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) store_piece_rows<LDH>(T2, i, t, c, h, uhp[i][t]);   // -eta u rows [tok][hid]
+          ask_bar(jn);   // the next mini-batch's output-branch images (the helpers made sure of its group before B1)
+          bf16x8 ut[4], gt[4][2];
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gt[s][fb] = piece_tr<LDX>(s_gz2, fb, s, lane);
+          WAVE_SYNC();
+#pragma unroll
+          for (int s = 0; s < 4; s++) ut[s] = piece_tr<LDH>(T2, 0, s, lane);
+          SCHED_FENCE();
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int fb = 0; fb < 2; fb++) gW2s.b[0][fb] = MFMA(ut[s], gt[s][fb], gW2s.b[0][fb]);   // (-eta u)^T gZ2
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) dx2[i][e] = q[i][e] * -eta_i[i];
+          WAVE_SYNC();
+        }
+        mlp_back(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                    // B3: dZ2 of block 1; the next mini-batch's tiles
+        __builtin_amdgcn_sched_barrier(0);
+        const int gave_up = flag(0);
+        mlp_back(1);
+        ask_step(kn, jn);
+        add_gb1(gb1_t);
+        if (gave_up != 0) return;
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();   // the last dZ1 is out
+    acc_store_rows(gW1s, gbuf(p.grad_L_W1_init + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
+    acc_store_rows(gW2s, gbuf(p.grad_L_W2_init + (size_t)bh * HID * FD), 0, FD, hid0, 0, c, h);
+    if (lane < BW_NS) p.grad_L_b1_init[(size_t)bh * HID + hid0 + lane] = s_gb1w[lane];
+    return;
+  }
+
+  // ================================================================== helper waves
+  const int q8 = lane >> 3, f0 = 8 * (lane & 7), t_in = 8 * u + q8;   // LayerNorm lanes: token t_in of a block, features f0 ..
+  const unsigned voff = (t_in * FD + f0) * 2;
+  constexpr unsigned HALF_TILE = TILE_BYTES / 2;                        // 32 tokens
+  int* const w_status = p.status;
+  bool gave_up = false;
+  __syncthreads();   // flags
+  auto wait_for = [&](int* word, int target) {
+    if (lane == 0 && !wait_word(word, target, w_status, p.wait_limit)) s_flag[0] = 1;
+  };
+  // group number `done` (from the end) has been replayed
+  auto wait_group = [&](int done) { wait_for(words + done % n_replay, done / n_replay + 1); };
+  // What one mini-batch needs from HBM besides the operand images: a chunk of 16 bytes per lane and token block of each
+  // tile - the lanes that hold a chunk are the LayerNorm lanes of that token and those features.
+  struct Ahead {
+    bf16x8 xq[2], xk[2], gz[2], gzb[2], xh[2], go[2];
+    float sd[2];
+    bf16 eta[2], deta[2];
+  } nx;
+  auto ask = [&](int k, int j) {
+    const int set = (p.K - 1 - k) % n_sets, mb = k * cgs + j;
+    asm volatile("" : "+s"(ka));
+    const gptr_t gq = gbuf(ka->XQ + ox), gk = gbuf(ka->XK + ox), gz = gbuf(WGRP(grad_l_wrt_Z2_group) + of);
+    const gptr_t gb = gbuf(WGRP(grad_x_hat_fused_group) + of), gx = gbuf(WGRP(x_hat_fused_group) + of);
+    const gptr_t gg = gbuf(WGRP(grad_output_fused_group) + of), gs = gbuf(WGRP(std_fused_group) + ot);
+    const gptr_t ge = gbuf(ka->last_eta + oe), gd = gbuf(ka->grad_L_last_eta + oe), zero = gbuf(zero_tile);
+    const bool ow = ka->overwrite != 0;
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      const unsigned xo = mb * TILE_BYTES + b * HALF_TILE, so = j * TILE_BYTES + b * HALF_TILE;
+      nx.gz[b] = g_ld8h(gz, voff, so);
+      nx.gzb[b] = g_ld_stream<bf16x8>(gb, voff, so);
+      nx.xq[b] = g_ld8h(gq, voff, xo);
+      nx.xk[b] = g_ld8h(gk, voff, xo);
+      nx.xh[b] = g_ld_stream<bf16x8>(gx, voff, so);
+      nx.go[b] = g_ld_stream<bf16x8>(gg, voff, so);
+      nx.sd[b] = g_ldf(gs, 4 * t_in, (j * CS + 32 * b) * 4);
+      nx.eta[b] = g_ldh(ge, 2 * t_in, (mb * CS + 32 * b) * 2);
+      nx.deta[b] = g_ldh(ow ? zero : gd, 2 * t_in, ow ? 0u : (mb * CS + 32 * b) * 2);
+    }
+  };
+  auto put = [&](int n) {   // tiles of the mini-batch that is walked as number n
+    bf16* const s_xk = reinterpret_cast<bf16*>(smem + BWW_XK + (n & 1) * SB_TILE);
+    bf16* const s_gz2 = reinterpret_cast<bf16*>(smem + BWW_GZ2 + (n & 1) * SB_TILE);
+    float* const s_eta = reinterpret_cast<float*>(smem + BWW_ETA) + (n & 1) * CS;
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      const int row = 32 * b + t_in;
+      ln_store_h(s_xq + xrow(row) + f0, nx.xq[b]);
+      ln_store_h(s_xk + xrow(row) + f0, nx.xk[b]);
+      ln_store_h(s_gz2 + row * LDX + f0, nx.gz[b]);
+      ln_store_h(s_gzb + row * LDX + f0, nx.gzb[b]);
+      if ((lane & 7) == 0) s_eta[row] = bf2f(nx.eta[b]);
+    }
+  };
+  const bool near = [&]() {
+    bool alive = true;
+    const bool one = on_one_xcd(words + BWW_XCD, 3, lane, w_status, p.wait_limit, alive);
+    if (!alive && lane == 0) s_flag[0] = 1;
+    return one;
+  }();
+  wait_group(0);   // (every helper wave itself)
+  {
+    const int j0 = min(cgs, p.NC - (p.K - 1) * cgs) - 1;
+    if (flag(0) == 0) {
+      ask(p.K - 1, j0);
+      put(0);
+    }
+  }
+  __syncthreads();
+  if (flag(0) != 0) return;
+  const gword64_t xch = (gword64_t)(p.xchg + (size_t)bh * BWW_XCHG_WORDS);
+  const float* const s_row = reinterpret_cast<const float*>(smem + BWW_P) + t_in * LDR + f0;
+  float gam[8];
+  ln_load_f32(gam, s_gam + f0);
+  const gptr_t bDETA = gbuf(p.grad_L_last_eta + oe);
+  __builtin_amdgcn_s_setprio(2);
+
+  int n = 0;
+  for (int k = p.K - 1; k >= 0; k--) {
+    const int n_mb = min(cgs, p.NC - k * cgs);
+    const int done = p.K - 1 - k;
+    const size_t ofin = uni64(((size_t)bh * 2 + (done & 1)) * cgs);
+    const gptr_t bFGY = gbuf(p.fin_gy + ofin * (2 * CS * FD));
+    for (int j = n_mb - 1; j >= 0; j--, n++) {
+      const int mb = k * cgs + j;
+      const bf16* const s_gz2 = reinterpret_cast<const bf16*>(smem + BWW_GZ2 + (n & 1) * SB_TILE);
+      const Ahead cur = nx;
+      // ---- ahead of time, while the compute waves are busy: the next mini-batch
+      const bool more = n + 1 < p.NC;
+      if (j == 0 && k > 0) wait_group(done + 1);
+      const int kn = j > 0 ? k : k - 1, jn = j > 0 ? j - 1 : cgs - 1;
+      // gradient wrt b2: what the output branch adds
+      if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_gzb, u, s, lane); }, ones, c, h);
+      if (more && flag(0) == 0) ask(kn, jn);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // g_y of the last mini-batch and the marks put back are in place
+      __syncthreads();   // B1
+      if (u == 0 && lane == 0 && n > 0) {
+        // all waves' stores of the last mini-batch were acknowledged before the barrier, all its reads are done
+        if (!near) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_store(words + BWW_GIVEN + 4 * half, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (j == n_mb - 1) __hip_atomic_store(words + BWW_WALKED + 4 * half, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float mine[8], d_mine, gy[8], dg[8], tot;
+      auto gather_send = [&](int blk) {   // this CU's sums over its 128 hidden columns; sent to the other CU
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+          f32x4 a[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) a[i] = *reinterpret_cast<const f32x4*>(s_row + i * (BWW_PTILE / 4) + 4 * q);
+          const f32x4 t = (a[0] + a[2]) + (a[1] + a[3]);
+#pragma unroll
+          for (int e = 0; e < 4; e++) mine[4 * q + e] = t[e];
+        }
+        const float* const d = s_deta + 32 * blk + t_in;
+        d_mine = (d[0] + d[2 * CS]) + (d[CS] + d[3 * CS]);
+        const gword64_t dst = xch + ((((n & 1) * 2 + half) * 2 + blk) * 4 + u) * (64 * BWW_WORDS) + lane;
+#pragma unroll
+        for (int i = 0; i < 4; i++) wd_put(dst + 64 * i, wd_pack(mine[2 * i], mine[2 * i + 1]), near);
+        wd_put(dst + 256, wd_pack(d_mine, 0.f), near);
+      };
+      auto finish_block = [&](int blk) {
+        const int tok = 32 * blk + t_in;
+        const gword64_t src = xch + ((((n & 1) * 2 + 1 - half) * 2 + blk) * 4 + u) * (64 * BWW_WORDS) + lane;
+        uint64_t wv[BWW_WORDS];
+        if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+#pragma unroll
+        for (int i = 0; i < BWW_WORDS; i++) wd_put(src + 64 * i, ~0ull, near);
+        float gg[8], gb[8], xh[8], go[8], gz[8], dz[8];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          gg[2 * i] = mine[2 * i] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[i]));
+          gg[2 * i + 1] = mine[2 * i + 1] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[i] >> 32));
+        }
+        const float d_sum = d_mine + __builtin_bit_cast(float, static_cast<uint32_t>(wv[4]));
+        ln_load_f32(gb, s_gb2 + f0);
+        ln_cvt8(xh, cur.xh[blk]);
+        ln_cvt8(go, cur.go[blk]);
+        ln_cvt8(gz, cur.gz[blk]);
+        tot = walk_layernorm(gg, gb, -bf2f(cur.eta[blk]), xh, go, gz, gam, cur.sd[blk], gy, dg, dz) + d_sum;
+        ln_store(s_dz2 + tok * LDX + f0, dz);
+      };
+      // what the block gives to the caller and to the grad_L_XK workgroup, once the other waves have what they wait for
+      auto store_block = [&](int blk) {
+        if (half == 0) {   // both halves hold these; one writes them
+          if ((lane & 7) == 0) g_sth(bDETA, 2 * t_in, (mb * CS + 32 * blk) * 2, (bf16)((float)cur.deta[blk] - tot));
+          const unsigned o = 2 * j * 4 * HALF_TILE + 2 * blk * HALF_TILE;   // g_y and the norm-weight terms: two fp32 tiles per mini-batch
+          const f32x4 y0 = {gy[0], gy[1], gy[2], gy[3]}, y1 = {gy[4], gy[5], gy[6], gy[7]};
+          const f32x4 d0 = {dg[0], dg[1], dg[2], dg[3]}, d1 = {dg[4], dg[5], dg[6], dg[7]};
+          g_st_stream<f32x4>(bFGY, 2 * voff, o, y0);
+          g_st_stream<f32x4>(bFGY, 2 * voff + 16, o, y1);
+          g_st_stream<f32x4>(bFGY, 2 * voff, o + 2 * TILE_BYTES, d0);
+          g_st_stream<f32x4>(bFGY, 2 * voff + 16, o + 2 * TILE_BYTES, d1);
+        }
+      };
+      gather_send(0);
+      // (relaxed: the gathered values are in registers; a release would also wait for the words just sent)
+      if (lane == 0) __hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      // the group's hand-over set to the grad_L_XK workgroup is free (written from here on)
+      if (j == n_mb - 1 && done >= 2) wait_for(words + 24, done - 1);
+      finish_block(0);
+      __syncthreads();   // B2
+      gather_send(1);
+      store_block(0);
+      if (more) put(n + 1);   // XQ and gZ2_bar are read before B1 only, XK and gZ2 alternate
+      finish_block(1);
+      if (gave_up && lane == 0) s_flag[0] = 1;
+      __syncthreads();   // B3
+      if (flag(0) != 0) return;
+      store_block(1);
+      if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_dz2, u, s, lane); }, ones, c, h);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (u == 0 && lane == 0) {
+    if (!near) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __hip_atomic_store(words + BWW_GIVEN + 4 * half, p.NC, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(words + BWW_WALKED + 4 * half, p.K, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (u < 2 && half == 0 && lane < 32) p.grad_L_b2_init[(size_t)bh * FD + 32 * u + lane] = s_gb2[32 * u + lane];
+#undef WGRP
+#undef WW_LANE
+}
+
+// The workgroup that reads ahead of the walk (see bwd_prefetch in ttt_mlp_bwd.hip): one dword of every 128-byte line that the
+// walk and the grad_L_XK workgroup will ask for, two mini-batches ahead of the walk, which asks for most of it one ahead.
+constexpr int BWW_AHEAD = 2;
+TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const int bh) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int v = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cgs = p.cgs, n_replay = p.n_replay, n_sets = p.n_sets;
+  int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
+  int* const s_flag = reinterpret_cast<int*>(smem + BWW_FLAG);
+  const size_t ox = uni64((size_t)bh * p.NC * (CS * FD)), of = uni64((size_t)bh * cgs * (CS * FD)), oh = uni64((size_t)bh * cgs * (CS * HID));
+  const unsigned line_t = 128u * lane, line_i = 128u * (tid & 255);   // this thread's line of a tile / of an image
+  const bool up = v >= 4;
+  int n = 0, seen = 0;
+  for (int k = p.K - 1; k >= 0; k--) {
+    const int n_mb = min(cgs, p.NC - k * cgs);
+    const int done = p.K - 1 - k, set = done % n_sets;
+    if (!wait_at_least(words + done % n_replay, done / n_replay + 1, p.status, s_flag, p.wait_limit)) return;
+#define PGRP(name) (set ? p.alt_##name[set - 1] : p.name)
+    // wave v: tile v (two inputs, four of the set); waves 0-3 / 4-7: one image each of a pair
+    gptr_t tile = gbuf(p.XQ + ox);
+    unsigned tile0 = k * cgs * TILE_BYTES;
+    if (v == 1) tile = gbuf(p.XK + ox);
+    if (v >= 2) tile0 = 0;
+    if (v == 2) tile = gbuf(PGRP(grad_l_wrt_Z2_group) + of);
+    if (v == 3) tile = gbuf(PGRP(grad_x_hat_fused_group) + of);
+    if (v == 4) tile = gbuf(PGRP(x_hat_fused_group) + of);
+    if (v >= 5) tile = gbuf(PGRP(grad_output_fused_group) + of);
+    const gptr_t img0 = up ? gbuf(PGRP(Z1_bar_group) + oh) : gbuf(PGRP(X2_bar_group) + oh);
+    const gptr_t img1 = up ? gbuf(PGRP(grad_l_wrt_Z1_group) + oh) : gbuf(PGRP(Z1_group) + oh);
+    const gptr_t img2 = gbuf(PGRP(W1_init_group) + oh), img3 = gbuf(PGRP(X2_group) + oh);
+#undef PGRP
+    for (int j = n_mb - 1; j >= 0; j--, n++) {
+      if (seen < n + 1 - BWW_AHEAD) {
+        const int s = wait_for_pace(words + BWW_GIVEN, n + 1 - BWW_AHEAD, p.status, s_flag, p.wait_limit);
+        if (s == 0) return;
+        seen = s - 1;
+      }
+      if (seen > n) continue;   // the walk is past this mini-batch already
+      const unsigned ho = j * IMG_BYTES, before = (j > 0 ? j - 1 : 0) * IMG_BYTES;
+      unsigned got[5] = {0, 0, 0, 0, 0};
+      got[1] = g_ld<unsigned>(img0, line_i, ho);
+      got[2] = g_ld<unsigned>(img1, line_i, up ? before : ho);
+      got[3] = g_ld<unsigned>(img2, line_i, 2 * ho + (up ? IMG_BYTES : 0));
+      if (v < 6) got[0] = g_ld<unsigned>(tile, line_t, tile0 + j * TILE_BYTES);
+      if (up) got[4] = g_ld<unsigned>(img3, line_i, before);   // W1 before the step, for the grad_L_XK workgroup
+#pragma unroll
+      for (int i = 0; i < 5; i++) asm volatile("" ::"v"(got[i]));   // landed; nothing is done with them
+    }
+  }
+}
+
+// Per (batch, head): two workgroups that walk, one for grad_L_XK, one that reads ahead (PREFETCH), NREPLAY that replay; laid out like
+// the wide forward's.
+template <int NREPLAY, bool PREFETCH>
+__global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_wide_kernel(const BwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int PER = NREPLAY + 3 + (PREFETCH ? 1 : 0);
+  constexpr bool IMG = NREPLAY > 2;   // with the replay to spare it also evaluates the GELU family for the walk
+  const int b = blockIdx.x;
+  int bh = (b / (8 * PER)) * 8 + (b & 7);
+  const int role = (b >> 3) % PER;
+  if (bh >= p.nbh) return;
+  bh += p.bh0;
+  if (role < 2) {
+    bwd_wide_walk<IMG>(p, smem, bh, role);
+  } else if (role == 2) {
+    if (threadIdx.x == 0) say_xcd(p.sync + (size_t)bh * BWD_SYNC_STRIDE + BWW_XCD + 2);
+    bwd_finish_dxk<IMG, true>(p, smem, bh);
+  } else if (PREFETCH && role == PER - 1) {
+    bwd_wide_prefetch(p, smem, bh);
+  } else {
+    bwd_body<1, IMG, true, true>(p, smem, bh, role - 3, p.K - 1, 0);
+  }
+}
+
+// Clears the synchronisation words and marks every word of the exchange empty.
+__global__ void ttt_mlp_bwd_wide_clear(int* w, int n, uint4* x, int nx) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) w[i] = 0;
+  if (i < nx) x[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+}
+
+}  // namespace ttt
+
+hipError_t ttt_mlp_bwd_wide_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
+  const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
+  int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
+  const int nx = p.nbh * (ttt::BWW_XCHG_WORDS / 2);
+  hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n,
+                     reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
+  const dim3 grid((p.nbh + 7) / 8 * 8 * (p.n_replay + 3 + p.n_prefetch)), block(ttt::BW_THREADS);
+  auto launch = [&](auto kernel) -> hipError_t {
+    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
+    return hipGetLastError();
+  };
+  if (p.n_prefetch) {
+    if (p.n_replay == 4) return launch(ttt::ttt_mlp_bwd_wide_kernel<4, true>);
+    return launch(ttt::ttt_mlp_bwd_wide_kernel<3, true>);
+  }
+  return launch(ttt::ttt_mlp_bwd_wide_kernel<2, false>);
+}

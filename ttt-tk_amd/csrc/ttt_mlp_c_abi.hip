@@ -249,8 +249,7 @@ int launch_fwd_segments(ttt::FwdParams p, const SegmentPlan& plan, int cus, hipS
   p.seg_len = plan.seg_len;
   return launch_segments(p, plan, cus, [stream](const ttt::FwdParams& q) { return ttt_mlp_fwd_enqueue(q, stream); });
 }
-// Backward: segment 0 = the last groups of every sequence.  The third parked norm-gradient sum needs a second
-// mini-batch slot in x_hat_ln_group, hence cgs >= 2 (plan_bwd_segments).
+// Backward: segment 0 = the last groups of every sequence.
 int launch_bwd_segments(ttt::BwdParams p, const SegmentPlan& plan, int cus, hipStream_t stream) {
   p.seg_groups = plan.groups;
   return launch_segments(p, plan, cus, [stream](const ttt::BwdParams& q) { return ttt_mlp_bwd_enqueue(q, stream); });
@@ -266,10 +265,11 @@ SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, in
 // 256-byte aligned.
 struct BwdWorkspace {
   static constexpr int PER_SET = 11;
-  static constexpr int PARTS = 8 + PER_SET * 3;
+  static constexpr int ALT_SETS = ttt::BWD_MAX_SETS - 1;
+  static constexpr int PARTS = 8 + PER_SET * ALT_SETS;
   size_t off[PARTS];
   size_t total;
-  BwdWorkspace(long long n, long long cgs, int alt_sets, bool finish) {
+  BwdWorkspace(long long n, long long cgs, int alt_sets, bool finish, bool wide) {
     const size_t slot = (size_t)n * (size_t)cgs;
     const size_t tile = TTT_MLP_CS * TTT_MLP_F * 2, img = TTT_MLP_CS * TTT_MLP_HID * 2, vec = TTT_MLP_CS * 4;
     const size_t norm = (size_t)n * 8 * 2 * TTT_MLP_F * sizeof(float);
@@ -280,17 +280,41 @@ struct BwdWorkspace {
     size_t o = 0;
     auto put = [&](int i, size_t bytes) { off[i] = o; o += (bytes + 255) & ~(size_t)255; };
     put(0, ttt::bwd_sync_ints(n) * sizeof(int));
-    put(1, 2 * norm);
+    put(1, ttt::BWD_MAX_SETS * norm);
     put(2, norm);
     put(3, (size_t)n * img);
     // hand-over to the grad_L_XK workgroup: one image (dZ1) and two fp32 tiles (g_y, norm-weight gradient terms) per slot, two sets
-    put(4, 0);
+    put(4, wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);   // walk on two workgroups: what they exchange
     put(5, 0);
     put(6, finish ? 2 * slot * img : 0);
     put(7, finish ? 2 * slot * 4 * tile : 0);
-    for (int s = 0; s < 3; s++)
+    for (int s = 0; s < ALT_SETS; s++)
       for (int t = 0; t < PER_SET; t++) put(8 + PER_SET * s + t, s < alt_sets ? per_set[t] : 0);
     total = o;
+  }
+};
+
+// Replaying workgroups per pair when the walk of each of the n pairs runs on two CUs of one XCD (with one more for grad_L_XK),
+// 0 if it does not: as for the forward, the workgroups of ceil(n / 8) pairs must fit an eighth of the CUs.  The walk takes
+// a mini-batch in a third of the time of a replay, so four replaying workgroups keep up with it, two are what bounds it.
+int bwd_wide_replays(long long n, int cus) {
+#ifdef TTT_STAGE_CLOCKS   // the stage clocks are those of the kernels with the walk on one workgroup
+  return 0;
+#endif
+  const long long per_xcd = (n + 7) / 8;
+  if (n <= 0) return 0;
+  return 8 * per_xcd <= cus / 8 ? 4 : 7 * per_xcd <= cus / 8 ? 3 : 5 * per_xcd <= cus / 8 ? 2 : 0;
+}
+// Shape of the backward's launch with several workgroups per pair.
+struct BwdShape {
+  int n_replay, n_sets;
+  bool finish, wide;
+  BwdShape(const LaunchPlan& pl, int cus) {
+    const int r = bwd_wide_replays(pl.n_rest, cus);
+    wide = r > 0;
+    n_replay = wide ? r : pl.per_pair >= 3 ? 2 : 1;
+    n_sets = wide ? r + 2 : 2 * n_replay;
+    finish = wide || pl.per_pair == 4;
   }
 };
 
@@ -356,8 +380,8 @@ extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_grou
   if (B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16)) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
   if (!pl.rest_split) return 0;
-  const int n_replay = pl.per_pair >= 3 ? 2 : 1;
-  return BwdWorkspace(pl.n_rest, checkpoint_group_size, 2 * n_replay - 1, pl.per_pair == 4).total;
+  const BwdShape sh(pl, device_cus());
+  return BwdWorkspace(pl.n_rest, checkpoint_group_size, sh.n_sets - 1, sh.finish, sh.wide).total;
 }
 
 extern "C" size_t ttt_mlp_bwd_status_offset(int B, int NH) {
@@ -372,9 +396,10 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const int n_replay = pl.per_pair >= 3 ? 2 : 1, alt_sets = 2 * n_replay - 1;
-  const bool finish = pl.per_pair == 4;
-  const BwdWorkspace w(pl.n_rest, p.cgs, alt_sets, finish);
+  const BwdShape sh(pl, device_cus());
+  const int alt_sets = sh.n_sets - 1;
+  const bool finish = sh.finish;
+  const BwdWorkspace w(pl.n_rest, p.cgs, alt_sets, finish, sh.wide);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   {
@@ -400,9 +425,10 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   const size_t norm = 8 * 2 * TTT_MLP_F;
   p.bh0 = static_cast<int>(pl.n_single);
   p.nbh = static_cast<int>(pl.n_rest);
-  p.n_replay = n_replay;
+  p.n_replay = sh.n_replay;
+  p.n_sets = sh.n_sets;
   p.n_finish = finish ? 1 : 0;
-  p.n_prefetch = pl.prefetch ? 1 : 0;
+  p.n_prefetch = (sh.wide ? sh.n_replay > 2 : pl.prefetch) ? 1 : 0;
   p.wait_limit = g_wait_limit;
   if (finish) {
     p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[6]) - b0 * 2 * img;
@@ -411,7 +437,7 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   int* words = reinterpret_cast<int*>(base + w.off[0]);
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
-  p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * 2 * norm;
+  p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * ttt::BWD_MAX_SETS * norm;
   p.norm_park = reinterpret_cast<float*>(base + w.off[2]) - b0 * norm;
   p.walk_park = reinterpret_cast<__bf16*>(base + w.off[3]) - b0 * (TTT_MLP_CS * TTT_MLP_HID);
   for (int s = 0; s < alt_sets; s++) {
@@ -427,6 +453,10 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
     p.alt_grad_output_fused_group[s] = reinterpret_cast<__bf16*>(base + o[8]) - b0 * tile;
     p.alt_std_fused_group[s] = reinterpret_cast<float*>(base + o[9]) - b0 * vec;
     p.alt_W1_init_group[s] = reinterpret_cast<float*>(base + o[10]) - b0 * img;   // [cgs][64][256] floats = 2 images per slot
+  }
+  if (sh.wide) {
+    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
+    return static_cast<int>(ttt_mlp_bwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
   }
   return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
 }

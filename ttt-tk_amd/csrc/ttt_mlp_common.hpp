@@ -494,6 +494,28 @@ TTT_DEV int wait_for_pace(int* word, int target, int* status, int* s_flag, uint6
   __syncthreads();
   return *s_flag;
 }
+// Two words: waits until both have reached `target`, orders what follows after them, and returns the smaller value seen (at
+// least `target`), or -1 if the wait gave up.
+TTT_DEV int wait_for_both(int* a, int* b, int target, int* status, int* s_flag, uint64_t limit) {
+  __syncthreads();   // the last value of the flag has been read by every wave
+  if (threadIdx.x == 0) {
+    int seen;
+    const uint64_t t0 = wall_clock64();
+    while ((seen = min(__hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                       __hip_atomic_load(b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < target) {
+      if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
+        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        seen = -1;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    *s_flag = seen;
+  }
+  __syncthreads();
+  return *s_flag;
+}
 // Everything this workgroup has written (or read) so far is ordered before the new value of `word`: every
 // wave drains its own outstanding memory operations (a workgroup-scope release alone does not wait for
 // stores that are still in flight), the barrier collects the waves, then one thread writes the L2 back at

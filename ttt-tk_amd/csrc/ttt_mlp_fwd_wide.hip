@@ -17,6 +17,7 @@
 // clocks per mini-batch; 1 pair of 32,768 tokens: 4.22 -> 2.70 ms).  Of the 13.1 k: block 0's products 2.2 k, block 1's 3.7 k
 // while block 0's sums cross (gather and send 1.1 k, 1.3 k under way, LayerNorm 0.8 k), then the same 3.4 k for block 1's
 // sums with block 0's weight step beside it, block 1's weight step and the split of the new state 3.3 k.
+#include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
 
 namespace ttt {
@@ -41,38 +42,6 @@ constexpr int WD_B2P = WD_BET + FD * 4;                  // [8 groups of 8 token
 constexpr int WD_FLAG = WD_B2P + 8 * FD * 4;             // [0] non-zero: a wait gave up; [1] helper waves that have left their shares of b2
 constexpr int WD_BYTES = WD_FLAG + 16;
 static_assert(WD_BYTES <= SM_FWD_BYTES, "the launch asks for SM_FWD_BYTES (the output branch's carve-up)");
-
-typedef __attribute__((address_space(1))) uint64_t* gword64_t;
-constexpr uint32_t WD_EMPTY = 0xffffffffu;
-// Two fp32 values as one 8-byte word of the exchange; the mark itself is never sent (a NaN stays a NaN).
-TTT_DEV uint64_t wd_pack(float a, float b) {
-  const uint32_t lo = min(__builtin_bit_cast(uint32_t, a), WD_EMPTY - 1), hi = min(__builtin_bit_cast(uint32_t, b), WD_EMPTY - 1);
-  return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-// A word for the other CU.  On one XCD the L2 is where both meet: a plain store reaches it and the partner's agent-scope
-// load is answered by it (2.9 k clocks for 16 KiB both ways; agent-scope stores 3.4-4.5 k).
-TTT_DEV void wd_put(gword64_t q, uint64_t x, bool near) {
-  if (near) __hip_atomic_store(q, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-  else __hip_atomic_store(q, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Waits until the four words of every lane have arrived.  False: gave up (status word raised).
-TTT_DEV bool wd_take(gword64_t q, uint64_t (&w)[4], int* status, uint64_t limit) {
-  uint64_t t0 = 0;
-  for (unsigned n = 0;; n++) {
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 4; k++) w[k] = __hip_atomic_load(q + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int k = 0; k < 4; k++) ok = ok && static_cast<uint32_t>(w[k]) != WD_EMPTY && static_cast<uint32_t>(w[k] >> 32) != WD_EMPTY;
-    if (__all(ok)) return true;
-    const uint64_t now = wall_clock64();
-    if (n == 0) t0 = now;
-    else if (now - t0 > limit || ((n & 63) == 0 && __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-      __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return false;
-    }
-  }
-}
 
 // Synchronisation words of a pair: 0 / 8 mini-batches handed over by the two halves, 16 / 20 mini-batches finished by the
 // output workgroups, 24 .. the XCD each workgroup of the pair runs on (+ 1).
@@ -100,11 +69,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   int* const w_status = p.status;
   const int n_wg = 2 + p.n_out;
-  if (tid == 0) {
-    unsigned xcc;
-    asm volatile("s_getreg_b32 %0, hwreg(20, 0, 4)" : "=s"(xcc));   // XCC_ID
-    __hip_atomic_store(words + WDW_XCD + half, static_cast<int>(xcc) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (tid == 0) say_xcd(words + WDW_XCD + half);
   if (tid < FD) {
     s_b2[tid] = p.b2[(size_t)bh * FD + tid];
     s_gam[tid] = p.ttt_norm_weight[head * FD + tid];
@@ -394,24 +359,9 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   load_xk(0);
   put_xk(0);
   __syncthreads();   // the flag is clear
-  bool near = true;
-  {
-    bool alive = true;
-    if (lane < n_wg) {
-      int x;
-      const uint64_t t0 = wall_clock64();
-      while ((x = __hip_atomic_load(words + WDW_XCD + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
-        if (__hip_atomic_load(w_status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > p.wait_limit) {
-          __hip_atomic_store(w_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          alive = false;
-          break;
-        }
-      }
-      near = x == __builtin_amdgcn_readfirstlane(x);
-    }
-    near = __all(near);
-    if (!__all(alive) && lane == 0) *s_flag = 1;
-  }
+  bool alive = true;
+  const bool near = on_one_xcd(words + WDW_XCD, n_wg, lane, w_status, p.wait_limit, alive);
+  if (!alive && lane == 0) *s_flag = 1;
   __syncthreads();
   if (flag() != 0) return;
   const gword64_t xch = (gword64_t)(p.xchg + (size_t)bh * FWD_XCHG_WORDS);
@@ -551,11 +501,7 @@ __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     return;
   }
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
-  if (threadIdx.x == 0) {
-    unsigned xcc;
-    asm volatile("s_getreg_b32 %0, hwreg(20, 0, 4)" : "=s"(xcc));
-    __hip_atomic_store(words + WDW_XCD + role, static_cast<int>(xcc) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (threadIdx.x == 0) say_xcd(words + WDW_XCD + role);
   fwd_output_branch<1, true>(p, smem, bh, role - 2);
 }
 

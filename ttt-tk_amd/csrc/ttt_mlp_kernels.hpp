@@ -43,6 +43,8 @@ constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 1024;  // 8-byte words of a pair's ex
 constexpr int FWD_IMG_BYTES = 64 * 256 * 2 * 2;  // W1 and W2 as bf16 operands
 constexpr int FWD_BIAS_FLOATS = 256 + 64;
 
+constexpr int BWD_MAX_SETS = 6;   // sets of per-group tensors in use at once, at most
+
 struct BwdParams {
   const __bf16 *XQ, *XK, *XV, *last_eta;
   const float *ttt_norm_weight, *ttt_norm_bias;
@@ -64,13 +66,13 @@ struct BwdParams {
   // checkpoint groups (taking turns), one walks them backwards.  Group number g (0 = the last group of the
   // sequence) is replayed into set g % (2 * n_replay) of the per-group tensors that carry it to the walk:
   // set 0 = the caller's tensors, sets 1.. = alt_*[set - 1] from the workspace.
-  __bf16 *alt_X2_group[3], *alt_Z1_group[3], *alt_Z1_bar_group[3], *alt_X2_bar_group[3];
-  __bf16 *alt_grad_l_wrt_Z2_group[3], *alt_grad_l_wrt_Z1_group[3];
-  __bf16 *alt_x_hat_fused_group[3], *alt_grad_x_hat_fused_group[3], *alt_grad_output_fused_group[3];
-  float* alt_std_fused_group[3];
-  float* alt_W1_init_group[3];
-  float* norm_partial;   // [B*NH][2][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients, by group parity
-  float* norm_park;      // [B*NH][8 waves][2][64]: n_replay = 1: the share of the parity that is not being added to
+  __bf16 *alt_X2_group[BWD_MAX_SETS - 1], *alt_Z1_group[BWD_MAX_SETS - 1], *alt_Z1_bar_group[BWD_MAX_SETS - 1], *alt_X2_bar_group[BWD_MAX_SETS - 1];
+  __bf16 *alt_grad_l_wrt_Z2_group[BWD_MAX_SETS - 1], *alt_grad_l_wrt_Z1_group[BWD_MAX_SETS - 1];
+  __bf16 *alt_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_output_fused_group[BWD_MAX_SETS - 1];
+  float* alt_std_fused_group[BWD_MAX_SETS - 1];
+  float* alt_W1_init_group[BWD_MAX_SETS - 1];
+  float* norm_partial;   // [B*NH][BWD_MAX_SETS][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set
+  float* norm_park;      // [B*NH][8 waves][2][64]: their sum over the groups walked so far (without a grad_L_XK workgroup)
   __bf16* walk_park;     // [B*NH][64][256]: one register image the walking workgroup parks across its LayerNorm stage
   int n_replay;
   // n_finish = 1: a further workgroup forms grad_L_XK, grad_L_XV and the walk's share of the norm gradients from
@@ -84,6 +86,10 @@ struct BwdParams {
   // line that the walk is about to ask for, one mini-batch ahead of it, so that the walk's own requests are
   // answered by the L2 the two share instead of by HBM.
   int n_prefetch;
+  // Walk on two workgroups (ttt_mlp_bwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
+  // 256 8-byte words]; n_replay = 2 .. 4 and n_sets sets of the per-group tensors; n_finish = 1, n_prefetch = 0.
+  unsigned long long* xchg;
+  int n_sets;
   int* sync;
   int* status;    // the status word behind the synchronisation words
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
@@ -106,6 +112,12 @@ struct BwdParams {
 // no data is ordered by it), word 24 the groups the grad_L_XK workgroup has finished - then one status
 // word (non-zero: a wait gave up).
 constexpr int BWD_SYNC_STRIDE = 32;
+// With the walk on two workgroups: words 0 .. 3 groups replayed by each replaying workgroup, BWW_WALKED + 0 / 4 groups and
+// BWW_GIVEN + 0 / 4 mini-batches done by the two halves of the walk, 24 as above, BWW_XCD .. the XCDs of the two halves
+// and the grad_L_XK workgroup.
+constexpr int BWW_WORDS = 5;                                // per lane: 8 fp32 sums and the token's share of d eta
+constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 80 KiB
+constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26;
 inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }
 
 // ---- optional stage clocks.  A library built with -DTTT_STAGE_CLOCKS (stage_clocks.py builds one beside the product
@@ -176,6 +188,8 @@ hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream)
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
 // p.sync == nullptr: one workgroup per (batch, head); otherwise two (replay / reverse walk).
 hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream);
+// The walk of every pair on two workgroups, p.n_replay replaying ones and one for grad_L_XK.
+hipError_t ttt_mlp_bwd_wide_enqueue(const ttt::BwdParams& p, hipStream_t stream);
 // Replays checkpoint group 0 and writes the sixteen per-group tensors row-major (side path, one workgroup per pair).
 hipError_t ttt_mlp_export_group0_enqueue(const ttt::BwdParams& p, hipStream_t stream);
 extern "C" int ttt_mlp_fwd_lds_bytes();

@@ -184,19 +184,17 @@ TTT_DEV void ln_load_f32(float (&x)[8], const float* p) {
 #pragma unroll
   for (int e = 0; e < 4; e++) { x[e] = a[e]; x[4 + e] = b[e]; }
 }
-// Sum of the four pair sums of this lane's token / features, (P0 + P1) + (P2 + P3): the order in which two CUs that hold two
-// pairs each form it.  `row` points at this token's row of the first pair's region; the regions of successive pairs are
-// 2 regions apart.
+// Sum of the four pair sums of this lane's token / features.  `row` points at this token's row of the
+// first pair's region; the regions of successive pairs are 2 regions apart.
 TTT_DEV void ln_gather(float (&z)[8], const float* row) {
+  f32x4 a = *reinterpret_cast<const f32x4*>(row), b = *reinterpret_cast<const f32x4*>(row + 4);
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
-    f32x4 a[4];
-#pragma unroll
-    for (int pp = 0; pp < 4; pp++) a[pp] = *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN + 4 * q);
-    const f32x4 t = (a[0] + a[1]) + (a[2] + a[3]);
-#pragma unroll
-    for (int e = 0; e < 4; e++) z[4 * q + e] = t[e];
+  for (int pp = 1; pp < 4; pp++) {
+    a += *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN);
+    b += *reinterpret_cast<const f32x4*>(row + pp * 2 * RGN + 4);
   }
+#pragma unroll
+  for (int e = 0; e < 4; e++) { z[e] = a[e]; z[4 + e] = b[e]; }
 }
 TTT_DEV float sum8(const float (&x)[8]) {
   float s = 0.f;
@@ -223,45 +221,11 @@ TTT_DEV float ln_normalize(float (&z)[8], float* std_out) {
   *std_out = v * rstd;  // sqrt(v)
   return rstd;
 }
-// Second-order pass through the fused LayerNorm loss for the 8 features of this lane's token.  gg: the sum over the hidden
-// dimension of what the weight step backwards gives (gradient wrt dl/dZ2 before the bias term and -eta); gb: gradient
-// wrt b2; xh, go, gz: x_hat, grad_output and dl/dZ2 of the loss.  Out: gy (gradient wrt y), dg (norm-weight gradient
-// terms), dz = dZ2; returns sum_F gz * gb, the bias part of d eta.
-TTT_DEV float walk_layernorm(float (&gg)[8], const float (&gb)[8], float neg_eta, const float (&xh)[8], const float (&go)[8],
-                             const float (&gz)[8], const float (&gam)[8], float sdf, float (&gy)[8], float (&dg)[8], float (&dz)[8]) {
-#pragma clang fp contract(off)   // which product of a sum of two is fused is written out: every launch shape gives the same bits
-#pragma unroll
-  for (int e = 0; e < 8; e++) gg[e] = (gg[e] + gb[e]) * neg_eta;   // grad wrt dl/dZ2
-  const float rsd = 1.f / sdf;
-  const float eta_bias = oct_sum(dot8(gz, gb));
-  const float s0 = oct_sum(sum8(gg)), a = oct_sum(dot8(gg, xh));
-  float bb = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; e++) bb = __builtin_fmaf(go[e] * gam[e], xh[e], bb);
-  bb = oct_sum(bb);
-  const float inv = rsd * (1.f / FD);
-  float sg = 0.f, sx = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const float ggx = __builtin_fmaf(-__builtin_fmaf(xh[e], a, s0), 1.f / FD, gg[e]) * rsd;
-    gy[e] = gam[e] * ggx;
-    dg[e] = __builtin_fmaf(go[e], ggx, gy[e] * xh[e]);
-    dz[e] = __builtin_fmaf(-__builtin_fmaf(go[e] * gam[e], a, gg[e] * bb), inv, gy[e] * gam[e]);
-    sg = __builtin_fmaf(-__builtin_fmaf(dz[e], xh[e], gg[e] * gz[e]), rsd, sg);
-    sx += dz[e];
-  }
-  sg = oct_sum(sg);
-  sx = oct_sum(sx);
-#pragma unroll
-  for (int e = 0; e < 8; e++) dz[e] = __builtin_fmaf(__builtin_fmaf(sg, xh[e], -sx * rsd), 1.f / FD, dz[e] * rsd);
-  return eta_bias;
-}
 // acc[f0 + e] += sum over this wave's tokens of x[e]   (wave-private LDS vector).  The 8 tokens sit in the lanes
 // that share lane % 8: lanes 8 apart inside a row of 16 (one rotation), then the four rows, two values per swap
 // (row_pair_sum2, half_sum2): in the end row r of one register holds the total of x[r], of the other that of
 // x[4 + r], and lanes 0..7 of every row add their two totals to the vector.
 TTT_DEV void ln_token_sum_add(float* s_acc, const float (&x)[8], int lane, int f0) {
-#pragma clang fp contract(off)   // not with the products that formed x: every launch shape gives the same bits
   float y[8];
 #pragma unroll
   for (int e = 0; e < 8; e++)
@@ -581,20 +545,32 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   // does not depend on who replays them.  The running sum sits in HBM (slot 0 of the park, 4 KiB): with one workgroup per
   // (batch, head) in the caller's x_hat_ln_group, where the walk's sum waits behind it (slot 1) while the LDS accumulators
   // serve a replay, otherwise in the workspace, added to by the walk (by the grad_L_XK workgroup where there is one).
-  const gptr_t gPark = ROLE == 0 ? gbuf(p.x_hat_ln_group + (size_t)bh * cgs * (CS * FD))
-                                 : gbuf(p.norm_park + (size_t)bh * (BW_NWAVE * 2 * FD));
+  // (Its address is formed where it is used: kept over the loop it costs the walk two registers it does not have.)
+  auto park = [&]() {
+    size_t o = uni64(ROLE == 0 ? (size_t)bh * cgs * (CS * FD) : (size_t)bh * (BW_NWAVE * 2 * FD));
+    asm volatile("" : "+s"(o));
+    return ROLE == 0 ? gbuf(p.x_hat_ln_group + o) : gbuf(p.norm_park + o);
+  };
+  auto group_sums = [&](int set) {   // of this wave
+    size_t o = uni64(((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD);
+    asm volatile("" : "+s"(o));
+    return gbuf(p.norm_partial + o);
+  };
   constexpr unsigned PARK_BYTES = BW_NWAVE * 2 * FD * 4;
   if (ROLE == 0 ? seg_first : (ROLE == 2 && !FIN)) {   // the running sum starts at zero
-    g_stf(gPark, np_off, 0, 0.f);
-    g_stf(gPark, np_off, FD * 4, 0.f);
+    g_stf(park(), np_off, 0, 0.f);
+    g_stf(park(), np_off, FD * 4, 0.f);
   }
   if (ROLE == 0 && !seg_first) {   // the walk's sum as the segment before this one left it
-    s_dgw[lane] = g_ldf(gPark, np_off, PARK_BYTES);
-    s_dbw[lane] = g_ldf(gPark, np_off, PARK_BYTES + FD * 4);
+    s_dgw[lane] = g_ldf(park(), np_off, PARK_BYTES);
+    s_dbw[lane] = g_ldf(park(), np_off, PARK_BYTES + FD * 4);
   }
   auto add_to_running_sum = [&](float a0, float a1) {
-    g_stf(gPark, np_off, 0, g_ldf(gPark, np_off, 0) + a0);
-    g_stf(gPark, np_off, FD * 4, g_ldf(gPark, np_off, FD * 4) + a1);
+    LANE_VARS;
+    const gptr_t g = park();
+    const unsigned o = (v * 2 * FD + lane) * 4;
+    g_stf(g, o, 0, g_ldf(g, o, 0) + a0);
+    g_stf(g, o, FD * 4, g_ldf(g, o, FD * 4) + a1);
   };
 
   TTT_STAGES_BEGIN();
@@ -624,8 +600,8 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         acc_store_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_store_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
         WAVE_SYNC();
-        g_stf(gPark, np_off, PARK_BYTES, s_dgw[lane]);   // the walk's sum out
-        g_stf(gPark, np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
+        g_stf(park(), np_off, PARK_BYTES, s_dgw[lane]);   // the walk's sum out
+        g_stf(park(), np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
         s_dgw[lane] = 0.f;
         s_dbw[lane] = 0.f;
       }
@@ -1070,9 +1046,10 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       }
       if constexpr (ROLE == 1) {
         WAVE_SYNC();   // this group's norm-gradient sums go with it
-        float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
-        np[lane] = s_dgw[lane];
-        np[FD + lane] = s_dbw[lane];
+        LANE_VARS;
+        const gptr_t g = group_sums(set);
+        g_stf(g, 4 * lane, 0, s_dgw[lane]);
+        g_stf(g, 4 * lane, FD * 4, s_dbw[lane]);
       }
       // running gradients back into registers
       if constexpr (ROLE == 0) {
@@ -1080,8 +1057,8 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         acc_load_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
         WAVE_SYNC();
         add_to_running_sum(s_dgw[lane], s_dbw[lane]);
-        s_dgw[lane] = g_ldf(gPark, np_off, PARK_BYTES);
-        s_dbw[lane] = g_ldf(gPark, np_off, PARK_BYTES + FD * 4);
+        s_dgw[lane] = g_ldf(park(), np_off, PARK_BYTES);
+        s_dbw[lane] = g_ldf(park(), np_off, PARK_BYTES + FD * 4);
         WAVE_SYNC();
       }
       if constexpr (ROLE == 1) publish(w_replayed, done / n_replay + 1);
@@ -1097,8 +1074,9 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       if constexpr (FIN) {   // the hand-over set of this group's parity is free once the group before last is finished
         if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return;
       } else {
-        const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
-        add_to_running_sum(np[lane], np[FD + lane]);
+        LANE_VARS;
+        const gptr_t g = group_sums(set);
+        add_to_running_sum(g_ldf(g, 4 * lane, 0), g_ldf(g, 4 * lane, FD * 4));
       }
     }
     // hand-over buffers of this group for the grad_L_XK workgroup (set = parity of the group)
@@ -1319,22 +1297,47 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         ln_cvt8(go, gof);
         ln_load(gz, s_gz2 + tok * LDX + f0);
         ln_load_f32(gam, s_gam + f0);
-        float gx[8], dg[8];
-        float tot = walk_layernorm(gg, gb, -s_eta[tok], xh, go, gz, gam, sdf, gy, dg, gx);
+        const float neg_eta = -s_eta[tok];
+#pragma unroll
+        for (int e = 0; e < 8; e++) gg[e] = (gg[e] + gb[e]) * neg_eta;   // grad wrt dl/dZ2
+        const float rsd = 1.f / sdf;
         // dEta: -(sum_F gZ2*(X2 gW2 + gb2) + sum_H gZ1*(XK gW1 + gb1))
         {
           LANE_VARS;
-          float d[BW_NWAVE];
+          float d[BW_NWAVE / 2];
 #pragma unroll
-          for (int u = 0; u < BW_NWAVE; u++) d[u] = s_deta[u * CS + tok];
-          tot += ((d[0] + d[4]) + (d[1] + d[5])) + ((d[2] + d[6]) + (d[3] + d[7]));
+          for (int u = 0; u < BW_NWAVE / 2; u++) d[u] = s_deta[u * CS + tok] + s_deta[(u + BW_NWAVE / 2) * CS + tok];
+          const float tot = oct_sum(dot8(gz, gb)) + ((d[0] + d[1]) + (d[2] + d[3]));
           if ((lane & 7) == 0) g_sth(bDETA, 2 * tok, mb * (CS * 2), (bf16)((float)deta_old - tot));
         }
+        // (the expressions are walk_layernorm's, ttt_mlp_bwd_wide.hip, which writes out what the compiler fuses here)
+        const float s0 = oct_sum(sum8(gg)), a = oct_sum(dot8(gg, xh));
+        float bb = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) bb = __builtin_fmaf(go[e] * gam[e], xh[e], bb);
+        bb = oct_sum(bb);
+        float gx[8], dg[8];
+        const float inv = rsd * (1.f / FD);
+        float sg = 0.f, sx = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float ggx = (gg[e] - (s0 + xh[e] * a) * (1.f / FD)) * rsd;
+          gy[e] = gam[e] * ggx;
+          dg[e] = go[e] * ggx + gy[e] * xh[e];
+          gx[e] = gy[e] * gam[e] - (go[e] * gam[e] * a + gg[e] * bb) * inv;
+          sg += (-gx[e] * xh[e] - gg[e] * gz[e]) * rsd;
+          sx += gx[e];
+        }
+        sg = oct_sum(sg);
+        sx = oct_sum(sx);
         if constexpr (!FIN) {   // with a grad_L_XK workgroup these token sums and grad_L_XV are formed there, from g_y and dg
           ln_token_sum_add(s_dgw, dg, lane, f0);
           ln_token_sum_add(s_dbw, gy, lane, f0);
+        }
 #pragma unroll
-          for (int e = 0; e < 8; e++) dxv_old[e] = (bf16)((float)dxv_old[e] - gy[e]);   // dXV accumulates -g_y
+        for (int e = 0; e < 8; e++) {
+          gx[e] = gx[e] * rsd + (sg * xh[e] - sx * rsd) * (1.f / FD);   // dZ2
+          if constexpr (!FIN) dxv_old[e] = (bf16)((float)dxv_old[e] - gy[e]);   // dXV accumulates -g_y
         }
         // g_y is needed again for dXK: park it (the XQ / E2 tiles are dead by now), or hand it over
         {
@@ -1496,8 +1499,8 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   // norm-weight / norm-bias gradients: sum the per-wave LDS accumulators
   if constexpr (FIN) return;   // with a grad_L_XK workgroup the walk holds no share of these sums: they are written there
   if (ROLE == 0 && !seg_last) {   // the next segment goes on with the walk's sum (the replay's is in place already)
-    g_stf(gPark, np_off, PARK_BYTES, s_dgw[lane]);
-    g_stf(gPark, np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
+    g_stf(park(), np_off, PARK_BYTES, s_dgw[lane]);
+    g_stf(park(), np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
     return;
   }
   if (tid < 2 * FD) {

@@ -36,6 +36,47 @@ constexpr int BWW_FLAG = BWW_ETA + 2 * CS * 4;            // [0] a wait gave up,
 constexpr int BWW_BYTES = BWW_FLAG + 16;
 static_assert(BWW_BYTES <= SM_BWD_BYTES, "the launch asks for SM_BWD_BYTES (the replay's carve-up)");
 
+// Second-order pass through the fused LayerNorm loss for the 8 features of this lane's token.  gg: the sum over the hidden
+// dimension of what the weight step backwards gives (gradient wrt dl/dZ2 before the bias term and -eta); gb: gradient
+// wrt b2; xh, go, gz: x_hat, grad_output and dl/dZ2 of the loss.  Out: gy (gradient wrt y), dg (norm-weight gradient
+// terms), dz = dZ2; returns sum_F gz * gb, the bias part of d eta.
+TTT_DEV float walk_layernorm(float (&gg)[8], const float (&gb)[8], float neg_eta, const float (&xh)[8], const float (&go)[8],
+                             const float (&gz)[8], const float (&gam)[8], float sdf, float (&gy)[8], float (&dg)[8], float (&dz)[8]) {
+#pragma clang fp contract(off)   // which product of a sum of two is fused is written out: every launch shape gives the same bits
+  float gs[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) gs[e] = gg[e] + gb[e];
+#pragma unroll
+  for (int e = 0; e < 8; e++) gg[e] = gs[e] * neg_eta;             // grad wrt dl/dZ2
+  const float rsd = 1.f / sdf;
+  const float eta_bias = oct_sum(dot8(gz, gb));
+  float s0 = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) s0 = __builtin_fmaf(gs[e], neg_eta, s0);
+  s0 = oct_sum(s0);
+  const float a = oct_sum(dot8(gg, xh));
+  float bb = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) bb = __builtin_fmaf(go[e] * gam[e], xh[e], bb);
+  bb = oct_sum(bb);
+  const float inv = rsd * (1.f / FD);
+  float sg = 0.f, sx = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const float ggx = __builtin_fmaf(-__builtin_fmaf(xh[e], a, s0), 1.f / FD, gg[e]) * rsd;
+    gy[e] = gam[e] * ggx;
+    dg[e] = __builtin_fmaf(go[e], ggx, gy[e] * xh[e]);
+    dz[e] = __builtin_fmaf(gy[e], gam[e], -(__builtin_fmaf(go[e] * gam[e], a, gg[e] * bb) * inv));
+    sg = __builtin_fmaf(-__builtin_fmaf(dz[e], xh[e], gg[e] * gz[e]), rsd, sg);
+    sx += dz[e];
+  }
+  sg = oct_sum(sg);
+  sx = oct_sum(sx);
+#pragma unroll
+  for (int e = 0; e < 8; e++) dz[e] = __builtin_fmaf(dz[e], rsd, __builtin_fmaf(sg, xh[e], -(sx * rsd)) * (1.f / FD));
+  return eta_bias;
+}
+
 template <bool IMG>
 TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh, const int half) {
   typedef __attribute__((address_space(3))) int* lint_t;
@@ -539,38 +580,58 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
         __hip_atomic_store(words + BWW_GIVEN + 4 * half, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (j == n_mb - 1) __hip_atomic_store(words + BWW_WALKED + 4 * half, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      float mine[8], d_mine, gy[8], dg[8], tot;
+      // the order of the one-workgroup kernel, ((P0 + P1) + P2) + P3 over the wave pairs: half 0 sends P0 + P1, half 1 P2 and P3
+      float m0[8], m1[8], d_mine, gy[8], dg[8], tot;
       auto gather_send = [&](int blk) {   // this CU's sums over its 128 hidden columns; sent to the other CU
 #pragma unroll
         for (int q = 0; q < 2; q++) {
           f32x4 a[4];
 #pragma unroll
           for (int i = 0; i < 4; i++) a[i] = *reinterpret_cast<const f32x4*>(s_row + i * (BWW_PTILE / 4) + 4 * q);
-          const f32x4 t = (a[0] + a[2]) + (a[1] + a[3]);
+          const f32x4 pa = a[0] + a[2], pb = a[1] + a[3];
 #pragma unroll
-          for (int e = 0; e < 4; e++) mine[4 * q + e] = t[e];
+          for (int e = 0; e < 4; e++) { m0[4 * q + e] = pa[e]; m1[4 * q + e] = pb[e]; }
         }
         const float* const d = s_deta + 32 * blk + t_in;
         d_mine = (d[0] + d[2 * CS]) + (d[CS] + d[3 * CS]);
         const gword64_t dst = xch + ((((n & 1) * 2 + half) * 2 + blk) * 4 + u) * (64 * BWW_WORDS) + lane;
+        if (half == 0) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) wd_put(dst + 64 * i, wd_pack(mine[2 * i], mine[2 * i + 1]), near);
-        wd_put(dst + 256, wd_pack(d_mine, 0.f), near);
+          for (int e = 0; e < 8; e++) m0[e] += m1[e];
+        } else {   // (d eta is half 0's to write)
+          wd_put(dst + 256, wd_pack(d_mine, 0.f), near);
+#pragma unroll
+          for (int i = 0; i < 4; i++) wd_put(dst + 64 * (5 + i), wd_pack(m1[2 * i], m1[2 * i + 1]), near);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) wd_put(dst + 64 * i, wd_pack(m0[2 * i], m0[2 * i + 1]), near);
       };
       auto finish_block = [&](int blk) {
         const int tok = 32 * blk + t_in;
         const gword64_t src = xch + ((((n & 1) * 2 + 1 - half) * 2 + blk) * 4 + u) * (64 * BWW_WORDS) + lane;
-        uint64_t wv[BWW_WORDS];
-        if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+        float gg[8], gb[8], xh[8], go[8], gz[8], dz[8], d_sum = 0.f;
+        if (half == 0) {
+          uint64_t wv[9];
+          if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
 #pragma unroll
-        for (int i = 0; i < BWW_WORDS; i++) wd_put(src + 64 * i, ~0ull, near);
-        float gg[8], gb[8], xh[8], go[8], gz[8], dz[8];
+          for (int i = 0; i < 9; i++) wd_put(src + 64 * i, ~0ull, near);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          gg[2 * i] = mine[2 * i] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[i]));
-          gg[2 * i + 1] = mine[2 * i + 1] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[i] >> 32));
+          for (int i = 0; i < 4; i++) {
+            gg[2 * i] = (m0[2 * i] + wd_lo(wv[i])) + wd_lo(wv[5 + i]);
+            gg[2 * i + 1] = (m0[2 * i + 1] + wd_hi(wv[i])) + wd_hi(wv[5 + i]);
+          }
+          d_sum = d_mine + wd_lo(wv[4]);
+        } else {
+          uint64_t wv[4];
+          if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+#pragma unroll
+          for (int i = 0; i < 4; i++) wd_put(src + 64 * i, ~0ull, near);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            gg[2 * i] = (wd_lo(wv[i]) + m0[2 * i]) + m1[2 * i];
+            gg[2 * i + 1] = (wd_hi(wv[i]) + m0[2 * i + 1]) + m1[2 * i + 1];
+          }
         }
-        const float d_sum = d_mine + __builtin_bit_cast(float, static_cast<uint32_t>(wv[4]));
         ln_load_f32(gb, s_gb2 + f0);
         ln_cvt8(xh, cur.xh[blk]);
         ln_cvt8(go, cur.go[blk]);

@@ -50,9 +50,7 @@ TTT_DEV bf16x8 pack8(const f32x16& x, int t) {
 // Two values at a time: one packed conversion for the high-order terms, a shift and a mask to read them back as
 // fp32, two subtractions, one packed conversion for the low-order terms (6 instructions per pair).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-// (No contraction of the subtraction with a product that formed a or b: the kernels that share a computation agree to the bit.)
 TTT_DEV void split2(float a, float b, bf16x2& hi, bf16x2& lo) {
-#pragma clang fp contract(off)
   const f32x2 ab = {a, b};
   hi = __builtin_convertvector(ab, bf16x2);
   const uint32_t hp = __builtin_bit_cast(uint32_t, hi);
@@ -76,6 +74,31 @@ TTT_DEV void split8(const float (&x)[8], bf16x8& hi, bf16x8& lo) {
     hi[j] = h2[0]; hi[j + 1] = h2[1];
     lo[j] = l2[0]; lo[j + 1] = l2[1];
   }
+}
+
+// The compiler may fuse the subtraction of a split with the product that formed the value, or the additions of a sum with
+// the products it adds.  Where two kernels have to agree to the bit on such a value, one of these says which it is.
+TTT_DEV void split8_plain(const f32x16& x, int t, bf16x8& hi, bf16x8& lo) {   // not fused
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const f32x2 ab = {x[8 * t + j], x[8 * t + j + 1]};
+    const bf16x2 h2 = __builtin_convertvector(ab, bf16x2);
+    const uint32_t hp = __builtin_bit_cast(uint32_t, h2);
+    const f32x2 r = {ab[0] - __builtin_bit_cast(float, hp << 16), ab[1] - __builtin_bit_cast(float, hp & 0xffff0000u)};
+    const bf16x2 l2 = __builtin_convertvector(r, bf16x2);
+    hi[j] = h2[0]; hi[j + 1] = h2[1];
+    lo[j] = l2[0]; lo[j + 1] = l2[1];
+  }
+}
+// Two products a * b, fused with the subtraction of the split.
+TTT_DEV void split2_product(float a0, float b0, float a1, float b1, bf16x2& hi, bf16x2& lo) {
+  const f32x2 ab = {a0 * b0, a1 * b1};
+  hi = __builtin_convertvector(ab, bf16x2);
+  const uint32_t hp = __builtin_bit_cast(uint32_t, hi);
+  const f32x2 r = {__builtin_fmaf(a0, b0, -__builtin_bit_cast(float, hp << 16)),
+                   __builtin_fmaf(a1, b1, -__builtin_bit_cast(float, hp & 0xffff0000u))};
+  lo = __builtin_convertvector(r, bf16x2);
 }
 
 TTT_DEV bf16x8 cat(bf16x4 lo, bf16x4 hi) { return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7); }
@@ -139,12 +162,7 @@ TTT_DEV float half_sum2(float s01, float s23) {
 // features f0 = 8 (l % 8) ... of it.  The tokens sit in the lanes that share lane % 8: lanes 8 apart inside a row of
 // 16 (one rotation), then the four rows, two values per swap: in the end row r of one register holds the total of
 // x[r], of the other that of x[4 + r], and lanes 0..7 of every row store their two totals.  Fixed order, fp32.
-TTT_DEV void ln_token_sum_store(float* vec, const float (&x)[8], int lane, int f0) {
-#pragma clang fp contract(off)   // not with the product that formed x: see split2
-  float y[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++)
-    y[e] = x[e] + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x[e]), 0x128, 0xF, 0xF, false));  // row_ror:8
+TTT_DEV void ln_token_sum_tail(float* vec, const float (&y)[8], int lane, int f0) {
   const float lo = half_sum2(row_pair_sum2(y[0], y[1]), row_pair_sum2(y[2], y[3]));
   const float hi = half_sum2(row_pair_sum2(y[4], y[5]), row_pair_sum2(y[6], y[7]));
   if ((lane & 8) == 0) {
@@ -152,6 +170,21 @@ TTT_DEV void ln_token_sum_store(float* vec, const float (&x)[8], int lane, int f
     d[0] = lo;
     d[4] = hi;
   }
+}
+TTT_DEV void ln_token_sum_store(float* vec, const float (&x)[8], int lane, int f0) {
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    y[e] = x[e] + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x[e]), 0x128, 0xF, 0xF, false));  // row_ror:8
+  ln_token_sum_tail(vec, y, lane, f0);
+}
+// The same for x[e] = t[e] * scale, the first addition fused with the product.
+TTT_DEV void ln_token_sum_store_product(float* vec, const float (&t)[8], float scale, int lane, int f0) {
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    y[e] = __builtin_fmaf(t[e], scale, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, t[e] * scale), 0x128, 0xF, 0xF, false)));
+  ln_token_sum_tail(vec, y, lane, f0);
 }
 
 // ---------------------------------------------------------------------------- shape-generic tiles

@@ -13,6 +13,8 @@ TTT_DEV uint64_t wd_pack(float a, float b) {
   const uint32_t lo = min(__builtin_bit_cast(uint32_t, a), WD_EMPTY - 1), hi = min(__builtin_bit_cast(uint32_t, b), WD_EMPTY - 1);
   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
+TTT_DEV float wd_lo(uint64_t x) { return __builtin_bit_cast(float, static_cast<uint32_t>(x)); }
+TTT_DEV float wd_hi(uint64_t x) { return __builtin_bit_cast(float, static_cast<uint32_t>(x >> 32)); }
 // A word for the other CU.  On one XCD the L2 is where both meet: a plain store reaches it and the partner's agent-scope
 // load is answered by it (2.9 k clocks for 16 KiB both ways; agent-scope stores 3.4-4.5 k).
 TTT_DEV void wd_put(gword64_t q, uint64_t x, bool near) {

@@ -219,19 +219,20 @@ TTT_DEV void fwd_body(const FwdParams& p, unsigned char* smem, const int bh, con
       }
       float z[8], gx[8];
       {
-        // ((P0 + P1) + (P2 + P3)) + b2: the order in which two CUs that hold two pairs each form it (ttt_mlp_fwd_wide.hip)
-        const float* row = s_P + tok * LDP + f0;
+        f32x4 a0 = *reinterpret_cast<const f32x4*>(s_b2 + f0);
+        f32x4 a1 = *reinterpret_cast<const f32x4*>(s_b2 + f0 + 4);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-          f32x4 a[4];
-#pragma unroll
-          for (int t = 0; t < 4; t++) a[t] = *reinterpret_cast<const f32x4*>(row + t * 64 * LDP + 4 * q);
-          const f32x4 s = ((a[0] + a[1]) + (a[2] + a[3])) + *reinterpret_cast<const f32x4*>(s_b2 + f0 + 4 * q);
-#pragma unroll
-          for (int e = 0; e < 4; e++) z[4 * q + e] = s[e];
+        for (int t = 0; t < 4; t++) {
+          a0 += *reinterpret_cast<const f32x4*>(s_P + t * 64 * LDP + tok * LDP + f0);
+          a1 += *reinterpret_cast<const f32x4*>(s_P + t * 64 * LDP + tok * LDP + f0 + 4);
         }
+#pragma unroll
+        for (int e = 0; e < 4; e++) { z[e] = a0[e]; z[4 + e] = a1[e]; }
       }
-      ln_loss_gradient(z, lds_get8h(s_xk + xrow(tok) + f0), lds_get8h(s_xv + xrow(tok) + f0), bf2f(s_eta[tok]), s_gam + f0, s_bet + f0, gx);
+      const float scale = ln_loss_gradient(z, lds_get8h(s_xk + xrow(tok) + f0), lds_get8h(s_xv + xrow(tok) + f0), bf2f(s_eta[tok]),
+                                           s_gam + f0, s_bet + f0, gx);
+#pragma unroll
+      for (int e = 0; e < 8; e++) gx[e] *= scale;
       ln_token_sum_store(reinterpret_cast<float*>(smem + SM_B2P) + v * FD, gx, lane, f0);   // b2's step, this wave's share
       bf16x8 o, ol;
       split8(gx, o, ol);

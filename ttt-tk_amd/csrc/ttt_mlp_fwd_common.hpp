@@ -186,8 +186,8 @@ TTT_DEV void output_layernorm(const float* s_P, const float* s_b2, const float* 
 }
 
 // LayerNorm-fused gradient of the reconstruction loss for the 8 features of this lane's token (8 lanes per token):
-// z = Z2 in, gx = G2 = -eta * dl/dZ2 out.
-TTT_DEV void ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, const float eta, const float* s_gam, const float* s_bet,
+// z = Z2 in; gx times the returned scale is G2 = -eta * dl/dZ2.
+TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, const float eta, const float* s_gam, const float* s_bet,
                               float (&gx)[8]) {
   float sum = 0.f;
 #pragma unroll
@@ -219,7 +219,8 @@ TTT_DEV void ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, c
   s2 = oct_sum(s2);
   const float scale = -eta * rstd * (1.f / FD);
 #pragma unroll
-  for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * scale;
+  for (int e = 0; e < 8; e++) gx[e] = FD * gx[e] - s1 - z[e] * s2;
+  return scale;
 }
 
 // Everything derived from the lane index is cheap to recompute and expensive to keep in a register

@@ -7,8 +7,8 @@
 //   waves 4-7                 the sums over the hidden dimension, their exchange with the other CU and the LayerNorm lanes
 // A mini-batch is taken in two blocks of 32 tokens, so that block 0's sums travel to the other CU and through the
 // LayerNorm while the compute waves form block 1, and block 1's while they apply block 0's share of the weight step.
-// What crosses the CUs is one fp32 tile per mini-batch and direction (16 KiB; both CUs form the LayerNorm of all
-// tokens, from the same sums in the same order).  No flags: a word is sent as it is and its slot holds an impossible
+// What crosses the CUs is one or two fp32 tiles per mini-batch and direction (16 / 32 KiB; both CUs form the LayerNorm of
+// all tokens, from the same sums in the same order).  No flags: a word is sent as it is and its slot holds an impossible
 // value (a NaN that is never sent) before and after; the receiver polls the data itself and puts the mark back.
 // One or two more workgroups per pair compute Out from the states left in a ring, as in the two-workgroup launch.
 // Every sum has the order of the one-workgroup kernel: results are the same to the bit.
@@ -181,7 +181,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
 #pragma unroll
         for (int t = 0; t < 2; t++) {
           bf16x8 xh;
-          split8(x2, t, xh, x2lo.v[0][2 * rb + t]);
+          split8_plain(x2, t, xh, x2lo.v[0][2 * rb + t]);
           store_piece_rows<FLD>(s_x2t, 0, 2 * rb + t, c, h, xh);
         }
         TTT_WAVE_SYNC();
@@ -283,28 +283,21 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
           __builtin_amdgcn_sched_barrier(0);
         }
         step_g2(1);
-#pragma unroll
-        for (int t = 0; t < 2; t++) {   // W2[shard, :] += X2^T G2
-          const bf16x8 xl = x2lo.v[0][2 * rb + t];
-#pragma unroll
-          for (int fb = 0; fb < 2; fb++) {
-            W2s.b[0][fb] = MFMA(xl, gh[t][fb], W2s.b[0][fb]);
-            W2s.b[0][fb] = MFMA(xh[t], gl[t][fb], W2s.b[0][fb]);
-            W2s.b[0][fb] = MFMA(xh[t], gh[t][fb], W2s.b[0][fb]);
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          g1[i] *= d1[rb][i];
-          colsum += g1[i];
-        }
         bf16x8 g1h[2], g1l[2];
 #pragma unroll
-        for (int t = 0; t < 2; t++) split8(g1, t, g1h[t], g1l[t]);
-#pragma unroll
-        for (int k = 0; k < 12; k++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one matrix product,
-          __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);   // seven vector instructions
+        for (int k = 0; k < 12; k++) {   // W2[shard, :] += X2^T G2; with each of the first eight products two values of G1
+          const int t = k / 6, fb = (k / 3) % 2, o = k % 3;
+          W2s.b[0][fb] = MFMA(o == 0 ? x2lo.v[0][2 * rb + t] : xh[t], o == 1 ? gl[t][fb] : gh[t][fb], W2s.b[0][fb]);
+          __builtin_amdgcn_sched_barrier(0);
+          if (k < 8) {
+            bf16x2 h2, l2;
+            split2_product(g1[2 * k], d1[rb][2 * k], g1[2 * k + 1], d1[rb][2 * k + 1], h2, l2);
+            colsum = __builtin_fmaf(g1[2 * k + 1], d1[rb][2 * k + 1], __builtin_fmaf(g1[2 * k], d1[rb][2 * k], colsum));
+            const int j = (2 * k) % 8;
+            g1h[k / 4][j] = h2[0]; g1h[k / 4][j + 1] = h2[1];
+            g1l[k / 4][j] = l2[0]; g1l[k / 4][j + 1] = l2[1];
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
 #pragma unroll
         for (int t = 0; t < 2; t++)     // W1[:, shard] += XK^T G1
@@ -370,48 +363,70 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   float b2v[8], b2L = s_b2[lane];                     // b2 of this lane's features, and of feature `lane` (wave 4 stores that one)
 #pragma unroll
   for (int e = 0; e < 8; e++) b2v[e] = s_b2[f0 + e];
-  float gx[8];                                        // G2 of the last block: its token sums are formed while the next block's sums travel
+  float gx[8], scale = 0.f;                           // G2 of the last block (gx * scale): its token sums are formed while the next block's sums travel
   __builtin_amdgcn_s_setprio(2);                      // these waves' few instructions are what the other four wait for
   int seen0 = 0, seen1 = 0;                           // mini-batches the output workgroups are known to have finished
   bool gave_up = false;
 
-  auto gather_send = [&](int mb, int blk, float (&z)[8]) {   // this CU's sum over its 128 hidden columns; sent to the other CU
+  // The sum has the order of the one-workgroup kernel, (((b2 + P0) + P1) + P2) + P3 over the wave pairs: half 0 holds P0 and P1 and
+  // sends b2 + P0 + P1, half 1 sends P2 and P3.
+  float m0[8], m1[8];
+  auto gather_send = [&](int mb, int blk) {
 #pragma unroll
     for (int q = 0; q < 2; q++) {
       f32x4 a[4];
 #pragma unroll
       for (int k = 0; k < 4; k++)
         a[k] = *reinterpret_cast<const f32x4*>((blk == 0 ? s_row0 + k * (WD_PTILE / 4) : s_row1 + k * (WD_P1TILE / 4)) + 4 * q);
-      const f32x4 s = (a[0] + a[2]) + (a[1] + a[3]);
+      const f32x4 pa = a[0] + a[2], pb = a[1] + a[3];
 #pragma unroll
-      for (int e = 0; e < 4; e++) z[4 * q + e] = s[e];
+      for (int e = 0; e < 4; e++) { m0[4 * q + e] = pa[e]; m1[4 * q + e] = pb[e]; }
     }
-    const gword64_t dst = xch + ((((mb & 1) * 2 + half) * 2 + blk) * 4 + u) * 256 + lane;
+    const gword64_t dst = xch + ((((mb & 1) * 2 + half) * 2 + blk) * 4 + u) * 512 + lane;
+    if (half == 0) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) wd_put(dst + 64 * k, wd_pack(z[2 * k], z[2 * k + 1]), near);
+      for (int e = 0; e < 8; e++) m0[e] = (b2v[e] + m0[e]) + m1[e];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) wd_put(dst + 256 + 64 * k, wd_pack(m1[2 * k], m1[2 * k + 1]), near);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) wd_put(dst + 64 * k, wd_pack(m0[2 * k], m0[2 * k + 1]), near);
   };
-  auto finish_block = [&](int mb, int blk, const float (&mine)[8], bf16x8 xk, bf16x8 xv, bf16 eta) {
+  auto finish_block = [&](int mb, int blk, bf16x8 xk, bf16x8 xv, bf16 eta) {
     const int tok = 32 * blk + t_in;
-    const gword64_t src = xch + ((((mb & 1) * 2 + 1 - half) * 2 + blk) * 4 + u) * 256 + lane;
-    uint64_t wv[4];
-    if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
-#pragma unroll
-    for (int k = 0; k < 4; k++) wd_put(src + 64 * k, ~0ull, near);
+    const gword64_t src = xch + ((((mb & 1) * 2 + 1 - half) * 2 + blk) * 4 + u) * 512 + lane;
     float z[8];
+    if (half == 0) {
+      uint64_t wv[8];
+      if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      z[2 * k] = mine[2 * k] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[k]));
-      z[2 * k + 1] = mine[2 * k + 1] + __builtin_bit_cast(float, static_cast<uint32_t>(wv[k] >> 32));
+      for (int k = 0; k < 8; k++) wd_put(src + 64 * k, ~0ull, near);
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        z[2 * k] = (m0[2 * k] + wd_lo(wv[k])) + wd_lo(wv[4 + k]);
+        z[2 * k + 1] = (m0[2 * k + 1] + wd_hi(wv[k])) + wd_hi(wv[4 + k]);
+      }
+    } else {
+      uint64_t wv[4];
+      if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+#pragma unroll
+      for (int k = 0; k < 4; k++) wd_put(src + 64 * k, ~0ull, near);
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        z[2 * k] = (wd_lo(wv[k]) + m0[2 * k]) + m1[2 * k];
+        z[2 * k + 1] = (wd_hi(wv[k]) + m0[2 * k + 1]) + m1[2 * k + 1];
+      }
     }
+    scale = ln_loss_gradient(z, xk, xv, bf2f(eta), s_gam + f0, s_bet + f0, gx);
+    f32x16 g2;
 #pragma unroll
-    for (int e = 0; e < 8; e++) z[e] += b2v[e];
-    ln_loss_gradient(z, xk, xv, bf2f(eta), s_gam + f0, s_bet + f0, gx);
+    for (int e = 0; e < 8; e++) { g2[e] = gx[e] * scale; g2[8 + e] = 0.f; }
     bf16x8 o, ol;
-    split8(gx, o, ol);
+    split8_plain(g2, 0, o, ol);
     lds_put16(s_g2 + tok * FLD + f0, __builtin_bit_cast(u32x4, o));
     lds_put16(s_g2l + tok * FLD + f0, __builtin_bit_cast(u32x4, ol));
   };
-
   // b2 after mini-batch m: + the sum over the tokens of G2, eight shares in a fixed order.  Every lane keeps its own features.
   auto step_b2 = [&](int m) {
 #pragma unroll
@@ -444,10 +459,9 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     }
     load_xk(mb + 1 < p.NC ? mb + 1 : mb);
     __syncthreads();   // B1
-    float mine[8];
-    gather_send(mb, 0, mine);
+    gather_send(mb, 0);
     put_xk(mb + 1);   // the buffer was last read a mini-batch ago
-    finish_block(mb, 0, mine, xk[0], xv[0], eta[0]);
+    finish_block(mb, 0, xk[0], xv[0], eta[0]);
     if (u == 3 && mb >= FWD_WIDE_RING) {
       // the slot this mini-batch's state goes to is free once the output branch is done with mini-batch mb - RING
       const int old = mb - FWD_WIDE_RING, o = old % p.n_out, need = old / p.n_out + 1;
@@ -467,15 +481,15 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       }
     }
     __syncthreads();   // B2
-    gather_send(mb, 1, mine);
-    ln_token_sum_store(s_b2p + u * FD, gx, lane, f0);
-    finish_block(mb, 1, mine, xk[1], xv[1], eta[1]);
+    gather_send(mb, 1);
+    ln_token_sum_store_product(s_b2p + u * FD, gx, scale, lane, f0);
+    finish_block(mb, 1, xk[1], xv[1], eta[1]);
     if (gave_up && lane == 0) *s_flag = 1;
     __syncthreads();   // B3
     if (flag() != 0) return;
     if (u == 0 && lane == 0 && mb > 0) give(mb);   // the stores of the last mini-batch's state were acknowledged before B3
     // b2's step, while the compute waves are busy: the four helper waves wait for each other's shares (all of them come here)
-    ln_token_sum_store(s_b2p + (4 + u) * FD, gx, lane, f0);
+    ln_token_sum_store_product(s_b2p + (4 + u) * FD, gx, scale, lane, f0);
     if (lane == 0) __hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     while (__hip_atomic_load(s_flag + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < 4 * (mb + 1)) __builtin_amdgcn_s_sleep(1);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");

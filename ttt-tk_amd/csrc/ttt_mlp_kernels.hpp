@@ -24,7 +24,7 @@ struct FwdParams {
   int* sync;
   int* status;    // the status word behind the synchronisation words
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
-  // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2048 fp32],
+  // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2 x 2048 fp32],
   // and the output workgroups per pair (1 or 2); the ring then has FWD_WIDE_RING slots.
   unsigned long long* xchg;
   int n_out;
@@ -39,7 +39,7 @@ struct FwdParams {
 };
 constexpr int FWD_RING_MAX = 32;               // most mini-batches per hand-over (8 or 32 are compiled)
 constexpr int FWD_WIDE_RING = 8;               // ring slots with the recurrence on two workgroups
-constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 1024;  // 8-byte words of a pair's exchange: 64 KiB
+constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 2048;  // 8-byte words of a pair's exchange: 128 KiB
 constexpr int FWD_IMG_BYTES = 64 * 256 * 2 * 2;  // W1 and W2 as bf16 operands
 constexpr int FWD_BIAS_FLOATS = 256 + 64;
 
@@ -115,8 +115,8 @@ constexpr int BWD_SYNC_STRIDE = 32;
 // With the walk on two workgroups: words 0 .. 3 groups replayed by each replaying workgroup, BWW_WALKED + 0 / 4 groups and
 // BWW_GIVEN + 0 / 4 mini-batches done by the two halves of the walk, 24 as above, BWW_XCD .. the XCDs of the two halves
 // and the grad_L_XK workgroup.
-constexpr int BWW_WORDS = 5;                                // per lane: 8 fp32 sums and the token's share of d eta
-constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 80 KiB
+constexpr int BWW_WORDS = 9;                                // per lane: two times 8 fp32 sums and the token's share of d eta
+constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 144 KiB
 constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26;
 inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }
 

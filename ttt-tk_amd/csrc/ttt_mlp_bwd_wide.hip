@@ -482,10 +482,13 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   const unsigned voff = (t_in * FD + f0) * 2;
   constexpr unsigned HALF_TILE = TILE_BYTES / 2;                        // 32 tokens
   int* const w_status = p.status;
+  // A wave that gives up keeps that to itself until the stage whose closing barrier precedes the reads of s_flag[0] (B3, or the
+  // barrier that opens the walk): all eight waves then read the same value and leave together, or none does.  Raised at the
+  // top of a mini-batch it could be seen by one wave and missed by another, which then waited for the first without a limit.
   bool gave_up = false;
   __syncthreads();   // flags
   auto wait_for = [&](int* word, int target) {
-    if (lane == 0 && !wait_word(word, target, w_status, p.wait_limit)) s_flag[0] = 1;
+    if (!__all(lane != 0 || wait_word(word, target, w_status, p.wait_limit))) gave_up = true;
   };
   // group number `done` (from the end) has been replayed
   auto wait_group = [&](int done) { wait_for(words + done % n_replay, done / n_replay + 1); };
@@ -535,17 +538,18 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   const bool near = [&]() {
     bool alive = true;
     const bool one = on_one_xcd(words + BWW_XCD, 3, lane, w_status, p.wait_limit, alive);
-    if (!alive && lane == 0) s_flag[0] = 1;
+    if (!alive) gave_up = true;
     return one;
   }();
   wait_group(0);   // (every helper wave itself)
   {
     const int j0 = min(cgs, p.NC - (p.K - 1) * cgs) - 1;
-    if (flag(0) == 0) {
+    if (!gave_up) {
       ask(p.K - 1, j0);
       put(0);
     }
   }
+  if (gave_up && lane == 0) s_flag[0] = 1;
   __syncthreads();
   if (flag(0) != 0) return;
   const gword64_t xch = (gword64_t)(p.xchg + (size_t)bh * BWW_XCHG_WORDS);
@@ -571,7 +575,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       const int kn = j > 0 ? k : k - 1, jn = j > 0 ? j - 1 : cgs - 1;
       // gradient wrt b2: what the output branch adds
       if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_gzb, u, s, lane); }, ones, c, h);
-      if (more && flag(0) == 0) ask(kn, jn);
+      if (more && !gave_up) ask(kn, jn);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // g_y of the last mini-batch and the marks put back are in place
       __syncthreads();   // B1
       if (u == 0 && lane == 0 && n > 0) {

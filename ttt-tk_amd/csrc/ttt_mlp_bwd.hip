@@ -451,7 +451,6 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   float* s_dgw = s_red + (v * 2 + 0) * FD;
   float* s_dbw = s_red + (v * 2 + 1) * FD;
   if (lane < FD) { s_dgw[lane] = 0.f; s_dbw[lane] = 0.f; }
-  const unsigned np_off = (v * 2 * FD + lane) * 4;   // this lane's two words of the wave's accumulators: +0, +FD*4
   float* s_gy = reinterpret_cast<float*>(smem + SB_XQ) + tok * FD + f0;   // this lane's part of the g_y park
   bf16x8 ones;
 #pragma unroll
@@ -551,6 +550,11 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     asm volatile("" : "+s"(o));
     return ROLE == 0 ? gbuf(p.x_hat_ln_group + o) : gbuf(p.norm_park + o);
   };
+  // (also formed where it is used) this lane's two words of the wave's accumulators: +0, +FD*4
+  auto np_off = [&]() {
+    LANE_VARS;
+    return (v * 2 * FD + lane) * 4u;
+  };
   auto group_sums = [&](int set) {   // of this wave
     size_t o = uni64(((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD);
     asm volatile("" : "+s"(o));
@@ -558,20 +562,14 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   };
   constexpr unsigned PARK_BYTES = BW_NWAVE * 2 * FD * 4;
   if (ROLE == 0 ? seg_first : (ROLE == 2 && !FIN)) {   // the running sum starts at zero
-    g_stf(park(), np_off, 0, 0.f);
-    g_stf(park(), np_off, FD * 4, 0.f);
+    const gptr_t g = park();
+    g_stf(g, (v * 2 * FD + lane) * 4, 0, 0.f);
+    g_stf(g, (v * 2 * FD + lane) * 4, FD * 4, 0.f);
   }
   if (ROLE == 0 && !seg_first) {   // the walk's sum as the segment before this one left it
-    s_dgw[lane] = g_ldf(park(), np_off, PARK_BYTES);
-    s_dbw[lane] = g_ldf(park(), np_off, PARK_BYTES + FD * 4);
+    s_dgw[lane] = g_ldf(park(), np_off(), PARK_BYTES);
+    s_dbw[lane] = g_ldf(park(), np_off(), PARK_BYTES + FD * 4);
   }
-  auto add_to_running_sum = [&](float a0, float a1) {
-    LANE_VARS;
-    const gptr_t g = park();
-    const unsigned o = (v * 2 * FD + lane) * 4;
-    g_stf(g, o, 0, g_ldf(g, o, 0) + a0);
-    g_stf(g, o, FD * 4, g_ldf(g, o, FD * 4) + a1);
-  };
 
   TTT_STAGES_BEGIN();
   for (int k = k_hi; k >= k_lo; k--) {
@@ -600,8 +598,10 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         acc_store_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_store_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
         WAVE_SYNC();
-        g_stf(park(), np_off, PARK_BYTES, s_dgw[lane]);   // the walk's sum out
-        g_stf(park(), np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
+        const gptr_t g = park();
+        const unsigned o = np_off();
+        g_stf(g, o, PARK_BYTES, s_dgw[lane]);   // the walk's sum out
+        g_stf(g, o, PARK_BYTES + FD * 4, s_dbw[lane]);
         s_dgw[lane] = 0.f;
         s_dbw[lane] = 0.f;
       }
@@ -1053,12 +1053,20 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       }
       // running gradients back into registers
       if constexpr (ROLE == 0) {
+        LANE_VARS;
+        // one round trip to HBM for the four words and the gradients (200 pairs x 100 mini-batches, 7 groups: 5.42 ms forward +
+        // backward with a word at a time and their address kept over the loops, 5.36 so)
+        const gptr_t g = park();
+        const unsigned o = np_off();
+        const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4), w0 = g_ldf(g, o, PARK_BYTES), w1 = g_ldf(g, o, PARK_BYTES + FD * 4);
         acc_load_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_load_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
         WAVE_SYNC();
-        add_to_running_sum(s_dgw[lane], s_dbw[lane]);
-        s_dgw[lane] = g_ldf(park(), np_off, PARK_BYTES);
-        s_dbw[lane] = g_ldf(park(), np_off, PARK_BYTES + FD * 4);
+        const float a0 = r0 + s_dgw[lane], a1 = r1 + s_dbw[lane];   // the running sum
+        s_dgw[lane] = w0;
+        s_dbw[lane] = w1;
+        g_stf(g, o, 0, a0);
+        g_stf(g, o, FD * 4, a1);
         WAVE_SYNC();
       }
       if constexpr (ROLE == 1) publish(w_replayed, done / n_replay + 1);
@@ -1075,8 +1083,13 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return;
       } else {
         LANE_VARS;
-        const gptr_t g = group_sums(set);
-        add_to_running_sum(g_ldf(g, 4 * lane, 0), g_ldf(g, 4 * lane, FD * 4));
+        const gptr_t gs = group_sums(set);   // the running sum
+        const float a0 = g_ldf(gs, 4 * lane, 0), a1 = g_ldf(gs, 4 * lane, FD * 4);
+        const gptr_t g = park();
+        const unsigned o = (v * 2 * FD + lane) * 4;
+        const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);
+        g_stf(g, o, 0, r0 + a0);
+        g_stf(g, o, FD * 4, r1 + a1);
       }
     }
     // hand-over buffers of this group for the grad_L_XK workgroup (set = parity of the group)
@@ -1499,8 +1512,8 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   // norm-weight / norm-bias gradients: sum the per-wave LDS accumulators
   if constexpr (FIN) return;   // with a grad_L_XK workgroup the walk holds no share of these sums: they are written there
   if (ROLE == 0 && !seg_last) {   // the next segment goes on with the walk's sum (the replay's is in place already)
-    g_stf(park(), np_off, PARK_BYTES, s_dgw[lane]);
-    g_stf(park(), np_off, PARK_BYTES + FD * 4, s_dbw[lane]);
+    g_stf(park(), np_off(), PARK_BYTES, s_dgw[lane]);
+    g_stf(park(), np_off(), PARK_BYTES + FD * 4, s_dbw[lane]);
     return;
   }
   if (tid < 2 * FD) {

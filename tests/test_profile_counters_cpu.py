@@ -61,6 +61,25 @@ def test_stage_names_come_from_the_kernels_header_and_fit_the_slots():
         assert f"TTT_STAGE({n})" in bsrc, n
 
 
+def test_the_launches_on_two_cus_have_stage_clocks_too():
+    """The kernels that run up to 80 (forward) and 48 pairs (backward) carry stages of their own for both kinds of waves, and
+    the instrumented library launches them as the product does."""
+    import re
+    import stage_clocks as sc
+    csrc = os.path.join(PKG, "csrc")
+    header = open(os.path.join(csrc, "ttt_mlp_kernels.hpp")).read()
+    for enum, source in (("FwdWideStage", "ttt_mlp_fwd_wide.hip"), ("BwdWideStage", "ttt_mlp_bwd_wide.hip")):
+        names = sc.stage_names(header, enum)
+        text = open(os.path.join(csrc, source)).read()
+        marked = set(re.findall(r"\b[FB]W[CH]_\w+", " ".join(re.findall(r"TTT_STAGE\((.*)\);", text))))
+        assert marked == {n for n, _ in names} and all(desc for _, desc in names) and len(names) <= sc.SLOTS
+        assert text.count("TTT_STAGES_BEGIN();") == text.count("TTT_STAGES_END(") == 2, "one table for each kind of waves"
+    role = dict(re.findall(r"STAGE_ROLE_(\w+) = (\d)", header))
+    assert {k: int(v) for k, v in role.items()} == {"OUT": sc.OUT, "HALF": sc.HALF, "WALK": sc.WALK, "DXK": sc.DXK, "WALK_HALF": sc.WALK_HALF}
+    plans = open(os.path.join(csrc, "ttt_mlp_c_abi.hip")).read()
+    assert plans.count("#ifndef TTT_STAGE_CLOCKS") == 1 and "return 0;\n#endif" not in plans
+
+
 def test_the_product_library_contains_no_stage_clocks():
     import ctypes
     lib = ctypes.CDLL(os.path.join(PKG, "libttt_mlp.so"))

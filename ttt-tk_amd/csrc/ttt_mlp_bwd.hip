@@ -1500,7 +1500,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #undef bFGY
 #undef WALK_FETCH
   }
-  TTT_STAGES_END(p.stage_clocks == nullptr ? nullptr : p.stage_clocks + ((size_t)bh * 4 + (ROLE == 1 ? turn : 2)) * (BW_NWAVE * STAGE_SLOTS));
+  TTT_STAGES_END(bh, ROLE == 1 ? turn : STAGE_ROLE_WALK);
   if constexpr (ROLE == 1) return;
 
   // ---- outputs that are written once
@@ -1704,6 +1704,7 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
           n_seen = wait_for_both(w_sync + BWW_GIVEN, w_sync + BWW_GIVEN + 4, n_step, p.status, s_flag, p.wait_limit);
           if (n_seen < 0) return;
         }
+        TTT_STAGE(BS_X_GROUP);
       } else if (k == 0 && (j == n_mb - 1 || (j & (FIN_CHUNK - 1)) == FIN_CHUNK - 1)) {
         if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return;
         TTT_STAGE(BS_X_GROUP);
@@ -1812,7 +1813,7 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
     publish(w_finished, done + 1);
     TTT_STAGE(BS_PUBLISH);
   }
-  TTT_STAGES_END(p.stage_clocks == nullptr ? nullptr : p.stage_clocks + ((size_t)bh * 4 + 3) * (BW_NWAVE * STAGE_SLOTS));
+  TTT_STAGES_END(bh, STAGE_ROLE_DXK);
   // norm-weight / norm-bias gradients: the replay's sum + the walk's, in the order of the other launch shapes
   __syncthreads();
   s_P[v * 2 * FD + lane] = nr0;

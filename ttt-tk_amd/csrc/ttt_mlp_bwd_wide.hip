@@ -208,6 +208,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       WAVE_SYNC();
     };
     int n = 0;   // mini-batches walked
+    TTT_STAGES_BEGIN();
     group_images(0);
     ask_bar(min(cgs, p.NC - (p.K - 1) * cgs) - 1);
     ask_step(p.K - 1, min(cgs, p.NC - (p.K - 1) * cgs) - 1);
@@ -245,6 +246,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
           add_gb1(t);
         }
         ask_gelu(1, j);
+        TTT_STAGE(BWC_BAR_TERMS);
         // ---- the weight step, backwards (state BEFORE this mini-batch), one token block at a time
         bf16x8 t2p[2][2], uhp[2][2], d1p[2][2];   // d1p: gelu'(Z1)
         float eta_i[2];
@@ -351,7 +353,9 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
         step_back(0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // dZ1 of the last mini-batch is out (and everything asked for is here)
         __builtin_amdgcn_sched_barrier(0);
+        TTT_STAGE(BWC_STEP0);
         __syncthreads();                                    // B1: block 0's sums
+        TTT_STAGE(BWC_B1);
         __builtin_amdgcn_sched_barrier(0);
         step_back(1);
         // ---- inner MLP backwards and the updates of the running gradients, token block i
@@ -407,7 +411,9 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
           }
         };
         __builtin_amdgcn_sched_barrier(0);
+        TTT_STAGE(BWC_STEP1);
         __syncthreads();                                    // B2: block 1's sums; dZ2 of block 0
+        TTT_STAGE(BWC_B2);
         __builtin_amdgcn_sched_barrier(0);
         if (j == 0) group_images((done + 1) % n_sets);
         const int kn = j > 0 || k == 0 ? k : k - 1, jn = j > 0 ? j - 1 : cgs - 1;   // (behind the last mini-batch: dropped)
@@ -458,17 +464,22 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
             for (int e = 0; e < 16; e++) dx2[i][e] = q[i][e] * -eta_i[i];
           WAVE_SYNC();
         }
+        TTT_STAGE(BWC_PRODUCTS);
         mlp_back(0);
         __builtin_amdgcn_sched_barrier(0);
+        TTT_STAGE(BWC_MLP0);
         __syncthreads();                                    // B3: dZ2 of block 1; the next mini-batch's tiles
+        TTT_STAGE(BWC_B3);
         __builtin_amdgcn_sched_barrier(0);
         const int gave_up = flag(0);
         mlp_back(1);
         ask_step(kn, jn);
         add_gb1(gb1_t);
+        TTT_STAGE(BWC_MLP1);
         if (gave_up != 0) return;
       }
     }
+    TTT_STAGES_END(bh, STAGE_ROLE_WALK_HALF + half);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();   // the last dZ1 is out
     acc_store_rows(gW1s, gbuf(p.grad_L_W1_init + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
@@ -560,6 +571,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   __builtin_amdgcn_s_setprio(2);
 
   int n = 0;
+  TTT_STAGES_BEGIN();
   for (int k = p.K - 1; k >= 0; k--) {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k;
@@ -577,7 +589,9 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_gzb, u, s, lane); }, ones, c, h);
       if (more && !gave_up) ask(kn, jn);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // g_y of the last mini-batch and the marks put back are in place
+      TTT_STAGE(BWH_ASK);
       __syncthreads();   // B1
+      TTT_STAGE(BWH_B1);
       if (u == 0 && lane == 0 && n > 0) {
         // all waves' stores of the last mini-batch were acknowledged before the barrier, all its reads are done
         if (!near) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -617,6 +631,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
         if (half == 0) {
           uint64_t wv[9];
           if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+          TTT_STAGE(blk == 0 ? BWH_TAKE0 : BWH_TAKE1);
 #pragma unroll
           for (int i = 0; i < 9; i++) wd_put(src + 64 * i, ~0ull, near);
 #pragma unroll
@@ -628,6 +643,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
         } else {
           uint64_t wv[4];
           if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+          TTT_STAGE(blk == 0 ? BWH_TAKE0 : BWH_TAKE1);
 #pragma unroll
           for (int i = 0; i < 4; i++) wd_put(src + 64 * i, ~0ull, near);
 #pragma unroll
@@ -661,19 +677,27 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       if (lane == 0) __hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       // the group's hand-over set to the grad_L_XK workgroup is free (written from here on)
       if (j == n_mb - 1 && done >= 2) wait_for(words + 24, done - 1);
+      TTT_STAGE(BWH_SEND0);
       finish_block(0);
+      TTT_STAGE(BWH_LN0);
       __syncthreads();   // B2
+      TTT_STAGE(BWH_B2);
       gather_send(1);
       store_block(0);
       if (more) put(n + 1);   // XQ and gZ2_bar are read before B1 only, XK and gZ2 alternate
+      TTT_STAGE(BWH_SEND1);
       finish_block(1);
       if (gave_up && lane == 0) s_flag[0] = 1;
+      TTT_STAGE(BWH_LN1);
       __syncthreads();   // B3
+      TTT_STAGE(BWH_B3);
       if (flag(0) != 0) return;
       store_block(1);
       if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_dz2, u, s, lane); }, ones, c, h);
+      TTT_STAGE(BWH_STORE1);
     }
   }
+  TTT_STAGES_END(bh, STAGE_ROLE_WALK_HALF + half);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (u == 0 && lane == 0) {

@@ -298,9 +298,6 @@ struct BwdWorkspace {
 // 0 if it does not: as for the forward, the workgroups of ceil(n / 8) pairs must fit an eighth of the CUs.  The walk takes
 // a mini-batch in a third of the time of a replay, so four replaying workgroups keep up with it, two are what bounds it.
 int bwd_wide_replays(long long n, int cus) {
-#ifdef TTT_STAGE_CLOCKS   // the stage clocks are those of the kernels with the walk on one workgroup
-  return 0;
-#endif
   const long long per_xcd = (n + 7) / 8;
   if (n <= 0) return 0;
   return 8 * per_xcd <= cus / 8 ? 4 : 7 * per_xcd <= cus / 8 ? 3 : 5 * per_xcd <= cus / 8 ? 2 : 0;
@@ -339,9 +336,6 @@ struct FwdWorkspace {
 // XCD, 0 if it does not: the workgroups of a pair share an XCD and wait for each other, so those of ceil(n / 8) pairs
 // must fit its CUs (an eighth of the device's).  One output workgroup keeps up with the recurrence only just; two where they fit.
 int fwd_wide_outputs(long long n, int cus) {
-#ifdef TTT_STAGE_CLOCKS   // the stage clocks are those of the one- and two-workgroup kernels
-  return 0;
-#endif
   const long long per_xcd = (n + 7) / 8;
   return n <= 0 ? 0 : 4 * per_xcd <= cus / 8 ? 2 : 3 * per_xcd <= cus / 8 ? 1 : 0;
 }

@@ -399,16 +399,16 @@ TTT_DEV float bf2f(bf16 x) { return (float)x; }
 #ifdef TTT_STAGE_CLOCKS
 #define TTT_STAGES_BEGIN() unsigned stage_acc[STAGE_SLOTS] = {}; unsigned stage_last = (unsigned)clock64()
 #define TTT_STAGE(i) do { const unsigned t_ = (unsigned)clock64(); stage_acc[i] += t_ - stage_last; stage_last = t_; } while (0)
-// `buf` = this workgroup's [8 waves][STAGE_SLOTS] part of the buffer
-#define TTT_STAGES_END(buf)                                                                                \
+#define TTT_STAGES_END(bh, role)                                                                           \
   do {                                                                                                     \
-    if ((buf) != nullptr && (threadIdx.x & 63) == 0)                                                       \
-      for (int i_ = 0; i_ < STAGE_SLOTS; i_++) (buf)[(threadIdx.x >> 6) * STAGE_SLOTS + i_] = stage_acc[i_]; \
+    if (p.stage_clocks != nullptr && (threadIdx.x & 63) == 0)                                              \
+      for (int i_ = 0; i_ < STAGE_SLOTS; i_++)                                                             \
+        p.stage_clocks[(((size_t)(bh) * STAGE_ROLES + (role)) * 8 + (threadIdx.x >> 6)) * STAGE_SLOTS + i_] = stage_acc[i_]; \
   } while (0)
 #else
 #define TTT_STAGES_BEGIN() ((void)0)
 #define TTT_STAGE(i) ((void)0)
-#define TTT_STAGES_END(buf) ((void)0)
+#define TTT_STAGES_END(bh, role) ((void)0)
 #endif
 
 // ---------------------------------------------------------------------------- tanh-GELU family

@@ -429,7 +429,7 @@ TTT_DEV void fwd_body(const FwdParams& p, unsigned char* smem, const int bh, con
   // a segment that is not the sequence's last leaves the checkpoint the next one starts from (b2 in LDS: every wave is
   // past the barrier that closes the last mini-batch)
   if (mb1 < p.NC) store_checkpoint(mb1 / p.cgs);
-  TTT_STAGES_END(p.stage_clocks == nullptr ? nullptr : p.stage_clocks + ((size_t)bh * 2 + 0) * (FW_NWAVE * STAGE_SLOTS));
+  TTT_STAGES_END(bh, 0);
 }
 
 __global__ __launch_bounds__(FW_THREADS) void ttt_mlp_fwd_kernel(const FwdParams p) {

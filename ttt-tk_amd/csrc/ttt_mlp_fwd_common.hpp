@@ -332,7 +332,7 @@ TTT_DEV void fwd_output_branch(const FwdParams& p, unsigned char* smem, const in
     } else if (at == ring - 1 || mb == p.NC - 1) publish(w_taken, grp + 1);
     TTT_STAGE(FS_PUBLISH);
   }
-  TTT_STAGES_END(p.stage_clocks == nullptr ? nullptr : p.stage_clocks + ((size_t)bh * 2 + 1) * (FW_NWAVE * STAGE_SLOTS));
+  TTT_STAGES_END(bh, STAGE_ROLE_OUT + turn);
 }
 
 }  // namespace ttt

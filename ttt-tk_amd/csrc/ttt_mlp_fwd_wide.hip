@@ -128,6 +128,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     bf16x8 xk[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) xk[s] = xpiece_rows(reinterpret_cast<const bf16*>(smem + WD_XK), 0, s, c, h);
+    TTT_STAGES_BEGIN();
     for (int mb = 0; mb < p.NC; mb++) {
       const bf16* const s_xk = reinterpret_cast<const bf16*>(smem + WD_XK + (mb & 1) * SM_TILE);
       if (mb % p.cgs == 0) {   // checkpoint: the state before this mini-batch
@@ -213,7 +214,9 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       load_xk(mb, 1);
       z2_block(0, s_P0);
       __builtin_amdgcn_sched_barrier(0);
+      TTT_STAGE(FWC_BLOCK0);
       __syncthreads();                                    // B1: block 0's partial sums
+      TTT_STAGE(FWC_B1);
       __builtin_amdgcn_sched_barrier(0);
       z1_block(1, true);
       bf16x8 wh[4], wl[4];   // W2[shard, :] with F contracted: its terms as rows [F][hid], read back transposed
@@ -308,13 +311,17 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
           }
       };
       __builtin_amdgcn_sched_barrier(0);
+      TTT_STAGE(FWC_BLOCK1);
       __syncthreads();                                    // B2: block 1's partial sums; G2 of block 0
+      TTT_STAGE(FWC_B2);
       __builtin_amdgcn_sched_barrier(0);
       update_block(0);
       step_operands(1);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last mini-batch's images, issued a block ago, are out
       __builtin_amdgcn_sched_barrier(0);
+      TTT_STAGE(FWC_STEP0);
       __syncthreads();                                    // B3: G2 of block 1
+      TTT_STAGE(FWC_B3);
       __builtin_amdgcn_sched_barrier(0);
       const int gave_up = flag();
       update_block(1);
@@ -322,8 +329,10 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       load_xk(mb + 1, 0);   // (put there before B2)
       cvt_chain_split(W2s, w2h, w2l);
       cvt_chain_split(W1s, w1h, w1l);
+      TTT_STAGE(FWC_STEP1);
       if (gave_up != 0) return;
     }
+    TTT_STAGES_END(bh, STAGE_ROLE_HALF + half);
 #pragma unroll
     for (int k = 0; k < 8; k++) store_image(p.NC - 1, k);
 #undef WD_LANE
@@ -367,6 +376,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   __builtin_amdgcn_s_setprio(2);                      // these waves' few instructions are what the other four wait for
   int seen0 = 0, seen1 = 0;                           // mini-batches the output workgroups are known to have finished
   bool gave_up = false;
+  TTT_STAGES_BEGIN();
 
   // The sum has the order of the one-workgroup kernel, (((b2 + P0) + P1) + P2) + P3 over the wave pairs: half 0 holds P0 and P1 and
   // sends b2 + P0 + P1, half 1 sends P2 and P3.
@@ -400,6 +410,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     if (half == 0) {
       uint64_t wv[8];
       if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+      TTT_STAGE(blk == 0 ? FWH_TAKE0 : FWH_TAKE1);
 #pragma unroll
       for (int k = 0; k < 8; k++) wd_put(src + 64 * k, ~0ull, near);
 #pragma unroll
@@ -410,6 +421,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     } else {
       uint64_t wv[4];
       if (!wd_take(src, wv, w_status, p.wait_limit)) gave_up = true;
+      TTT_STAGE(blk == 0 ? FWH_TAKE0 : FWH_TAKE1);
 #pragma unroll
       for (int k = 0; k < 4; k++) wd_put(src + 64 * k, ~0ull, near);
 #pragma unroll
@@ -458,9 +470,12 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       eta[k] = g_ldh(gEta, 2 * t_in, mb * (CS * 2) + k * CS);
     }
     load_xk(mb + 1 < p.NC ? mb + 1 : mb);
+    TTT_STAGE(FWH_ASK);
     __syncthreads();   // B1
+    TTT_STAGE(FWH_B1);
     gather_send(mb, 0);
     put_xk(mb + 1);   // the buffer was last read a mini-batch ago
+    TTT_STAGE(FWH_SEND0);
     finish_block(mb, 0, xk[0], xv[0], eta[0]);
     if (u == 3 && mb >= FWD_WIDE_RING) {
       // the slot this mini-batch's state goes to is free once the output branch is done with mini-batch mb - RING
@@ -480,12 +495,17 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
         else seen1 = seen;
       }
     }
+    TTT_STAGE(FWH_LN0);
     __syncthreads();   // B2
+    TTT_STAGE(FWH_B2);
     gather_send(mb, 1);
     ln_token_sum_store_product(s_b2p + u * FD, gx, scale, lane, f0);
+    TTT_STAGE(FWH_SEND1);
     finish_block(mb, 1, xk[1], xv[1], eta[1]);
     if (gave_up && lane == 0) *s_flag = 1;
+    TTT_STAGE(FWH_LN1);
     __syncthreads();   // B3
+    TTT_STAGE(FWH_B3);
     if (flag() != 0) return;
     if (u == 0 && lane == 0 && mb > 0) give(mb);   // the stores of the last mini-batch's state were acknowledged before B3
     // b2's step, while the compute waves are busy: the four helper waves wait for each other's shares (all of them come here)
@@ -494,7 +514,9 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     while (__hip_atomic_load(s_flag + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < 4 * (mb + 1)) __builtin_amdgcn_s_sleep(1);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     step_b2(mb);
+    TTT_STAGE(FWH_B2STEP);
   }
+  TTT_STAGES_END(bh, STAGE_ROLE_HALF + half);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (u == 0 && lane == 0) give(p.NC);

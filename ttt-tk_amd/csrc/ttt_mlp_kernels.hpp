@@ -34,7 +34,7 @@ struct FwdParams {
   // segment before it left (an earlier launch on the same stream) and leaves the one the next starts from.
   int seg_len, job0;
 #ifdef TTT_STAGE_CLOCKS
-  unsigned* stage_clocks;   // [B*NH][2 roles][8 waves][STAGE_SLOTS] or nullptr (see below)
+  unsigned* stage_clocks;   // [B*NH][STAGE_ROLES][8 waves][STAGE_SLOTS] or nullptr (see below)
 #endif
 };
 constexpr int FWD_RING_MAX = 32;               // most mini-batches per hand-over (8 or 32 are compiled)
@@ -101,7 +101,7 @@ struct BwdParams {
   // stream) left them, and the norm-gradient sums from the pair's slots of x_hat_ln_group.
   int seg_groups, job0;
 #ifdef TTT_STAGE_CLOCKS
-  unsigned* stage_clocks;   // [B*NH][4 roles][8 waves][STAGE_SLOTS] or nullptr (see below)
+  unsigned* stage_clocks;   // [B*NH][STAGE_ROLES][8 waves][STAGE_SLOTS] or nullptr (see below)
 #endif
 };
 
@@ -125,9 +125,12 @@ inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE 
 // spent in each; every wave stores its sums when the kernel ends.  The product library
 // is built without the macro and contains none of this.  Reading the clock is a scalar-memory operation: every
 // boundary also waits for the wave's outstanding LDS reads, which makes an instrumented kernel some 10 % slower.
-// Slot of a workgroup in the buffer: forward 0 = the recurrence (or the one workgroup), 1 = the output branch;
-// backward 0 / 1 = the replaying workgroups, 2 = the reverse walk (or the one workgroup), 3 = unused.
+// Role of a workgroup in the buffer: forward 0 = the recurrence (or the one workgroup), 1 / 2 = the output branch, 3 / 4 = the halves
+// of a recurrence on two workgroups; backward 0 .. 3 = the replaying workgroups, 4 = the reverse walk (or the one
+// workgroup), 5 = the grad_L_XK workgroup, 6 / 7 = the halves of a walk on two workgroups.
 constexpr int STAGE_SLOTS = 24;
+constexpr int STAGE_ROLES = 8;
+constexpr int STAGE_ROLE_OUT = 1, STAGE_ROLE_HALF = 3, STAGE_ROLE_WALK = 4, STAGE_ROLE_DXK = 5, STAGE_ROLE_WALK_HALF = 6;
 enum FwdStage {
   FS_TOP,            // barrier that opens the mini-batch, checkpoint store, wait for the other workgroup
   FS_F1_GELU,        // Z1 = XK W1 + b1, GELU and its derivative
@@ -171,13 +174,58 @@ enum BwdStage {
   BS_X_SUMS,         // grad_L_XK workgroup: pair sum, grad_L_XK / grad_L_XV, token sums of the norm gradients, barrier
   BS_COUNT
 };
-static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS, "stage slots");
+// The recurrence and the walk on two workgroups: their waves 0-3 (compute) and 4-7 (helpers) go through stages of their own.
+enum FwdWideStage {
+  FWC_BLOCK0,        // compute: checkpoint store, Z1, GELU and partial Z2 of token block 0
+  FWC_B1,            // compute: barrier behind it
+  FWC_BLOCK1,        // compute: the same for block 1, W2's terms transposed, the last state's images stored
+  FWC_B2,            // compute: barrier behind it (block 0's sums have crossed and been normalised)
+  FWC_STEP0,         // compute: G1 of block 0 and its share of the weight step
+  FWC_B3,            // compute: barrier behind it (the same for block 1's sums)
+  FWC_STEP1,         // compute: the same for block 1, the new state split into its terms
+  FWH_ASK,           // helpers: the next inputs asked for, what the last mini-batch left in flight waited for
+  FWH_B1,            // helpers: wait for block 0's partial sums
+  FWH_SEND0,         // helpers: sum over this CU's hidden columns, sent to the other CU
+  FWH_TAKE0,         // helpers: wait for the other CU's share of block 0
+  FWH_LN0,           // helpers: LayerNorm and loss gradient of block 0, G2 to LDS, free ring slot waited for
+  FWH_B2,            // helpers: wait for block 1's partial sums
+  FWH_SEND1,         // helpers: as for block 0, with block 0's token sums for b2
+  FWH_TAKE1,         // helpers: wait for the other CU's share of block 1
+  FWH_LN1,           // helpers: LayerNorm and loss gradient of block 1, G2 to LDS
+  FWH_B3,            // helpers: wait for block 0's weight step
+  FWH_B2STEP,        // helpers: state announced, step of b2
+  FWX_COUNT
+};
+enum BwdWideStage {
+  BWC_BAR_TERMS,     // compute: what the output branch adds to the running gradients
+  BWC_STEP0,         // compute: weight step backwards, partial sums of token block 0
+  BWC_B1,            // compute: barrier behind it
+  BWC_STEP1,         // compute: the same for block 1
+  BWC_B2,            // compute: barrier behind it (block 0's sums have crossed, dZ2 of block 0 is there)
+  BWC_PRODUCTS,      // compute: products of the inner MLP backwards that do not need the sums
+  BWC_MLP0,          // compute: inner MLP backwards and updates, block 0
+  BWC_B3,            // compute: barrier behind it (the same for block 1's sums)
+  BWC_MLP1,          // compute: inner MLP backwards and updates, block 1
+  BWH_ASK,           // helpers: next group waited for, gradient wrt b2, the next mini-batch's tiles asked for
+  BWH_B1,            // helpers: wait for block 0's partial sums
+  BWH_SEND0,         // helpers: last mini-batch announced, sum over this CU's hidden columns, sent to the other CU
+  BWH_TAKE0,         // helpers: wait for the other CU's share of block 0
+  BWH_LN0,           // helpers: second-order LayerNorm pass of block 0, dZ2 to LDS
+  BWH_B2,            // helpers: wait for block 1's partial sums
+  BWH_SEND1,         // helpers: as for block 0, with block 0's outputs stored and the next mini-batch's tiles put into LDS
+  BWH_TAKE1,         // helpers: wait for the other CU's share of block 1
+  BWH_LN1,           // helpers: second-order LayerNorm pass of block 1, dZ2 to LDS
+  BWH_B3,            // helpers: wait for block 0's inner MLP backwards
+  BWH_STORE1,        // helpers: block 1's outputs stored, gradient wrt b2
+  BWX_COUNT
+};
+static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <= STAGE_SLOTS && BWX_COUNT <= STAGE_SLOTS, "stage slots");
 
 }  // namespace ttt
 
 #ifdef TTT_STAGE_CLOCKS
-// Device buffers the next launches write their stage clocks to (nullptr: none): forward [B*NH][2][8][STAGE_SLOTS],
-// backward [B*NH][4][8][STAGE_SLOTS] unsigned ints, zero-filled by the caller.
+// Device buffers the next launches write their stage clocks to (nullptr: none): [B*NH][STAGE_ROLES][8][STAGE_SLOTS]
+// unsigned ints each, zero-filled by the caller.
 extern "C" void ttt_mlp_set_stage_clocks(unsigned* forward, unsigned* backward);
 #endif
 

@@ -6,10 +6,11 @@
 
 Loads the library built with -DTTT_STAGE_CLOCKS (the product library contains no clocks), runs the forward and the
 backward of the workload once each the way the operator module would (same launch plan, workspace from torch), and
-prints for every kind of workgroup - forward: recurrence / output branch; backward: replay / reverse walk - the
-clocks per mini-batch that its waves spent in each stage, averaged over the (batch, head) pairs: the mean over
-the 8 waves and the slowest wave.  The stage names and their descriptions are read from the two enums in
-csrc/ttt_mlp_kernels.hpp.  Reading the clock is a scalar-memory operation that also waits for the wave's
+prints for every kind of workgroup - forward: recurrence / output branch; backward: replay / reverse walk / grad_L_XK
+workgroup - the clocks per mini-batch that its waves spent in each stage, averaged over the (batch, head) pairs: the mean
+over the 8 waves and the slowest wave.  Where the recurrence or the walk runs on two workgroups, their compute waves and
+their helper waves go through stages of their own and get a table each.  The stage names and their descriptions are read
+from the enums in csrc/ttt_mlp_kernels.hpp.  --shape B,NH,NC,CGS takes another shape than the benchmark's.  Reading the clock is a scalar-memory operation that also waits for the wave's
 outstanding LDS reads, so an instrumented kernel runs some 10 % slower than the product kernel; the launch times of
 both are printed side by side.
 """
@@ -24,6 +25,8 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SLOTS = 24
+ROLES = 8     # of a workgroup: csrc/ttt_mlp_kernels.hpp
+OUT, HALF, WALK, DXK, WALK_HALF = 1, 3, 4, 5, 6
 WAVES = 8
 WORKLOADS = {   # B, NH, NC, checkpoint_group_size, std of the eta logits
     "c3": (1, 48, 256, 16, 1.0),
@@ -47,8 +50,8 @@ PER_WAVE = False
 
 
 def table(title, clocks, names, per_mb):
-    """clocks: tensor [pairs][8 waves][SLOTS] of summed clocks; per_mb: mini-batches each wave went through."""
-    mean_w = clocks.double().mean(dim=0) / per_mb          # [8][SLOTS]
+    """clocks: tensor [pairs][waves][SLOTS] of summed clocks; per_mb: mini-batches each wave went through."""
+    mean_w = clocks.double().mean(dim=0) / per_mb          # [waves][SLOTS]
     tot = mean_w.sum(dim=1)                                # per wave
     lines = [f"{title}: {tot.mean().item():9.0f} clocks per mini-batch (mean over the waves; slowest wave {tot.max().item():.0f})"]
     for i, (name, desc) in enumerate(names):
@@ -56,7 +59,7 @@ def table(title, clocks, names, per_mb):
         if mx <= 0:
             continue
         if PER_WAVE:
-            lines.append(f"  {name:18s} {m:8.0f}   waves 0-7: " + " ".join(f"{x:6.0f}" for x in mean_w[:, i].tolist()))
+            lines.append(f"  {name:18s} {m:8.0f}   wave by wave: " + " ".join(f"{x:6.0f}" for x in mean_w[:, i].tolist()))
         else:
             lines.append(f"  {name:18s} {m:8.0f} {100 * m / tot.mean().item():5.1f} %   slowest wave {mx:8.0f}   {desc}")
     return lines
@@ -65,6 +68,7 @@ def table(title, clocks, names, per_mb):
 def main() -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--workload", choices=sorted(WORKLOADS), default="c4")
+    ap.add_argument("--shape", default=None, metavar="B,NH,NC,CGS", help="this shape instead of a named workload")
     ap.add_argument("--out", default=None, help="also write the tables to this file")
     ap.add_argument("--per-wave", action="store_true", help="every stage's clocks wave by wave instead of share and description")
     a = ap.parse_args()
@@ -81,7 +85,13 @@ def main() -> int:
         raise SystemExit(f"{STAGES_LIB} is missing or older than the product library: run  python ttt-tk_amd/build.py --stages  first")
     header = open(os.path.join(HERE, "csrc", "ttt_mlp_kernels.hpp")).read()
     fwd_names, bwd_names = stage_names(header, "FwdStage"), stage_names(header, "BwdStage")
-    B, NH, NC, cgs, eta_std = WORKLOADS[a.workload]
+    fwd_wide_names, bwd_wide_names = stage_names(header, "FwdWideStage"), stage_names(header, "BwdWideStage")
+    if a.shape:
+        B, NH, NC, cgs, eta_std = *(int(x) for x in a.shape.split(",")), 1.0
+        label, option = "custom", f"--shape {a.shape}"
+    else:
+        B, NH, NC, cgs, eta_std = WORKLOADS[a.workload]
+        label, option = a.workload, f"--workload {a.workload}"
     BH, K = B * NH, host.num_checkpoints(NC, cgs)
     dev = torch.device("cuda:0")
     t = make_device_inputs(B, NH, NC, eta_std, dev)
@@ -133,8 +143,8 @@ def main() -> int:
     plain_ms = (timed(pf), timed(pb))
 
     lib = ctypes.CDLL(STAGES_LIB)
-    cf = torch.zeros(BH, 2, WAVES, SLOTS, dtype=torch.int32, device=dev)
-    cb = torch.zeros(BH, 4, WAVES, SLOTS, dtype=torch.int32, device=dev)
+    cf = torch.zeros(BH, ROLES, WAVES, SLOTS, dtype=torch.int32, device=dev)
+    cb = torch.zeros(BH, ROLES, WAVES, SLOTS, dtype=torch.int32, device=dev)
     lib.ttt_mlp_set_stage_clocks.restype = None
     sf, sb, keep1 = launches(lib)
     lib.ttt_mlp_set_stage_clocks(ctypes.c_void_p(0), ctypes.c_void_p(0))
@@ -150,8 +160,8 @@ def main() -> int:
     cf, cb = cf.cpu().long() & 0xFFFFFFFF, cb.cpu().long() & 0xFFFFFFFF
 
     props = torch.cuda.get_device_properties(0)
-    out = [f"Stage clocks of the TTT-MLP kernels, workload {a.workload}: B={B} NH={NH} NC={NC} checkpoint_group_size={cgs} on {props.name} ({props.multi_processor_count} CUs)",
-           f"Command: python ttt-tk_amd/build.py --stages && python ttt-tk_amd/stage_clocks.py --workload {a.workload}",
+    out = [f"Stage clocks of the TTT-MLP kernels, workload {label}: B={B} NH={NH} NC={NC} checkpoint_group_size={cgs} on {props.name} ({props.multi_processor_count} CUs)",
+           f"Command: python ttt-tk_amd/build.py --stages && python ttt-tk_amd/stage_clocks.py {option}",
            f"Launch times: forward {plain_ms[0]:.2f} ms, backward {plain_ms[1]:.2f} ms (product library); "
            f"{stage_ms[0]:.2f} ms, {stage_ms[1]:.2f} ms with the clocks compiled in",
            "Clocks are shader clocks per mini-batch and wave, averaged over the (batch, head) pairs whose workgroup of that kind ran;",
@@ -160,30 +170,45 @@ def main() -> int:
     def present(x):   # pairs whose workgroup of this kind wrote anything
         return x[x.sum(dim=(1, 2)) > 0]
 
-    one_f, rec, outb = present(cf[:, 0]), None, present(cf[:, 1])
-    if len(outb):   # pairs with two workgroups: slot 0 is the recurrence alone
-        two = cf[:, 1].sum(dim=(1, 2)) > 0
-        rec, one_f = cf[two, 0], cf[~two, 0]
-        one_f = present(one_f)
-    if len(one_f):
-        out += table(f"forward, one workgroup per pair ({len(one_f)} pairs)", one_f, fwd_names, NC) + [""]
-    if rec is not None:
-        out += table(f"forward, recurrence workgroup ({len(rec)} pairs)", rec, fwd_names, NC) + [""]
-        out += table(f"forward, output-branch workgroup ({len(outb)} pairs)", outb, fwd_names, NC) + [""]
-    r0, r1, walk = cb[:, 0], cb[:, 1], cb[:, 2]
-    has_r0, has_r1 = r0.sum(dim=(1, 2)) > 0, r1.sum(dim=(1, 2)) > 0
-    single = present(walk[~has_r0])
-    if len(single):
-        out += table(f"backward, one workgroup per pair ({len(single)} pairs)", single, bwd_names, NC) + [""]
-    if has_r0.any():
-        n_rep = 2 if has_r1.any() else 1
-        groups0 = (K + n_rep - 1) // n_rep   # groups (counted from the end) replayed by the first replaying workgroup
-        mb0 = NC - (K - groups0) * cgs if n_rep == 1 else sum(min(cgs, NC - (K - 1 - g) * cgs) for g in range(0, K, 2))
-        out += table(f"backward, replaying workgroup 0 of {n_rep} ({int(has_r0.sum())} pairs, {mb0} of the {NC} mini-batches)", r0[has_r0], bwd_names, mb0) + [""]
-        out += table(f"backward, reverse-walk workgroup ({int(has_r0.sum())} pairs)", walk[has_r0], bwd_names, NC) + [""]
-        fin = cb[:, 3]
-        if (fin.sum(dim=(1, 2)) > 0).any():
-            out += table(f"backward, grad_L_XK workgroup ({int((fin.sum(dim=(1, 2)) > 0).sum())} pairs)", present(fin), bwd_names, NC) + [""]
+    def ran(x):       # which pairs had a workgroup of this kind
+        return x.sum(dim=(1, 2)) > 0
+
+    def halves(clocks, role):   # both workgroups of every pair, as if they were pairs of their own
+        return torch.cat((present(clocks[:, role]), present(clocks[:, role + 1])))
+
+    def mini_batches(turn, n):  # of the groups (counted from the end) that replaying workgroup `turn` of n takes
+        return sum(min(cgs, NC - (K - 1 - g) * cgs) for g in range(turn, K, n))
+
+    wide_f, split_f = ran(cf[:, HALF]), ran(cf[:, OUT]) & ~ran(cf[:, HALF])
+    one_f = ran(cf[:, 0]) & ~split_f
+    if one_f.any():
+        out += table(f"forward, one workgroup per pair ({int(one_f.sum())} pairs)", cf[one_f, 0], fwd_names, NC) + [""]
+    if split_f.any():
+        out += table(f"forward, recurrence workgroup ({int(split_f.sum())} pairs)", cf[split_f, 0], fwd_names, NC) + [""]
+        out += table(f"forward, output-branch workgroup ({int(split_f.sum())} pairs)", cf[split_f, OUT], fwd_names, NC) + [""]
+    if wide_f.any():
+        both = halves(cf, HALF)
+        n_out = 2 if ran(cf[:, OUT + 1]).any() else 1
+        out += table(f"forward, recurrence on two workgroups, compute waves ({int(wide_f.sum())} pairs)", both[:, :4], fwd_wide_names, NC) + [""]
+        out += table("forward, recurrence on two workgroups, helper waves", both[:, 4:], fwd_wide_names, NC) + [""]
+        out += table(f"forward, output-branch workgroup 0 of {n_out}", cf[wide_f, OUT], fwd_names, -(-NC // n_out)) + [""]
+    n_rep = sum(bool(ran(cb[:, r]).any()) for r in range(4))
+    wide_b, rep0 = ran(cb[:, WALK_HALF]), ran(cb[:, 0])
+    walk_b = ran(cb[:, WALK])
+    if (walk_b & ~rep0).any():
+        one_b = walk_b & ~rep0
+        out += table(f"backward, one workgroup per pair ({int(one_b.sum())} pairs)", cb[one_b, WALK], bwd_names, NC) + [""]
+    if rep0.any():
+        mb0 = mini_batches(0, n_rep)
+        out += table(f"backward, replaying workgroup 0 of {n_rep} ({int(rep0.sum())} pairs, {mb0} of the {NC} mini-batches)", cb[rep0, 0], bwd_names, mb0) + [""]
+    if (walk_b & rep0).any():
+        out += table(f"backward, reverse-walk workgroup ({int((walk_b & rep0).sum())} pairs)", cb[walk_b & rep0, WALK], bwd_names, NC) + [""]
+    if wide_b.any():
+        both = halves(cb, WALK_HALF)
+        out += table(f"backward, walk on two workgroups, compute waves ({int(wide_b.sum())} pairs)", both[:, :4], bwd_wide_names, NC) + [""]
+        out += table("backward, walk on two workgroups, helper waves", both[:, 4:], bwd_wide_names, NC) + [""]
+    if ran(cb[:, DXK]).any():
+        out += table(f"backward, grad_L_XK workgroup ({int(ran(cb[:, DXK]).sum())} pairs)", present(cb[:, DXK]), bwd_names, NC) + [""]
     text = "\n".join(out)
     print(text)
     if a.out:

@@ -136,6 +136,27 @@ def measured_traffic_checked(workload, which):
     return measured_traffic(workload, which), None
 
 
+def launched_kernel(which, pairs, NC, cgs, cus, overlapped):
+    """Kernel(s) that a forward (which = 0) or backward (1) of this shape launches; one is compiled per combination of roles."""
+    import ctypes
+    lib = ctypes.CDLL(os.path.join(ROOT, "ttt-tk_amd", "libttt_mlp.so"))
+    one_each = ("ttt_mlp_fwd_kernel", "ttt_mlp_bwd_kernel")[which]
+    seg, launches = ctypes.c_int(), ctypes.c_int()
+    lib.ttt_mlp_segment_plan(which, ctypes.c_longlong(pairs), cus, NC, cgs, 1 if overlapped else 0, ctypes.byref(seg), ctypes.byref(launches))
+    if seg.value > 0:
+        return f"{one_each} x {launches.value} (sequences cut at checkpoints)"
+    if not overlapped:
+        return one_each
+    one, rest, per = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
+    lib.ttt_mlp_launch_plan(which, ctypes.c_longlong(pairs), cus, ctypes.byref(one), ctypes.byref(rest), ctypes.byref(per))
+    if which == 0:   # <mini-batches per hand-over>
+        several = "ttt_mlp_fwd_wide_kernel" if per.value > 2 else f"ttt_mlp_fwd_split_kernel<{32 if NC >= 512 else 8}>"
+    else:            # <replaying workgroups, grad_L_XK workgroup> / <replaying workgroups, workgroup that reads ahead>
+        several = {2: "ttt_mlp_bwd_split_kernel<1, false>", 3: "ttt_mlp_bwd_split_kernel<2, false>", 4: "ttt_mlp_bwd_split_kernel<2, true>",
+                   5: "ttt_mlp_bwd_wide_kernel<2, false>", 7: "ttt_mlp_bwd_wide_kernel<3, true>", 8: "ttt_mlp_bwd_wide_kernel<4, true>"}.get(per.value, "")
+    return f"{one_each} + {several}" if one.value else several
+
+
 def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibrate_copy=False):
     """Times `steps` forward (+ backward) steps of one workload and returns the figures of its JSON block."""
     import torch
@@ -194,28 +215,9 @@ def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibra
     bwd_tflops = BWD_G * G_FLOP * mb_steps / (bwd_ms * 1e-3) / 1e12 if backward else 0.0
     fwd_tflops = FWD_G * G_FLOP * mb_steps / (fwd_ms * 1e-3) / 1e12
     all_tflops = (FWD_G + (BWD_G if backward else 0)) * G_FLOP * mb_steps / (ms_per_step * 1e-3) / 1e12
-    # one kernel per combination of roles: ttt_mlp_bwd_split_kernel<replaying workgroups, grad_L_XK workgroup>
-    bwd_kernel = "ttt_mlp_bwd_kernel"
-    fwd_kernel = "ttt_mlp_fwd_kernel" if ext.last_forward_mode() == 0 else f"ttt_mlp_fwd_split_kernel<{32 if NC >= 512 else 8}>"
-    import ctypes
-    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(host.__file__)), "libttt_mlp.so"))
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-
-    def cut(which, overlapped):   # launches of a call whose sequences are cut at checkpoints (0: they are not)
-        seg, launches = ctypes.c_int(), ctypes.c_int()
-        lib.ttt_mlp_segment_plan(which, ctypes.c_longlong(B * NH), cus, NC, cgs, 1 if overlapped else 0, ctypes.byref(seg), ctypes.byref(launches))
-        return launches.value if seg.value > 0 else 0
-
-    if cut(0, ext.last_forward_mode() == 1):
-        fwd_kernel = f"ttt_mlp_fwd_kernel x {cut(0, ext.last_forward_mode() == 1)} (sequences cut at checkpoints)"
-    if backward and cut(1, ext.last_backward_mode() == 1):
-        bwd_kernel = f"ttt_mlp_bwd_kernel x {cut(1, ext.last_backward_mode() == 1)} (sequences cut at checkpoints)"
-    elif backward and ext.last_backward_mode() == 1:
-        one, rest, per = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
-        lib.ttt_mlp_launch_plan(1, ctypes.c_longlong(B * NH), cus, ctypes.byref(one), ctypes.byref(rest), ctypes.byref(per))
-        bwd_kernel = f"ttt_mlp_bwd_split_kernel<{2 if per.value >= 3 else 1}, {'true' if per.value >= 4 else 'false'}>"
-        if one.value:
-            bwd_kernel = "ttt_mlp_bwd_kernel + " + bwd_kernel
+    fwd_kernel = launched_kernel(0, B * NH, NC, cgs, cus, ext.last_forward_mode() == 1)
+    bwd_kernel = launched_kernel(1, B * NH, NC, cgs, cus, ext.last_backward_mode() == 1) if backward else None
     traffic, note = measured_traffic_checked(name, "bwd" if backward else "fwd")
     # the dominant kernel: the backward (the forward where there is no backward)
     roofline = {"bound": "mfma", "kernel": bwd_kernel if backward else fwd_kernel,

@@ -136,20 +136,24 @@ int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* args, void* stream);
 /* Same for the remat backward. */
 int ttt_mlp_bwd_launch(const ttt_mlp_bwd_args* args, void* stream);
 
-/* The same backward (bit-identical results) with two to five workgroups per
- * (batch, head) where the device has CUs to spare: one or two recompute checkpoint
- * group after checkpoint group, one walks each recomputed group backwards, a
- * fourth forms grad_L_XK, grad_L_XV and part of the norm gradients from what the
+/* The same backward (bit-identical results) with two to eight workgroups per
+ * (batch, head) where the device has CUs to spare: one to four recompute checkpoint
+ * group after checkpoint group, one walks each recomputed group backwards - or two,
+ * which hold half of the hidden columns each and exchange partial sums - another
+ * forms grad_L_XK, grad_L_XV and part of the norm gradients from what the
  * walk hands it, so that only the chain through the running gradients stays on
- * the critical path, and a fifth (with a multiple of 8 pairs, if 5*n fits) only
- * reads ahead of the walk so that the walk's requests hit the L2.  The reference launcher
+ * the critical path, and one more only reads ahead of the walk so that the walk's
+ * requests hit the L2.  The reference launcher
  * (kernels/ttt_backward/ttt.cu:1451-1917) has no counterpart: it spreads one
  * (batch, head) over a cluster of four thread blocks instead.
  * Workgroups that wait for each other must be resident together (one per CU),
  * so the pairs are covered by up to two launches in a row: the largest multiple
- * of the CU count with one workgroup per pair, then the remaining n pairs with
- * four each if 4*n fits the CUs, else three if 3*n fits, else two if 2*n fits.
- * ttt_mlp_bwd_workspace_bytes() returns 0 when neither does (n = 0 or 2*n > CUs of
+ * of the CU count with one workgroup per pair, then the remaining n pairs.  Where
+ * the workgroups of ceil(n/8) pairs fit an eighth of the CUs the walk takes two: eight
+ * per pair (four recomputing, one reading ahead), else seven (three), else
+ * five (two recomputing, none reading ahead) - up to 32, 32 and 48 pairs on 256 CUs.
+ * Otherwise four per pair if 4*n fits the CUs, else three if 3*n fits, else two if 2*n fits.
+ * ttt_mlp_bwd_workspace_bytes() returns 0 when none does (n = 0 or 2*n > CUs of
  * the current device); the launcher then returns TTT_MLP_ERR_NO_ROOM and the caller
  * uses ttt_mlp_bwd_launch.
  * The caller owns the device workspace (256-byte aligned, contents unspecified
@@ -230,8 +234,10 @@ const char* ttt_mlp_error_string(int code);
 /* How an overlapped launch of `pairs` = B*NH (batch, head) pairs is laid out on a device with
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
  * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  which = 0
- * forward (1 or 2 roles per pair; see ttt_mlp_fwd_workspace_bytes for what a role takes), 1 backward (1 to 5: one or two that replay the checkpoint groups, one that walks
- * them backwards, one for grad_L_XK / grad_L_XV, one that fetches the walk's operands into the L2 ahead of it). */
+ * forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk),
+ * 3 (two replay), 4 (and one for grad_L_XK / grad_L_XV), 5, 7 or 8 (walk on two, grad_L_XK, two, three or four that
+ * replay; with three or four one more that reads ahead).  More than 2 forward and more than 4 backward: the workgroups of
+ * a pair share an XCD, and those of ceil(*other_pairs / 8) pairs fit an eighth of the CUs. */
 int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long* one_workgroup_pairs,
                         long long* other_pairs, int* workgroups_per_other_pair);
 

@@ -141,20 +141,25 @@ int make_bwd_params(const ttt_mlp_bwd_args* a, ttt::BwdParams& p) {
   return TTT_MLP_OK;
 }
 
-// Two workgroups per (batch, head) wait for each other, so all of them must be resident at once: one
+// Several workgroups per (batch, head) wait for each other, so all of them must be resident at once: one
 // workgroup fills a CU (LDS), hence such a launch may not exceed the CUs of the current device.  The
 // (batch, head) pairs are therefore covered by two launches in a row: as many full rounds of one
-// workgroup per pair as there are (a multiple of the CU count), then the rest - with two workgroups per
-// pair if that fits the device (split), otherwise with one.
+// workgroup per pair as there are (a multiple of the CU count), then the rest - with several workgroups per
+// pair if two each fit the device (split), otherwise with one.
+// With the recurrence (walk) of a pair on two CUs (wide) the workgroups of a pair share an XCD: the grid is padded to a
+// multiple of 8 pairs and dealt to the 8 XCDs in turn, so those of ceil(pairs / 8) pairs must fit an eighth of the CUs.
 struct LaunchPlan {
   long long n_single = 0;   // pairs 0 .. n_single-1: one workgroup each
   long long n_rest = 0;     // pairs n_single .. n_single+n_rest-1
   bool rest_split = false;
-  int per_pair = 1;         // workgroups per pair of the rest: 2, or 3 / 4 where the kernel can use them and they fit
-  bool prefetch = false;    // backward with 4 per pair: a fifth that fetches ahead of the walk
+  bool wide = false;
+  int per_pair = 1;         // workgroups per pair of the rest, in every role
+  int n_out = 0;            // forward, wide: that compute Out
+  int n_replay = 0;         // backward: that replay checkpoint groups
+  bool finish = false;      // backward: one more for grad_L_XK / grad_L_XV
+  bool prefetch = false;    // backward: and one that fetches ahead of the walk
 };
-// `three_way`: the backward can use three to five workgroups per pair, the forward two.
-LaunchPlan plan_for(long long BH, int cus, bool three_way) {
+LaunchPlan plan_for(long long BH, int cus, bool backward) {
   LaunchPlan pl;
   if (BH <= 0 || cus <= 0) {
     pl.n_single = BH > 0 ? BH : 0;
@@ -163,19 +168,45 @@ LaunchPlan plan_for(long long BH, int cus, bool three_way) {
   pl.n_single = BH / cus * cus;
   pl.n_rest = BH - pl.n_single;
   pl.rest_split = pl.n_rest > 0 && 2 * pl.n_rest <= cus;
-  if (!pl.rest_split) { pl.n_single = BH; pl.n_rest = 0; }
-  else pl.per_pair = !three_way ? 2 : 4 * pl.n_rest <= cus ? 4 : 3 * pl.n_rest <= cus ? 3 : 2;
-  // the fifth workgroup helps only from the walk's own XCD, which the kernel arranges for a multiple of 8 pairs
-  pl.prefetch = pl.per_pair == 4 && 5 * pl.n_rest <= cus && pl.n_rest % 8 == 0;
+  if (!pl.rest_split) {
+    pl.n_single = BH;
+    pl.n_rest = 0;
+    return pl;
+  }
+  const long long per_xcd = (pl.n_rest + 7) / 8;
+  const auto fits_xcd = [&](int per) { return per * per_xcd <= cus / 8; };
+  if (!backward) {
+    // one output workgroup keeps up with a recurrence on two CUs only just; two where they fit
+    pl.n_out = fits_xcd(4) ? 2 : fits_xcd(3) ? 1 : 0;
+    pl.wide = pl.n_out > 0;
+    pl.per_pair = 2 + pl.n_out;
+    return pl;
+  }
+  // Two replaying workgroups bound a walk on two CUs (48 pairs x 4,096 mini-batches: 20 us per replayed mini-batch, 10.1 us per
+  // walked one).  Four leave it to itself, also where they evaluate the GELU family for it (32 pairs x 512: 25 us per
+  // replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).
+  pl.n_replay = fits_xcd(8) ? 4 : fits_xcd(7) ? 3 : fits_xcd(5) ? 2 : 0;
+  pl.wide = pl.n_replay > 0;
+  if (pl.wide) {
+    pl.finish = true;
+    pl.prefetch = pl.n_replay > 2;
+    pl.per_pair = 2 + pl.n_replay + 1 + (pl.prefetch ? 1 : 0);
+    return pl;
+  }
+  pl.finish = 4 * pl.n_rest <= cus;
+  pl.n_replay = 3 * pl.n_rest <= cus ? 2 : 1;
+  // the fetching workgroup helps only from the walk's own XCD, which the kernel arranges for a multiple of 8 pairs
+  pl.prefetch = pl.finish && 5 * pl.n_rest <= cus && pl.n_rest % 8 == 0;
+  pl.per_pair = 1 + pl.n_replay + (pl.finish ? 1 : 0) + (pl.prefetch ? 1 : 0);
   return pl;
 }
-LaunchPlan plan_launches(long long BH, bool three_way) {
+int device_cus() {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 0;
-  if (g_cu_budget > 0 && g_cu_budget < cus) cus = g_cu_budget;
-  return plan_for(BH, cus, three_way);
+    return 0;
+  return g_cu_budget > 0 && g_cu_budget < cus ? g_cu_budget : cus;
 }
+LaunchPlan plan_launches(long long BH, bool backward) { return plan_for(BH, device_cus(), backward); }
 
 // More (batch, head) pairs than CUs, one workgroup each: the hardware runs them in rounds, and a last round that is
 // not full leaves CUs idle for a whole sequence.  The forward can cut every sequence into segments at checkpoint
@@ -222,16 +253,10 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long a
 long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, bool with_workspace, bool backward) {
   if (cus <= 0) return (long long)NC * 1000;
   if (with_workspace && pl.rest_split) {
-    const int rest = !backward ? 755 : pl.per_pair == 2 ? 560 : pl.per_pair == 3 ? 400 : 300;
+    const int rest = !backward ? 755 : pl.n_replay == 1 ? 560 : !pl.finish ? 400 : 300;
     return (pl.n_single / cus * 1000 + rest) * NC;
   }
   return (pairs + cus - 1) / cus * 1000 * NC;
-}
-int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  return g_cu_budget > 0 && g_cu_budget < cus ? g_cu_budget : cus;
 }
 // The launches of a call with the sequences cut: `cus` jobs each, in job order, on the one stream.
 template <class Params, class Enqueue>
@@ -294,26 +319,8 @@ struct BwdWorkspace {
   }
 };
 
-// Replaying workgroups per pair when the walk of each of the n pairs runs on two CUs of one XCD (with one more for grad_L_XK),
-// 0 if it does not: as for the forward, the workgroups of ceil(n / 8) pairs must fit an eighth of the CUs.  The walk takes
-// a mini-batch in a third of the time of a replay, so four replaying workgroups keep up with it, two are what bounds it.
-int bwd_wide_replays(long long n, int cus) {
-  const long long per_xcd = (n + 7) / 8;
-  if (n <= 0) return 0;
-  return 8 * per_xcd <= cus / 8 ? 4 : 7 * per_xcd <= cus / 8 ? 3 : 5 * per_xcd <= cus / 8 ? 2 : 0;
-}
-// Shape of the backward's launch with several workgroups per pair.
-struct BwdShape {
-  int n_replay, n_sets;
-  bool finish, wide;
-  BwdShape(const LaunchPlan& pl, int cus) {
-    const int r = bwd_wide_replays(pl.n_rest, cus);
-    wide = r > 0;
-    n_replay = wide ? r : pl.per_pair >= 3 ? 2 : 1;
-    n_sets = wide ? r + 2 : 2 * n_replay;
-    finish = wide || pl.per_pair == 4;
-  }
-};
+// Sets of the per-group tensors that carry replayed groups to the walk.
+int bwd_sets(const LaunchPlan& pl) { return pl.wide ? pl.n_replay + 2 : 2 * pl.n_replay; }
 
 // Workspace of the forward's two-workgroup mode: synchronisation words, then per (batch, head) a ring of
 // 2 * FWD_RING_MAX slots of state images and of bias vectors.
@@ -331,14 +338,6 @@ struct FwdWorkspace {
     total = o;
   }
 };
-
-// Output workgroups per pair when the recurrence of each of the n pairs of a several-workgroup launch runs on two CUs of one
-// XCD, 0 if it does not: the workgroups of a pair share an XCD and wait for each other, so those of ceil(n / 8) pairs
-// must fit its CUs (an eighth of the device's).  One output workgroup keeps up with the recurrence only just; two where they fit.
-int fwd_wide_outputs(long long n, int cus) {
-  const long long per_xcd = (n + 7) / 8;
-  return n <= 0 ? 0 : 4 * per_xcd <= cus / 8 ? 2 : 3 * per_xcd <= cus / 8 ? 1 : 0;
-}
 
 int check_workspace(const void* workspace) {
   if (workspace == nullptr) return TTT_MLP_ERR_BAD_ARG;
@@ -373,9 +372,7 @@ extern "C" int ttt_mlp_bwd_export_group0(const ttt_mlp_bwd_args* a, void* stream
 extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_group_size) {
   if (B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16)) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
-  if (!pl.rest_split) return 0;
-  const BwdShape sh(pl, device_cus());
-  return BwdWorkspace(pl.n_rest, checkpoint_group_size, sh.n_sets - 1, sh.finish, sh.wide).total;
+  return pl.rest_split ? BwdWorkspace(pl.n_rest, checkpoint_group_size, bwd_sets(pl) - 1, pl.finish, pl.wide).total : 0;
 }
 
 extern "C" size_t ttt_mlp_bwd_status_offset(int B, int NH) {
@@ -390,10 +387,8 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const BwdShape sh(pl, device_cus());
-  const int alt_sets = sh.n_sets - 1;
-  const bool finish = sh.finish;
-  const BwdWorkspace w(pl.n_rest, p.cgs, alt_sets, finish, sh.wide);
+  const int alt_sets = bwd_sets(pl) - 1;
+  const BwdWorkspace w(pl.n_rest, p.cgs, alt_sets, pl.finish, pl.wide);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   {
@@ -419,12 +414,12 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   const size_t norm = 8 * 2 * TTT_MLP_F;
   p.bh0 = static_cast<int>(pl.n_single);
   p.nbh = static_cast<int>(pl.n_rest);
-  p.n_replay = sh.n_replay;
-  p.n_sets = sh.n_sets;
-  p.n_finish = finish ? 1 : 0;
-  p.n_prefetch = (sh.wide ? sh.n_replay > 2 : pl.prefetch) ? 1 : 0;
+  p.n_replay = pl.n_replay;
+  p.n_sets = bwd_sets(pl);
+  p.n_finish = pl.finish ? 1 : 0;
+  p.n_prefetch = pl.prefetch ? 1 : 0;
   p.wait_limit = g_wait_limit;
-  if (finish) {
+  if (pl.finish) {
     p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[6]) - b0 * 2 * img;
     p.fin_gy = reinterpret_cast<float*>(base + w.off[7]) - b0 * 2 * 2 * tile;
   }
@@ -448,7 +443,7 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
     p.alt_std_fused_group[s] = reinterpret_cast<float*>(base + o[9]) - b0 * vec;
     p.alt_W1_init_group[s] = reinterpret_cast<float*>(base + o[10]) - b0 * img;   // [cgs][64][256] floats = 2 images per slot
   }
-  if (sh.wide) {
+  if (pl.wide) {
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
     return static_cast<int>(ttt_mlp_bwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
   }
@@ -470,7 +465,7 @@ extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
 extern "C" size_t ttt_mlp_fwd_workspace_bytes(int B, int NH) {
   if (B <= 0 || NH <= 0) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, false);
-  return pl.rest_split ? FwdWorkspace(pl.n_rest, fwd_wide_outputs(pl.n_rest, device_cus())).total : 0;
+  return pl.rest_split ? FwdWorkspace(pl.n_rest, pl.n_out).total : 0;
 }
 
 extern "C" size_t ttt_mlp_fwd_status_offset(int B, int NH) {
@@ -485,8 +480,7 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, false);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const int n_out = fwd_wide_outputs(pl.n_rest, device_cus());
-  const FwdWorkspace w(pl.n_rest, n_out);
+  const FwdWorkspace w(pl.n_rest, pl.n_out);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   {
@@ -514,8 +508,8 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
   p.wait_limit = g_wait_limit;
-  if (n_out > 0) {
-    p.n_out = n_out;
+  if (pl.wide) {
+    p.n_out = pl.n_out;
     p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * ttt::FWD_WIDE_RING * (ttt::FWD_IMG_BYTES / 2);
     p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
@@ -583,7 +577,7 @@ extern "C" int ttt_mlp_fwd_launch_static(const ttt_mlp_fwd_args* a, int* sticky_
   if (pairs > STATIC_MAX_PAIRS) return TTT_MLP_ERR_SCRATCH;
   const LaunchPlan pl = plan_launches(pairs, false);
   if (!pl.rest_split || pl.n_single != 0) return TTT_MLP_ERR_NO_ROOM;
-  const FwdWorkspace w(pl.n_rest, fwd_wide_outputs(pl.n_rest, device_cus()));
+  const FwdWorkspace w(pl.n_rest, pl.n_out);
   static_assert(static_scratch_bytes() % 256 == 0, "scratch parts are 256-byte aligned");
   if (w.total > static_scratch_bytes()) return TTT_MLP_ERR_SCRATCH;
   void* ws = nullptr;
@@ -606,7 +600,7 @@ extern "C" int ttt_mlp_launch_plan(int which, long long pairs, int compute_units
   const LaunchPlan pl = plan_for(pairs, compute_units, which == 1);
   *one_workgroup_pairs = pl.n_single;
   *other_pairs = pl.n_rest;
-  *workgroups_per_other_pair = pl.n_rest > 0 ? pl.per_pair + (pl.prefetch ? 1 : 0) : 0;
+  *workgroups_per_other_pair = pl.n_rest > 0 ? pl.per_pair : 0;
   return TTT_MLP_OK;
 }
 

@@ -95,6 +95,8 @@ def short_name(kernel_name: str) -> str:
 
 
 def is_ours(name: str) -> bool:
+    if "clear" in name or "zero_words" in name:   # the small kernels that clear words ahead of a launch
+        return False
     return "ttt_mlp_fwd" in name or "ttt_mlp_bwd" in name or "ttt_mlp_export" in name
 
 
@@ -209,7 +211,7 @@ def profile(workload: str, raw_dir: str, limit_s: int):
     geo = kernel_geometry()
     kernels = {}
     for name, st in stats.items():
-        if not is_ours(name) or "zero_words" in name:
+        if not is_ours(name):
             continue
         key = short_name(name)
         g = geo["fwd" if "fwd" in key else "bwd"]

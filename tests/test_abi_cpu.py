@@ -222,6 +222,8 @@ def test_launch_plan_keeps_waiting_workgroups_within_the_device(lib):
                 assert per in ((0, 2, 3, 4) if which == 0 else (0, 2, 3, 4, 5, 7, 8))
                 if per > (2, 4)[which]:            # the workgroups of a pair on one XCD, the grid padded to a multiple of 8 pairs
                     assert -(-rest // 8) * per <= cus // 8
+                if which == 1 and per == 4:        # a fifth workgroup on the walk's XCD never has room beside a walk on one CU
+                    assert not (5 * rest <= cus and rest % 8 == 0)
     assert lib.ttt_mlp_launch_plan(2, ctypes.c_longlong(1), 1, None, None, None) == 1001
 
 

@@ -6,9 +6,10 @@
 // activations are saved, then the group is walked backwards producing the ten output gradients.
 //
 // Mapping: workgroups of 8 wavefronts (two per SIMD, at most 256 registers each); one per (batch,
-// head), or two to five where the device has CUs to spare - then one or two replay the checkpoint
-// groups (taking turns), one walks them backwards, a group or more behind, a fourth forms
-// grad_L_XK from what the walk hands it, and a fifth reads ahead of the walk into the L2.  Wave v owns hidden columns [32v, 32v+32).  All [tokens x hidden] activations live in
+// head), or two to four where the device has CUs to spare - then one or two replay the checkpoint
+// groups (taking turns), one walks them backwards, a group or more behind, and a fourth forms
+// grad_L_XK from what the walk hands it (with the walk itself on two workgroups: ttt_mlp_bwd_wide.hip, which takes the
+// roles of the others from here).  Wave v owns hidden columns [32v, 32v+32).  All [tokens x hidden] activations live in
 // registers in the "Q" orientation (accumulator rows = hidden, lane = token), so per-token scalars
 // (eta, dEta partial sums) are per-lane values.  An activation that is also needed with tokens as the
 // contraction index is bounced once through a wave-private LDS tile (row store + transposing read).
@@ -132,22 +133,6 @@ TTT_DEV void acc_store_rows(const AccT<RB, CB>& a, gptr_t g, unsigned off, int l
       for (int i = 0; i < 16; i++)
         g_stf(g, vo, off + ((r0 + 32 * rb + 8 * (i >> 2) + (i & 3)) * ld + c0 + 32 * cb) * 4, a.b[rb][cb][i]);
 }
-// Same, but accumulator rows are tensor COLUMNS (the tile holds the transpose of the block).
-template <int RB, int CB>
-TTT_DEV void acc_load_cols(AccT<RB, CB>& a, gptr_t g, unsigned off, int ld, int r0, int c0, int c, int h) {
-  const unsigned vo = (c * ld + 4 * h) * 4;
-#pragma unroll
-  for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-    for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; g4++) {
-        const f32x4 x = g_ld4f(g, vo, off + ((r0 + 32 * cb) * ld + c0 + 32 * rb + 8 * g4) * 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++) a.b[rb][cb][4 * g4 + e] = x[e];
-      }
-}
-
 // ------------------------------------------------------------------ LayerNorm-lane helpers
 // A lane of a LayerNorm stage owns token `tok` and the 8 features f0 .. f0+7.
 TTT_DEV void ln_load(float (&x)[8], const bf16* p) {      // p 8-byte aligned
@@ -362,7 +347,7 @@ TTT_DEV void stage3_store(const Staged3& s, bf16* sa, bf16* sb, bf16* sc, bf16* 
 
 // Piece s of W2[shard] before mini-batch j of the group as an operand (lane = hid row, contraction =
 // F): the image the replay stored after mini-batch j-1, or straight from the fp32 checkpoint.
-// STREAM: the caller reads the image once (the grad_L_XK workgroup), so it need not stay in the L2.
+// STREAM: the second and last read of the image on this CU, so it need not stay in the L2.
 template <bool STREAM = false>
 TTT_DEV bf16x8 w2_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int s, int hid0, int c, int h, unsigned t16) {
   // the image offset is clamped so that the load stays inside the buffer even if it is hoisted above the branch
@@ -371,9 +356,8 @@ TTT_DEV bf16x8 w2_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int s, i
   return r;
 }
 // Piece (row block rb, k-step s) of W1[:, shard]^T before mini-batch j (lane = F row, contraction = hid).
-template <bool STREAM = false>
 TTT_DEV bf16x8 w1_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int rb, int s, int hid0, int c, int h, unsigned t16) {
-  bf16x8 r = image_load<STREAM>(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, 2 * rb + s, t16);
+  bf16x8 r = image_load<false>(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, 2 * rb + s, t16);
   if (j == 0) r = piece_from_f32(ck, ck_off, HID, 32 * rb, hid0, s, c, h);
   return r;
 }
@@ -1122,7 +1106,10 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     }
     if constexpr (ROLE != 1) WALK_FETCH(n_mb - 1);
     if constexpr (ROLE != 1)
-    for (int j = n_mb - 1; j >= 0; j--) {
+    for (int jj = n_mb - 1; jj >= 0; jj--) {
+      // (in a scalar register: left to itself the compiler keeps sums of the images' offsets in vector registers over the whole
+      // mini-batch and spills them, up to 14 reloads, each of which waits for every load under way; 51 pairs x 77: 1.60 ms)
+      const int j = ROLE == 2 ? __builtin_amdgcn_readfirstlane(jj) : jj;
       const int mb = k * cgs + j;
       REFRESH_OFFSETS();
       LANE_VARS;
@@ -1180,13 +1167,6 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       // gb2 holds its value after the first update
 
       TTT_STAGE(BS_W_BAR_TERMS);
-      // How far the walk is, for the workgroup that fetches ahead of it: said here, a quarter into the mini-batch, so
-      // that the next mini-batch's lines reach the L2 in time for the first of them (requested during this
-      // mini-batch's updates) and stay there no longer than needed (said at the top: c4 backward +0.3 ms; two stages
-      // further on: +1.9 ms, the lines come too late).
-      if constexpr (ROLE == 2 && FIN) {
-        if (threadIdx.x == 0) __hip_atomic_store(w_sync + 20, p.NC - mb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
       // ---- the weight step, backwards (uses the state BEFORE this mini-batch).
       //      Parked across the LayerNorm stage: X2 in T0; packed d1 = gelu'(Z1), g1 = -eta * dl/dZ1 and
       //      t2 = -eta * (gZ2 W2^T) * (XK gW1 + gb1) * gelu''(Z1).
@@ -1833,71 +1813,13 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
 #undef FIN_LANE
 
 #ifndef TTT_BWD_ROLES_ONLY
-// ------------------------------------------------------------------ the workgroup that fetches ahead of the walk
-// The walk asks per mini-batch for 240 KiB that a replaying workgroup wrote a checkpoint group earlier (six register
-// images, four tiles) or that the caller passed in (two tiles): none of it is in the L2 by then, and one CU cannot
-// keep enough requests in flight to hide the way to HBM.  This workgroup computes nothing: it goes through the walk's
-// mini-batches in the walk's order, PREFETCH_AHEAD of them ahead of it, and reads one dword of every 128-byte line
-// the walk will ask for.  Placed on the walk's XCD, it leaves the lines in the L2 that the walk's requests go to.
-// Purely a hint: the values are dropped, nothing is written except the status word of a wait that gives up, and
-// the walk's results do not depend on whether, when or where this workgroup runs.
-constexpr int PREFETCH_AHEAD = 1;
-TTT_DEV void bwd_prefetch(const BwdParams& p, unsigned char* smem, const int bh) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int v = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cgs = p.cgs, n_replay = p.n_replay, n_sets = 2 * n_replay;
-  int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
-  int* const w_step = w_sync + 20;
-  int* const s_flag = reinterpret_cast<int*>(smem + SB_FLAG);
-  const size_t ox = uni64((size_t)bh * p.NC * (CS * FD)), of = uni64((size_t)bh * cgs * (CS * FD));
-  const size_t oh = uni64((size_t)bh * cgs * (CS * HID)), opk = uni64((size_t)bh * cgs * (FD * HID));
-  const unsigned line_t = 128u * lane, line_i = 128u * (tid & 255);   // this thread's line of a tile / of an image
-  int n = 0;   // mini-batches the walk has before the one at hand
-  for (int k = p.K - 1; k >= 0; k--) {
-    const int n_mb = min(cgs, p.NC - k * cgs);
-    const int done = p.K - 1 - k, set = done % n_sets;
-    // the group has been replayed: what is fetched is what the walk will read
-    if (!wait_at_least(w_sync + 8 * (done % n_replay), done / n_replay + 1, p.status, s_flag, p.wait_limit)) return;
-#define PGRP(name) (set ? p.alt_##name[set - 1] : p.name)
-    // wave v fetches tile v (v < 6): the two inputs (indexed by the mini-batch's place in the sequence), then four of the set
-    gptr_t tile = gbuf(p.XQ + ox);
-    unsigned tile0 = k * cgs * TILE_BYTES;
-    if (v == 1) tile = gbuf(p.XK + ox);
-    if (v >= 2) tile0 = 0;
-    if (v == 2) tile = gbuf(PGRP(grad_l_wrt_Z2_group) + of);
-    if (v == 3) tile = gbuf(PGRP(grad_x_hat_fused_group) + of);
-    if (v == 4) tile = gbuf(PGRP(x_hat_fused_group) + of);
-    if (v >= 5) tile = gbuf(PGRP(grad_output_fused_group) + of);
-    // and half of three of the six images: waves 0-3 X2_bar, GELU, GELU''; waves 4-7 gZ1_bar, GELU', W2 before the step
-    const bool up = v >= 4;
-    const gptr_t img0 = up ? gbuf(PGRP(Z1_bar_group) + oh) : gbuf(PGRP(X2_bar_group) + oh);
-    const gptr_t img1 = up ? gbuf(PGRP(W1_init_group) + opk) : gbuf(PGRP(Z1_group) + oh);
-    const gptr_t img2 = up ? gbuf(PGRP(grad_l_wrt_Z1_group) + oh) : gbuf(PGRP(W1_init_group) + opk);
-#undef PGRP
-    for (int j = n_mb - 1; j >= 0; j--, n++) {
-      const int seen = wait_for_pace(w_step, n + 1 - PREFETCH_AHEAD, p.status, s_flag, p.wait_limit);
-      if (seen == 0) return;
-      if (seen - 1 > n + 1) continue;   // the walk is past this mini-batch already
-      const unsigned ho = j * IMG_BYTES;
-      unsigned got[4] = {0, 0, 0, 0};
-      if (v < 6) got[0] = g_ld<unsigned>(tile, line_t, tile0 + j * TILE_BYTES);
-      got[1] = g_ld<unsigned>(img0, line_i, ho);
-      got[2] = g_ld<unsigned>(img1, line_i, up ? 2 * ho : ho);
-      if (!up) got[3] = g_ld<unsigned>(img2, line_i, 2 * ho + IMG_BYTES);
-      else if (j > 0) got[3] = g_ld<unsigned>(img2, line_i, ho - IMG_BYTES);
-#pragma unroll
-      for (int i = 0; i < 4; i++) asm volatile("" ::"v"(got[i]));   // landed; nothing is done with them
-    }
-  }
-}
-
 // n_replay + 1 (+ 1) workgroups per (batch, head).  Workgroups are dealt to the 8 XCDs in turn, so with a
 // multiple of 8 (batch, head) pairs the workgroups of a pair are placed 8 apart: same XCD, same L2.
 // One kernel per combination, so that each holds only the code (and the register allocation) of its own roles.
 template <int NREPLAY, bool FINISH>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_split_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int b = blockIdx.x, per = NREPLAY + 1 + (FINISH ? 1 + p.n_prefetch : 0);
+  const int b = blockIdx.x, per = NREPLAY + 1 + (FINISH ? 1 : 0);
   int bh, role;
   if (p.nbh % 8 == 0) {
     bh = (b / (8 * per)) * 8 + (b & 7);
@@ -1910,10 +1832,7 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_split_kernel(const Bwd
   constexpr bool IMG = NREPLAY == 2;   // two replaying workgroups also evaluate the GELU family for the walk
   if (role < NREPLAY) bwd_body<1, IMG, FINISH>(p, smem, bh, role, p.K - 1, 0);
   else if (role == NREPLAY) bwd_body<2, IMG, FINISH>(p, smem, bh, 0, p.K - 1, 0);
-  else if constexpr (FINISH) {
-    if (role == NREPLAY + 1) bwd_finish_dxk<true, false>(p, smem, bh);
-    else bwd_prefetch(p, smem, bh);
-  }
+  else if constexpr (FINISH) bwd_finish_dxk<true, false>(p, smem, bh);
 }
 
 __global__ void ttt_mlp_zero_words(int* w, int n) {
@@ -1937,7 +1856,7 @@ hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
   hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n);
-  const dim3 grid((p.n_replay + 1 + p.n_finish + p.n_prefetch) * p.nbh), block(ttt::BW_THREADS);
+  const dim3 grid((p.n_replay + 1 + p.n_finish) * p.nbh), block(ttt::BW_THREADS);
   auto launch = [&](auto kernel) -> hipError_t {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
     if (err != hipSuccess) return err;

@@ -158,7 +158,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       }
     };
     // Operands are asked for one to two stages ahead.  One CU cannot keep enough requests in flight to hide the way to HBM (80 KiB
-    // asked for in a row take 9 k clocks to issue), so another workgroup brings the lines into the L2 before (bwd_wide_prefetch);
+    // asked for in a row take 9 k clocks to issue), so another workgroup brings the lines into the L2 before (bwd_wide_prefetch, with three or four replaying ones);
     // what the grad_L_XK workgroup reads next is left there.
     auto ask_bar = [&](int j) {
       WW_LANE;
@@ -710,8 +710,13 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
 #undef WW_LANE
 }
 
-// The workgroup that reads ahead of the walk (see bwd_prefetch in ttt_mlp_bwd.hip): one dword of every 128-byte line that the
-// walk and the grad_L_XK workgroup will ask for, two mini-batches ahead of the walk, which asks for most of it one ahead.
+// The workgroup that reads ahead of the walk.  The walk asks per mini-batch for 240 KiB that a replaying workgroup wrote a
+// checkpoint group earlier or that the caller passed in: none of it is in the L2 by then, and a CU whose registers and LDS are
+// full cannot keep enough requests in flight to hide the way to HBM.  This one computes nothing: it reads one dword of every
+// 128-byte line that the walk and the grad_L_XK workgroup will ask for, two mini-batches ahead of the walk, which asks for
+// most of it one ahead.  On the walk's XCD it leaves the lines in the L2 that the walk's requests go to.  Purely a hint: the
+// values are dropped, nothing is written except the status word of a wait that gives up, and the results do not depend on
+// whether, when or where this workgroup runs.
 constexpr int BWW_AHEAD = 2;
 TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const int bh) {
   const int tid = threadIdx.x, lane = tid & 63;

@@ -157,7 +157,7 @@ struct LaunchPlan {
   int n_out = 0;            // forward, wide: that compute Out
   int n_replay = 0;         // backward: that replay checkpoint groups
   bool finish = false;      // backward: one more for grad_L_XK / grad_L_XV
-  bool prefetch = false;    // backward: and one that fetches ahead of the walk
+  bool prefetch = false;    // backward, wide: and one that fetches ahead of the walk
 };
 LaunchPlan plan_for(long long BH, int cus, bool backward) {
   LaunchPlan pl;
@@ -195,9 +195,7 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
   }
   pl.finish = 4 * pl.n_rest <= cus;
   pl.n_replay = 3 * pl.n_rest <= cus ? 2 : 1;
-  // the fetching workgroup helps only from the walk's own XCD, which the kernel arranges for a multiple of 8 pairs
-  pl.prefetch = pl.finish && 5 * pl.n_rest <= cus && pl.n_rest % 8 == 0;
-  pl.per_pair = 1 + pl.n_replay + (pl.finish ? 1 : 0) + (pl.prefetch ? 1 : 0);
+  pl.per_pair = 1 + pl.n_replay + (pl.finish ? 1 : 0);
   return pl;
 }
 int device_cus() {

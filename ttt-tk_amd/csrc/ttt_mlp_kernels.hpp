@@ -82,14 +82,14 @@ struct BwdParams {
   __bf16* fin_dz;
   float* fin_gy;
   int n_finish;
-  // n_prefetch = 1 (with n_finish = 1 only): one more workgroup reads nothing for itself; it touches every cache
-  // line that the walk is about to ask for, one mini-batch ahead of it, so that the walk's own requests are
-  // answered by the L2 the two share instead of by HBM.
-  int n_prefetch;
   // Walk on two workgroups (ttt_mlp_bwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
-  // 256 8-byte words]; n_replay = 2 .. 4 and n_sets sets of the per-group tensors; n_finish = 1, n_prefetch = 0.
+  // 256 8-byte words]; n_replay = 2 .. 4 and n_sets sets of the per-group tensors; n_finish = 1.
+  // n_prefetch = 1 (with three or four replaying workgroups): one more workgroup reads nothing for itself; it touches every
+  // cache line that the walk is about to ask for, ahead of it, so that the walk's own requests are answered by the L2 the
+  // two share instead of by HBM.
   unsigned long long* xchg;
   int n_sets;
+  int n_prefetch;
   int* sync;
   int* status;    // the status word behind the synchronisation words
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
@@ -106,10 +106,9 @@ struct BwdParams {
 };
 
 // Layout of `sync` (ints): 32 per (batch, head) - words 0 and 8 count the groups replayed by the first /
-// second replaying workgroup (norm_partial is written before the last count), word 16 the groups the
+// second replaying workgroup (norm_partial is written with the group), word 16 the groups the
 // reverse walk has finished, word 12 the mini-batches of the last group it walks that it has handed to the grad_L_XK
-// workgroup (that group is handed over in chunks), word 20 the mini-batches it has started (a pacing hint for the prefetching workgroup,
-// no data is ordered by it), word 24 the groups the grad_L_XK workgroup has finished - then one status
+// workgroup (that group is handed over in chunks), word 24 the groups the grad_L_XK workgroup has finished - then one status
 // word (non-zero: a wait gave up).
 constexpr int BWD_SYNC_STRIDE = 32;
 // With the walk on two workgroups: words 0 .. 3 groups replayed by each replaying workgroup, BWW_WALKED + 0 / 4 groups and

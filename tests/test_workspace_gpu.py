@@ -101,3 +101,67 @@ def test_compute_unit_budget_turns_the_waiting_launches_off():
             assert torch.equal(got[k], r), k
     finally:
         ext.set_compute_units(0)
+
+
+@pytest.mark.parametrize("NH,NC,cgs", [(8, 3, 4), (8, 7, 4), (3, 9, 4), (8, 48, 4), (40, 5, 4), (8, 5, 1)])
+def test_short_sequences_and_small_workspaces(NH, NC, cgs):
+    """One set of per-group tensors per checkpoint group is enough for a short sequence (K groups, the caller's own set among
+    them), and a workspace too small for three or four recomputing workgroups still serves two; results do not change."""
+    import ctypes
+    import os
+    import test_time_training as ext
+    import ttt_mlp_host as host
+    from test_overlapped_abi_gpu import LIB, _args
+    lib = ctypes.CDLL(LIB)
+    lib.ttt_mlp_bwd_workspace_bytes.restype = ctypes.c_size_t
+    dev = torch.device("cuda:0")
+    B, K = 1, host.num_checkpoints(NC, cgs)
+    print(f"case B={B} NH={NH} NC={NC} cgs={cgs} K={K}", flush=True)
+    d = orc.make_inputs(B, NH, NC, seed=7)
+    t = {k: d[k].to(dev).contiguous() for k in FWD_KEYS + UP_KEYS}
+    t.update(host.alloc_forward_buffers(B, NH, NC, cgs, dev))
+    t.update(host.alloc_backward_buffers(B, NH, NC, cgs, dev))
+    ext.set_overlap(False)
+    try:
+        ref = _run(host, t, cgs)
+    finally:
+        ext.set_overlap(True)
+    least, most = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.ttt_mlp_bwd_workspace_range(B, NH, cgs, K, ctypes.byref(least), ctypes.byref(most)) == 0
+    full = lib.ttt_mlp_bwd_workspace_bytes(B, NH, cgs)
+    sets = 6 if NH <= 32 else 4
+    per_set = NH * cgs * (7 * 32768 + 4 * 8192 + 256)      # seven images, four tiles, a vector per slot
+    assert full - most.value == max(0, sets - K) * per_set
+    assert most.value - least.value == (min(sets, K) - min(4, K)) * per_set
+    ba = _args(host.BWD_ORDER, t, cgs, B, NH, NC, K)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for nbytes in (most.value, least.value):
+        host.zero_accumulating_grads(t)
+        for k in host.GRAD_NAMES[:6]:
+            t[k].fill_(7.0)
+        ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=dev)
+        assert lib.ttt_mlp_bwd_launch_within(ctypes.byref(ba), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(least.value - 1), stream) == 1006
+        assert lib.ttt_mlp_bwd_launch_within(ctypes.byref(ba), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(nbytes), stream) == 0
+        torch.cuda.synchronize()
+        for k in host.GRAD_NAMES:
+            assert torch.equal(t[k], ref[k]), (nbytes, k)
+    # the operator: what it allocates, and what it does with a caller's tensor of either size
+    if K >= 2:
+        del ws
+        host.zero_accumulating_grads(t)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated(dev)
+        torch.cuda.reset_peak_memory_stats(dev)
+        host.backward(t, cgs)
+        assert ext.last_backward_mode() == 1
+        assert torch.cuda.max_memory_allocated(dev) - before <= most.value + 512
+        try:
+            for nbytes, mode in ((least.value, 1), (least.value - 1, 0)):
+                host.set_workspace(torch.empty(nbytes, dtype=torch.uint8, device=dev))
+                host.zero_accumulating_grads(t)
+                host.backward(t, cgs)
+                assert ext.last_backward_mode() == mode
+                for k in host.GRAD_NAMES:
+                    assert torch.equal(t[k], ref[k]), (nbytes, k)
+        finally:
+            host.set_workspace(None)

@@ -8,7 +8,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
-#include "../../include/ttt_mlp.h"
+#include "ttt_mlp_operator.h"
 
 namespace {
 
@@ -277,13 +277,15 @@ torch::Tensor ttt_backward(
   // With few (batch, head) pairs most CUs would idle: then a second workgroup per pair recomputes the
   // checkpoint groups ahead of the reverse walk.  Its workspace (further sets of the per-group tensors): the
   // caller's (set_workspace) or torch's caching allocator's.
-  const size_t ws_bytes = (g_overlap && K >= 2 && !sequences_cut(1, B * NH, NC, checkpoint_group_size))
-                              ? ttt_mlp_bwd_workspace_bytes((int32_t)B, (int32_t)NH, checkpoint_group_size) : 0;
-  const Workspace ws = take_workspace(ws_bytes, XQ.device());
+  size_t least = 0, ws_bytes = 0;
+  if (g_overlap && K >= 2 && !sequences_cut(1, B * NH, NC, checkpoint_group_size))
+    (void)ttt_mlp_bwd_workspace_range((int32_t)B, (int32_t)NH, checkpoint_group_size, (int32_t)K, &least, &ws_bytes);
+  Workspace ws = take_workspace(ws_bytes, XQ.device());
+  if (ws.ptr == nullptr && least < ws_bytes) ws = take_workspace(ws_bytes = least, XQ.device());   // fewer sets before one workgroup per pair
   if (ws.ptr != nullptr) {
     g_last_backward_mode = 1;
     const char* status = static_cast<const char*>(ws.ptr) + ttt_mlp_bwd_status_offset((int32_t)B, (int32_t)NH);
-    int rc = ttt_mlp_bwd_launch_overlapped(&a, ws.ptr, ws_bytes, stream);
+    int rc = ttt_mlp_bwd_launch_within(&a, ws.ptr, ws_bytes, stream);
     if (rc == 0 && g_fill_group_tensors) rc = ttt_mlp_bwd_export_group0(&a, stream);
     finish(rc, stream, "ttt_backward", XQ.device(), status);
   } else {
@@ -344,7 +346,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           return (unsigned long long)(f > b ? f : b);
         },
         "Bytes of workspace that let ttt_forward and ttt_backward of this shape use several workgroups per (batch, head) "
-        "(0: the shape runs with one workgroup per pair and needs none).");
+        "(0: the shape runs with one workgroup per pair and needs none).  Serves every sequence length; a backward over fewer "
+        "checkpoint groups takes less of it, and with less than it the backward recomputes with fewer workgroups first.");
   m.def("set_workspace", [](c10::optional<torch::Tensor> ws) {
           if (!ws.has_value()) { delete g_workspace; g_workspace = nullptr; return; }
           TORCH_CHECK(ws->device().is_cuda() && ws->is_contiguous() && ws->scalar_type() == torch::kUInt8 && ws->dim() == 1,
@@ -356,8 +359,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         },
         "Hand the operators a workspace (1-D uint8 GPU tensor of at least workspace_bytes(...) bytes) that they use for "
         "every later call instead of allocating one: with it ttt_forward / ttt_backward allocate nothing and do not query "
-        "the device's free memory; a call whose shape needs more than the tensor holds, or that runs on another device, "
-        "uses one workgroup per (batch, head).  The contents are scratch; calls that overlap in time must not share it.  "
+        "the device's free memory; a backward that does not fit the tensor recomputes with fewer workgroups if that does, and a "
+        "call that still needs more than it holds, or that runs on another device, uses one workgroup per (batch, head).  The contents are scratch; calls that overlap in time must not share it.  "
         "None returns to the default (workspace from torch's caching allocator per call).");
   m.def("set_compute_units", [](int n) { ttt_mlp_set_compute_units(n); },
         "CUs the multi-workgroup launches may count on (their workgroups wait for each other and must all be resident): "

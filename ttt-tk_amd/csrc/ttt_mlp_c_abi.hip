@@ -2,7 +2,7 @@
 // one asynchronous kernel launch.  Nothing here allocates or synchronises.
 #include <atomic>
 
-#include "../../include/ttt_mlp.h"
+#include "ttt_mlp_operator.h"
 #include "ttt_mlp_kernels.hpp"
 
 namespace {
@@ -282,17 +282,34 @@ SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, in
   return plan_segments(pairs, cus, NC, cgs, uncut_x1000(pl, pairs, cus, NC, with_workspace, true));
 }
 
-// Workspace of the backward with 2 or 3 workgroups per pair, for n (batch, head) pairs: the synchronisation
-// words, the replay's shares of the norm gradients (two sums per pair + one parking slot), then 1 or 3
-// alternate sets of the ten per-group tensors that carry a replayed group to the reverse walk; each part
-// 256-byte aligned.
+// Sets of the per-group tensors that carry replayed groups to the walk, used in turn: two per replaying workgroup, or one each
+// and two more where four of them run ahead of a walk on two CUs.  Set 0 is the caller's own; a sequence of K groups uses K.
+int bwd_sets(const LaunchPlan& pl) { return pl.wide ? pl.n_replay + 2 : 2 * pl.n_replay; }
+int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K < bwd_sets(pl) ? K : bwd_sets(pl)); }
+// The launch with less workspace for the same pairs: two replaying workgroups instead of three or four.
+LaunchPlan bwd_reduced(LaunchPlan pl) {
+  if (pl.wide && pl.n_replay > 2) {
+    pl.n_replay = 2;
+    pl.prefetch = false;
+    pl.per_pair = 5;
+  }
+  return pl;
+}
+// Workspace of the backward with several workgroups per pair, for n (batch, head) pairs of K groups: the synchronisation
+// words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
+// CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
+// gradient terms, per slot, two sets), then the sets of per-group tensors beyond the caller's; each part 256-byte aligned.
 struct BwdWorkspace {
   static constexpr int PER_SET = 11;
   static constexpr int ALT_SETS = ttt::BWD_MAX_SETS - 1;
-  static constexpr int PARTS = 8 + PER_SET * ALT_SETS;
+  static constexpr int FIRST_SET = 7;
+  static constexpr int PARTS = FIRST_SET + PER_SET * ALT_SETS;
   size_t off[PARTS];
   size_t total;
-  BwdWorkspace(long long n, long long cgs, int alt_sets, bool finish, bool wide) {
+  int alt_sets;
+  BwdWorkspace(const LaunchPlan& pl, long long cgs, long long K) {
+    const long long n = pl.n_rest;
+    alt_sets = bwd_sets_used(pl, K) - 1;
     const size_t slot = (size_t)n * (size_t)cgs;
     const size_t tile = TTT_MLP_CS * TTT_MLP_F * 2, img = TTT_MLP_CS * TTT_MLP_HID * 2, vec = TTT_MLP_CS * 4;
     const size_t norm = (size_t)n * 8 * 2 * TTT_MLP_F * sizeof(float);
@@ -306,19 +323,14 @@ struct BwdWorkspace {
     put(1, ttt::BWD_MAX_SETS * norm);
     put(2, norm);
     put(3, (size_t)n * img);
-    // hand-over to the grad_L_XK workgroup: one image (dZ1) and two fp32 tiles (g_y, norm-weight gradient terms) per slot, two sets
-    put(4, wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);   // walk on two workgroups: what they exchange
-    put(5, 0);
-    put(6, finish ? 2 * slot * img : 0);
-    put(7, finish ? 2 * slot * 4 * tile : 0);
+    put(4, pl.wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);
+    put(5, pl.finish ? 2 * slot * img : 0);
+    put(6, pl.finish ? 2 * slot * 4 * tile : 0);
     for (int s = 0; s < ALT_SETS; s++)
-      for (int t = 0; t < PER_SET; t++) put(8 + PER_SET * s + t, s < alt_sets ? per_set[t] : 0);
+      for (int t = 0; t < PER_SET; t++) put(FIRST_SET + PER_SET * s + t, s < alt_sets ? per_set[t] : 0);
     total = o;
   }
 };
-
-// Sets of the per-group tensors that carry replayed groups to the walk.
-int bwd_sets(const LaunchPlan& pl) { return pl.wide ? pl.n_replay + 2 : 2 * pl.n_replay; }
 
 // Workspace of the forward's two-workgroup mode: synchronisation words, then per (batch, head) a ring of
 // 2 * FWD_RING_MAX slots of state images and of bias vectors.
@@ -370,7 +382,16 @@ extern "C" int ttt_mlp_bwd_export_group0(const ttt_mlp_bwd_args* a, void* stream
 extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_group_size) {
   if (B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16)) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
-  return pl.rest_split ? BwdWorkspace(pl.n_rest, checkpoint_group_size, bwd_sets(pl) - 1, pl.finish, pl.wide).total : 0;
+  return pl.rest_split ? BwdWorkspace(pl, checkpoint_group_size, ttt::BWD_MAX_SETS).total : 0;
+}
+
+extern "C" int ttt_mlp_bwd_workspace_range(int B, int NH, int checkpoint_group_size, int K, size_t* least, size_t* most) {
+  if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || K <= 0)
+    return TTT_MLP_ERR_BAD_ARG;
+  const LaunchPlan pl = plan_launches((long long)B * NH, true);
+  *least = pl.rest_split ? BwdWorkspace(bwd_reduced(pl), checkpoint_group_size, K).total : 0;
+  *most = pl.rest_split ? BwdWorkspace(pl, checkpoint_group_size, K).total : 0;
+  return TTT_MLP_OK;
 }
 
 extern "C" size_t ttt_mlp_bwd_status_offset(int B, int NH) {
@@ -385,8 +406,18 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const int alt_sets = bwd_sets(pl) - 1;
-  const BwdWorkspace w(pl.n_rest, p.cgs, alt_sets, pl.finish, pl.wide);
+  if (workspace_bytes < BwdWorkspace(pl, p.cgs, ttt::BWD_MAX_SETS).total) return TTT_MLP_ERR_WORKSPACE;
+  return ttt_mlp_bwd_launch_within(a, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  ttt::BwdParams p;
+  if (int rc = make_bwd_params(a, p)) return rc;
+  if (int rc = check_workspace(workspace)) return rc;
+  LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
+  if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
+  if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
+  const BwdWorkspace w(pl, p.cgs, p.K);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   {
@@ -418,8 +449,8 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   p.n_prefetch = pl.prefetch ? 1 : 0;
   p.wait_limit = g_wait_limit;
   if (pl.finish) {
-    p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[6]) - b0 * 2 * img;
-    p.fin_gy = reinterpret_cast<float*>(base + w.off[7]) - b0 * 2 * 2 * tile;
+    p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[5]) - b0 * 2 * img;
+    p.fin_gy = reinterpret_cast<float*>(base + w.off[6]) - b0 * 2 * 2 * tile;
   }
   int* words = reinterpret_cast<int*>(base + w.off[0]);
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
@@ -427,8 +458,18 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * ttt::BWD_MAX_SETS * norm;
   p.norm_park = reinterpret_cast<float*>(base + w.off[2]) - b0 * norm;
   p.walk_park = reinterpret_cast<__bf16*>(base + w.off[3]) - b0 * (TTT_MLP_CS * TTT_MLP_HID);
-  for (int s = 0; s < alt_sets; s++) {
-    const size_t* o = w.off + 8 + BwdWorkspace::PER_SET * s;
+  // (sets that a sequence this short does not come to: the walk asks for operands of the group behind its last one and drops
+  // them, so their pointers are the caller's own tensors)
+  for (int s = w.alt_sets; s < ttt::BWD_MAX_SETS - 1; s++) {
+    p.alt_X2_group[s] = p.X2_group; p.alt_Z1_group[s] = p.Z1_group;
+    p.alt_Z1_bar_group[s] = p.Z1_bar_group; p.alt_X2_bar_group[s] = p.X2_bar_group;
+    p.alt_grad_l_wrt_Z2_group[s] = p.grad_l_wrt_Z2_group; p.alt_grad_l_wrt_Z1_group[s] = p.grad_l_wrt_Z1_group;
+    p.alt_x_hat_fused_group[s] = p.x_hat_fused_group; p.alt_grad_x_hat_fused_group[s] = p.grad_x_hat_fused_group;
+    p.alt_grad_output_fused_group[s] = p.grad_output_fused_group; p.alt_std_fused_group[s] = p.std_fused_group;
+    p.alt_W1_init_group[s] = p.W1_init_group;
+  }
+  for (int s = 0; s < w.alt_sets; s++) {
+    const size_t* o = w.off + BwdWorkspace::FIRST_SET + BwdWorkspace::PER_SET * s;
     p.alt_X2_group[s] = reinterpret_cast<__bf16*>(base + o[0]) - b0 * img;
     p.alt_Z1_group[s] = reinterpret_cast<__bf16*>(base + o[1]) - b0 * img;
     p.alt_Z1_bar_group[s] = reinterpret_cast<__bf16*>(base + o[2]) - b0 * img;

@@ -587,7 +587,9 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       const int kn = j > 0 ? k : k - 1, jn = j > 0 ? j - 1 : cgs - 1;
       // gradient wrt b2: what the output branch adds
       if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_gzb, u, s, lane); }, ones, c, h);
-      if (more && !gave_up) ask(kn, jn);
+      // (everybody is still here, so the flag reads 0; read at this place it holds these loads back until the sums above are
+      // through, 0.729 instead of 0.732 ms for 24 pairs x 64 mini-batches)
+      if (more && flag(0) == 0) ask(kn, jn);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // g_y of the last mini-batch and the marks put back are in place
       TTT_STAGE(BWH_ASK);
       __syncthreads();   // B1

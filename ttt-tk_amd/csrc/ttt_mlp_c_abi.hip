@@ -211,7 +211,7 @@ LaunchPlan plan_launches(long long BH, bool backward) { return plan_for(BH, devi
 // boundaries instead - a segment starts from the checkpoint before its first mini-batch, which the segment before it
 // left in the caller's checkpoint tensors - and launch the (segment, pair) jobs segment-major, one launch per `cus`
 // jobs: a pair's earlier segment is always in an earlier launch (pairs >= cus), and the rounds are a fraction of a
-// sequence long, so 384 pairs on 256 CUs take 3 launches of half a sequence, 1.5 sequences instead of 2 (or 1.76 with
+// sequence long, so 384 pairs on 256 CUs take 3 launches of half a sequence, 1.5 sequences instead of 2 (or 1.7 with
 // the last 128 pairs on two workgroups each).  Same arithmetic on the same state: results do not change.
 struct SegmentPlan {
   int seg_len = 0;      // mini-batches per segment, a multiple of cgs; 0 = sequences are not cut
@@ -219,20 +219,19 @@ struct SegmentPlan {
   int launches = 1;
   long long jobs = 0;
 };
-#ifndef TTT_CUT_PERCENT
-#define TTT_CUT_PERCENT 99   // a cut must gain 1 % by the estimate below
-#endif
 // `alt_x1000`: what the alternative costs, in thousandths of a mini-batch of one workgroup.
 SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long alt_x1000) {
   SegmentPlan best;
 #ifndef TTT_STAGE_CLOCKS   // the stage clocks are kept per pair and sequence
   if (pairs <= cus || pairs > (1 << 27) || cus <= 0 || NC <= 0 || cgs <= 0) return best;   // (job numbers are ints)
   const int K = (NC + cgs - 1) / cgs;
-  long long best_t = alt_x1000 * TTT_CUT_PERCENT / 100;
+  long long best_t = alt_x1000;
   for (int S = 2; S <= 8 && S <= K; S++) {
     const int groups = (K + S - 1) / S, segs = (K + groups - 1) / groups;
     const long long len = (long long)groups * cgs, jobs = segs * pairs, launches = (jobs + cus - 1) / cus;
-    const long long t = launches * (len * 1000 + 2000);   // + 2 mini-batches' worth per launch: gaps, state in and out
+    // + a mini-batch's worth per launch: gaps, state in and out (5 launches of 128 mini-batches, 320 pairs: 29.4 ms against 31.3
+    // uncut; 11 of 64, 352 pairs: 32.4 against 33.9; 3 of 256, 384 pairs: 35.1 against 34.8)
+    const long long t = launches * (len * 1000 + 1000);
     if (t < best_t) {
       best_t = t;
       best.seg_len = static_cast<int>(len);
@@ -245,15 +244,18 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long a
   return best;
 }
 // Thousandths of a one-workgroup mini-batch that the pairs take uncut: full rounds, and the rest either one more
-// round or, with several workgroups per pair, a shorter one - measured with every CU busy: the forward's recurrence
-// workgroup runs at 0.755 of one workgroup's time per mini-batch; the backward's walk with one replaying workgroup
-// at 0.56, and about 0.4 / 0.3 with more workgroups per pair.
-long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, bool with_workspace, bool backward) {
+// round or, with several workgroups per pair, a shorter one.  Measured on 256 CUs as what the rest adds to a full round
+// (6.5 ms forward, 23.1 ms backward for 512 mini-batches), at the most pairs of a shape: forward 530 (4 pairs, 430 for 64), 550
+// (80), 710 (128).  The backward's walk waits for the first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at
+// K = 16, 320 at 4; 48 pairs 265 and 335, 64 pairs 350 and 435, 80 pairs 435 and 515, 128 pairs 500 and 605.
+long long rest_x1000(const LaunchPlan& pl, int K, bool backward) {
+  if (!backward) return pl.n_out == 2 ? 530 : pl.n_out == 1 ? 550 : 710;
+  const int walk = pl.wide ? (pl.n_replay > 2 ? 210 : 235) : pl.finish ? 325 : pl.n_replay == 2 ? 405 : 485;
+  return walk + 470 / K;
+}
+long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace, bool backward) {
   if (cus <= 0) return (long long)NC * 1000;
-  if (with_workspace && pl.rest_split) {
-    const int rest = !backward ? 755 : pl.n_replay == 1 ? 560 : !pl.finish ? 400 : 300;
-    return (pl.n_single / cus * 1000 + rest) * NC;
-  }
+  if (with_workspace && pl.rest_split) return (pl.n_single / cus * 1000 + rest_x1000(pl, (NC + cgs - 1) / cgs, backward)) * NC;
   return (pairs + cus - 1) / cus * 1000 * NC;
 }
 // The launches of a call with the sequences cut: `cus` jobs each, in job order, on the one stream.
@@ -279,7 +281,7 @@ int launch_bwd_segments(ttt::BwdParams p, const SegmentPlan& plan, int cus, hipS
 }
 SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace) {
   if (cgs < 2) return SegmentPlan{};
-  return plan_segments(pairs, cus, NC, cgs, uncut_x1000(pl, pairs, cus, NC, with_workspace, true));
+  return plan_segments(pairs, cus, NC, cgs, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, true));
 }
 
 // Sets of the per-group tensors that carry replayed groups to the walk, used in turn: two per replaying workgroup, or one each
@@ -494,7 +496,7 @@ extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
   if (int rc = make_fwd_params(a, p)) return rc;
   const long long pairs = (long long)p.B * p.NH;
   const int cus = device_cus();
-  const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(LaunchPlan{}, pairs, cus, p.NC, false, false));
+  const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(LaunchPlan{}, pairs, cus, p.NC, p.cgs, false, false));
   if (seg.seg_len > 0) return launch_fwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
   p.bh0 = 0;
   p.nbh = p.B * p.NH;
@@ -527,7 +529,7 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
     // workspace then only has its words cleared (callers read the status word behind them)
     const long long pairs = (long long)p.B * p.NH;
     const int cus = device_cus();
-    const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(pl, pairs, cus, p.NC, true, false));
+    const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(pl, pairs, cus, p.NC, p.cgs, true, false));
     if (seg.seg_len > 0) {
       if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_rest)),
                                                  static_cast<hipStream_t>(stream)))
@@ -652,7 +654,7 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
   const LaunchPlan pl = plan_for(pairs, compute_units, which == 1);
   const SegmentPlan seg = which == 1 ? plan_bwd_segments(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0)
                                      : plan_segments(pairs, compute_units, NC, checkpoint_group_size,
-                                                     uncut_x1000(pl, pairs, compute_units, NC, with_workspace != 0, false));
+                                                     uncut_x1000(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0, false));
   *segment_minibatches = seg.seg_len;
   *launches = seg.seg_len > 0 ? seg.launches : (with_workspace != 0 && pl.rest_split && pl.n_single > 0 ? 2 : 1);
   return TTT_MLP_OK;

@@ -245,7 +245,7 @@ int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long
  * where that shortens the call: a forward segment starts from the checkpoint that the segment before it left in
  * the caller's checkpoint tensors; a backward segment (the sequence's last groups first) takes the running
  * gradients from grad_L_W1/b1/W2/b2_init, where the one before it left them, and the norm-gradient sums from
- * x_hat_ln_group (needs checkpoint_group_size >= 2).  The (segment, pair) jobs are launched `compute_units` at a
+ * x_hat_ln_group.  The (segment, pair) jobs are launched `compute_units` at a
  * time, so a last round that is not full costs a fraction of a sequence instead of a whole one (384 pairs on
  * 256 CUs: 3 launches of half a sequence).  Results do not change by a bit.  This query (no device needed) says
  * what the launchers do for `pairs` pairs of `NC` mini-batches (which = 0 forward, 1 backward; compute_units = 0:

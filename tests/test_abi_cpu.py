@@ -234,8 +234,7 @@ def test_export_of_group_zero_validates_like_the_backward(lib):
 def test_segment_plan_cuts_sequences_where_a_last_round_would_idle(lib):
     """More pairs than CUs: the sequences are cut at checkpoint boundaries and the (segment, pair) jobs launched a
     device's worth at a time, when that is shorter than whole rounds (or than a last round with several workgroups per
-    pair).  A pair's earlier segment must sit in an earlier launch, the segments are whole checkpoint groups, and the
-    backward needs two mini-batch slots of x_hat_ln_group for its parked sums."""
+    pair).  A pair's earlier segment must sit in an earlier launch, and the segments are whole checkpoint groups."""
     def plan(which, pairs, cus, NC, cgs, ws):
         a, b = ctypes.c_int(-1), ctypes.c_int(-1)
         assert lib.ttt_mlp_segment_plan(which, ctypes.c_longlong(pairs), cus, NC, cgs, ws, ctypes.byref(a), ctypes.byref(b)) == 0
@@ -248,7 +247,7 @@ def test_segment_plan_cuts_sequences_where_a_last_round_would_idle(lib):
             assert plan(which, 512, 256, 512, 32, ws)[0] == 0         # full rounds
             assert plan(which, 384, 256, 512, 512, ws)[0] == 0        # one checkpoint group: nowhere to cut
     assert plan(0, 257, 256, 512, 32, 1) == (64, 9)                   # 8 segments: 9 launches of an eighth
-    assert plan(1, 384, 256, 512, 1, 0)[0] == 0                       # backward, groups of one mini-batch
+    assert plan(1, 384, 256, 512, 1, 0) == (256, 3)                   # groups of one mini-batch
     assert plan(0, 384, 256, 512, 1, 0)[0] > 0
     assert plan(0, 384, 256, 512, 32, 1) == plan(0, 384, 256, 512, 32, 0)
     # few groups: a rest with several workgroups per pair waits for its first group's replay, so the cut pays for less

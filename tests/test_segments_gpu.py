@@ -27,7 +27,7 @@ def _plan(lib, which, pairs, cus, NC, cgs, with_workspace):
     return seg.value, launches.value
 
 
-@pytest.mark.parametrize("NC,cgs", [(96, 8), (100, 8), (90, 3)])
+@pytest.mark.parametrize("NC,cgs", [(96, 8), (100, 8), (90, 3), (90, 1)])
 def test_cut_sequences_give_the_same_forward(NC, cgs):
     import test_time_training as ext
     import ttt_mlp_host as host

@@ -280,7 +280,7 @@ int launch_bwd_segments(ttt::BwdParams p, const SegmentPlan& plan, int cus, hipS
   return launch_segments(p, plan, cus, [stream](const ttt::BwdParams& q) { return ttt_mlp_bwd_enqueue(q, stream); });
 }
 SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace) {
-  if (cgs < 2) return SegmentPlan{};
+  // (the two norm sums that a segment leaves behind, 4 KiB each, fill one 8 KiB slot of x_hat_ln_group)
   return plan_segments(pairs, cus, NC, cgs, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, true));
 }
 

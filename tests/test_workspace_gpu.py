@@ -154,7 +154,8 @@ def test_short_sequences_and_small_workspaces(NH, NC, cgs):
         torch.cuda.reset_peak_memory_stats(dev)
         host.backward(t, cgs)
         assert ext.last_backward_mode() == 1
-        assert torch.cuda.max_memory_allocated(dev) - before <= most.value + 512
+        # (the caching allocator rounds to 512 bytes and hands out a block of up to 1 MiB more rather than split it; a set is 2 MiB or more)
+        assert torch.cuda.max_memory_allocated(dev) - before <= most.value + 512 + (1 << 20)
         try:
             for nbytes, mode in ((least.value, 1), (least.value - 1, 0)):
                 host.set_workspace(torch.empty(nbytes, dtype=torch.uint8, device=dev))

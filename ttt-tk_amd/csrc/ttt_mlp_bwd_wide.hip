@@ -776,8 +776,8 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_wide_kernel(const BwdP
   constexpr int PER = NREPLAY + 3 + (PREFETCH ? 1 : 0);
   constexpr bool IMG = NREPLAY > 2;   // with the replay to spare it also evaluates the GELU family for the walk
   const int b = blockIdx.x;
-  int bh = (b / (8 * PER)) * 8 + (b & 7);
-  const int role = (b >> 3) % PER;
+  int bh = p.scatter ? b / PER : (b / (8 * PER)) * 8 + (b & 7);
+  const int role = (p.scatter ? b : b >> 3) % PER;
   if (bh >= p.nbh) return;
   bh += p.bh0;
   if (role < 2) {

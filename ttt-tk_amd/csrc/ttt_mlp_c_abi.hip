@@ -412,7 +412,8 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   return ttt_mlp_bwd_launch_within(a, workspace, workspace_bytes, stream);
 }
 
-extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter) {
   ttt::BwdParams p;
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
@@ -486,9 +487,15 @@ extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* worksp
   }
   if (pl.wide) {
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
+    p.scatter = scatter ? 1 : 0;
     return static_cast<int>(ttt_mlp_bwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
   }
   return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
+}
+}  // namespace
+
+extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  return bwd_launch(a, workspace, workspace_bytes, stream, false);
 }
 
 extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
@@ -515,7 +522,8 @@ extern "C" size_t ttt_mlp_fwd_status_offset(int B, int NH) {
   return pl.rest_split ? (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE * sizeof(int) : 0;
 }
 
-extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter) {
   ttt::FwdParams p;
   if (int rc = make_fwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
@@ -554,12 +562,24 @@ extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* wo
     p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * ttt::FWD_WIDE_RING * (ttt::FWD_IMG_BYTES / 2);
     p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
+    p.scatter = scatter ? 1 : 0;
     return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
   }
   p.ring_log2 = p.NC >= 512 ? 5 : 3;   // 32 or 8 mini-batches per hand-over
   p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * 2 * ttt::FWD_RING_MAX * (ttt::FWD_IMG_BYTES / 2);
   p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * 2 * ttt::FWD_RING_MAX * ttt::FWD_BIAS_FLOATS;
   return static_cast<int>(ttt_mlp_fwd_enqueue(p, static_cast<hipStream_t>(stream)));
+}
+}  // namespace
+
+extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  return fwd_launch(a, workspace, workspace_bytes, stream, false);
+}
+
+extern "C" int ttt_mlp_launch_scattered(int which, const void* args, void* workspace, size_t workspace_bytes, void* stream) {
+  if (which == 0) return fwd_launch(static_cast<const ttt_mlp_fwd_args*>(args), workspace, workspace_bytes, stream, true);
+  if (which == 1) return bwd_launch(static_cast<const ttt_mlp_bwd_args*>(args), workspace, workspace_bytes, stream, true);
+  return TTT_MLP_ERR_BAD_ARG;
 }
 
 // ---------------------------------------------------------------------------------------------------------

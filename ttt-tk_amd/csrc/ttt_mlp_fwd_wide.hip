@@ -528,8 +528,8 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
 __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_kernel(const FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x, per = 2 + p.n_out;
-  int bh = (b / (8 * per)) * 8 + (b & 7);
-  const int role = (b >> 3) % per;
+  int bh = p.scatter ? b / per : (b / (8 * per)) * 8 + (b & 7);
+  const int role = (p.scatter ? b : b >> 3) % per;
   if (bh >= p.nbh) return;
   bh += p.bh0;
   if (role < 2) {

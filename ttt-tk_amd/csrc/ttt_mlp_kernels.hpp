@@ -26,8 +26,9 @@ struct FwdParams {
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
   // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2 x 2048 fp32],
   // and the output workgroups per pair (1 or 2); the ring then has FWD_WIDE_RING slots.
+  // scatter: the workgroups of a pair on consecutive XCDs instead of on one, for tests.
   unsigned long long* xchg;
-  int n_out;
+  int n_out, scatter;
   int bh0, nbh;   // this launch covers (batch, head) pairs bh0 .. bh0 + nbh - 1
   // One workgroup per pair, sequence cut into segments (seg_len > 0, a multiple of cgs): workgroup i of the launch
   // runs job job0 + i, job q = segment q / (B*NH) of pair q % (B*NH); a segment starts from the checkpoint that the
@@ -87,9 +88,10 @@ struct BwdParams {
   // n_prefetch = 1 (with three or four replaying workgroups): one more workgroup reads nothing for itself; it touches every
   // cache line that the walk is about to ask for, ahead of it, so that the walk's own requests are answered by the L2 the
   // two share instead of by HBM.
+  // scatter: the workgroups of a pair on consecutive XCDs instead of on one, for tests.
   unsigned long long* xchg;
   int n_sets;
-  int n_prefetch;
+  int n_prefetch, scatter;
   int* sync;
   int* status;    // the status word behind the synchronisation words
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up

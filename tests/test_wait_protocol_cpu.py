@@ -58,3 +58,14 @@ def test_leaving_is_decided_between_barriers_by_all_waves_alike(source, function
     assert any("W" in x for x in kinds[1]) and any("R" in x for x in kinds[0])
     for i, (a, b) in enumerate(zip(*kinds)):
         assert not ("W" in a + b and "R" in a + b), f"interval {i}: the word is written while it is read ({a!r}, {b!r})"
+
+
+def test_the_count_of_gathered_sums_orders_what_it_counts():
+    """The compute waves overwrite block 0's partial sums once four helpers have counted up: a release before the count, an
+    acquire behind the wait (in the forward, the shares of b2 the same way)."""
+    text = re.sub(r"//[^\n]*", "", open(os.path.join(CSRC, "ttt_mlp_bwd_wide.hip")).read())
+    assert re.search(r'fence\(__ATOMIC_RELEASE, "workgroup", "local"\);\s*if \(lane == 0\) __hip_atomic_fetch_add\(s_flag \+ 1', text)
+    assert re.search(r'while \(flag\(1\) < 4 \* \(n \+ 1\)\)[^;]*;\s*__builtin_amdgcn_fence\(__ATOMIC_ACQUIRE, "workgroup", "local"\)', text)
+    text = open(os.path.join(CSRC, "ttt_mlp_fwd_wide.hip")).read()
+    assert "__hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELEASE" in text
+    assert re.search(r'while \(__hip_atomic_load\(s_flag \+ 1[^;]*;\s*__builtin_amdgcn_fence\(__ATOMIC_ACQUIRE, "workgroup"\)', text)

@@ -339,6 +339,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
           const float a = half_sum_valu(de);
           if (i == 1) {   // block 0's sums have been gathered (long since)
             while (flag(1) < 4 * (n + 1)) __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
           }
           if (h == 0) s_deta[u * CS + 32 * i + c] = a;
 #pragma unroll
@@ -675,7 +676,8 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
         }
       };
       gather_send(0);
-      // (relaxed: the gathered values are in registers; a release would also wait for the words just sent)
+      // (a release of LDS only: one of everything would also wait for the words just sent)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
       if (lane == 0) __hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       // the group's hand-over set to the grad_L_XK workgroup is free (written from here on)
       if (j == n_mb - 1 && done >= 2) wait_for(words + 24, done - 1);

@@ -16,12 +16,12 @@ constexpr int64_t F = TTT_MLP_F, CS = TTT_MLP_CS, HID = TTT_MLP_HID;
 bool g_synchronize = true;  // upstream blocks the host until the kernel has finished
 bool g_fill_group_tensors = false;   // leave the values of checkpoint group 0 in the sixteen *_group tensors
 bool g_accumulate = true;            // grad_L_XQ / XK / XV / last_eta are added to (upstream behaviour) rather than overwritten
-bool g_overlap = true;      // two workgroups per (batch, head) whenever they fit the device
+bool g_overlap = true;      // several workgroups per (batch, head) whenever they fit the device
 unsigned long long g_wait_ticks = 2000000000ull;   // mirrors the library's limit, for the error text
 torch::Tensor* g_sticky = nullptr;   // a device int, non-zero once a launch that nobody waited for gave up a wait (never freed:
                                      // a static tensor would be destroyed after the runtime at process exit)
 torch::Tensor* g_workspace = nullptr;   // caller-owned workspace of the multi-workgroup launches (set_workspace); never freed here
-int g_last_forward_mode = -1;    // 0 = one workgroup per (batch, head), 1 = two
+int g_last_forward_mode = -1;    // 0 = one workgroup per (batch, head), 1 = several
 int g_last_backward_mode = -1;
 
 void check_tensor(const torch::Tensor& t, const char* name, c10::ScalarType dtype, std::initializer_list<int64_t> shape) {
@@ -307,7 +307,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("abi_version", []() { return ttt_mlp_abi_version(); });
   // Also not upstream: choice of the launch shape (results are bit-identical either way).
   m.def("set_overlap", [](bool on) { g_overlap = on; },
-        "Use a second workgroup per (batch, head) when the device has room: the forward's output branch, the "
+        "Use several workgroups per (batch, head) when the device has room: the forward's output branch, the "
         "backward's recomputation of checkpoint groups (default true).");
   m.def("set_fill_group_tensors", [](bool on) { g_fill_group_tensors = on; },
         "After ttt_backward, leave the values of checkpoint group 0 in the sixteen *_group tensors, row-major, as the "
@@ -366,7 +366,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "CUs the multi-workgroup launches may count on (their workgroups wait for each other and must all be resident): "
         "say so when the process runs under a CU mask or beside a kernel that holds CUs; 0 (default) = all of the device.");
   m.def("last_forward_mode", []() { return g_last_forward_mode; },
-        "0: the last ttt_forward used one workgroup per (batch, head); 1: two; -1: none yet.");
+        "0: the last ttt_forward used one workgroup per (batch, head); 1: several; -1: none yet.");
   m.def("last_backward_mode", []() { return g_last_backward_mode; },
-        "0: the last ttt_backward used one workgroup per (batch, head); 1: two; -1: none yet.");
+        "0: the last ttt_backward used one workgroup per (batch, head); 1: several; -1: none yet.");
 }

@@ -364,20 +364,21 @@ TTT_DEV bf16x8 w1_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int rb, 
 
 constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK workgroup within the last group walked (a power of two)
 
-// ------------------------------------------------------------------ two workgroups per (batch, head)
+// ------------------------------------------------------------------ several workgroups per (batch, head)
 // The replay of a checkpoint group needs only the checkpoint, so it can run ahead of the reverse walk
-// on another CU: one workgroup replays group after group into two alternating sets of the per-group
-// tensors, the other walks each group backwards as soon as it is complete.  They signal through two
-// counters in HBM (agent scope); both are resident at once because the launcher uses this mode only
-// when the grid fits the CUs of the device.  A wait that sees no progress for SPIN_LIMIT ticks of the
-// 100 MHz clock raises the status word and both workgroups leave, so every wave always exits.
+// on other CUs: n_replay workgroups replay group after group, in turn, into alternating sets of the per-group
+// tensors, another walks each group backwards as soon as it is complete.  They signal through
+// counters in HBM (agent scope); all are resident at once because the launcher uses this mode only
+// when the grid fits the CUs of the device.  A wait that sees no progress for p.wait_limit ticks of the
+// 100 MHz clock raises the status word and all of them leave, so every wave always exits.
 // ROLE 0: replay and reverse walk of every group in one workgroup; 1: replays only - every n_replay-th group,
 // starting with group number `turn` (counted from the end of the sequence); 2: the reverse walks only.
-// IMG (with two replaying workgroups): the replay has time to spare and evaluates gelu, gelu', gelu'' of the
-// rounded Z1 for the walk, which gets them as three images instead of the image of Z1.  Same values either way.
-// FIN: grad_L_XK is a leaf of the walk - it needs the running gradients, but nothing needs it.  With a
-// fourth workgroup the walk hands over the operands of its two products (gW1, G1, dZ1 as register images)
-// and g_y, and that workgroup (bwd_finish_dxk) forms the products, their pair sum and the final sum.
+// IMG (two replaying workgroups, with the walk on two CUs three or four): the replay has time to spare and evaluates gelu,
+// gelu', gelu'' of the rounded Z1 for the walk, which gets them as three images instead of the image of Z1.  Same values
+// either way.
+// FIN: grad_L_XK is a leaf of the walk - it needs the running gradients, but nothing needs it.  Where one more workgroup
+// fits, the walk hands it dZ1 (a register image) and two fp32 tiles, g_y and the norm-weight gradient terms, and that
+// workgroup (bwd_finish_dxk) forms grad_L_XK, grad_L_XV and the norm gradients.
 // WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
 template <int ROLE, bool IMG, bool FIN, bool WIDE = false>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; the other roles take
@@ -459,7 +460,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   typedef const __attribute__((address_space(4))) BwdParams* KernArgs;
   KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
 #define REFRESH_OFFSETS() asm volatile("" : "+s"(ka), "+s"(ox), "+s"(oe), "+s"(of), "+s"(oh), "+s"(ot), "+s"(opk), "+s"(ock))
-  // per-group tensors: the caller's (set 0) or, in two-workgroup mode, the alternate set
+  // per-group tensors: the caller's (set 0) or, with several workgroups, one of the alternate sets
 #define GRP(name) (set ? ka->alt_##name[set - 1] : ka->name)
 #define bXQ gbuf(ka->XQ + ox)
 #define bXK gbuf(ka->XK + ox)

@@ -334,7 +334,7 @@ struct BwdWorkspace {
   }
 };
 
-// Workspace of the forward's two-workgroup mode: synchronisation words, then per (batch, head) a ring of
+// Workspace of the forward with several workgroups per pair: synchronisation words, then per (batch, head) a ring of
 // 2 * FWD_RING_MAX slots of state images and of bias vectors.
 // With the recurrence on two workgroups (n_out > 0) the ring has FWD_WIDE_RING slots, and the exchange follows.
 struct FwdWorkspace {

@@ -15,8 +15,12 @@ TTT_DEV uint64_t wd_pack(float a, float b) {
 }
 TTT_DEV float wd_lo(uint64_t x) { return __builtin_bit_cast(float, static_cast<uint32_t>(x)); }
 TTT_DEV float wd_hi(uint64_t x) { return __builtin_bit_cast(float, static_cast<uint32_t>(x >> 32)); }
-// A word for the other CU.  On one XCD the L2 is where both meet: a plain store reaches it and the partner's agent-scope
-// load is answered by it (2.9 k clocks for 16 KiB both ways; agent-scope stores 3.4-4.5 k).
+// A word for the other CU.  On one XCD the L2 is where both meet: the L1 writes through, so a plain store (wavefront scope)
+// reaches it and the partner's agent-scope load is answered by it (2.9 k clocks for 16 KiB both ways; agent-scope stores
+// 3.4-4.5 k).  For the same reason counters need no release where all of a pair share an XCD (give in ttt_mlp_fwd_wide.hip,
+// BWW_GIVEN in ttt_mlp_bwd_wide.hip): a wave's vmcnt(0) says that its stores are in the L2, a barrier collects the waves,
+// and the reader's acquire drops what its own L1 holds.  This is how gfx950 works, not what the memory model promises;
+// `near` false (no common XCD) takes agent scope and release fences throughout.
 TTT_DEV void wd_put(gword64_t q, uint64_t x, bool near) {
   if (near) __hip_atomic_store(q, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   else __hip_atomic_store(q, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -13,10 +13,11 @@
 // One or two more workgroups per pair compute Out from the states left in a ring, as in the two-workgroup launch.
 // Every sum has the order of the one-workgroup kernel: results are the same to the bit.
 //
-// What bounds it: the chain.  48 pairs, 16,384 tokens: 2.24 ms with the recurrence on one CU, 1.45 ms here (5.7 us or 13.1 k
-// clocks per mini-batch; 1 pair of 32,768 tokens: 4.22 -> 2.70 ms).  Of the 13.1 k: block 0's products 2.2 k, block 1's 3.7 k
-// while block 0's sums cross (gather and send 1.1 k, 1.3 k under way, LayerNorm 0.8 k), then the same 3.4 k for block 1's
-// sums with block 0's weight step beside it, block 1's weight step and the split of the new state 3.3 k.
+// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.57 ms here (6.1 us per
+// mini-batch), 48 x 4,096: 32.5 -> 24.2 ms.  With the stage clocks in, 14.3 k clocks: block 0's products 2.7 k; block 1's 3.7 k
+// while block 0's sums cross (gather and send 1.25 k, 1.1 k under way, LayerNorm 1.8 k) and 0.75 k of waiting for them;
+// block 0's weight step 2.0 k while block 1's sums cross and 2.35 k of waiting for those; block 1's weight step and the
+// split of the new state 2.65 k.
 #include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
 

@@ -63,10 +63,11 @@ struct BwdParams {
   float *grad_L_W1_init, *grad_L_b1_init, *grad_L_W2_init, *grad_L_b2_init;
   __bf16 *grad_L_last_eta, *grad_L_XQ, *grad_L_XK, *grad_L_XV;
   int B, NH, NC, K, cgs;
-  // Several workgroups per (batch, head) only (sync != nullptr): n_replay = 1 or 2 workgroups replay the
-  // checkpoint groups (taking turns), one walks them backwards.  Group number g (0 = the last group of the
-  // sequence) is replayed into set g % (2 * n_replay) of the per-group tensors that carry it to the walk:
-  // set 0 = the caller's tensors, sets 1.. = alt_*[set - 1] from the workspace.
+  // Several workgroups per (batch, head) only (sync != nullptr): n_replay workgroups replay the checkpoint groups (taking
+  // turns; 1 or 2, with the walk on two workgroups 2 to 4), one or two walk them backwards.  Group number g (0 = the last
+  // group of the sequence) is replayed into set g % n_sets of the per-group tensors that carry it to the walk:
+  // set 0 = the caller's tensors, sets 1.. = alt_*[set - 1] from the workspace; n_sets = 2 * n_replay, with the walk on two
+  // workgroups n_replay + 2 (the kernels with the walk on one do not read it).
   __bf16 *alt_X2_group[BWD_MAX_SETS - 1], *alt_Z1_group[BWD_MAX_SETS - 1], *alt_Z1_bar_group[BWD_MAX_SETS - 1], *alt_X2_bar_group[BWD_MAX_SETS - 1];
   __bf16 *alt_grad_l_wrt_Z2_group[BWD_MAX_SETS - 1], *alt_grad_l_wrt_Z1_group[BWD_MAX_SETS - 1];
   __bf16 *alt_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_output_fused_group[BWD_MAX_SETS - 1];
@@ -84,7 +85,7 @@ struct BwdParams {
   float* fin_gy;
   int n_finish;
   // Walk on two workgroups (ttt_mlp_bwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
-  // 256 8-byte words]; n_replay = 2 .. 4 and n_sets sets of the per-group tensors; n_finish = 1.
+  // 256 8-byte words]; n_finish = 1.
   // n_prefetch = 1 (with three or four replaying workgroups): one more workgroup reads nothing for itself; it touches every
   // cache line that the walk is about to ask for, ahead of it, so that the walk's own requests are answered by the L2 the
   // two share instead of by HBM.
@@ -107,7 +108,7 @@ struct BwdParams {
 #endif
 };
 
-// Layout of `sync` (ints): 32 per (batch, head) - words 0 and 8 count the groups replayed by the first /
+// Layout of `sync` (ints): 32 per (batch, head).  Walk on one workgroup: words 0 and 8 count the groups replayed by the first /
 // second replaying workgroup (norm_partial is written with the group), word 16 the groups the
 // reverse walk has finished, word 12 the mini-batches of the last group it walks that it has handed to the grad_L_XK
 // workgroup (that group is handed over in chunks), word 24 the groups the grad_L_XK workgroup has finished - then one status

@@ -220,7 +220,7 @@ struct SegmentPlan {
   long long jobs = 0;
 };
 // `alt_x1000`: what the alternative costs, in thousandths of a mini-batch of one workgroup.
-SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long alt_x1000) {
+SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backward, long long alt_x1000) {
   SegmentPlan best;
 #ifndef TTT_STAGE_CLOCKS   // the stage clocks are kept per pair and sequence
   if (pairs <= cus || pairs > (1 << 27) || cus <= 0 || NC <= 0 || cgs <= 0) return best;   // (job numbers are ints)
@@ -229,9 +229,14 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long a
   for (int S = 2; S <= 8 && S <= K; S++) {
     const int groups = (K + S - 1) / S, segs = (K + groups - 1) / groups;
     const long long len = (long long)groups * cgs, jobs = segs * pairs, launches = (jobs + cus - 1) / cus;
-    // + a mini-batch's worth per launch: gaps, state in and out (5 launches of 128 mini-batches, 320 pairs: 29.4 ms against 31.3
-    // uncut; 11 of 64, 352 pairs: 32.4 against 33.9; 3 of 256, 384 pairs: 35.1 against 34.8)
-    const long long t = launches * (len * 1000 + 1000);
+    // A launch takes what the longest segment in it takes.  All have `len` mini-batches except the one with the sequence's last
+    // group (the forward's last, the backward's first) and the one with the groups left over (the last): how many launches
+    // hold nothing but those?
+    const long long left = (long long)(K - (segs - 1) * groups) * cgs, missing = (long long)K * cgs - NC;
+    const long long len0 = backward ? len - missing : len, len_last = backward ? left : left - missing;
+    const long long n0 = pairs / cus, n_last = launches - ((segs - 1) * pairs + cus - 1) / cus;
+    // + a mini-batch's worth per launch: gaps, state in and out (measured 0.7 to 2 forward, about 1 backward)
+    const long long t = 1000 * (n0 * len0 + n_last * len_last + (launches - n0 - n_last) * len + launches);
     if (t < best_t) {
       best_t = t;
       best.seg_len = static_cast<int>(len);
@@ -244,19 +249,23 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, long long a
   return best;
 }
 // Thousandths of a one-workgroup mini-batch that the pairs take uncut: full rounds, and the rest either one more
-// round or, with several workgroups per pair, a shorter one.  Measured on 256 CUs as what the rest adds to a full round
-// (6.5 ms forward, 23.1 ms backward for 512 mini-batches), at the most pairs of a shape: forward 530 (4 pairs, 430 for 64), 550
-// (80), 710 (128).  The backward's walk waits for the first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at
-// K = 16, 320 at 4; 48 pairs 265 and 335, 64 pairs 350 and 435, 80 pairs 435 and 515, 128 pairs 500 and 605.
-long long rest_x1000(const LaunchPlan& pl, int K, bool backward) {
-  if (!backward) return pl.n_out == 2 ? 530 : pl.n_out == 1 ? 550 : 710;
+// round or, with several workgroups per pair, a shorter one.  Measured on 256 CUs as what the rest adds to full rounds
+// (6.5 ms forward, 23.1 ms backward for 512 mini-batches), at the most pairs of a shape.  Forward: 530 per mini-batch (4 pairs; 430
+// for 64), 545 (80 pairs) and 650 (128 pairs), and the mini-batches by which Out trails.  The backward's walk waits for the
+// first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at K = 16, 320 at 4; 48 pairs 265 and 335, 64 pairs 350 and
+// 435, 80 pairs 435 and 515, 128 pairs 500 and 605.
+// A last round that is not full is 5 % shorter than a full one (400 to 456 pairs).
+// What the estimate decides: 312 pairs x 101 mini-batches in 4 groups, forward 1.70 ms cut, 1.93 uncut; 384 x 31 in 16, 0.65 and
+// 0.78; 276 x 329 in 22, backward 17.5 and 18.7; 330 x 395 in 18, 24.3 and 27.3; 384 x 512 in 16, 35.1 and 34.8.
+long long rest_x1000(const LaunchPlan& pl, int NC, int K, bool backward) {
+  if (!backward) return pl.n_out == 2 ? 525LL * NC + 3000 : pl.n_out == 1 ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
   const int walk = pl.wide ? (pl.n_replay > 2 ? 210 : 235) : pl.finish ? 325 : pl.n_replay == 2 ? 405 : 485;
-  return walk + 470 / K;
+  return (long long)(walk + 470 / K) * NC;
 }
 long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace, bool backward) {
   if (cus <= 0) return (long long)NC * 1000;
-  if (with_workspace && pl.rest_split) return (pl.n_single / cus * 1000 + rest_x1000(pl, (NC + cgs - 1) / cgs, backward)) * NC;
-  return (pairs + cus - 1) / cus * 1000 * NC;
+  if (with_workspace && pl.rest_split) return pl.n_single / cus * 1000 * NC + rest_x1000(pl, NC, (NC + cgs - 1) / cgs, backward);
+  return (pairs + cus - 1) / cus * (pairs % cus != 0 ? 950 : 1000) * NC;
 }
 // The launches of a call with the sequences cut: `cus` jobs each, in job order, on the one stream.
 template <class Params, class Enqueue>
@@ -281,7 +290,7 @@ int launch_bwd_segments(ttt::BwdParams p, const SegmentPlan& plan, int cus, hipS
 }
 SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace) {
   // (the two norm sums that a segment leaves behind, 4 KiB each, fill one 8 KiB slot of x_hat_ln_group)
-  return plan_segments(pairs, cus, NC, cgs, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, true));
+  return plan_segments(pairs, cus, NC, cgs, true, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, true));
 }
 
 // Sets of the per-group tensors that carry replayed groups to the walk, used in turn: two per replaying workgroup, or one each
@@ -503,7 +512,7 @@ extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
   if (int rc = make_fwd_params(a, p)) return rc;
   const long long pairs = (long long)p.B * p.NH;
   const int cus = device_cus();
-  const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(LaunchPlan{}, pairs, cus, p.NC, p.cgs, false, false));
+  const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, false, uncut_x1000(LaunchPlan{}, pairs, cus, p.NC, p.cgs, false, false));
   if (seg.seg_len > 0) return launch_fwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
   p.bh0 = 0;
   p.nbh = p.B * p.NH;
@@ -537,7 +546,7 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
     // workspace then only has its words cleared (callers read the status word behind them)
     const long long pairs = (long long)p.B * p.NH;
     const int cus = device_cus();
-    const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, uncut_x1000(pl, pairs, cus, p.NC, p.cgs, true, false));
+    const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, false, uncut_x1000(pl, pairs, cus, p.NC, p.cgs, true, false));
     if (seg.seg_len > 0) {
       if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_rest)),
                                                  static_cast<hipStream_t>(stream)))
@@ -673,7 +682,7 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
     return TTT_MLP_ERR_BAD_ARG;
   const LaunchPlan pl = plan_for(pairs, compute_units, which == 1);
   const SegmentPlan seg = which == 1 ? plan_bwd_segments(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0)
-                                     : plan_segments(pairs, compute_units, NC, checkpoint_group_size,
+                                     : plan_segments(pairs, compute_units, NC, checkpoint_group_size, false,
                                                      uncut_x1000(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0, false));
   *segment_minibatches = seg.seg_len;
   *launches = seg.seg_len > 0 ? seg.launches : (with_workspace != 0 && pl.rest_split && pl.n_single > 0 ? 2 : 1);

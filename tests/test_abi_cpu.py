@@ -246,6 +246,7 @@ def test_segment_plan_cuts_sequences_where_a_last_round_would_idle(lib):
             assert plan(which, 256, 256, 512, 32, ws)[0] == 0
             assert plan(which, 512, 256, 512, 32, ws)[0] == 0         # full rounds
             assert plan(which, 384, 256, 512, 512, ws)[0] == 0        # one checkpoint group: nowhere to cut
+            assert ws == 0 or plan(which, 260, 256, 5, 2, ws) == (0, 2)   # what the tests of a rest behind a full round count on
     assert plan(0, 257, 256, 512, 32, 1) == (64, 9)                   # 8 segments: 9 launches of an eighth
     assert plan(1, 384, 256, 512, 1, 0) == (256, 3)                   # groups of one mini-batch
     assert plan(0, 384, 256, 512, 1, 0)[0] > 0

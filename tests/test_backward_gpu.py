@@ -17,7 +17,7 @@ UP_KEYS = ("grad_L_W1_last", "grad_L_b1_last", "grad_L_W2_last", "grad_L_b2_last
 def run_fwd_bwd(d, cgs, hw_forward=True, scratch_fill=None, overlap=None):
     """Forward on the GPU (or oracle checkpoints when hw_forward is False), then backward on the GPU.
     scratch_fill: value written into the sixteen *_group workspace tensors before the backward.
-    overlap: None = the operator's own choice; False / True = one / two workgroups per (batch, head),
+    overlap: None = the operator's own choice; False / True = one / several workgroups per (batch, head),
     and the mode that actually ran is asserted."""
     import ttt_mlp_host as host
     import test_time_training as ext
@@ -149,15 +149,15 @@ def test_bit_reproducible_and_independent_of_workspace_contents(B, NH, NC, cgs):
 @pytest.mark.parametrize("B,NH,NC,cgs", [
     (1, 2, 9, 1),        # nine groups of one mini-batch: the sets are reused, the replays wait for the walk
     (2, 3, 9, 4),        # ragged last group (walked first), (batch, head) count not a multiple of 8
-    (1, 8, 24, 8),       # multiple of 8: the two workgroups of a pair are placed on one XCD
+    (1, 8, 24, 8),       # a grid that needs no padding to a multiple of 8 pairs
     (2, 8, 10, 5),       # two groups only
     (1, 4, 33, 2),       # seventeen groups
-    (2, 130, 5, 2),      # more pairs than CUs: 256 with one workgroup each, then the last 4 with four
+    (2, 130, 5, 2),      # more pairs than CUs: 256 with one workgroup each, then the last 4 with eight
     (1, 72, 5, 2),       # too many pairs for four workgroups each: two replay, one walks (and forms grad_L_XK itself)
     (1, 96, 5, 2),       # too many pairs for three: one replays all groups, one walks
 ])
 def test_overlapped_backward_is_bit_identical(B, NH, NC, cgs):
-    """Recomputing the groups on a second workgroup changes the schedule, not one bit of the results."""
+    """Recomputing the groups on further workgroups changes the schedule, not one bit of the results."""
     print(f"case B={B} NH={NH} NC={NC} cgs={cgs}", flush=True)
     d = orc.make_inputs(B, NH, NC, seed=11)
     randomize_affine(d, 11)

@@ -14,7 +14,7 @@ FWD_KEYS = ("XQ", "XK", "XV", "last_eta", "ttt_norm_weight", "ttt_norm_bias", "W
 
 
 def _run_forward(d, cgs, overlap=None):
-    """overlap: None = the operator's own choice; False / True = one / two workgroups per (batch, head),
+    """overlap: None = the operator's own choice; False / True = one / several workgroups per (batch, head),
     and the mode that actually ran is asserted."""
     import ttt_mlp_host as host
     import test_time_training as ext
@@ -80,11 +80,11 @@ def test_forward_matches_oracle(B, NH, NC, cgs, seed, rand_affine):
     (2, 3, 9, 4),        # one full hand-over and a ragged one; (batch, head) count not a multiple of 8
     (1, 8, 40, 8),       # five hand-overs: both halves of the ring are reused, the recurrence waits for the output branch
     (1, 4, 33, 16),
-    (2, 130, 5, 2),      # more pairs than CUs: a full round with one workgroup each, the remaining 4 pairs with two
+    (2, 130, 5, 2),      # more pairs than CUs: a full round with one workgroup each, the remaining 4 pairs with four
     (1, 72, 5, 2),
 ])
 def test_overlapped_forward_is_bit_identical(B, NH, NC, cgs):
-    """Computing Out on a second workgroup changes the schedule, not one bit of the results."""
+    """Computing Out on further workgroups changes the schedule, not one bit of the results."""
     print(f"case B={B} NH={NH} NC={NC} cgs={cgs}", flush=True)
     d = orc.make_inputs(B, NH, NC, seed=21, with_grads=False)
     g = torch.Generator().manual_seed(121)

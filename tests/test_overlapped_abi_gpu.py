@@ -31,7 +31,7 @@ def _args(order, t, cgs, B, NH, NC, K):
     return Args(*[t[k].data_ptr() for k in order], cgs, B, NH, NC, K)
 
 
-# 8 pairs: the backward runs with a fifth workgroup per pair that fetches ahead of the walk (a multiple of 8 pairs)
+# up to 32 pairs the backward runs with eight workgroups per pair (four replay, the walk takes two), at 48 with five
 @pytest.mark.parametrize("B,NH,NC,cgs", [(1, 2, 1, 1), (1, 3, 5, 8), (2, 2, 17, 4), (1, 8, 13, 4), (2, 4, 3, 8),
                                           (1, 16, 9, 4), (3, 8, 5, 2), (1, 48, 19, 8)])
 def test_overlapped_launchers_through_ctypes(B, NH, NC, cgs):
@@ -78,7 +78,7 @@ def test_overlapped_launchers_through_ctypes(B, NH, NC, cgs):
         assert torch.equal(results[0][k], results[1][k]), k
 
 
-@pytest.mark.parametrize("NH", [2, 8])   # 8 pairs: with the workgroup that fetches ahead of the walk
+@pytest.mark.parametrize("NH", [2, 8])   # a grid padded to a multiple of 8 pairs, and a full one
 def test_a_wait_that_gives_up_is_reported_and_every_wave_exits(NH):
     """Forced from the host: with a wait limit of one clock tick the first workgroup that has to wait for its
     partner gives up at once, raises the status word, and all workgroups of the launch leave.  The operator

@@ -160,9 +160,9 @@ torch::Tensor ttt_forward(const torch::Tensor XQ, const torch::Tensor XK, const 
   a.B = (int32_t)B; a.NH = (int32_t)NH; a.NC = (int32_t)NC; a.K = (int32_t)K;
   const c10::DeviceGuard guard(XQ.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(XQ.device().index()).stream();
-  // With few (batch, head) pairs most CUs would idle: then a second workgroup per pair computes Out behind
+  // With few (batch, head) pairs most CUs would idle: then further workgroups per pair compute Out behind
   // the state recurrence.  Its workspace: the caller's (set_workspace) or torch's caching allocator's.
-  // (more pairs than CUs and sequences that the launcher cuts at checkpoints: no second workgroup, no workspace)
+  // (more pairs than CUs and sequences that the launcher cuts at checkpoints: one workgroup each, no workspace)
   const size_t ws_bytes = (g_overlap && NC >= 2 && !sequences_cut(0, B * NH, NC, checkpoint_group_size))
                               ? ttt_mlp_fwd_workspace_bytes((int32_t)B, (int32_t)NH) : 0;
   const Workspace ws = take_workspace(ws_bytes, XQ.device());
@@ -274,7 +274,7 @@ torch::Tensor ttt_backward(
   a.overwrite = g_accumulate ? 0 : 1;
   const c10::DeviceGuard guard(XQ.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(XQ.device().index()).stream();
-  // With few (batch, head) pairs most CUs would idle: then a second workgroup per pair recomputes the
+  // With few (batch, head) pairs most CUs would idle: then further workgroups per pair recompute the
   // checkpoint groups ahead of the reverse walk.  Its workspace (further sets of the per-group tensors): the
   // caller's (set_workspace) or torch's caching allocator's.
   size_t least = 0, ws_bytes = 0;

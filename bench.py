@@ -102,7 +102,7 @@ def cpu_baseline(NH, cgs, nc_sample, backward=True):
 
 
 METRICS = {
-    # the metric string follows the workload; c4's is BASELINE.json's
+    # the metric string follows the workload; c4's is the one the metric is quoted with
     "c2": "TTT-MLP forward tokens/sec on 1 MI355X (B=1,NH=48,16K tok); % bf16 MFMA peak",
     "c3": "TTT-MLP fwd+bwd tokens/sec on 1 MI355X (B=1,NH=48,16K tok); % bf16 MFMA peak",
     "c4": "TTT-MLP fwd+bwd tokens/sec on 1 MI355X (B=1,NH=48,256K tok); % bf16 MFMA peak",

@@ -1,6 +1,6 @@
 """CPU oracle for the non-causal TTT-MLP forward scan and its remat backward.
 
-THIS FILE IS TEST INFRASTRUCTURE.  It is a checker: only the test-suite, the
+THIS FILE IS TEST INFRASTRUCTURE.  Only the test-suite, the
 smoke check and the benchmark's ``cpu_baseline`` leg may import it.  The shipped
 operator never calls anything in here and has no CPU fallback.
 

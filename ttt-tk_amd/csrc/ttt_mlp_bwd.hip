@@ -6,10 +6,9 @@
 // activations are saved, then the group is walked backwards producing the ten output gradients.
 //
 // Mapping: workgroups of 8 wavefronts (two per SIMD, at most 256 registers each); one per (batch,
-// head), or two to four where the device has CUs to spare - then one or two replay the checkpoint
-// groups (taking turns), one walks them backwards, a group or more behind, and a fourth forms
-// grad_L_XK from what the walk hands it (with the walk itself on two workgroups: ttt_mlp_bwd_wide.hip, which takes the
-// roles of the others from here).  Wave v owns hidden columns [32v, 32v+32).  All [tokens x hidden] activations live in
+// head), or two or three where the device has CUs to spare - then one or two replay the checkpoint groups (taking
+// turns) and one walks them backwards, a group or more behind.  With more room: ttt_mlp_bwd_wide.hip, which takes the
+// roles from here (others form grad_L_XK from what the walk hands them).  Wave v owns hidden columns [32v, 32v+32).  All [tokens x hidden] activations live in
 // registers in the "Q" orientation (accumulator rows = hidden, lane = token), so per-token scalars
 // (eta, dEta partial sums) are per-lane values.  An activation that is also needed with tokens as the
 // contraction index is bounced once through a wave-private LDS tile (row store + transposing read).
@@ -366,14 +365,13 @@ constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK wo
 
 // ------------------------------------------------------------------ several workgroups per (batch, head)
 // The replay of a checkpoint group needs only the checkpoint, so it can run ahead of the reverse walk
-// on other CUs: n_replay workgroups replay group after group, in turn, into alternating sets of the per-group
+// on other CUs: one or more workgroups replay group after group, in turn, into alternating sets of the per-group
 // tensors, another walks each group backwards as soon as it is complete.  They signal through
 // counters in HBM (agent scope); all are resident at once because the launcher uses this mode only
 // when the grid fits the CUs of the device.  A wait that sees no progress for p.wait_limit ticks of the
 // 100 MHz clock raises the status word and all of them leave, so every wave always exits.
-// ROLE 0: replay and reverse walk of every group in one workgroup; 1: replays only - every n_replay-th group,
-// starting with group number `turn` (counted from the end of the sequence); 2: the reverse walks only.
-// IMG (two replaying workgroups, with the walk on two CUs three or four): the replay has time to spare and evaluates gelu,
+// ROLE 0: replay and reverse walk of every group in one workgroup; 1: one replay (k_hi = k_lo); 2: the reverse walks only.
+// IMG (two replaying workgroups per pair and the walk on one CU, three or four and the walk on two): the replay has time to spare and evaluates gelu,
 // gelu', gelu'' of the rounded Z1 for the walk, which gets them as three images instead of the image of Z1.  Same values
 // either way.
 // FIN: grad_L_XK is a leaf of the walk - it needs the running gradients, but nothing needs it.  Where one more workgroup
@@ -381,9 +379,9 @@ constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK wo
 // workgroup (bwd_finish_dxk) forms grad_L_XK, grad_L_XV and the norm gradients.
 // WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
 template <int ROLE, bool IMG, bool FIN, bool WIDE = false>
-// k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; the other roles take
-// the whole sequence, K - 1 .. 0).
-TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int turn, const int k_hi, const int k_lo) {
+// k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; ROLE 2: K - 1 .. 0).
+// False: a wait gave up.
+TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi, const int k_lo) {
   static_assert(!(ROLE == 0 && (IMG || FIN)), "one workgroup per (batch, head) does everything itself");
   bf16* s_xq = reinterpret_cast<bf16*>(smem + SB_XQ);
   bf16* s_xk = reinterpret_cast<bf16*>(smem + SB_XK);
@@ -426,9 +424,9 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   if (tid < FD) {
     s_gam[tid] = p.ttt_norm_weight[head * FD + tid];
     s_bet[tid] = p.ttt_norm_bias[head * FD + tid];
-    s_gb2[tid] = (seg_first ? p.grad_L_b2_last : p.grad_L_b2_init)[(size_t)bh * FD + tid];
+    if (ROLE != 1) s_gb2[tid] = (seg_first ? p.grad_L_b2_last : p.grad_L_b2_init)[(size_t)bh * FD + tid];
   }
-  if (tid < HID) s_gb1[tid] = (seg_first ? p.grad_L_b1_last : p.grad_L_b1_init)[(size_t)bh * HID + tid];
+  if (ROLE != 1 && tid < HID) s_gb1[tid] = (seg_first ? p.grad_L_b1_last : p.grad_L_b1_init)[(size_t)bh * HID + tid];
   // Norm-weight / norm-bias gradients accumulate per wave in LDS (summed over the wave's 8 tokens
   // with cross-lane adds in a fixed order); summed over the waves at the end.  The replay and the
   // reverse walk each contribute, and their sums are kept apart (so that the result does not depend on
@@ -518,10 +516,10 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     acc_load_rows(gW1s, gbuf((seg_first ? p.grad_L_W1_last : p.grad_L_W1_init) + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
     acc_load_rows(gW2s, gbuf((seg_first ? p.grad_L_W2_last : p.grad_L_W2_init) + (size_t)bh * HID * FD), 0, FD, hid0, 0, c, h);
   }
-  int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;   // + 0, + 8: groups replayed by workgroup 0 / 1
+  int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;   // + s: the group last replayed into set s
   int* const w_walked = w_sync + (WIDE ? BWW_WALKED : 16);
   int* const w_finished = w_sync + 24;
-  const int n_replay = ROLE == 0 ? 1 : p.n_replay, n_sets = WIDE ? p.n_sets : 2 * n_replay;
+  const int n_sets = ROLE == 0 ? 1 : p.n_sets;
   int* const w_status = p.status;
   int* const s_flag = reinterpret_cast<int*>(smem + SB_FLAG);
 
@@ -560,19 +558,18 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   for (int k = k_hi; k >= k_lo; k--) {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k;                    // number of this group, counted from the end of the sequence
-    if (ROLE == 1 && done % n_replay != turn) continue;
     const int set = ROLE == 0 ? 0 : done % n_sets;
-    int* const w_replayed = w_sync + (WIDE ? 1 : 8) * (done % n_replay);
+    int* const w_replayed = w_sync + set;
     REFRESH_OFFSETS();
     const size_t slot = (size_t)bh * p.K + k;
     const unsigned ckW = static_cast<unsigned>(k) * (FD * HID * 4u);   // byte offset of this group's checkpoint in bCW1 / bCW2
     // ================================================================= replay
     if constexpr (ROLE != 2) {
       if constexpr (ROLE == 1) {   // the set is free once the reverse walk is done with the group that used it last
-        if (done >= n_sets && !wait_at_least(w_walked, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
-        if (WIDE && done >= n_sets && !wait_at_least(w_walked + 4, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
+        if (done >= n_sets && !wait_at_least(w_walked, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
+        if (WIDE && done >= n_sets && !wait_at_least(w_walked + 4, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
         if constexpr (FIN) {   // ... and so is the workgroup that reads the before-state images for grad_L_XK
-          if (done >= n_sets && !wait_at_least(w_finished, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return;
+          if (done >= n_sets && !wait_at_least(w_finished, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
         }
         WAVE_SYNC();
         s_dgw[lane] = 0.f;   // (every lane its own words)
@@ -1054,7 +1051,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         g_stf(g, o, FD * 4, a1);
         WAVE_SYNC();
       }
-      if constexpr (ROLE == 1) publish(w_replayed, done / n_replay + 1);
+      if constexpr (ROLE == 1) publish(w_replayed, done + 1);
       TTT_STAGE(BS_PUBLISH);
     }
 
@@ -1063,9 +1060,9 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     // wave covers the latency, while holding requests in registers across stages costs more in spills
     // than it gains (measured).
     if constexpr (ROLE == 2) {
-      if (!wait_at_least(w_replayed, done / n_replay + 1, w_status, s_flag, p.wait_limit)) return;
+      if (!wait_at_least(w_replayed, done + 1, w_status, s_flag, p.wait_limit)) return false;
       if constexpr (FIN) {   // the hand-over set of this group's parity is free once the group before last is finished
-        if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return;
+        if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return false;
       } else {
         LANE_VARS;
         const gptr_t gs = group_sums(set);   // the running sum
@@ -1481,8 +1478,8 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #undef bFGY
 #undef WALK_FETCH
   }
-  TTT_STAGES_END(bh, ROLE == 1 ? turn : STAGE_ROLE_WALK);
-  if constexpr (ROLE == 1) return;
+  TTT_STAGES_END(bh, ROLE == 1 ? 0 : STAGE_ROLE_WALK);
+  if constexpr (ROLE == 1) return true;
 
   // ---- outputs that are written once
   acc_store_rows(gW1s, gbuf(p.grad_L_W1_init + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
@@ -1491,11 +1488,11 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   if (tid < HID) p.grad_L_b1_init[(size_t)bh * HID + tid] = s_gb1[tid];
   if (tid < FD) p.grad_L_b2_init[(size_t)bh * FD + tid] = s_gb2[tid];
   // norm-weight / norm-bias gradients: sum the per-wave LDS accumulators
-  if constexpr (FIN) return;   // with a grad_L_XK workgroup the walk holds no share of these sums: they are written there
+  if constexpr (FIN) return true;   // with a grad_L_XK workgroup the walk holds no share of these sums: they are written there
   if (ROLE == 0 && !seg_last) {   // the next segment goes on with the walk's sum (the replay's is in place already)
     g_stf(park(), np_off(), PARK_BYTES, s_dgw[lane]);
     g_stf(park(), np_off(), PARK_BYTES + FD * 4, s_dbw[lane]);
-    return;
+    return true;
   }
   if (tid < 2 * FD) {
     const int which = tid / FD, f = tid % FD;
@@ -1509,6 +1506,7 @@ TTT_DEV void bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     }
     (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = sr + s;
   }
+  return true;
 }
 #undef REFRESH_OFFSETS
 #undef LANE_VARS
@@ -1549,18 +1547,22 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_kernel(const BwdParams
     k_hi = p.K - 1 - seg * p.seg_groups;
     k_lo = k_hi - p.seg_groups + 1 > 0 ? k_hi - p.seg_groups + 1 : 0;
   }
-  bwd_body<0, false, false>(p, smem, bh, 0, k_hi, k_lo);
+  bwd_body<0, false, false>(p, smem, bh, k_hi, k_lo);
 }
 #endif
 
 // grad_L_XK on a workgroup of its own: for every mini-batch of every group, as soon as the walk is done with the
 // group, dk = gW1 G1^T + W1 dZ1^T (W1 before the step: from the replay's image, or the checkpoint), its sum over
 // the hidden dimension, + g_y, accumulated into grad_L_XK.  Same wave / lane roles and the same order of every
-// sum as in the walk, so the result is the same to the bit.
-template <bool IMG, bool WIDE>
-TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int bh) {
+// sum as in the walk, so the result is the same to the bit.  OWN: the whole sequence (k_hi = K - 1); otherwise fewer such
+// workgroups than pairs take the groups in turn and this is group k_hi, with what is carried from group to group (the copy of
+// the gradient wrt W1 and the norm-gradient sums) parked in between.  False: a wait gave up.
+template <bool IMG, bool WIDE, bool OWN>
+TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi) {
   float* s_P = reinterpret_cast<float*>(smem + SB_P);
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // nothing derived from it is kept over the caller's loop over groups
+  const int lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int v = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pp = v & 3, r = v >> 2;
   const int tb[2] = {r, 1 - r};
@@ -1569,7 +1571,7 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
   float* s_own = s_P + (pp * 2 + r) * RGN;
   float* s_partner = s_P + (pp * 2 + (1 - r)) * RGN;
   const float* s_lnrow = s_P + (1 - r) * RGN + (tok & 31) * LDR + f0;
-  const int cgs = p.cgs, n_sets = WIDE ? p.n_sets : 2 * p.n_replay;
+  const int cgs = p.cgs, n_sets = p.n_sets;
   const unsigned t16 = 16 * tid, vln = (tok * FD + f0) * 2;
   int* const w_sync = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   int* const w_walked = w_sync + 16;
@@ -1589,13 +1591,26 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
   // This workgroup keeps its own copy of the running gradient wrt W1: both terms the walk adds to it per
   // mini-batch (XQ^T gZ1_bar and XK^T dZ1) are formed from data that reaches this workgroup anyway, in the walk's order.
   AccT<2, 1> gW1s;
-  acc_load_rows(gW1s, gbuf(p.grad_L_W1_last + (size_t)bh * FD * HID), 0, HID, 0, hid0, c, h);
+  const bool first = OWN || k_hi == p.K - 1;
+  float* const park = p.fin_park + (size_t)bh * FIN_PARK_FLOATS;
+  if (!first && !wait_at_least(w_finished, p.K - 1 - k_hi, p.status, s_flag, p.wait_limit)) return false;   // the group before is parked
+  acc_load_rows(gW1s, gbuf(first ? p.grad_L_W1_last + (size_t)bh * FD * HID : park), 0, HID, 0, hid0, c, h);
   // the walk's share of the norm-weight / norm-bias gradients: per wave, summed in the walk's order
   float* s_red = reinterpret_cast<float*>(smem + SB_RED);
   float* s_dgw = s_red + (v * 2 + 0) * FD;
   float* s_dbw = s_red + (v * 2 + 1) * FD;
-  if (lane < FD) { s_dgw[lane] = 0.f; s_dbw[lane] = 0.f; }
-  int n_step = 0, n_seen = 0;
+  float nr0 = 0.f, nr1 = 0.f;   // the replay's share: this lane's two words of the wave's running sum
+  {
+    float w0 = 0.f, w1 = 0.f;
+    if (!first) {
+      const float* const q = park + FD * HID + v * 4 * FD + lane;
+      w0 = q[0]; w1 = q[FD]; nr0 = q[2 * FD]; nr1 = q[3 * FD];
+    }
+    s_dgw[lane] = w0;
+    s_dbw[lane] = w1;
+  }
+  // mini-batches walked before group k_hi (the ragged group is the first), and how many of them are known to have been
+  int n_step = first ? 0 : p.NC - (k_hi + 1) * cgs, n_seen = 0;
   int lane_v = lane;
 #define FIN_LANE                                                                                  \
   asm volatile("" : "+v"(lane_v));                                                                \
@@ -1604,14 +1619,14 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
   const unsigned t16 = 16 * tid, vln = (tok * FD + f0) * 2;                                       \
   const float* s_lnrow = s_P + (1 - r) * RGN + (tok & 31) * LDR + f0;                             \
   (void)h; (void)c; (void)t16; (void)vln; (void)s_lnrow
-  float nr0 = 0.f, nr1 = 0.f;   // the replay's share: this lane's two words of the wave's running sum
   TTT_STAGES_BEGIN();
-  for (int k = p.K - 1; k >= 0; k--) {
+  int k = k_hi;
+  do {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k, set = done % n_sets;
     // the walk hands over whole groups, except the last one it walks (k = 0): that one in chunks of FIN_CHUNK mini-batches
     // (WIDE: every mini-batch is announced by both halves of the walk)
-    if (!WIDE && k > 0 && !wait_at_least(w_walked, done + 1, p.status, s_flag, p.wait_limit)) return;
+    if (!WIDE && k > 0 && !wait_at_least(w_walked, done + 1, p.status, s_flag, p.wait_limit)) return false;
     TTT_STAGE(BS_X_GROUP);
     const size_t ofin = uni64(((size_t)bh * 2 + (done & 1)) * cgs);
     const size_t o_img = uni64((size_t)bh * cgs * (CS * HID)), o_tile = uni64((size_t)bh * cgs * (CS * FD));
@@ -1683,11 +1698,11 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
       if constexpr (WIDE) {
         if (++n_step > n_seen) {
           n_seen = wait_for_both(w_sync + BWW_GIVEN, w_sync + BWW_GIVEN + 4, n_step, p.status, s_flag, p.wait_limit);
-          if (n_seen < 0) return;
+          if (n_seen < 0) return false;
         }
         TTT_STAGE(BS_X_GROUP);
       } else if (k == 0 && (j == n_mb - 1 || (j & (FIN_CHUNK - 1)) == FIN_CHUNK - 1)) {
-        if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return;
+        if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return false;
         TTT_STAGE(BS_X_GROUP);
       }
       if (j == n_mb - 1) {   // the group's norm-gradient sums: published with it, and the walk has acquired it
@@ -1791,10 +1806,17 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
       __syncthreads();   // the readers of the pair sums are done before the next mini-batch's take their place
       TTT_STAGE(BS_X_SUMS);
     }
+    if (!OWN && k > 0) {   // another workgroup goes on with the next group
+      FIN_LANE;
+      acc_store_rows(gW1s, gbuf(park), 0, HID, 0, hid0, c, h);
+      float* const q = park + FD * HID + v * 4 * FD + lane;
+      q[0] = s_dgw[lane]; q[FD] = s_dbw[lane]; q[2 * FD] = nr0; q[3 * FD] = nr1;
+    }
     publish(w_finished, done + 1);
     TTT_STAGE(BS_PUBLISH);
-  }
+  } while (OWN && --k >= 0);
   TTT_STAGES_END(bh, STAGE_ROLE_DXK);
+  if (!OWN && k > 0) return true;
   // norm-weight / norm-bias gradients: the replay's sum + the walk's, in the order of the other launch shapes
   __syncthreads();
   s_P[v * 2 * FD + lane] = nr0;
@@ -1810,30 +1832,34 @@ TTT_DEV void bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
     }
     (which == 0 ? p.grad_L_ttt_norm_weight : p.grad_L_ttt_norm_bias)[(size_t)bh * FD + f] = sr + s;
   }
+  return true;
 }
 #undef FIN_LANE
 
 #ifndef TTT_BWD_ROLES_ONLY
-// n_replay + 1 (+ 1) workgroups per (batch, head).  Workgroups are dealt to the 8 XCDs in turn, so with a
+// NREPLAY + 1 workgroups per (batch, head): one walks.  Workgroups are dealt to the 8 XCDs in turn, so with a
 // multiple of 8 (batch, head) pairs the workgroups of a pair are placed 8 apart: same XCD, same L2.
-// One kernel per combination, so that each holds only the code (and the register allocation) of its own roles.
-template <int NREPLAY, bool FINISH>
+template <int NREPLAY>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_split_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int b = blockIdx.x, per = NREPLAY + 1 + (FINISH ? 1 : 0);
+  constexpr int PER = NREPLAY + 1;
+  constexpr bool IMG = NREPLAY == 2;   // two replaying workgroups also evaluate the GELU family for the walk
+  const int b = blockIdx.x;
   int bh, role;
   if (p.nbh % 8 == 0) {
-    bh = (b / (8 * per)) * 8 + (b & 7);
-    role = (b >> 3) % per;
+    bh = (b / (8 * PER)) * 8 + (b & 7);
+    role = (b >> 3) % PER;
   } else {
-    bh = b / per;
-    role = b % per;
+    bh = b / PER;
+    role = b % PER;
   }
   bh += p.bh0;
-  constexpr bool IMG = NREPLAY == 2;   // two replaying workgroups also evaluate the GELU family for the walk
-  if (role < NREPLAY) bwd_body<1, IMG, FINISH>(p, smem, bh, role, p.K - 1, 0);
-  else if (role == NREPLAY) bwd_body<2, IMG, FINISH>(p, smem, bh, 0, p.K - 1, 0);
-  else if constexpr (FINISH) bwd_finish_dxk<true, false>(p, smem, bh);
+  if (role == NREPLAY) {
+    bwd_body<2, IMG, false>(p, smem, bh, p.K - 1, 0);
+    return;
+  }
+  for (int k = p.K - 1 - role; k >= 0; k -= NREPLAY)
+    if (!bwd_body<1, IMG, false>(p, smem, bh, k, k)) return;
 }
 
 __global__ void ttt_mlp_zero_words(int* w, int n) {
@@ -1857,16 +1883,14 @@ hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
   hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n);
-  const dim3 grid((p.n_replay + 1 + p.n_finish) * p.nbh), block(ttt::BW_THREADS);
+  const dim3 grid((p.n_replay + 1) * p.nbh), block(ttt::BW_THREADS);
   auto launch = [&](auto kernel) -> hipError_t {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };
-  if (p.n_finish) return launch(ttt::ttt_mlp_bwd_split_kernel<2, true>);
-  if (p.n_replay == 2) return launch(ttt::ttt_mlp_bwd_split_kernel<2, false>);
-  return launch(ttt::ttt_mlp_bwd_split_kernel<1, false>);
+  return p.n_replay == 2 ? launch(ttt::ttt_mlp_bwd_split_kernel<2>) : launch(ttt::ttt_mlp_bwd_split_kernel<1>);
 }
 #else
 }  // namespace ttt

@@ -7,8 +7,9 @@
 //                             gradient wrt b2, and the next mini-batch's tiles through their registers into LDS
 // The sum that crosses (the gradient wrt dl/dZ2, one fp32 tile per mini-batch and direction) is taken in two blocks of 32
 // tokens: block 0's travels while block 1 is computed, block 1's while the products that do not wait for it run.
-// Two to four further workgroups per pair replay checkpoint groups in turn (bwd_body<1>), one forms grad_L_XK / grad_L_XV and
-// the norm gradients (bwd_finish_dxk).  Every sum has the order of the one-workgroup kernel: same results to the bit.
+// Further workgroups replay checkpoint groups in turn (bwd_body<1>) or form grad_L_XK / grad_L_XV and the norm gradients
+// (bwd_finish_dxk), whole ones for each pair or shared by the pairs of an XCD; that launch also runs with the walk on one CU
+// (ttt_mlp_bwd_gang_kernel).  Every sum has the order of the one-workgroup kernel: same results to the bit.
 //
 // 48 pairs x 256 mini-batches 3.60 ms with the walk on one CU, 3.03 ms here; 48 x 4,096 49.8 -> 41.2 ms; 32 x 512 6.73 -> 5.10 ms.
 // With the stage clocks in, 21.8 k clocks per mini-batch at 48 pairs, 19.2 k at 32.  At 48 the two replaying workgroups bound
@@ -91,7 +92,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   const int u = w & 3;                                   // number among its kind
   const int v = 2 * half + (u & 1) + 4 * (u >> 1);       // compute wave u: hidden block, = wave of the one-workgroup kernel
   const int head = bh % p.NH, hid0 = BW_NS * v;
-  const int cgs = p.cgs, n_sets = p.n_sets, n_replay = p.n_replay;
+  const int cgs = p.cgs, n_sets = p.n_sets;
   bf16* const s_xq = reinterpret_cast<bf16*>(smem + BWW_XQ);
   bf16* const s_gzb = reinterpret_cast<bf16*>(smem + BWW_GZB);
   bf16* const s_dz2 = reinterpret_cast<bf16*>(smem + BWW_DZ2);
@@ -507,7 +508,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
     if (!__all(lane != 0 || wait_word(word, target, w_status, p.wait_limit))) gave_up = true;
   };
   // group number `done` (from the end) has been replayed
-  auto wait_group = [&](int done) { wait_for(words + done % n_replay, done / n_replay + 1); };
+  auto wait_group = [&](int done) { wait_for(words + done % n_sets, done + 1); };
   // What one mini-batch needs from HBM besides the operand images: a chunk of 16 bytes per lane and token block of each
   // tile - the lanes that hold a chunk are the LayerNorm lanes of that token and those features.
   struct Ahead {
@@ -553,7 +554,8 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   };
   const bool near = [&]() {
     bool alive = true;
-    const bool one = on_one_xcd(words + BWW_XCD, 3, lane, w_status, p.wait_limit, alive);
+    bool one = on_one_xcd(words + BWW_XCD, 2, lane, w_status, p.wait_limit, alive);
+    one = workers_here(words + BWW_WORKERS, p.n_finish + p.n_replay, w_status, p.wait_limit, alive) && one;
     if (!alive) gave_up = true;
     return one;
   }();
@@ -729,7 +731,7 @@ constexpr int BWW_AHEAD = 2;
 TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const int bh) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int v = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cgs = p.cgs, n_replay = p.n_replay, n_sets = p.n_sets;
+  const int cgs = p.cgs, n_sets = p.n_sets;
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   int* const s_flag = reinterpret_cast<int*>(smem + BWW_FLAG);
   const size_t ox = uni64((size_t)bh * p.NC * (CS * FD)), of = uni64((size_t)bh * cgs * (CS * FD)), oh = uni64((size_t)bh * cgs * (CS * HID));
@@ -739,7 +741,7 @@ TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const in
   for (int k = p.K - 1; k >= 0; k--) {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k, set = done % n_sets;
-    if (!wait_at_least(words + done % n_replay, done / n_replay + 1, p.status, s_flag, p.wait_limit)) return;
+    if (!wait_at_least(words + set, done + 1, p.status, s_flag, p.wait_limit)) return;
 #define PGRP(name) (set ? p.alt_##name[set - 1] : p.name)
     // wave v: tile v (two inputs, four of the set); waves 0-3 / 4-7: one image each of a pair
     gptr_t tile = gbuf(p.XQ + ox);
@@ -774,27 +776,57 @@ TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const in
   }
 }
 
-// Per (batch, head): two workgroups that walk, one for grad_L_XK, one that reads ahead (PREFETCH), NREPLAY that replay; laid out like
-// the wide forward's.
-template <int NREPLAY, bool PREFETCH>
-__global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_wide_kernel(const BwdParams p) {
+// The workgroups of a gang: gang g has pairs g, g + 8, .. and, as workgroups are dealt to the 8 XCDs in turn, one XCD.  WALKERS of
+// them walk each pair, the others work for all of its pairs: n_replay take the replays in turn, ordered by group and then by
+// pair (all walks go at one pace), n_finish the finishing of the groups (grad_L_XK and the norm gradients) in the same
+// order, PREFETCH: one per pair reads ahead of its walk.  With a finishing workgroup for each pair it stays with that
+// pair; with fewer, the last group of each pair is finished by a replaying workgroup, all of them together.
+// Nobody waits for a later job than his own: a replay waits for the set of n_sets groups ago to be walked and finished, the
+// finishing of a group for its walk and the group before, a walk for its replay and the finishing of two groups ago; so of
+// the jobs not yet done the first can always go on.
+template <bool WIDE, bool IMG, bool PREFETCH, bool OWN>
+__global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int PER = NREPLAY + 3 + (PREFETCH ? 1 : 0);
-  constexpr bool IMG = NREPLAY > 2;   // with the replay to spare it also evaluates the GELU family for the walk
-  const int b = blockIdx.x;
-  int bh = p.scatter ? b / PER : (b / (8 * PER)) * 8 + (b & 7);
-  const int role = (p.scatter ? b : b >> 3) % PER;
-  if (bh >= p.nbh) return;
-  bh += p.bh0;
-  if (role < 2) {
-    bwd_wide_walk<IMG>(p, smem, bh, role);
-  } else if (role == 2) {
-    if (threadIdx.x == 0) say_xcd(p.sync + (size_t)bh * BWD_SYNC_STRIDE + BWW_XCD + 2);
-    bwd_finish_dxk<IMG, true>(p, smem, bh);
-  } else if (PREFETCH && role == PER - 1) {
-    bwd_wide_prefetch(p, smem, bh);
+  const int b = blockIdx.x, walkers = (WIDE ? 2 : 1) * p.gang_pairs;
+  const int slots = walkers + p.n_finish + p.n_replay + (PREFETCH ? p.gang_pairs : 0);
+  const int gang = uni(p.scatter ? b / slots : b & 7);   // (a division leaves its result in a vector register)
+  int slot = uni(p.scatter ? b % slots : b >> 3);
+  const int pairs = (p.nbh - gang + 7) / 8;   // of this gang
+  if (pairs <= 0) return;
+  const int bh0 = p.bh0 + gang;
+  if (slot < walkers) {
+    const int i = WIDE ? slot >> 1 : slot;
+    if (i >= pairs) return;
+    if constexpr (WIDE) bwd_wide_walk<IMG>(p, smem, bh0 + 8 * i, slot & 1);
+    else bwd_body<2, IMG, true>(p, smem, bh0 + 8 * i, p.K - 1, 0);
+    return;
+  }
+  slot -= walkers;
+  if constexpr (PREFETCH) {
+    if (slot >= p.n_finish + p.n_replay) {
+      const int i = slot - (p.n_finish + p.n_replay);
+      if (i < pairs) bwd_wide_prefetch(p, smem, bh0 + 8 * i);
+      return;
+    }
+  }
+  if (WIDE && threadIdx.x < pairs) say_worker(p.sync + (size_t)(bh0 + 8 * (int)threadIdx.x) * BWD_SYNC_STRIDE + BWW_WORKERS);
+  const bool replays = slot >= p.n_finish;
+  const int r = slot - p.n_finish;
+  if (replays) {
+    for (int job = r; job < p.K * pairs; job += p.n_replay) {
+      const int done = uni(job / pairs), k = p.K - 1 - done;
+      if (!bwd_body<1, IMG, true, WIDE>(p, smem, bh0 + 8 * (job - done * pairs), k, k)) return;
+    }
+  }
+  if constexpr (OWN) {
+    if (!replays && slot < pairs) bwd_finish_dxk<IMG, WIDE, true>(p, smem, bh0 + 8 * slot, p.K - 1);
   } else {
-    bwd_body<1, IMG, true, true>(p, smem, bh, role - 3, p.K - 1, 0);
+    // (n_replay >= pairs: one of the last groups each)
+    const int last = (p.K - 1) * pairs, end = replays ? last + pairs : last;
+    for (int job = replays ? last + r : slot; job < end; job += replays ? p.n_replay : p.n_finish) {
+      const int done = uni(job / pairs);
+      if (!bwd_finish_dxk<IMG, WIDE, false>(p, smem, bh0 + 8 * (job - done * pairs), p.K - 1 - done)) return;
+    }
   }
 }
 
@@ -807,22 +839,22 @@ __global__ void ttt_mlp_bwd_wide_clear(int* w, int n, uint4* x, int nx) {
 
 }  // namespace ttt
 
-hipError_t ttt_mlp_bwd_wide_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
+hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-  const int nx = p.nbh * (ttt::BWW_XCHG_WORDS / 2);
+  const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
   hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n,
                      reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
-  const dim3 grid((p.nbh + 7) / 8 * 8 * (p.n_replay + 3 + p.n_prefetch)), block(ttt::BW_THREADS);
+  const int slots = (p.wide ? 2 : 1) * p.gang_pairs + p.n_finish + p.n_replay + (p.n_prefetch ? p.gang_pairs : 0);
+  const dim3 grid(8 * slots), block(ttt::BW_THREADS);
   auto launch = [&](auto kernel) -> hipError_t {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };
-  if (p.n_prefetch) {
-    if (p.n_replay == 4) return launch(ttt::ttt_mlp_bwd_wide_kernel<4, true>);
-    return launch(ttt::ttt_mlp_bwd_wide_kernel<3, true>);
-  }
-  return launch(ttt::ttt_mlp_bwd_wide_kernel<2, false>);
+  const bool own = p.n_finish == p.gang_pairs;
+  if (p.n_prefetch) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, true, true, true>);
+  if (p.wide) return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true>) : launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, false>);
+  return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, true>) : launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, false>);
 }

@@ -146,19 +146,41 @@ int make_bwd_params(const ttt_mlp_bwd_args* a, ttt::BwdParams& p) {
 // (batch, head) pairs are therefore covered by two launches in a row: as many full rounds of one
 // workgroup per pair as there are (a multiple of the CU count), then the rest - with several workgroups per
 // pair if two each fit the device (split), otherwise with one.
-// With the recurrence (walk) of a pair on two CUs (wide) the workgroups of a pair share an XCD: the grid is padded to a
-// multiple of 8 pairs and dealt to the 8 XCDs in turn, so those of ceil(pairs / 8) pairs must fit an eighth of the CUs.
+// With the recurrence (walk) of a pair on two CUs (wide), or workgroups that serve several pairs (gang), the workgroups of a
+// pair share an XCD: the grid is padded to a multiple of 8 pairs and dealt to the 8 XCDs in turn, so those of
+// ceil(pairs / 8) pairs must fit an eighth of the CUs.
 struct LaunchPlan {
   long long n_single = 0;   // pairs 0 .. n_single-1: one workgroup each
   long long n_rest = 0;     // pairs n_single .. n_single+n_rest-1
   bool rest_split = false;
   bool wide = false;
-  int per_pair = 1;         // workgroups per pair of the rest, in every role
+  int per_pair = 1;         // workgroups per pair of the rest, in every role (whole ones, at most five, where some are shared)
   int n_out = 0;            // forward, wide: that compute Out
-  int n_replay = 0;         // backward: that replay checkpoint groups
-  bool finish = false;      // backward: one more for grad_L_XK / grad_L_XV
-  bool prefetch = false;    // backward, wide: and one that fetches ahead of the walk
+  int gang = 0;             // backward: pairs of an XCD that share workgroups, 0: whole ones, that replay or walk, for each pair
+  int n_replay = 0;         // backward: that replay checkpoint groups, of a gang or of a pair
+  int n_finish = 0;         // backward, of a gang: for grad_L_XK / grad_L_XV
+  bool prefetch = false;    // backward, wide: and one per pair that fetches ahead of the walk
+  int sets = 0;             // backward: sets of the per-group tensors
 };
+// Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
+// of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others.
+constexpr int COST_REPLAY = 443, COST_FINISH = 200, COST_REPLAY_IMG = 488, COST_FINISH_IMG = 185;
+// `workers` of an XCD divided between replaying and finishing for its `pairs`, so that the slower of the two is as fast as can be;
+// a finishing workgroup for each pair, which then follows its walk closely, where the replay still keeps up with `walk`.
+void divide_workers(int pairs, int workers, int walk, int replay, int finish, int* n_replay, int* n_finish) {
+  *n_finish = pairs;
+  if (workers - pairs < pairs || replay * pairs > walk * (workers - pairs)) {
+    int best = 0;
+    for (int f = 1; f < pairs && workers - f >= pairs; f++) {
+      const int r = workers - f, tr = replay * pairs / r, tf = finish * pairs / f, t = tr > tf ? tr : tf;
+      if (best == 0 || t < best) {
+        best = t;
+        *n_finish = f;
+      }
+    }
+  }
+  *n_replay = workers - *n_finish;
+}
 LaunchPlan plan_for(long long BH, int cus, bool backward) {
   LaunchPlan pl;
   if (BH <= 0 || cus <= 0) {
@@ -182,20 +204,42 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     pl.per_pair = 2 + pl.n_out;
     return pl;
   }
-  // Two replaying workgroups bound a walk on two CUs (48 pairs x 4,096 mini-batches: 20 us per replayed mini-batch, 10.1 us per
-  // walked one).  Four leave it to itself, also where they evaluate the GELU family for it (32 pairs x 512: 25 us per
-  // replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).
-  pl.n_replay = fits_xcd(8) ? 4 : fits_xcd(7) ? 3 : fits_xcd(5) ? 2 : 0;
-  pl.wide = pl.n_replay > 0;
-  if (pl.wide) {
-    pl.finish = true;
-    pl.prefetch = pl.n_replay > 2;
-    pl.per_pair = 2 + pl.n_replay + 1 + (pl.prefetch ? 1 : 0);
+  // Four replaying workgroups per pair leave a walk on two CUs to itself, also where they evaluate the GELU family for it (32 pairs x 512:
+  // 25 us per replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).
+  const int on_xcd = cus / 8, pairs = static_cast<int>(per_xcd);
+  if (fits_xcd(7)) {
+    const int each = fits_xcd(8) ? 4 : 3;
+    pl.wide = pl.prefetch = true;
+    pl.gang = pl.n_finish = pairs;
+    pl.n_replay = each * pairs;
+    pl.per_pair = each + 4;
+    pl.sets = each + 2;
     return pl;
   }
-  pl.finish = 4 * pl.n_rest <= cus;
+  // Two replaying workgroups per pair bound a walk on two CUs (48 pairs x 4,096 mini-batches: 20 us per replayed mini-batch, 10.1 us
+  // per walked one); a third for some of the pairs gained nothing (48 x 512: 5.95 ms with 12 or 14 of them on an XCD).  With less
+  // room than that the workgroups of an XCD that replay and those that finish serve all of its pairs.  The walks take two CUs
+  // each from 4.5 CUs per pair on (56 pairs x 512 7.75 -> 6.85 ms, 51 x 77 1.46 -> 1.22 ms against one CU each and four whole
+  // workgroups per pair; but 64 x 512 8.30 ms so, 8.13 with one CU each), one from 3 CUs on (72 x 512 9.57 -> 8.96 ms, 80 x 512
+  // 9.71 -> 9.35 ms against three whole workgroups per pair; but 96 x 512 11.3 ms so, 10.3 with two).
+  if (3 * pairs <= on_xcd) {
+    pl.wide = 9 * pairs <= 2 * on_xcd;
+    pl.gang = pairs;
+    if (fits_xcd(5)) {
+      pl.n_finish = pairs;
+      pl.n_replay = 2 * pairs;
+    } else if (pl.wide) {
+      divide_workers(pairs, on_xcd - 2 * pairs, 215, COST_REPLAY, COST_FINISH, &pl.n_replay, &pl.n_finish);
+    } else {
+      divide_workers(pairs, on_xcd - pairs, 330, COST_REPLAY_IMG, COST_FINISH_IMG, &pl.n_replay, &pl.n_finish);
+    }
+    pl.per_pair = on_xcd / pairs < 5 ? on_xcd / pairs : 5;
+    pl.sets = 4;
+    return pl;
+  }
   pl.n_replay = 3 * pl.n_rest <= cus ? 2 : 1;
-  pl.per_pair = 1 + pl.n_replay + (pl.finish ? 1 : 0);
+  pl.per_pair = pl.n_replay + 1;
+  pl.sets = 2 * pl.n_replay;
   return pl;
 }
 int device_cus() {
@@ -252,14 +296,14 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backwa
 // round or, with several workgroups per pair, a shorter one.  Measured on 256 CUs as what the rest adds to full rounds
 // (6.5 ms forward, 23.1 ms backward for 512 mini-batches), at the most pairs of a shape.  Forward: 530 per mini-batch (4 pairs; 430
 // for 64), 545 (80 pairs) and 650 (128 pairs), and the mini-batches by which Out trails.  The backward's walk waits for the
-// first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at K = 16, 320 at 4; 48 pairs 265 and 335, 64 pairs 350 and
-// 435, 80 pairs 435 and 515, 128 pairs 500 and 605.
+// first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at K = 16, 320 at 4; 48 pairs 265 and 335, 56 pairs 290 at
+// K = 16, 64 pairs 350 and 435, 80 pairs 410 at K = 16, 85 pairs 435 and 515 at 4, 128 pairs 500 and 605.
 // A last round that is not full is 5 % shorter than a full one (400 to 456 pairs).
 // What the estimate decides: 312 pairs x 101 mini-batches in 4 groups, forward 1.70 ms cut, 1.93 uncut; 384 x 31 in 16, 0.65 and
 // 0.78; 276 x 329 in 22, backward 17.5 and 18.7; 330 x 395 in 18, 24.3 and 27.3; 384 x 512 in 16, 35.1 and 34.8.
 long long rest_x1000(const LaunchPlan& pl, int NC, int K, bool backward) {
   if (!backward) return pl.n_out == 2 ? 525LL * NC + 3000 : pl.n_out == 1 ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
-  const int walk = pl.wide ? (pl.n_replay > 2 ? 210 : 235) : pl.finish ? 325 : pl.n_replay == 2 ? 405 : 485;
+  const int walk = pl.prefetch ? 210 : pl.wide ? (pl.gang > 6 ? 290 : 235) : pl.gang > 8 ? 380 : pl.gang ? 325 : pl.n_replay == 2 ? 405 : 485;
   return (long long)(walk + 470 / K) * NC;
 }
 long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace, bool backward) {
@@ -293,27 +337,27 @@ SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, in
   return plan_segments(pairs, cus, NC, cgs, true, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, true));
 }
 
-// Sets of the per-group tensors that carry replayed groups to the walk, used in turn: two per replaying workgroup, or one each
-// and two more where four of them run ahead of a walk on two CUs.  Set 0 is the caller's own; a sequence of K groups uses K.
-int bwd_sets(const LaunchPlan& pl) { return pl.wide ? pl.n_replay + 2 : 2 * pl.n_replay; }
-int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K < bwd_sets(pl) ? K : bwd_sets(pl)); }
-// The launch with less workspace for the same pairs: two replaying workgroups instead of three or four.
+// Sets of the per-group tensors that carry replayed groups to the walk, used in turn.  Set 0 is the caller's own; a sequence of K
+// groups uses K.
+int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K < pl.sets ? K : pl.sets); }
+// The launch with less workspace for the same pairs: two replaying workgroups per pair instead of three or four.
 LaunchPlan bwd_reduced(LaunchPlan pl) {
-  if (pl.wide && pl.n_replay > 2) {
-    pl.n_replay = 2;
+  if (pl.prefetch) {
+    pl.n_replay = 2 * pl.gang;
     pl.prefetch = false;
     pl.per_pair = 5;
+    pl.sets = 4;
   }
   return pl;
 }
 // Workspace of the backward with several workgroups per pair, for n (batch, head) pairs of K groups: the synchronisation
 // words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
 // CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
-// gradient terms, per slot, two sets), then the sets of per-group tensors beyond the caller's; each part 256-byte aligned.
+// gradient terms, per slot, two sets), what fewer of those than pairs park between two groups, then the sets of per-group tensors beyond the caller's; each part 256-byte aligned.
 struct BwdWorkspace {
   static constexpr int PER_SET = 11;
   static constexpr int ALT_SETS = ttt::BWD_MAX_SETS - 1;
-  static constexpr int FIRST_SET = 7;
+  static constexpr int FIRST_SET = 8;
   static constexpr int PARTS = FIRST_SET + PER_SET * ALT_SETS;
   size_t off[PARTS];
   size_t total;
@@ -335,8 +379,9 @@ struct BwdWorkspace {
     put(2, norm);
     put(3, (size_t)n * img);
     put(4, pl.wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);
-    put(5, pl.finish ? 2 * slot * img : 0);
-    put(6, pl.finish ? 2 * slot * 4 * tile : 0);
+    put(5, pl.gang ? 2 * slot * img : 0);
+    put(6, pl.gang ? 2 * slot * 4 * tile : 0);
+    put(7, pl.n_finish < pl.gang ? (size_t)n * ttt::FIN_PARK_FLOATS * sizeof(float) : 0);
     for (int s = 0; s < ALT_SETS; s++)
       for (int t = 0; t < PER_SET; t++) put(FIRST_SET + PER_SET * s + t, s < alt_sets ? per_set[t] : 0);
     total = o;
@@ -455,14 +500,17 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   const size_t norm = 8 * 2 * TTT_MLP_F;
   p.bh0 = static_cast<int>(pl.n_single);
   p.nbh = static_cast<int>(pl.n_rest);
+  p.gang_pairs = pl.gang;
   p.n_replay = pl.n_replay;
-  p.n_sets = bwd_sets(pl);
-  p.n_finish = pl.finish ? 1 : 0;
+  p.n_sets = pl.sets;
+  p.n_finish = pl.n_finish;
   p.n_prefetch = pl.prefetch ? 1 : 0;
+  p.wide = pl.wide ? 1 : 0;
   p.wait_limit = g_wait_limit;
-  if (pl.finish) {
+  if (pl.gang) {
     p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[5]) - b0 * 2 * img;
     p.fin_gy = reinterpret_cast<float*>(base + w.off[6]) - b0 * 2 * 2 * tile;
+    p.fin_park = reinterpret_cast<float*>(base + w.off[7]) - b0 * ttt::FIN_PARK_FLOATS;
   }
   int* words = reinterpret_cast<int*>(base + w.off[0]);
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
@@ -494,10 +542,10 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
     p.alt_std_fused_group[s] = reinterpret_cast<float*>(base + o[9]) - b0 * vec;
     p.alt_W1_init_group[s] = reinterpret_cast<float*>(base + o[10]) - b0 * img;   // [cgs][64][256] floats = 2 images per slot
   }
-  if (pl.wide) {
+  if (pl.gang) {
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
     p.scatter = scatter ? 1 : 0;
-    return static_cast<int>(ttt_mlp_bwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
+    return static_cast<int>(ttt_mlp_bwd_gang_enqueue(p, static_cast<hipStream_t>(stream)));
   }
   return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
 }

@@ -403,7 +403,7 @@ TTT_DEV float bf2f(bf16 x) { return (float)x; }
   do {                                                                                                     \
     if (p.stage_clocks != nullptr && (threadIdx.x & 63) == 0)                                              \
       for (int i_ = 0; i_ < STAGE_SLOTS; i_++)                                                             \
-        p.stage_clocks[(((size_t)(bh) * STAGE_ROLES + (role)) * 8 + (threadIdx.x >> 6)) * STAGE_SLOTS + i_] = stage_acc[i_]; \
+        atomicAdd(&p.stage_clocks[(((size_t)(bh) * STAGE_ROLES + (role)) * 8 + (threadIdx.x >> 6)) * STAGE_SLOTS + i_], stage_acc[i_]); \
   } while (0)
 #else
 #define TTT_STAGES_BEGIN() ((void)0)

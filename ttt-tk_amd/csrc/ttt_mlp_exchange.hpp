@@ -69,6 +69,31 @@ TTT_DEV bool on_one_xcd(int* words, int n, int lane, int* status, uint64_t limit
   alive = __all(ok);
   return __all(here);
 }
+// The workgroups that work for several pairs: each adds itself to a pair's word, a byte per XCD; true: all `total` of them are on
+// the caller's.
+TTT_DEV void say_worker(int* word) {
+  unsigned xcc;
+  asm volatile("s_getreg_b32 %0, hwreg(20, 0, 4)" : "=s"(xcc));   // XCC_ID
+  __hip_atomic_fetch_add(reinterpret_cast<uint64_t*>(word), 1ull << (8 * (xcc & 7)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+TTT_DEV bool workers_here(int* word, int total, int* status, uint64_t limit, bool& alive) {
+  unsigned xcc;
+  asm volatile("s_getreg_b32 %0, hwreg(20, 0, 4)" : "=s"(xcc));
+  uint64_t x;
+  bool ok = true;
+  const uint64_t t0 = wall_clock64();
+  while (((x = __hip_atomic_load(reinterpret_cast<uint64_t*>(word), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) * 0x0101010101010101ull) >> 56 <
+         static_cast<uint64_t>(total)) {
+    if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
+      __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ok = false;
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  alive = __all(ok) && alive;
+  return __all(((x >> (8 * (xcc & 7))) & 255) == static_cast<uint64_t>(total));
+}
 // One thread: waits until `word` has reached `target` and orders what follows after it.  False: gave up.
 TTT_DEV bool wait_word(int* word, int target, int* status, uint64_t limit) {
   const uint64_t t0 = wall_clock64();

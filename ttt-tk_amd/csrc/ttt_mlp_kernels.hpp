@@ -63,11 +63,9 @@ struct BwdParams {
   float *grad_L_W1_init, *grad_L_b1_init, *grad_L_W2_init, *grad_L_b2_init;
   __bf16 *grad_L_last_eta, *grad_L_XQ, *grad_L_XK, *grad_L_XV;
   int B, NH, NC, K, cgs;
-  // Several workgroups per (batch, head) only (sync != nullptr): n_replay workgroups replay the checkpoint groups (taking
-  // turns; 1 or 2, with the walk on two workgroups 2 to 4), one or two walk them backwards.  Group number g (0 = the last
-  // group of the sequence) is replayed into set g % n_sets of the per-group tensors that carry it to the walk:
-  // set 0 = the caller's tensors, sets 1.. = alt_*[set - 1] from the workspace; n_sets = 2 * n_replay, with the walk on two
-  // workgroups n_replay + 2 (the kernels with the walk on one do not read it).
+  // Several workgroups per (batch, head) only (sync != nullptr): replays, the walk and, in a gang, the finishing of the groups
+  // on workgroups of their own.  Group number g (0 = the last group of the sequence) is replayed into set g % n_sets of the
+  // per-group tensors that carry it to the walk: set 0 = the caller's tensors, sets 1.. = alt_*[set - 1] from the workspace.
   __bf16 *alt_X2_group[BWD_MAX_SETS - 1], *alt_Z1_group[BWD_MAX_SETS - 1], *alt_Z1_bar_group[BWD_MAX_SETS - 1], *alt_X2_bar_group[BWD_MAX_SETS - 1];
   __bf16 *alt_grad_l_wrt_Z2_group[BWD_MAX_SETS - 1], *alt_grad_l_wrt_Z1_group[BWD_MAX_SETS - 1];
   __bf16 *alt_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_output_fused_group[BWD_MAX_SETS - 1];
@@ -76,20 +74,23 @@ struct BwdParams {
   float* norm_partial;   // [B*NH][BWD_MAX_SETS][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set
   float* norm_park;      // [B*NH][8 waves][2][64]: their sum over the groups walked so far (without a grad_L_XK workgroup)
   __bf16* walk_park;     // [B*NH][64][256]: one register image the walking workgroup parks across its LayerNorm stage
-  int n_replay;
-  // n_finish = 1: a further workgroup forms grad_L_XK, grad_L_XV and the walk's share of the norm gradients from
-  // what the walk hands it per mini-batch - one register image (dZ1: [B*NH][2 sets][cgs][64][256] bf16) and two
-  // fp32 tiles (g_y and the norm-weight gradient terms: [B*NH][2][cgs][2][64][64]); the two sets alternate by
-  // group.  It keeps its own copy of the running gradient wrt W1 and forms G1 = -eta * dl/dZ1 itself.
+  // Gang (gang_pairs > 0: pairs per XCD, gang g = pairs g, g + 8, ..; ttt_mlp_bwd_wide.hip): n_replay workgroups replay for all of
+  // its pairs, n_finish form grad_L_XK, grad_L_XV and the walk's share of the norm gradients from what the walk hands over per
+  // mini-batch - one register image (dZ1: [B*NH][2 sets][cgs][64][256] bf16) and two fp32 tiles (g_y and the norm-weight
+  // gradient terms: [B*NH][2][cgs][2][64][64]); the two sets alternate by group.  They keep their own copy of the running
+  // gradient wrt W1 and form G1 = -eta * dl/dZ1 themselves; fin_park: [B*NH][FIN_PARK_FLOATS], that copy and the norm-gradient
+  // sums between two groups of a pair (n_finish < gang_pairs only).
+  int gang_pairs, n_replay, n_finish;
   __bf16* fin_dz;
   float* fin_gy;
-  int n_finish;
-  // Walk on two workgroups (ttt_mlp_bwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
-  // 256 8-byte words]; n_finish = 1.
-  // n_prefetch = 1 (with three or four replaying workgroups): one more workgroup reads nothing for itself; it touches every
+  float* fin_park;
+  // wide: the walk on two workgroups, which exchange through xchg, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
+  // 256 8-byte words].
+  // n_prefetch = 1 (with three or four replaying workgroups per pair): one more per pair reads nothing for itself; it touches every
   // cache line that the walk is about to ask for, ahead of it, so that the walk's own requests are answered by the L2 the
   // two share instead of by HBM.
-  // scatter: the workgroups of a pair on consecutive XCDs instead of on one, for tests.
+  // scatter: the workgroups of a gang on consecutive XCDs instead of on one, for tests.
+  int wide;
   unsigned long long* xchg;
   int n_sets;
   int n_prefetch, scatter;
@@ -108,18 +109,17 @@ struct BwdParams {
 #endif
 };
 
-// Layout of `sync` (ints): 32 per (batch, head).  Walk on one workgroup: words 0 and 8 count the groups replayed by the first /
-// second replaying workgroup (norm_partial is written with the group), word 16 the groups the
-// reverse walk has finished, word 12 the mini-batches of the last group it walks that it has handed to the grad_L_XK
-// workgroup (that group is handed over in chunks), word 24 the groups the grad_L_XK workgroup has finished - then one status
-// word (non-zero: a wait gave up).
+// Layout of `sync` (ints): 32 per (batch, head).  Words 0 .. 5: the group last replayed into each set, its number from the end + 1
+// (norm_partial is written with the group).  Walk on one workgroup: word 16 the groups it has finished, word 12 the
+// mini-batches of the last group it walks that it has handed on (that group is handed over in chunks).  Word 24 the groups
+// whose finishing is done - then one status word behind all of them (non-zero: a wait gave up).
 constexpr int BWD_SYNC_STRIDE = 32;
-// With the walk on two workgroups: words 0 .. 3 groups replayed by each replaying workgroup, BWW_WALKED + 0 / 4 groups and
-// BWW_GIVEN + 0 / 4 mini-batches done by the two halves of the walk, 24 as above, BWW_XCD .. the XCDs of the two halves
-// and the grad_L_XK workgroup.
+// With the walk on two workgroups: BWW_WALKED + 0 / 4 groups and BWW_GIVEN + 0 / 4 mini-batches done by its two halves,
+// BWW_XCD .. their XCDs, BWW_WORKERS (two words) the gang's other workgroups by XCD.
 constexpr int BWW_WORDS = 9;                                // per lane: two times 8 fp32 sums and the token's share of d eta
 constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 144 KiB
-constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26;
+constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26, BWW_WORKERS = 28;
+constexpr int FIN_PARK_FLOATS = 64 * 256 + 8 * 4 * 64;
 inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }
 
 // ---- optional stage clocks.  A library built with -DTTT_STAGE_CLOCKS (stage_clocks.py builds one beside the product
@@ -238,8 +238,8 @@ hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream)
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
 // p.sync == nullptr: one workgroup per (batch, head); otherwise two (replay / reverse walk).
 hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream);
-// The walk of every pair on two workgroups, p.n_replay replaying ones and one for grad_L_XK.
-hipError_t ttt_mlp_bwd_wide_enqueue(const ttt::BwdParams& p, hipStream_t stream);
+// Gangs: p.gang_pairs pairs per XCD, walked by one or two workgroups each (p.wide), and workgroups that serve all of them.
+hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream);
 // Replays checkpoint group 0 and writes the sixteen per-group tensors row-major (side path, one workgroup per pair).
 hipError_t ttt_mlp_export_group0_enqueue(const ttt::BwdParams& p, hipStream_t stream);
 extern "C" int ttt_mlp_fwd_lds_bytes();

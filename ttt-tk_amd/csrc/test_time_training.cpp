@@ -8,6 +8,9 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <mutex>
+#include <vector>
+
 #include "ttt_mlp_operator.h"
 
 namespace {
@@ -18,8 +21,6 @@ bool g_fill_group_tensors = false;   // leave the values of checkpoint group 0 i
 bool g_accumulate = true;            // grad_L_XQ / XK / XV / last_eta are added to (upstream behaviour) rather than overwritten
 bool g_overlap = true;      // several workgroups per (batch, head) whenever they fit the device
 unsigned long long g_wait_ticks = 2000000000ull;   // mirrors the library's limit, for the error text
-torch::Tensor* g_sticky = nullptr;   // a device int, non-zero once a launch that nobody waited for gave up a wait (never freed:
-                                     // a static tensor would be destroyed after the runtime at process exit)
 torch::Tensor* g_workspace = nullptr;   // caller-owned workspace of the multi-workgroup launches (set_workspace); never freed here
 int g_last_forward_mode = -1;    // 0 = one workgroup per (batch, head), 1 = several
 int g_last_backward_mode = -1;
@@ -46,44 +47,100 @@ void check_eta(const torch::Tensor& t, const char* name, int64_t B, int64_t NH, 
 const uint16_t* bfp(const torch::Tensor& t) { return reinterpret_cast<const uint16_t*>(t.data_ptr<at::BFloat16>()); }
 uint16_t* bfp_mut(const torch::Tensor& t) { return reinterpret_cast<uint16_t*>(t.data_ptr<at::BFloat16>()); }
 
-// `status` (may be null): device address of the status word of a launch with several workgroups per
-// (batch, head); it can only be looked at when the host waits for the stream anyway.
 std::string gave_up_text() {
   return "a workgroup waited " + std::to_string(g_wait_ticks / 100000000.0) + " s for its partner and gave up (were all "
          "compute units available to this launch?); the outputs are invalid - set_overlap(False) avoids the mode";
 }
 
-// The device int that collects the status words of launches the host did not wait for.
-int* sticky_word(const torch::Device& dev) {
-  if (g_sticky == nullptr || g_sticky->device() != dev)
-    g_sticky = new torch::Tensor(torch::zeros({1}, torch::TensorOptions().dtype(torch::kInt32).device(dev)));
-  return g_sticky->data_ptr<int>();
-}
-
-void finish(int rc, hipStream_t stream, const char* what, const torch::Device& dev, const void* status = nullptr) {
-  TORCH_CHECK(rc == TTT_MLP_OK, what, " launch failed: ", ttt_mlp_error_string(rc));
-  if (!g_synchronize && status != nullptr) {
-    // nobody looks at the status word before the workspace goes back to the allocator: fold it into a word that stays
-    rc = ttt_mlp_status_accumulate(status, sticky_word(dev), stream);
-    TORCH_CHECK(rc == TTT_MLP_OK, what, " launch failed: ", ttt_mlp_error_string(rc));
-  }
-  if (g_synchronize) {
-    hipError_t e = hipStreamSynchronize(stream);
-    TORCH_CHECK(e == hipSuccess, what, " execution failed: ", hipGetErrorString(e));
-    if (status != nullptr) {
-      int word = 0;
-      e = hipMemcpy(&word, status, sizeof(int), hipMemcpyDeviceToHost);
-      TORCH_CHECK(e == hipSuccess, what, " execution failed: ", hipGetErrorString(e));
-      TORCH_CHECK(word == 0, what, ": ", gave_up_text());
+// Ints in host memory that the device writes when a wait gives up, so that after its own wait for the stream the host knows without
+// a copy from the device (a second wait: forward of 2 pairs x 4 mini-batches 75.3 us with it, 62.8 us so).  One block, allocated at the first
+// launch that needs one and kept for the process; word 0 collects the launches that nobody waits for, the others serve one
+// waiting call each.
+struct ReportWords {
+  static constexpr int WORDS = 64, STRIDE = 16;   // ints; a cache line each
+  std::mutex mutex;
+  int* block = nullptr;
+  bool asked = false;
+  std::vector<int> unused;
+  bool ready() {   // (mutex held)
+    if (!asked) {
+      asked = true;
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // the caller may be recording a graph
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      void* p = nullptr;
+      if (hipHostMalloc(&p, WORDS * STRIDE * sizeof(int), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+        block = static_cast<int*>(p);
+        for (int i = 0; i < WORDS * STRIDE; i++) block[i] = 0;
+        for (int i = 1; i < WORDS; i++) unused.push_back(i);
+      } else {
+        (void)hipGetLastError();
+      }
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
     }
+    return block != nullptr;
   }
+  int* collecting() {
+    const std::lock_guard<std::mutex> lock(mutex);
+    return ready() ? block : nullptr;
+  }
+  int* take() {   // nullptr: none left
+    const std::lock_guard<std::mutex> lock(mutex);
+    if (!ready() || unused.empty()) return nullptr;
+    int* const w = block + unused.back() * STRIDE;
+    unused.pop_back();
+    __atomic_store_n(w, 0, __ATOMIC_RELAXED);
+    return w;
+  }
+  void give(int* w) {
+    const std::lock_guard<std::mutex> lock(mutex);
+    unused.push_back(static_cast<int>(w - block) / STRIDE);
+  }
+};
+ReportWords& report_words() {
+  static ReportWords* const words = new ReportWords;   // (not destroyed: launches may outlive the end of main)
+  return *words;
+}
+int g_unwaited_device = -1;   // of the last launch with several workgroups per pair that nobody waited for
+
+// A launch with several workgroups per (batch, head): enqueued by `launch(report word)`, waited for and checked unless the host
+// does not wait.  `status`: device address of the launch's status word.
+template <class Launch>
+void run_overlapped(Launch launch, hipStream_t stream, const char* what, const torch::Device& dev, const void* status) {
+  struct Word {
+    int* w;
+    ~Word() { if (w != nullptr) report_words().give(w); }
+  } word{g_synchronize ? report_words().take() : nullptr};
+  int* const collecting = g_synchronize ? nullptr : report_words().collecting();
+  TORCH_CHECK(g_synchronize || collecting != nullptr, what, ": no host memory for the status of a launch that is not waited for");
+  const int rc = launch(g_synchronize ? word.w : collecting);
+  TORCH_CHECK(rc == TTT_MLP_OK, what, " launch failed: ", ttt_mlp_error_string(rc));
+  if (!g_synchronize) {
+    g_unwaited_device = dev.index();
+    return;
+  }
+  hipError_t e = hipStreamSynchronize(stream);
+  TORCH_CHECK(e == hipSuccess, what, " execution failed: ", hipGetErrorString(e));
+  int gave_up = 0;
+  if (word.w != nullptr) gave_up = __atomic_load_n(word.w, __ATOMIC_RELAXED);
+  else e = hipMemcpy(&gave_up, status, sizeof(int), hipMemcpyDeviceToHost);
+  TORCH_CHECK(e == hipSuccess, what, " execution failed: ", hipGetErrorString(e));
+  TORCH_CHECK(gave_up == 0, what, ": ", gave_up_text());
+}
+void finish(int rc, hipStream_t stream, const char* what) {
+  TORCH_CHECK(rc == TTT_MLP_OK, what, " launch failed: ", ttt_mlp_error_string(rc));
+  if (!g_synchronize) return;
+  const hipError_t e = hipStreamSynchronize(stream);
+  TORCH_CHECK(e == hipSuccess, what, " execution failed: ", hipGetErrorString(e));
 }
 
 // The multi-workgroup launches are an optimisation: not worth failing (or evicting the caller's cached
 // blocks) for.  They are used only if their workspace fits comfortably into what the device has free
-// (memory held by torch's caching allocator counts as free for torch, so this is conservative).
+// (memory held by torch's caching allocator counts as free for torch, so this is conservative).  A small one (a thousandth of
+// 288 GB) is not worth the question (the same forward 62.8 us with it, 52.6 us without): it is there, or the allocator says
+// that it is not.
+constexpr size_t SMALL_WORKSPACE = (size_t)256 << 20;
 bool workspace_is_affordable(size_t bytes) {
-  if (bytes == 0) return false;
+  if (bytes <= SMALL_WORKSPACE) return bytes > 0;
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
   return bytes <= free_b / 2;
@@ -113,8 +170,11 @@ Workspace take_workspace(size_t bytes, const torch::Device& dev) {
     return w;
   }
   if (!workspace_is_affordable(bytes)) return w;
-  w.held = torch::empty({(int64_t)bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(dev));
-  w.ptr = w.held.data_ptr();
+  try {
+    w.held = torch::empty({(int64_t)bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(dev));
+    w.ptr = w.held.data_ptr();
+  } catch (const c10::OutOfMemoryError&) {
+  }
   return w;
 }
 
@@ -169,10 +229,11 @@ torch::Tensor ttt_forward(const torch::Tensor XQ, const torch::Tensor XK, const 
   if (ws.ptr != nullptr) {
     g_last_forward_mode = 1;
     const char* status = static_cast<const char*>(ws.ptr) + ttt_mlp_fwd_status_offset((int32_t)B, (int32_t)NH);
-    finish(ttt_mlp_fwd_launch_overlapped(&a, ws.ptr, ws_bytes, stream), stream, "ttt_forward", XQ.device(), status);
+    run_overlapped([&](int* report) { return ttt_mlp_launch_reporting(0, &a, ws.ptr, ws_bytes, report, stream); }, stream, "ttt_forward",
+                   XQ.device(), status);
   } else {
     g_last_forward_mode = 0;
-    finish(ttt_mlp_fwd_launch(&a, stream), stream, "ttt_forward", XQ.device());
+    finish(ttt_mlp_fwd_launch(&a, stream), stream, "ttt_forward");
   }
   return Out;
 }
@@ -285,14 +346,15 @@ torch::Tensor ttt_backward(
   if (ws.ptr != nullptr) {
     g_last_backward_mode = 1;
     const char* status = static_cast<const char*>(ws.ptr) + ttt_mlp_bwd_status_offset((int32_t)B, (int32_t)NH);
-    int rc = ttt_mlp_bwd_launch_within(&a, ws.ptr, ws_bytes, stream);
-    if (rc == 0 && g_fill_group_tensors) rc = ttt_mlp_bwd_export_group0(&a, stream);
-    finish(rc, stream, "ttt_backward", XQ.device(), status);
+    run_overlapped([&](int* report) {
+      const int rc = ttt_mlp_launch_reporting(1, &a, ws.ptr, ws_bytes, report, stream);
+      return rc == 0 && g_fill_group_tensors ? ttt_mlp_bwd_export_group0(&a, stream) : rc;
+    }, stream, "ttt_backward", XQ.device(), status);
   } else {
     g_last_backward_mode = 0;
     int rc = ttt_mlp_bwd_launch(&a, stream);
     if (rc == 0 && g_fill_group_tensors) rc = ttt_mlp_bwd_export_group0(&a, stream);
-    finish(rc, stream, "ttt_backward", XQ.device());
+    finish(rc, stream, "ttt_backward");
   }
   return Out;
 }
@@ -319,18 +381,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "skip the read of the old values.");
   m.def("get_accumulate", []() { return g_accumulate; });
   m.def("check_last_status", []() {
-          if (g_sticky == nullptr) return;
-          const c10::DeviceGuard guard(g_sticky->device());
-          hipStream_t stream = c10::hip::getCurrentHIPStream(g_sticky->device().index()).stream();
-          hipError_t e = hipStreamSynchronize(stream);
+          if (g_unwaited_device < 0) return;
+          const c10::DeviceGuard guard(c10::Device(c10::kCUDA, static_cast<c10::DeviceIndex>(g_unwaited_device)));
+          const hipError_t e = hipStreamSynchronize(c10::hip::getCurrentHIPStream(g_unwaited_device).stream());
           TORCH_CHECK(e == hipSuccess, "check_last_status: ", hipGetErrorString(e));
-          int word = 0;
-          e = hipMemcpy(&word, g_sticky->data_ptr<int>(), sizeof(int), hipMemcpyDeviceToHost);
-          TORCH_CHECK(e == hipSuccess, "check_last_status: ", hipGetErrorString(e));
-          if (word != 0) {
-            (void)hipMemset(g_sticky->data_ptr<int>(), 0, sizeof(int));
+          if (__atomic_exchange_n(report_words().collecting(), 0, __ATOMIC_RELAXED) != 0)
             TORCH_CHECK(false, "ttt_forward / ttt_backward: ", gave_up_text());
-          }
         },
         "With set_synchronize(False) the operators cannot report a multi-workgroup launch whose workgroups gave up "
         "waiting for each other (the reference reports execution errors after its own synchronisation, "
@@ -353,7 +409,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           TORCH_CHECK(ws->device().is_cuda() && ws->is_contiguous() && ws->scalar_type() == torch::kUInt8 && ws->dim() == 1,
                       "set_workspace: a contiguous 1-D uint8 GPU tensor is expected");
           TORCH_CHECK(reinterpret_cast<uintptr_t>(ws->data_ptr()) % 256 == 0, "set_workspace: the tensor must be 256-byte aligned");
-          (void)sticky_word(ws->device());   // the one device word check_last_status reads exists before the first launch
+          (void)report_words().collecting();   // (allocated before the first launch)
           delete g_workspace;
           g_workspace = new torch::Tensor(*ws);
         },

@@ -831,9 +831,9 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
 }
 
 // Clears the synchronisation words and marks every word of the exchange empty.
-__global__ void ttt_mlp_bwd_wide_clear(int* w, int n, uint4* x, int nx) {
+__global__ void ttt_mlp_bwd_wide_clear(int* w, int n, const int* report, uint4* x, int nx) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) w[i] = 0;
+  clear_word(w, n, i, report);
   if (i < nx) x[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
 }
 
@@ -843,7 +843,7 @@ hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream)
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
   const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
-  hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n,
+  hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
                      reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
   const int slots = (p.wide ? 2 : 1) * p.gang_pairs + p.n_finish + p.n_replay + (p.n_prefetch ? p.gang_pairs : 0);
   const dim3 grid(8 * slots), block(ttt::BW_THREADS);

@@ -467,7 +467,7 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
 }
 
 namespace {
-int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter) {
+int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter, int* report) {
   ttt::BwdParams p;
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
@@ -507,6 +507,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   p.n_prefetch = pl.prefetch ? 1 : 0;
   p.wide = pl.wide ? 1 : 0;
   p.wait_limit = g_wait_limit;
+  p.report = report;
   if (pl.gang) {
     p.fin_dz = reinterpret_cast<__bf16*>(base + w.off[5]) - b0 * 2 * img;
     p.fin_gy = reinterpret_cast<float*>(base + w.off[6]) - b0 * 2 * 2 * tile;
@@ -552,7 +553,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
 }  // namespace
 
 extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
-  return bwd_launch(a, workspace, workspace_bytes, stream, false);
+  return bwd_launch(a, workspace, workspace_bytes, stream, false, nullptr);
 }
 
 extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
@@ -580,7 +581,7 @@ extern "C" size_t ttt_mlp_fwd_status_offset(int B, int NH) {
 }
 
 namespace {
-int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter) {
+int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream, bool scatter, int* report) {
   ttt::FwdParams p;
   if (int rc = make_fwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
@@ -614,6 +615,7 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
   p.wait_limit = g_wait_limit;
+  p.report = report;
   if (pl.wide) {
     p.n_out = pl.n_out;
     p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * ttt::FWD_WIDE_RING * (ttt::FWD_IMG_BYTES / 2);
@@ -630,12 +632,18 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
 }  // namespace
 
 extern "C" int ttt_mlp_fwd_launch_overlapped(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
-  return fwd_launch(a, workspace, workspace_bytes, stream, false);
+  return fwd_launch(a, workspace, workspace_bytes, stream, false, nullptr);
+}
+
+extern "C" int ttt_mlp_launch_reporting(int which, const void* args, void* workspace, size_t workspace_bytes, int* report, void* stream) {
+  if (which == 0) return fwd_launch(static_cast<const ttt_mlp_fwd_args*>(args), workspace, workspace_bytes, stream, false, report);
+  if (which == 1) return bwd_launch(static_cast<const ttt_mlp_bwd_args*>(args), workspace, workspace_bytes, stream, false, report);
+  return TTT_MLP_ERR_BAD_ARG;
 }
 
 extern "C" int ttt_mlp_launch_scattered(int which, const void* args, void* workspace, size_t workspace_bytes, void* stream) {
-  if (which == 0) return fwd_launch(static_cast<const ttt_mlp_fwd_args*>(args), workspace, workspace_bytes, stream, true);
-  if (which == 1) return bwd_launch(static_cast<const ttt_mlp_bwd_args*>(args), workspace, workspace_bytes, stream, true);
+  if (which == 0) return fwd_launch(static_cast<const ttt_mlp_fwd_args*>(args), workspace, workspace_bytes, stream, true, nullptr);
+  if (which == 1) return bwd_launch(static_cast<const ttt_mlp_bwd_args*>(args), workspace, workspace_bytes, stream, true, nullptr);
   return TTT_MLP_ERR_BAD_ARG;
 }
 

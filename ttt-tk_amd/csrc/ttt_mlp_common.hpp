@@ -485,6 +485,19 @@ TTT_DEV void eta_to_lds(gptr_t g, unsigned off, unsigned char* dst, int v, int l
 // resident at once because the launchers use such a mode only when the grid fits the CUs of the device.
 // A wait that sees no progress for `limit` ticks of the 100 MHz clock (20 s unless the host says otherwise)
 // raises the status word and makes all workgroups of the launch leave, so every wave always exits.
+// The words behind the status word name, as an address, one more int that hears of it (host memory the caller reads without a
+// copy; 0: none): put there by the kernel that clears the words ahead of the launch.
+constexpr int STATUS_WORDS = 32;    // the status word, a gap, the two halves of the address, unused
+TTT_DEV void clear_word(int* w, int n, int i, const int* report) {   // word i of n, the last STATUS_WORDS of them those
+  const uint64_t r = reinterpret_cast<uint64_t>(report);
+  const int k = i - (n - STATUS_WORDS);
+  if (i < n) w[i] = k == 2 ? static_cast<int>(static_cast<uint32_t>(r)) : k == 3 ? static_cast<int>(static_cast<uint32_t>(r >> 32)) : 0;
+}
+TTT_DEV void raise_status(int* status) {
+  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int* const report = reinterpret_cast<int*>(__hip_atomic_load(reinterpret_cast<uint64_t*>(status + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  if (report != nullptr) __hip_atomic_store(report, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 TTT_DEV bool wait_at_least(int* word, int target, int* status, int* s_flag, uint64_t limit) {
   __syncthreads();   // every wave has read the flag's last value (waits follow one another, here and in wait_for_pace)
   if (threadIdx.x == 0) {
@@ -494,7 +507,7 @@ TTT_DEV bool wait_at_least(int* word, int target, int* status, int* s_flag, uint
     // one acquire fence once the value is there
     while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_status(status);
         ok = 0;
         break;
       }
@@ -516,7 +529,7 @@ TTT_DEV int wait_for_pace(int* word, int target, int* status, int* s_flag, uint6
     const uint64_t t0 = wall_clock64();
     while ((seen = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_status(status);
         seen = -1;
         break;
       }
@@ -537,7 +550,7 @@ TTT_DEV int wait_for_both(int* a, int* b, int target, int* status, int* s_flag, 
     while ((seen = min(__hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
                        __hip_atomic_load(b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_status(status);
         seen = -1;
         break;
       }

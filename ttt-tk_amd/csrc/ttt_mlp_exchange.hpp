@@ -39,7 +39,7 @@ TTT_DEV bool wd_take(gword64_t q, uint64_t (&w)[N], int* status, uint64_t limit)
     const uint64_t now = wall_clock64();
     if (n == 0) t0 = now;
     else if (now - t0 > limit || ((n & 63) == 0 && __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-      __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      raise_status(status);
       return false;
     }
   }
@@ -59,7 +59,7 @@ TTT_DEV bool on_one_xcd(int* words, int n, int lane, int* status, uint64_t limit
     const uint64_t t0 = wall_clock64();
     while ((x = __hip_atomic_load(words + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_status(status);
         ok = false;
         break;
       }
@@ -85,7 +85,7 @@ TTT_DEV bool workers_here(int* word, int total, int* status, uint64_t limit, boo
   while (((x = __hip_atomic_load(reinterpret_cast<uint64_t*>(word), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) * 0x0101010101010101ull) >> 56 <
          static_cast<uint64_t>(total)) {
     if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-      __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      raise_status(status);
       ok = false;
       break;
     }
@@ -99,7 +99,7 @@ TTT_DEV bool wait_word(int* word, int target, int* status, uint64_t limit) {
   const uint64_t t0 = wall_clock64();
   while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
     if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
-      __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      raise_status(status);
       return false;
     }
     __builtin_amdgcn_s_sleep(4);

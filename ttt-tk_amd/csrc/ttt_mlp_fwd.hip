@@ -464,10 +464,7 @@ __global__ __launch_bounds__(FW_THREADS) void ttt_mlp_fwd_split_kernel(const Fwd
   else fwd_output_branch<RING, false>(p, smem, bh, 0);
 }
 
-__global__ void ttt_mlp_fwd_zero_words(int* w, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) w[i] = 0;
-}
+__global__ void ttt_mlp_fwd_zero_words(int* w, int n, const int* report) { clear_word(w, n, blockIdx.x * blockDim.x + threadIdx.x, report); }
 
 }  // namespace ttt
 
@@ -475,7 +472,7 @@ extern "C" int ttt_mlp_fwd_lds_bytes() { return ttt::SM_FWD_BYTES; }
 extern "C" int ttt_mlp_fwd_threads() { return ttt::FW_THREADS; }
 
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream) {
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n);
+  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, static_cast<const int*>(nullptr));
   return hipGetLastError();
 }
 
@@ -494,7 +491,7 @@ hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, hipStream_t stream) {
   if (e != hipSuccess) return e;
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n);
+  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
   if (p.ring_log2 == 5)
     hipLaunchKernelGGL(ttt::ttt_mlp_fwd_split_kernel<32>, dim3(2 * p.nbh), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
   else

@@ -486,7 +486,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
         const uint64_t t0 = wall_clock64();
         while ((seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(words + WDW_TAKEN + 4 * o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < need) {
           if (__hip_atomic_load(w_status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > p.wait_limit) {
-            __hip_atomic_store(w_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            raise_status(w_status);
             gave_up = true;
             break;
           }
@@ -543,9 +543,9 @@ __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 }
 
 // Clears the synchronisation words and marks every word of the exchange empty.
-__global__ void ttt_mlp_fwd_wide_clear(int* w, int n, uint4* x, int nx) {
+__global__ void ttt_mlp_fwd_wide_clear(int* w, int n, const int* report, uint4* x, int nx) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) w[i] = 0;
+  clear_word(w, n, i, report);
   for (int k = i; k < nx; k += gridDim.x * blockDim.x) x[k] = make_uint4(~0u, ~0u, ~0u, ~0u);
 }
 
@@ -559,7 +559,7 @@ hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream)
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
   const int nx = p.nbh * (ttt::FWD_XCHG_WORDS / 2);
   const int need = nx > n ? nx : n;
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n,
+  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n, p.report,
                      reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::FWD_XCHG_WORDS), nx);
   hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_kernel, dim3((p.nbh + 7) / 8 * 8 * (2 + p.n_out)), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
   return hipGetLastError();

@@ -23,6 +23,7 @@ struct FwdParams {
   int ring_log2;
   int* sync;
   int* status;    // the status word behind the synchronisation words
+  int* report;    // one more int, in host memory, that a wait that gives up is told to (or nullptr)
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
   // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2 x 2048 fp32],
   // and the output workgroups per pair (1 or 2); the ring then has FWD_WIDE_RING slots.
@@ -96,6 +97,7 @@ struct BwdParams {
   int n_prefetch, scatter;
   int* sync;
   int* status;    // the status word behind the synchronisation words
+  int* report;    // one more int, in host memory, that a wait that gives up is told to (or nullptr)
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
   int overwrite;  // non-zero: grad_L_XQ / XK / XV / last_eta are stored, not added to (every element is written exactly once)
   int bh0, nbh;   // this launch covers (batch, head) pairs bh0 .. bh0 + nbh - 1 (workspace pointers moved back by bh0 entries)
@@ -120,7 +122,7 @@ constexpr int BWW_WORDS = 9;                                // per lane: two tim
 constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 144 KiB
 constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26, BWW_WORKERS = 28;
 constexpr int FIN_PARK_FLOATS = 64 * 256 + 8 * 4 * 64;
-inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }
+inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }   // 32: STATUS_WORDS (ttt_mlp_common.hpp)
 
 // ---- optional stage clocks.  A library built with -DTTT_STAGE_CLOCKS (stage_clocks.py builds one beside the product
 // library) reads the shader clock at the boundaries of the stages named here and adds up, per wave, the clocks

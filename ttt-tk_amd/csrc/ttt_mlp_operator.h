@@ -1,6 +1,6 @@
 /* Entry points of libttt_mlp.so for the operator module in this folder and for the tests; not part of the C ABI in
- * include/ttt_mlp.h.  The first two let the operator take a workspace that fits the call at hand instead of one that fits
- * every call of its B, NH and checkpoint_group_size. */
+ * include/ttt_mlp.h.  The first three let the operator take a workspace that fits the call at hand instead of one that fits
+ * every call of its B, NH and checkpoint_group_size, and learn without a copy whether a wait gave up. */
 #ifndef TTT_MLP_OPERATOR_H_
 #define TTT_MLP_OPERATOR_H_
 
@@ -19,6 +19,11 @@ int ttt_mlp_bwd_workspace_range(int32_t B, int32_t NH, int32_t checkpoint_group_
 /* As ttt_mlp_bwd_launch_overlapped, with any workspace of at least *least bytes (ttt_mlp_bwd_workspace_range): the launch
  * of the plan from *most bytes on, the one with fewer sets below.  Same results, bit for bit. */
 int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
+
+/* ttt_mlp_fwd_launch_overlapped (which = 0, args a ttt_mlp_fwd_args) / ttt_mlp_bwd_launch_within (1) whose workgroups, if a wait
+ * gives up, also set *report, an int that the device can write and the host reads once the stream has been waited for (host
+ * memory; not written otherwise; nullptr: none). */
+int ttt_mlp_launch_reporting(int which, const void* args, void* workspace, size_t workspace_bytes, int* report, void* stream);
 
 /* ttt_mlp_fwd_launch_overlapped (which = 0, args a ttt_mlp_fwd_args) / ttt_mlp_bwd_launch_overlapped (1) with the workgroups
  * of a pair on consecutive XCDs where the recurrence or the walk takes two: what they do if a device does not place them on

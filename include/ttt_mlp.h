@@ -235,9 +235,9 @@ const char* ttt_mlp_error_string(int code);
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
  * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  which = 0
  * forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk),
- * 3 (two replay), 7 or 8 (walk on two, one for grad_L_XK / grad_L_XV, three or four that replay, one that reads ahead), and
- * 5, 4 or 3 where the CUs of an eighth of the device are not a whole number per pair: the whole ones of a pair's share, at
- * most 5, while the workgroups that replay and those for grad_L_XK serve all of those pairs.  More than 2 forward, and all
+ * 3 (two replay), 7 or 8 (walk on two, one for grad_L_XK / grad_L_XV, three, or four to eight, that replay, one that reads ahead), and
+ * 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly: the whole ones of a pair's share, at most 5, while
+ * the workgroups that replay and those for grad_L_XK may serve all of those pairs.  More than 2 forward, and all
  * backward but 2 and the 3 that has no eighth of the device for its pairs: the workgroups of a pair share an XCD, and those of
  * ceil(*other_pairs / 8) pairs fit an eighth of the CUs. */
 int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long* one_workgroup_pairs,

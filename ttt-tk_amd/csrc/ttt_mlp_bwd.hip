@@ -36,6 +36,8 @@
 // images X2_bar^T (X2_bar_group) and (dL/dZ1_bar)^T (Z1_bar_group); the two weight operand images
 // (X2_group: W1^T[shard], grad_l_wrt_Z1_group: W2[shard]^T); x_hat / grad_output of the fused LayerNorm
 // loss, dl/dZ2 and dL/dZ2_bar (grad_x_hat_fused_group) as bf16 [tok][F] tiles; the fused std in fp32.
+#include <type_traits>
+
 #include "ttt_mlp_common.hpp"
 #include "ttt_mlp_kernels.hpp"
 
@@ -363,6 +365,12 @@ TTT_DEV bf16x8 w1_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int rb, 
 
 constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK workgroup within the last group walked (a power of two)
 
+// What a set's word has come to when group number `done` has been replayed into it, in all of its parts.
+TTT_DEV int parts_until(const BwdParams& p, int done) {
+  const int use = uni(done / p.n_sets);   // (only the first use of a set can be in parts)
+  return use + (done - use * p.n_sets < p.n_shared ? p.n_parts : 1);
+}
+
 // ------------------------------------------------------------------ several workgroups per (batch, head)
 // The replay of a checkpoint group needs only the checkpoint, so it can run ahead of the reverse walk
 // on other CUs: one or more workgroups replay group after group, in turn, into alternating sets of the per-group
@@ -378,10 +386,13 @@ constexpr int FIN_CHUNK = 8;   // mini-batches per hand-over to the grad_L_XK wo
 // fits, the walk hands it dZ1 (a register image) and two fp32 tiles, g_y and the norm-weight gradient terms, and that
 // workgroup (bwd_finish_dxk) forms grad_L_XK, grad_L_XV and the norm gradients.
 // WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
-template <int ROLE, bool IMG, bool FIN, bool WIDE = false>
+// PARTS: several workgroups at once replay each of the p.n_shared groups walked first, a stretch of its mini-batches each.
+template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; ROLE 2: K - 1 .. 0).
+// part (PARTS): which of the p.n_parts stretches of the group's mini-batches this workgroup replays; it takes the state there from
+// the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).
 // False: a wait gave up.
-TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi, const int k_lo) {
+TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi, const int k_lo, const int part = 0) {
   static_assert(!(ROLE == 0 && (IMG || FIN)), "one workgroup per (batch, head) does everything itself");
   bf16* s_xq = reinterpret_cast<bf16*>(smem + SB_XQ);
   bf16* s_xk = reinterpret_cast<bf16*>(smem + SB_XK);
@@ -459,7 +470,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
 #define REFRESH_OFFSETS() asm volatile("" : "+s"(ka), "+s"(ox), "+s"(oe), "+s"(of), "+s"(oh), "+s"(ot), "+s"(opk), "+s"(ock))
   // per-group tensors: the caller's (set 0) or, with several workgroups, one of the alternate sets
-#define GRP(name) (set ? ka->alt_##name[set - 1] : ka->name)
+#define GRP(name) (ROLE != 0 && set ? ka->alt_##name[ROLE != 0 ? set - 1 : 0] : ka->name)
 #define bXQ gbuf(ka->XQ + ox)
 #define bXK gbuf(ka->XK + ox)
 #define bXV gbuf(ka->XV + ox)
@@ -523,8 +534,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   int* const w_status = p.status;
   int* const s_flag = reinterpret_cast<int*>(smem + SB_FLAG);
 
-  // The replay's share of the norm gradients is formed group by group and added to a running sum in the groups' order, so it
-  // does not depend on who replays them.  The running sum sits in HBM (slot 0 of the park, 4 KiB): with one workgroup per
+  // The replay's share of the norm gradients is formed by eighths of a group, which are summed, and added group by group to a
+  // running sum, in that order, so it does not depend on who replays what.  The running sum sits in HBM (slot 0 of the park, 4 KiB): with one workgroup per
   // (batch, head) in the caller's x_hat_ln_group, where the walk's sum waits behind it (slot 1) while the LDS accumulators
   // serve a replay, otherwise in the workspace, added to by the walk (by the grad_L_XK workgroup where there is one).
   // (Its address is formed where it is used: kept over the loop it costs the walk two registers it does not have.)
@@ -538,8 +549,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     LANE_VARS;
     return (v * 2 * FD + lane) * 4u;
   };
-  auto group_sums = [&](int set) {   // of this wave
-    size_t o = uni64(((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD);
+  const int eighth = (cgs + 7) / 8;   // mini-batches
+  auto group_sums = [&](int set, int e) {   // of this wave
+    size_t o = uni64((((size_t)bh * BWD_MAX_SETS + set) * 8 + e) * (BW_NWAVE * 2 * FD) + v * 2 * FD);
     asm volatile("" : "+s"(o));
     return gbuf(p.norm_partial + o);
   };
@@ -575,6 +587,17 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         s_dgw[lane] = 0.f;   // (every lane its own words)
         s_dbw[lane] = 0.f;
       }
+      // [j_first, j_end): what this workgroup replays of the group
+      int j_first = 0, j_end = n_mb;
+      if (PARTS && done < p.n_shared) {
+        const int n_eighths = (n_mb + eighth - 1) / eighth;
+        j_first = uni((p.part_start[part] * n_eighths / 8) * eighth);
+        j_end = uni(min((p.part_start[part + 1] * n_eighths / 8) * eighth, n_mb));
+        if (j_first >= j_end) {
+          publish_part(w_replayed);
+          continue;
+        }
+      }
       // park the running gradients while the forward state needs the registers
       if constexpr (ROLE == 0) {
         acc_store_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
@@ -595,19 +618,19 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       if (tid < HID) s_b1[tid] = p.b1_ck[slot * HID + tid];
       if (tid < FD) s_b2[tid] = p.b2_ck[slot * FD + tid];
 
+      // where XK of a mini-batch on the way to j_first sits: the two buffers in turn, so that the last one is in XQ's
+      auto light_xk = [&](int j) { return (j_first - 1 - j) & 1 ? SB_XK : SB_XQ; };
       {
         Staged3 st;
         stage3_load(st, bXQ, bXK, bXV, bETA, k * cgs, tid, t16);
-        stage3_store(st, s_xq, s_xk, s_e2, s_etah, tid);
+        const bool swap = PARTS && j_first > 0 && light_xk(0) == SB_XQ;
+        stage3_store(st, swap ? s_xk : s_xq, swap ? s_xq : s_xk, s_e2, s_etah, tid);
       }
       TTT_STAGE(BS_GROUP);
-      for (int j = 0; j < n_mb; j++) {
-        const int mb = k * cgs + j;
-        REFRESH_OFFSETS();
+      // The state through mini-batch j.  FULL: with everything the walk needs of it saved on the way.
+      auto step_state = [&](auto full, const int j, bf16* const xk_tile) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full)::value;
         LANE_VARS;
-        __syncthreads();   // the staged inputs (and, for j = 0, the biases) are visible
-        TTT_STAGE(BS_R_TOP);
-
         // Z1^T = W1s^T XK^T + b1  (rows hid, lane = tok); X2 rows [tok][hid] -> T0; gelu'(Z1) (fp32) and the
         // low-order term of X2 stay in registers.  The products that carry the state to the next mini-batch
         // take their fp32 operands in two bf16 terms (see split8).
@@ -622,7 +645,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             bf16x8 wh, wl, xk[2];
             split8(W1s.b[s >> 1][0], s & 1, wh, wl);
 #pragma unroll
-            for (int i = 0; i < 2; i++) xk[i] = xpiece_rows(s_xk, tb[i], s, c, h);
+            for (int i = 0; i < 2; i++) xk[i] = xpiece_rows(xk_tile, tb[i], s, c, h);
 #pragma unroll
             for (int i = 0; i < 2; i++) {
               x2.b[0][i] = MFMA(wl, xk[i], x2.b[0][i]);
@@ -634,9 +657,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
             for (int t = 0; t < 2; t++) {
               const bf16x8 zr = pack8(x2.b[0][i], t);
-              if constexpr (!IMG) {
+              if constexpr (FULL && !IMG) {
                 image_store<ROLE != 0>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
-              } else {
+              } else if constexpr (FULL) {
                 // The walk needs gelu, gelu' and gelu'' of the ROUNDED Z1 (what it would compute from the image
                 // of Z1); a replaying workgroup has the time to do that for it.
                 bf16x8 gv, av, bv;
@@ -709,7 +732,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           float go[8], gx[8];
           {
             float kv[8], vv[8], bet[8];
-            ln_load(kv, s_xk + xrow(tok) + f0);
+            ln_load(kv, xk_tile + xrow(tok) + f0);
             ln_load(vv, s_e2 + xrow(tok) + f0);
             ln_load_f32(bet, s_bet + f0);
 #pragma unroll
@@ -718,13 +741,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
               gx[e] = go[e] * gam[e];
             }
           }
-          ln_store_g<ROLE != 0>(bXHF, vln, j * TILE_BYTES, z);
-          ln_store_g<ROLE != 0>(bGOF, vln, j * TILE_BYTES, go);
+          if constexpr (FULL) {
+            ln_store_g<ROLE != 0>(bXHF, vln, j * TILE_BYTES, z);
+            ln_store_g<ROLE != 0>(bGOF, vln, j * TILE_BYTES, go);
+          }
           const float s1 = oct_sum(sum8(gx)), s2 = oct_sum(dot8(gx, z));
           const float sc = rstd * (1.f / FD), neg_eta = -bf2f(s_etah[tok]);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;   // dl/dZ2
-          ln_store_g<ROLE != 0>(bGZ2, vln, j * TILE_BYTES, gx);
+          if constexpr (FULL) ln_store_g<ROLE != 0>(bGZ2, vln, j * TILE_BYTES, gx);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] *= neg_eta;                             // G2, in two terms (the second in
           ln_token_sum_store(s_deta + v * CS, gx, lane, f0);   // b2's step: this wave's share (s_deta is the walk's otherwise)
@@ -734,9 +759,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             ln_store_h(s_gz2 + tok * LDX + f0, gh);
             ln_store_h(s_a + tok * LDX + f0, gl);
           }
-          if ((lane & 7) == 0) g_stf(bSDF, vtok, j * (CS * 4), sd);
+          if (FULL && (lane & 7) == 0) g_stf(bSDF, vtok, j * (CS * 4), sd);
         }
+        if (PARTS && FULL && j == j_first && j > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // XQ (see below)
         __syncthreads();
+        if constexpr (!FULL) {   // XV and eta have been read: the next ones'
+          LANE_VARS;
+          tile_to_lds<CPOL_NT>(bXV, (k * cgs + j + 1) * TILE_BYTES, smem + SB_E2, v, lane);
+          eta_to_lds(bETA, (k * cgs + j + 1) * (CS * 2), smem + SB_ETA, v, lane);
+        }
         if (v == 0) {   // b2 += sum over the tokens of G2: the eight waves' fp32 shares in a fixed order (next read: the output LayerNorm)
           LANE_VARS;
           float b = s_b2[lane];
@@ -803,7 +834,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           for (int s = 0; s < 4; s++) {                        // W1[:, shard] += XK^T G1
             bf16x8 xk[2];
 #pragma unroll
-            for (int fb = 0; fb < 2; fb++) xk[fb] = xpiece_tr(s_xk, fb, s, lane);               // XK^T: lane = F
+            for (int fb = 0; fb < 2; fb++) xk[fb] = xpiece_tr(xk_tile, fb, s, lane);               // XK^T: lane = F
             const bf16x8 gh = piece_tr<LDH>(T1, 0, s, lane), gl = piece_tr<LDH>(T2, 0, s, lane);   // G1: lane = hid
 #pragma unroll
             for (int fb = 0; fb < 2; fb++) {
@@ -838,6 +869,46 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           WAVE_SYNC();   // this wave's readers of T1 / T2 are done
         }
         TTT_STAGE(BS_R_WSTEP);
+      };
+      if constexpr (PARTS) {
+        for (int j = 0; j < j_first; j++) {
+          REFRESH_OFFSETS();
+          __syncthreads();   // the staged inputs (and, for j = 0, the biases) are visible
+          TTT_STAGE(BS_R_TOP);
+          {
+            LANE_VARS;
+            tile_to_lds<CPOL_NT>(bXK, (k * cgs + j + 1) * TILE_BYTES, smem + light_xk(j + 1), v, lane);   // (read last a mini-batch ago)
+          }
+          step_state(std::false_type{}, j, reinterpret_cast<bf16*>(smem + light_xk(j)));
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier
+        }
+      }
+      // The norm-gradient sums of an eighth of the group go out on their own, at the top of the next one, where their stores have a
+      // whole mini-batch to arrive (of one workgroup per (batch, head) the last eighth's stay in LDS).
+      auto eighth_out = [&](int e) {
+        WAVE_SYNC();
+        LANE_VARS;
+        const gptr_t g = ROLE == 1 ? group_sums(set, e) : park();
+        const unsigned o = ROLE == 1 ? 4 * lane : np_off(), so = ROLE == 1 ? 0 : (2 + e) * PARK_BYTES;
+        g_stf(g, o, so, s_dgw[lane]);
+        g_stf(g, o, so + FD * 4, s_dbw[lane]);
+        s_dgw[lane] = 0.f;
+        s_dbw[lane] = 0.f;
+        WAVE_SYNC();
+      };
+      int e = uni(PARTS ? j_first / eighth : 0), e_end = j_first + eighth;   // the eighth of the group that mini-batch j is in, and its end
+      for (int j = j_first; j < j_end; j++) {
+        const int mb = k * cgs + j;
+        REFRESH_OFFSETS();
+        LANE_VARS;
+        __syncthreads();   // the staged inputs (and, for j = 0, the biases) are visible
+        TTT_STAGE(BS_R_TOP);
+        if (j == e_end) {
+          eighth_out(e++);
+          e_end += eighth;
+        }
+        if (PARTS && j == j_first && j > 0) tile_to_lds<CPOL_NT>(bXQ, mb * TILE_BYTES, smem + SB_XQ, v, lane);   // XK was there until now
+        step_state(std::true_type{}, j, s_xk);
         // operand images of the state after this step, for the reverse walk; the image of W2 (lane = hid,
         // contraction = F) also serves the output branch below
         bf16x8 w2a[4];
@@ -921,7 +992,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           // Every reader of this mini-batch's XQ / XK / XV / eta is past the barriers of the pair sum: the next
           // mini-batch's leave HBM now - straight to LDS, no registers involved - and have the rest of this
           // mini-batch to arrive.
-          if (j + 1 < n_mb) {
+          if (j + 1 < j_end) {
             tile_to_lds<CPOL_NT>(bXQ, (mb + 1) * TILE_BYTES, smem + SB_XQ, v, lane);
             tile_to_lds<CPOL_NT>(bXK, (mb + 1) * TILE_BYTES, smem + SB_XK, v, lane);
             tile_to_lds<CPOL_NT>(bXV, (mb + 1) * TILE_BYTES, smem + SB_E2, v, lane);
@@ -1026,32 +1097,41 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier at the loop's top
         TTT_STAGE(BS_R_OUT_BACKWARD);
       }
-      if constexpr (ROLE == 1) {
-        WAVE_SYNC();   // this group's norm-gradient sums go with it
-        LANE_VARS;
-        const gptr_t g = group_sums(set);
-        g_stf(g, 4 * lane, 0, s_dgw[lane]);
-        g_stf(g, 4 * lane, FD * 4, s_dbw[lane]);
-      }
+      if constexpr (ROLE == 1) eighth_out(e);
       // running gradients back into registers
       if constexpr (ROLE == 0) {
         LANE_VARS;
-        // one round trip to HBM for the four words and the gradients (200 pairs x 100 mini-batches, 7 groups: 5.42 ms forward +
+        // one round trip to HBM for the words and the gradients (200 pairs x 100 mini-batches, 7 groups: 5.42 ms forward +
         // backward with a word at a time and their address kept over the loops, 5.36 so)
         const gptr_t g = park();
         const unsigned o = np_off();
         const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4), w0 = g_ldf(g, o, PARK_BYTES), w1 = g_ldf(g, o, PARK_BYTES + FD * 4);
+        float e0[7], e1[7];
+        const int n_out = (n_mb + eighth - 1) / eighth - 1;   // eighths that are out
+#pragma unroll
+        for (int e = 0; e < 7; e++) {
+          e0[e] = e < n_out ? g_ldf(g, o, (2 + e) * PARK_BYTES) : 0.f;
+          e1[e] = e < n_out ? g_ldf(g, o, (2 + e) * PARK_BYTES + FD * 4) : 0.f;
+        }
         acc_load_rows(gW1s, bPW1, 0, HID, 0, hid0, c, h);
         acc_load_rows(gW2s, bPW2, 0, FD, hid0, 0, c, h);
         WAVE_SYNC();
-        const float a0 = r0 + s_dgw[lane], a1 = r1 + s_dbw[lane];   // the running sum
+        float a0 = s_dgw[lane], a1 = s_dbw[lane];
+        if (n_out > 0) {
+          float t0 = e0[0], t1 = e1[0];
+#pragma unroll
+          for (int e = 1; e < 7; e++)
+            if (e < n_out) { t0 += e0[e]; t1 += e1[e]; }
+          a0 = t0 + a0;
+          a1 = t1 + a1;
+        }
         s_dgw[lane] = w0;
         s_dbw[lane] = w1;
-        g_stf(g, o, 0, a0);
-        g_stf(g, o, FD * 4, a1);
+        g_stf(g, o, 0, r0 + a0);   // the running sum
+        g_stf(g, o, FD * 4, r1 + a1);
         WAVE_SYNC();
       }
-      if constexpr (ROLE == 1) publish(w_replayed, done + 1);
+      if constexpr (ROLE == 1) publish_part(w_replayed);
       TTT_STAGE(BS_PUBLISH);
     }
 
@@ -1060,13 +1140,17 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     // wave covers the latency, while holding requests in registers across stages costs more in spills
     // than it gains (measured).
     if constexpr (ROLE == 2) {
-      if (!wait_at_least(w_replayed, done + 1, w_status, s_flag, p.wait_limit)) return false;
+      if (!wait_at_least(w_replayed, parts_until(p, done), w_status, s_flag, p.wait_limit)) return false;
       if constexpr (FIN) {   // the hand-over set of this group's parity is free once the group before last is finished
         if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return false;
       } else {
         LANE_VARS;
-        const gptr_t gs = group_sums(set);   // the running sum
-        const float a0 = g_ldf(gs, 4 * lane, 0), a1 = g_ldf(gs, 4 * lane, FD * 4);
+        float a0 = 0.f, a1 = 0.f;
+        for (int e = 0; e * eighth < n_mb; e++) {
+          const gptr_t gs = group_sums(set, e);
+          a0 = e > 0 ? a0 + g_ldf(gs, 4 * lane, 0) : g_ldf(gs, 4 * lane, 0);
+          a1 = e > 0 ? a1 + g_ldf(gs, 4 * lane, FD * 4) : g_ldf(gs, 4 * lane, FD * 4);
+        }
         const gptr_t g = park();
         const unsigned o = (v * 2 * FD + lane) * 4;
         const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);
@@ -1705,10 +1789,16 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
         if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return false;
         TTT_STAGE(BS_X_GROUP);
       }
-      if (j == n_mb - 1) {   // the group's norm-gradient sums: published with it, and the walk has acquired it
-        const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (BW_NWAVE * 2 * FD) + v * 2 * FD;
-        nr0 += np[lane];
-        nr1 += np[FD + lane];
+      if (j == n_mb - 1) {   // the group's norm-gradient sums, by eighths: published with it, and the walk has acquired it
+        const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (8 * BW_NWAVE * 2 * FD) + v * 2 * FD + lane;
+        const int eighth = (cgs + 7) / 8;
+        float a0 = np[0], a1 = np[FD];
+        for (int e = 1; e * eighth < n_mb; e++) {
+          a0 += np[e * (BW_NWAVE * 2 * FD)];
+          a1 += np[e * (BW_NWAVE * 2 * FD) + FD];
+        }
+        nr0 += a0;
+        nr1 += a1;
         ask_tiles(j);
         ask_g1b(j);
         ask_w2(j);

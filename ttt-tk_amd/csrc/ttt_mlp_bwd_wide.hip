@@ -508,7 +508,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
     if (!__all(lane != 0 || wait_word(word, target, w_status, p.wait_limit))) gave_up = true;
   };
   // group number `done` (from the end) has been replayed
-  auto wait_group = [&](int done) { wait_for(words + done % n_sets, done + 1); };
+  auto wait_group = [&](int done) { wait_for(words + done % n_sets, parts_until(p, done)); };
   // What one mini-batch needs from HBM besides the operand images: a chunk of 16 bytes per lane and token block of each
   // tile - the lanes that hold a chunk are the LayerNorm lanes of that token and those features.
   struct Ahead {
@@ -741,7 +741,7 @@ TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const in
   for (int k = p.K - 1; k >= 0; k--) {
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k, set = done % n_sets;
-    if (!wait_at_least(words + set, done + 1, p.status, s_flag, p.wait_limit)) return;
+    if (!wait_at_least(words + set, parts_until(p, done), p.status, s_flag, p.wait_limit)) return;
 #define PGRP(name) (set ? p.alt_##name[set - 1] : p.name)
     // wave v: tile v (two inputs, four of the set); waves 0-3 / 4-7: one image each of a pair
     gptr_t tile = gbuf(p.XQ + ox);
@@ -777,14 +777,14 @@ TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const in
 }
 
 // The workgroups of a gang: gang g has pairs g, g + 8, .. and, as workgroups are dealt to the 8 XCDs in turn, one XCD.  WALKERS of
-// them walk each pair, the others work for all of its pairs: n_replay take the replays in turn, ordered by group and then by
-// pair (all walks go at one pace), n_finish the finishing of the groups (grad_L_XK and the norm gradients) in the same
+// them walk each pair, the others work for all of its pairs: n_replay take the replays in turn, ordered by group, then by pair (all
+// walks go at one pace) and then by part of the group, n_finish the finishing of the groups (grad_L_XK and the norm gradients) in the same
 // order, PREFETCH: one per pair reads ahead of its walk.  With a finishing workgroup for each pair it stays with that
 // pair; with fewer, the last group of each pair is finished by a replaying workgroup, all of them together.
 // Nobody waits for a later job than his own: a replay waits for the set of n_sets groups ago to be walked and finished, the
 // finishing of a group for its walk and the group before, a walk for its replay and the finishing of two groups ago; so of
 // the jobs not yet done the first can always go on.
-template <bool WIDE, bool IMG, bool PREFETCH, bool OWN>
+template <bool WIDE, bool IMG, bool PREFETCH, bool OWN, bool PARTS>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x, walkers = (WIDE ? 2 : 1) * p.gang_pairs;
@@ -792,6 +792,12 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
   const int gang = uni(p.scatter ? b / slots : b & 7);   // (a division leaves its result in a vector register)
   int slot = uni(p.scatter ? b % slots : b >> 3);
   const int pairs = (p.nbh - gang + 7) / 8;   // of this gang
+  // Where every pair has as many replaying workgroups, what belongs to a pair is placed side by side (24 pairs x 512 4.66 ms, 4.70 by
+  // kind; the CUs that share an instruction cache are a few workgroups apart).
+  if (OWN && slots % p.gang_pairs == 0) {
+    const int per = uni(slots / p.gang_pairs), n = WIDE ? 2 : 1, i = uni(slot / per), role = slot - i * per;
+    slot = role < n ? n * i + role : role == n ? walkers + i : PREFETCH && role == per - 1 ? slots - p.gang_pairs + i : walkers + p.gang_pairs + (role - n - 1) * p.gang_pairs + i;
+  }
   if (pairs <= 0) return;
   const int bh0 = p.bh0 + gang;
   if (slot < walkers) {
@@ -813,9 +819,18 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
   const bool replays = slot >= p.n_finish;
   const int r = slot - p.n_finish;
   if (replays) {
-    for (int job = r; job < p.K * pairs; job += p.n_replay) {
-      const int done = uni(job / pairs), k = p.K - 1 - done;
-      if (!bwd_body<1, IMG, true, WIDE>(p, smem, bh0 + 8 * (job - done * pairs), k, k)) return;
+    const int shared = PARTS ? min(p.n_shared, p.K) : 0, shared_jobs = shared * pairs * p.n_parts, jobs = shared_jobs + (p.K - shared) * pairs;
+    for (int job = r; job < jobs; job += p.n_replay) {
+      int n = job, part = 0, before = 0;   // job -> number of the group and pair, ordered by group and then by pair
+      if (PARTS && job < shared_jobs) {
+        n = uni(job / p.n_parts);
+        part = job - n * p.n_parts;
+      } else {
+        n = job - shared_jobs;
+        before = shared;
+      }
+      const int q = uni(n / pairs), k = uni(p.K - 1 - (before + q));
+      if (!bwd_body<1, IMG, true, WIDE, PARTS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
     }
   }
   if constexpr (OWN) {
@@ -854,7 +869,8 @@ hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream)
     return hipGetLastError();
   };
   const bool own = p.n_finish == p.gang_pairs;
-  if (p.n_prefetch) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, true, true, true>);
-  if (p.wide) return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true>) : launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, false>);
-  return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, true>) : launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, false>);
+  if (p.n_prefetch) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, true, true, true, true>);
+  if (p.wide && p.n_shared > 0) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true, true>);
+  if (p.wide) return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true, false>) : launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, false, false>);
+  return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, true, false>) : launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, false, false>);
 }

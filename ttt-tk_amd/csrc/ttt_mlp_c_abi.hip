@@ -161,6 +161,8 @@ struct LaunchPlan {
   int n_finish = 0;         // backward, of a gang: for grad_L_XK / grad_L_XV
   bool prefetch = false;    // backward, wide: and one per pair that fetches ahead of the walk
   int sets = 0;             // backward: sets of the per-group tensors
+  int shared = 0;           // backward: groups, the first ones walked, that several workgroups at once replay
+  int parts = 1;            // backward: that many, a stretch of the group each
 };
 // Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
 // of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others.
@@ -181,6 +183,9 @@ void divide_workers(int pairs, int workers, int walk, int replay, int finish, in
   }
   *n_replay = workers - *n_finish;
 }
+// Where the stretches of a group begin, in eighths of it.  To the state at its first mini-batch a workgroup takes the half of every
+// replay before that carries the state, about a third of the whole, so the stretches get shorter.
+constexpr int PART_START[ttt::BWD_MAX_PARTS][ttt::BWD_MAX_PARTS + 1] = {{0, 8, 8, 8, 8}, {0, 5, 8, 8, 8}, {0, 4, 6, 8, 8}, {0, 3, 5, 7, 8}};
 LaunchPlan plan_for(long long BH, int cus, bool backward) {
   LaunchPlan pl;
   if (BH <= 0 || cus <= 0) {
@@ -205,15 +210,22 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     return pl;
   }
   // Four replaying workgroups per pair leave a walk on two CUs to itself, also where they evaluate the GELU family for it (32 pairs x 512:
-  // 25 us per replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).
+  // 25 us per replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).  What is left then is the walk's wait
+  // for the first group's replay: the first groups are replayed by two to four workgroups at once, and as many groups
+  // that way as it takes for a group replayed by one workgroup to be ready in time (three: replay of a group 57 k clocks a
+  // mini-batch, in two parts 35 k, in four 27 k; walk 19 k).  In ms, four replaying workgroups and whole groups -> so: 8 pairs x 64 in groups of 8
+  // 0.683 -> 0.617 (four parts, eight workgroups), 24 x 64 0.733 -> 0.691 and 24 x 512 in groups of 32 4.88 -> 4.64 (three, six),
+  // 32 x 512 5.12 -> 5.06 (two, four; all groups in parts: 5.25, the work done twice takes clock from the walk).
   const int on_xcd = cus / 8, pairs = static_cast<int>(per_xcd);
   if (fits_xcd(7)) {
-    const int each = fits_xcd(8) ? 4 : 3;
+    const int each = on_xcd / pairs - 4;
     pl.wide = pl.prefetch = true;
     pl.gang = pl.n_finish = pairs;
-    pl.n_replay = each * pairs;
-    pl.per_pair = each + 4;
-    pl.sets = each + 2;
+    pl.parts = each >= 8 ? 4 : each >= 6 ? 3 : each >= 4 ? 2 : 1;
+    pl.shared = each >= 4 ? 3 : 0;
+    pl.n_replay = (each >= 4 ? 2 * pl.parts : 3) * pairs;
+    pl.per_pair = each >= 4 ? 8 : 7;
+    pl.sets = each >= 4 ? 6 : 5;
     return pl;
   }
   // Two replaying workgroups per pair bound a walk on two CUs (48 pairs x 4,096 mini-batches: 20 us per replayed mini-batch, 10.1 us
@@ -228,6 +240,11 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     if (fits_xcd(5)) {
       pl.n_finish = pairs;
       pl.n_replay = 2 * pairs;
+      if (fits_xcd(6)) {   // (a third per pair pays once the first group is replayed in two parts: 40 x 512 5.67 -> 5.36 ms; five pairs on 32 CUs)
+        pl.n_replay = 3 * pairs;
+        pl.parts = 2;
+        pl.shared = 1;
+      }
     } else if (pl.wide) {
       divide_workers(pairs, on_xcd - 2 * pairs, 215, COST_REPLAY, COST_FINISH, &pl.n_replay, &pl.n_finish);
     } else {
@@ -344,6 +361,8 @@ int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K
 LaunchPlan bwd_reduced(LaunchPlan pl) {
   if (pl.prefetch) {
     pl.n_replay = 2 * pl.gang;
+    pl.parts = 1;
+    pl.shared = 0;
     pl.prefetch = false;
     pl.per_pair = 5;
     pl.sets = 4;
@@ -375,7 +394,7 @@ struct BwdWorkspace {
     size_t o = 0;
     auto put = [&](int i, size_t bytes) { off[i] = o; o += (bytes + 255) & ~(size_t)255; };
     put(0, ttt::bwd_sync_ints(n) * sizeof(int));
-    put(1, ttt::BWD_MAX_SETS * norm);
+    put(1, ttt::BWD_MAX_SETS * 8 * norm);
     put(2, norm);
     put(3, (size_t)n * img);
     put(4, pl.wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);
@@ -503,6 +522,9 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   p.gang_pairs = pl.gang;
   p.n_replay = pl.n_replay;
   p.n_sets = pl.sets;
+  p.n_shared = pl.shared;
+  p.n_parts = pl.parts;
+  for (int i = 0; i <= ttt::BWD_MAX_PARTS; i++) p.part_start[i] = PART_START[pl.parts - 1][i];
   p.n_finish = pl.n_finish;
   p.n_prefetch = pl.prefetch ? 1 : 0;
   p.wide = pl.wide ? 1 : 0;
@@ -516,7 +538,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   int* words = reinterpret_cast<int*>(base + w.off[0]);
   p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
-  p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * ttt::BWD_MAX_SETS * norm;
+  p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * ttt::BWD_MAX_SETS * 8 * norm;
   p.norm_park = reinterpret_cast<float*>(base + w.off[2]) - b0 * norm;
   p.walk_park = reinterpret_cast<__bf16*>(base + w.off[3]) - b0 * (TTT_MLP_CS * TTT_MLP_HID);
   // (sets that a sequence this short does not come to: the walk asks for operands of the group behind its last one and drops

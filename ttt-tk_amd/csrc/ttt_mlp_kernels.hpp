@@ -45,6 +45,7 @@ constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 2048;  // 8-byte words of a pair's ex
 constexpr int FWD_IMG_BYTES = 64 * 256 * 2 * 2;  // W1 and W2 as bf16 operands
 constexpr int FWD_BIAS_FLOATS = 256 + 64;
 
+constexpr int BWD_MAX_PARTS = 4;
 constexpr int BWD_MAX_SETS = 6;   // sets of per-group tensors in use at once, at most
 
 struct BwdParams {
@@ -72,7 +73,7 @@ struct BwdParams {
   __bf16 *alt_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_output_fused_group[BWD_MAX_SETS - 1];
   float* alt_std_fused_group[BWD_MAX_SETS - 1];
   float* alt_W1_init_group[BWD_MAX_SETS - 1];
-  float* norm_partial;   // [B*NH][BWD_MAX_SETS][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set
+  float* norm_partial;   // [B*NH][BWD_MAX_SETS][8][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set, by eighths of it
   float* norm_park;      // [B*NH][8 waves][2][64]: their sum over the groups walked so far (without a grad_L_XK workgroup)
   __bf16* walk_park;     // [B*NH][64][256]: one register image the walking workgroup parks across its LayerNorm stage
   // Gang (gang_pairs > 0: pairs per XCD, gang g = pairs g, g + 8, ..; ttt_mlp_bwd_wide.hip): n_replay workgroups replay for all of
@@ -82,6 +83,9 @@ struct BwdParams {
   // gradient wrt W1 and form G1 = -eta * dl/dZ1 themselves; fin_park: [B*NH][FIN_PARK_FLOATS], that copy and the norm-gradient
   // sums between two groups of a pair (n_finish < gang_pairs only).
   int gang_pairs, n_replay, n_finish;
+  // The first n_shared groups (at most n_sets) are replayed in n_parts stretches, by as many workgroups at once: part i its eighths
+  // part_start[i] .. part_start[i + 1] - 1.
+  int n_shared, n_parts, part_start[BWD_MAX_PARTS + 1];
   __bf16* fin_dz;
   float* fin_gy;
   float* fin_park;
@@ -111,8 +115,8 @@ struct BwdParams {
 #endif
 };
 
-// Layout of `sync` (ints): 32 per (batch, head).  Words 0 .. 5: the group last replayed into each set, its number from the end + 1
-// (norm_partial is written with the group).  Walk on one workgroup: word 16 the groups it has finished, word 12 the
+// Layout of `sync` (ints): 32 per (batch, head).  Words 0 .. 5: the parts of groups replayed into each set
+// so far (norm_partial is written with them).  Walk on one workgroup: word 16 the groups it has finished, word 12 the
 // mini-batches of the last group it walks that it has handed on (that group is handed over in chunks).  Word 24 the groups
 // whose finishing is done - then one status word behind all of them (non-zero: a wait gave up).
 constexpr int BWD_SYNC_STRIDE = 32;

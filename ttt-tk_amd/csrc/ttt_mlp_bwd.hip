@@ -145,19 +145,12 @@ TTT_DEV void ln_store_h(bf16* p, bf16x8 v) {
   *reinterpret_cast<bf16x4*>(p) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
   *reinterpret_cast<bf16x4*>(p + 4) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
 }
-TTT_DEV void ln_store(bf16* p, const float (&x)[8]) {
-  bf16x4 a, b;
-#pragma unroll
-  for (int e = 0; e < 4; e++) { a[e] = (bf16)x[e]; b[e] = (bf16)x[4 + e]; }
-  *reinterpret_cast<bf16x4*>(p) = a;
-  *reinterpret_cast<bf16x4*>(p + 4) = b;
-}
+template <bool PAIRS = false>
+TTT_DEV void ln_store(bf16* p, const float (&x)[8]) { ln_store_h(p, cvt8<PAIRS>(x)); }
 // 8 features of this lane's token to / from a [tok][F] bf16 tile in HBM (16 bytes per lane).
-template <bool STREAM = false>
+template <bool STREAM = false, bool PAIRS = false>
 TTT_DEV void ln_store_g(gptr_t b, unsigned voff, unsigned soff, const float (&x)[8]) {
-  bf16x8 v;
-#pragma unroll
-  for (int e = 0; e < 8; e++) v[e] = (bf16)x[e];
+  const bf16x8 v = cvt8<PAIRS>(x);
   if constexpr (STREAM) g_st_stream<bf16x8>(b, voff, soff, v);
   else g_st8h(b, voff, soff, v);
 }
@@ -288,16 +281,28 @@ TTT_DEV void acc_init_rows_lds(AccT<1, CB>& a, const float* s_vec, int h) {
 }
 
 TTT_DEV bf16x8 cvt8(const f32x4 lo, const f32x4 hi) {
-  bf16x8 o;
-#pragma unroll
-  for (int e = 0; e < 4; e++) { o[e] = (bf16)lo[e]; o[4 + e] = (bf16)hi[e]; }
-  return o;
+  const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  return cvt8(x);
 }
 // Piece (kappa order) straight from a row-major fp32 matrix in HBM: lane = row row0 + c, contraction =
 // columns col0 + 16 s ...; row0, col0, s wave-uniform.
 TTT_DEV bf16x8 piece_from_f32(gptr_t g, unsigned off, int ld, int row0, int col0, int s, int c, int h) {
   const unsigned vo = (c * ld + 4 * h) * 4, so = off + (row0 * ld + col0 + 16 * s) * 4;
   return cvt8(g_ld4f(g, vo, so), g_ld4f(g, vo, so + 32));
+}
+
+// gelu, gelu', gelu'' of eight bf16 values, rounded to bf16.
+template <bool PAIRS>
+TTT_DEV void gelu_images(const bf16x8 z, bf16x8& g, bf16x8& a, bf16x8& b) {
+#pragma unroll
+  for (int jj = 0; jj < 8; jj += 2) {
+    float g2[2], a2[2], b2[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) gelu_fdd((float)z[jj + q], g2[q], a2[q], b2[q]);
+    put_cvt<PAIRS>(g, jj, g2[0], g2[1]);
+    put_cvt<PAIRS>(a, jj, a2[0], a2[1]);
+    put_cvt<PAIRS>(b, jj, b2[0], b2[1]);
+  }
 }
 
 // Pair sum of a product z (rows F, column block 0 = the token block this wave keeps, column block 1 =
@@ -393,6 +398,7 @@ template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false>
 // the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).
 // False: a wait gave up.
 TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi, const int k_lo, const int part = 0) {
+  constexpr bool PAIRS = ROLE == 0;
   static_assert(!(ROLE == 0 && (IMG || FIN)), "one workgroup per (batch, head) does everything itself");
   bf16* s_xq = reinterpret_cast<bf16*>(smem + SB_XQ);
   bf16* s_xk = reinterpret_cast<bf16*>(smem + SB_XK);
@@ -656,37 +662,32 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-              const bf16x8 zr = pack8(x2.b[0][i], t);
+              const bf16x8 zr = pack8<PAIRS>(x2.b[0][i], t);
               if constexpr (FULL && !IMG) {
                 image_store<ROLE != 0>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
               } else if constexpr (FULL) {
                 // The walk needs gelu, gelu' and gelu'' of the ROUNDED Z1 (what it would compute from the image
                 // of Z1); a replaying workgroup has the time to do that for it.
                 bf16x8 gv, av, bv;
-#pragma unroll
-                for (int jj = 0; jj < 8; jj++) {
-                  float g, a, b;
-                  gelu_fdd((float)zr[jj], g, a, b);
-                  gv[jj] = (bf16)g;
-                  av[jj] = (bf16)a;
-                  bv[jj] = (bf16)b;
-                }
+                gelu_images<PAIRS>(zr, gv, av, bv);
                 image_store<ROLE != 0>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, gv);
                 image_store<ROLE != 0>(bDD, j * (2 * IMG_BYTES), 2 * tb[i] + t, t16, av);
                 image_store<ROLE != 0>(bDD, j * (2 * IMG_BYTES) + IMG_BYTES, 2 * tb[i] + t, t16, bv);
               }
               bf16x8 xv;
 #pragma unroll
-              for (int jj = 0; jj < 8; jj++) {
-                float g, d;
-                gelu_fd(x2.b[0][i][8 * t + jj], g, d);
-                const bf16 gh = (bf16)g;
-                xv[jj] = gh;
-                x2lo[i][t][jj] = (bf16)(g - (float)gh);
-                d1f[i][8 * t + jj] = d;
-                // pinned: left to itself the compiler finishes gelu' only where it is used, two stages on, and keeps
-                // three values per element alive until then instead of one (a dozen of them in scratch memory)
-                asm volatile("" : "+v"(d1f[i][8 * t + jj]));
+              for (int jj = 0; jj < 8; jj += 2) {
+                float g[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                  float d;
+                  gelu_fd(x2.b[0][i][8 * t + jj + q], g[q], d);
+                  d1f[i][8 * t + jj + q] = d;
+                  // pinned: left to itself the compiler finishes gelu' only where it is used, two stages on, and keeps
+                  // three values per element alive until then instead of one (a dozen of them in scratch memory)
+                  asm volatile("" : "+v"(d1f[i][8 * t + jj + q]));
+                }
+                put_split<PAIRS>(xv, x2lo[i][t], jj, g[0], g[1]);
               }
               store_piece_rows<LDH>(T0, tb[i], t, c, h, xv);
             }
@@ -742,14 +743,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             }
           }
           if constexpr (FULL) {
-            ln_store_g<ROLE != 0>(bXHF, vln, j * TILE_BYTES, z);
-            ln_store_g<ROLE != 0>(bGOF, vln, j * TILE_BYTES, go);
+            ln_store_g<ROLE != 0, PAIRS>(bXHF, vln, j * TILE_BYTES, z);
+            ln_store_g<ROLE != 0, PAIRS>(bGOF, vln, j * TILE_BYTES, go);
           }
           const float s1 = oct_sum(sum8(gx)), s2 = oct_sum(dot8(gx, z));
           const float sc = rstd * (1.f / FD), neg_eta = -bf2f(s_etah[tok]);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;   // dl/dZ2
-          if constexpr (FULL) ln_store_g<ROLE != 0>(bGZ2, vln, j * TILE_BYTES, gx);
+          if constexpr (FULL) ln_store_g<ROLE != 0, PAIRS>(bGZ2, vln, j * TILE_BYTES, gx);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] *= neg_eta;                             // G2, in two terms (the second in
           ln_token_sum_store(s_deta + v * CS, gx, lane, f0);   // b2's step: this wave's share (s_deta is the walk's otherwise)
@@ -816,11 +817,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             for (int t = 0; t < 2; t++) {
               bf16x8 gv, gvl;
 #pragma unroll
-              for (int jj = 0; jj < 8; jj++) {
-                const float g = g1.b[0][i][8 * t + jj] * d1f[i][8 * t + jj];
-                const bf16 gh = (bf16)g;
-                gv[jj] = gh;
-                gvl[jj] = (bf16)(g - (float)gh);
+              for (int jj = 0; jj < 8; jj += 2) {
+                const int k0 = 8 * t + jj, k1 = k0 + 1;
+                put_split<PAIRS>(gv, gvl, jj, g1.b[0][i][k0] * d1f[i][k0], g1.b[0][i][k1] * d1f[i][k1]);
               }
               store_piece_rows<LDH>(T1, tb[i], t, c, h, gv);      // G1 rows [tok][hid], two terms
               store_piece_rows<LDH>(T2, tb[i], t, c, h, gvl);
@@ -957,11 +956,12 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
             for (int t = 0; t < 2; t++) {
 #pragma unroll
-              for (int jj = 0; jj < 8; jj++) {
-                float g, d;
-                gelu_fd(z1b.b[0][i][8 * t + jj], g, d);
-                x2bQ[i][t][jj] = (bf16)g;
-                d1b[i][t][jj] = (bf16)d;
+              for (int jj = 0; jj < 8; jj += 2) {
+                float g[2], d[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) gelu_fd(z1b.b[0][i][8 * t + jj + q], g[q], d[q]);
+                put_cvt<PAIRS>(x2bQ[i][t], jj, g[0], g[1]);
+                put_cvt<PAIRS>(d1b[i][t], jj, d[0], d[1]);
               }
               asm volatile("" : "+v"(d1b[i][t]));   // finished here, not where it is used (see gelu'(Z1) above)
               store_piece_rows<LDH>(T0, tb[i], t, c, h, x2bQ[i][t]);
@@ -1019,8 +1019,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           const float sc = 1.f / (FD * sd);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;
-          ln_store(s_a + tok * LDX + f0, gx);            // gZ2_bar
-          ln_store_g<ROLE != 0>(bGZB, vln, j * TILE_BYTES, gx);
+          ln_store<PAIRS>(s_a + tok * LDX + f0, gx);            // gZ2_bar
+          ln_store_g<ROLE != 0, PAIRS>(bGZB, vln, j * TILE_BYTES, gx);
         }
         __syncthreads();
         TTT_STAGE(BS_R_OUT_LN);
@@ -1064,7 +1064,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
               for (int t = 0; t < 2; t++) {
                 bf16x8 gzb;
 #pragma unroll
-                for (int jj = 0; jj < 8; jj++) gzb[jj] = (bf16)(gz1b.b[0][i][8 * t + jj] * (float)d1b[i][t][jj]);
+                for (int jj = 0; jj < 8; jj += 2)
+                  put_cvt<PAIRS>(gzb, jj, gz1b.b[0][i][8 * t + jj] * (float)d1b[i][t][jj], gz1b.b[0][i][8 * t + jj + 1] * (float)d1b[i][t][jj + 1]);
                 store_piece_rows<LDH>(T1, tb[i], t, c, h, gzb);    // gZ1_bar rows [tok][hid]
               }
           }
@@ -1091,8 +1092,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           float z[8];
           ln_gather(z, s_lnrow);
 #pragma unroll
-          for (int e = 0; e < 8; e++) dxq_old[e] = (bf16)((float)dxq_old[e] + (z[e] + gO[e]));
-          g_st_stream<bf16x8>(bDXQ, vln, mb * TILE_BYTES, dxq_old);
+          for (int e = 0; e < 8; e++) z[e] = (float)dxq_old[e] + (z[e] + gO[e]);
+          g_st_stream<bf16x8>(bDXQ, vln, mb * TILE_BYTES, cvt8<PAIRS>(z));
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier at the loop's top
         TTT_STAGE(BS_R_OUT_BACKWARD);
@@ -1281,17 +1282,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           // fetched as three images that a replaying workgroup computed the same way
           bf16x8 ac[2], bc[2];
           if constexpr (!IMG) {
-            const bf16x8 zc[2] = {gq[i][0], gq[i][1]};
 #pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-              for (int jj = 0; jj < 8; jj++) {
-                float g, a, b;
-                gelu_fdd((float)zc[t][jj], g, a, b);
-                x2c[t][jj] = (bf16)g;
-                ac[t][jj] = (bf16)a;
-                bc[t][jj] = (bf16)b;
-              }
+            for (int t = 0; t < 2; t++) gelu_images<PAIRS>(gq[i][t], x2c[t], ac[t], bc[t]);
           } else {
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -1304,15 +1296,23 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           for (int t = 0; t < 2; t++) {
             bf16x8 t2c, g1c, uhc;
 #pragma unroll
-            for (int jj = 0; jj < 8; jj++) {
-              const float a = (float)ac[t][jj], b = (float)bc[t][jj];
-              const float r0 = R.b[0][0][8 * t + jj], sv = S.b[0][0][8 * t + jj];
-              const float gz1 = r0 * a;                                   // dl/dZ1
-              de[i] = __builtin_fmaf(gz1, sv, de[i]);
-              uc[t][jj] = (bf16)(sv * a);
-              uhc[jj] = (bf16)(-eta_i[i] * sv * a);
-              g1c[jj] = (bf16)(-eta_i[i] * gz1);
-              t2c[jj] = (bf16)(-eta_i[i] * r0 * sv * b);
+            for (int jj = 0; jj < 8; jj += 2) {
+              float u[2], uh[2], g[2], t2[2];
+#pragma unroll
+              for (int q = 0; q < 2; q++) {
+                const float a = (float)ac[t][jj + q], b = (float)bc[t][jj + q];
+                const float r0 = R.b[0][0][8 * t + jj + q], sv = S.b[0][0][8 * t + jj + q];
+                const float gz1 = r0 * a;                                   // dl/dZ1
+                de[i] = __builtin_fmaf(gz1, sv, de[i]);
+                u[q] = sv * a;
+                uh[q] = -eta_i[i] * sv * a;
+                g[q] = -eta_i[i] * gz1;
+                t2[q] = -eta_i[i] * r0 * sv * b;
+              }
+              put_cvt<PAIRS>(uc[t], jj, u[0], u[1]);
+              put_cvt<PAIRS>(uhc, jj, uh[0], uh[1]);
+              put_cvt<PAIRS>(g1c, jj, g[0], g[1]);
+              put_cvt<PAIRS>(t2c, jj, t2[0], t2[1]);
             }
             chunk_store(bPUH, 0, 2 * tb[i] + t, t16, uhc);
             // nothing stays in registers across the LayerNorm stage: g1 and t2 (and, without the images,
@@ -1341,7 +1341,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         }
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-          const float a = half_sum(de[i]);
+          const float a = half_sum_valu(de[i]);   // (a shuffle keeps a lane index over the loop, and reloads it here)
           if (h == 0) s_deta[v * CS + 32 * tb[i] + c] = a;
         }
         WAVE_SYNC();   // this wave's readers of T1 / T2 are done
@@ -1412,7 +1412,12 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           gx[e] = gx[e] * rsd + (sg * xh[e] - sx * rsd) * (1.f / FD);   // dZ2
-          if constexpr (!FIN) dxv_old[e] = (bf16)((float)dxv_old[e] - gy[e]);   // dXV accumulates -g_y
+        }
+        if constexpr (!FIN) {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = (float)dxv_old[e] - gy[e];   // dXV accumulates -g_y
+          dxv_old = cvt8<PAIRS>(x);
         }
         // g_y is needed again for dXK: park it (the XQ / E2 tiles are dead by now), or hand it over
         {
@@ -1429,7 +1434,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             *reinterpret_cast<f32x4*>(s_gy + 4) = hi;
           }
         }
-        ln_store(s_a + tok * LDX + f0, gx);
+        ln_store<PAIRS>(s_a + tok * LDX + f0, gx);
         if constexpr (!FIN) g_st_stream<bf16x8>(bDXV, vln, xo, dxv_old);
       }
       TTT_STAGE(BS_W_LN);
@@ -1485,10 +1490,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int jj = 0; jj < 8; jj++) {
-              const float d1v = (float)d1c[t][jj];
-              dzp[i][t][jj] = (bf16)__builtin_fmaf(dx2.b[0][0][8 * t + jj], d1v, (float)t2c[t][jj]);
-            }
+            for (int jj = 0; jj < 8; jj += 2)
+              put_cvt<PAIRS>(dzp[i][t], jj, __builtin_fmaf(dx2.b[0][0][8 * t + jj], (float)d1c[t][jj], (float)t2c[t][jj]),
+                                       __builtin_fmaf(dx2.b[0][0][8 * t + jj + 1], (float)d1c[t][jj + 1], (float)t2c[t][jj + 1]));
           uhp[i][0] = chunk_load(bPUH, 0, 2 * tb[i], t16);       // -eta * S * gelu', formed with S two stages back
           uhp[i][1] = chunk_load(bPUH, 0, 2 * tb[i] + 1, t16);
         }
@@ -1543,8 +1547,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         ln_gather(z, s_lnrow);
         ln_load_f32(gyv, s_gy);
 #pragma unroll
-        for (int e = 0; e < 8; e++) dxk_old[e] = (bf16)((float)dxk_old[e] + (z[e] + gyv[e]));
-        g_st_stream<bf16x8>(bDXK, vln, xo, dxk_old);
+        for (int e = 0; e < 8; e++) z[e] = (float)dxk_old[e] + (z[e] + gyv[e]);
+        g_st_stream<bf16x8>(bDXK, vln, xo, cvt8<PAIRS>(z));
       }
       TTT_STAGE(BS_W_DXK);
       if constexpr (ROLE == 2 && FIN) {
@@ -1883,14 +1887,14 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
       ln_gather(z, s_lnrow);
       const float gyv[8] = {gy_lo[0], gy_lo[1], gy_lo[2], gy_lo[3], gy_hi[0], gy_hi[1], gy_hi[2], gy_hi[3]};
       const float dgv[8] = {dg_lo[0], dg_lo[1], dg_lo[2], dg_lo[3], dg_hi[0], dg_hi[1], dg_hi[2], dg_hi[3]};
-      bf16x8 dxk_new, dxv_new;
+      float dxv_new[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        dxk_new[e] = (bf16)((float)dxk_ld[e] + (z[e] + gyv[e]));
-        dxv_new[e] = (bf16)((float)dxv_ld[e] - gyv[e]);                 // dXV accumulates -g_y
+        z[e] = (float)dxk_ld[e] + (z[e] + gyv[e]);
+        dxv_new[e] = (float)dxv_ld[e] - gyv[e];                         // dXV accumulates -g_y
       }
-      g_st_stream<bf16x8>(gDXK, vln, xo, dxk_new);
-      g_st_stream<bf16x8>(gDXV, vln, xo, dxv_new);
+      g_st_stream<bf16x8>(gDXK, vln, xo, cvt8(z));
+      g_st_stream<bf16x8>(gDXV, vln, xo, cvt8(dxv_new));
       ln_token_sum_add(s_dgw, dgv, lane, f0);
       ln_token_sum_add(s_dbw, gyv, lane, f0);
       __syncthreads();   // the readers of the pair sums are done before the next mini-batch's take their place

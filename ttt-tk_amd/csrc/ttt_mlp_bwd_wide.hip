@@ -569,7 +569,10 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
   }
   if (gave_up && lane == 0) s_flag[0] = 1;
   __syncthreads();
-  if (flag(0) != 0) return;
+  if (flag(0) != 0) {
+    if (lane == 0) report_status(w_status);
+    return;
+  }
   const gword64_t xch = (gword64_t)(p.xchg + (size_t)bh * BWW_XCHG_WORDS);
   const float* const s_row = reinterpret_cast<const float*>(smem + BWW_P) + t_in * LDR + f0;
   float gam[8];
@@ -701,7 +704,10 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       TTT_STAGE(BWH_LN1);
       __syncthreads();   // B3
       TTT_STAGE(BWH_B3);
-      if (flag(0) != 0) return;
+      if (flag(0) != 0) {
+        if (lane == 0) report_status(w_status);
+        return;
+      }
       store_block(1);
       if (u < 2) lds_rowsum_add_jit(s_gb2 + 32 * u, [&](int s) { return piece_tr<LDX>(s_dz2, u, s, lane); }, ones, c, h);
       TTT_STAGE(BWH_STORE1);

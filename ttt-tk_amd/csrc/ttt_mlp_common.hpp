@@ -36,10 +36,35 @@ constexpr float LN_EPS = 1e-8f;
 
 #define TTT_DEV __device__ __forceinline__
 
+// Two values converted into elements j, j + 1 of o.  PAIRS: as a pair, one instruction; written one by one the compiler often takes one
+// for each and a third to join them (a quarter of the backward's conversions, by its listing).  The kernel with one workgroup
+// per (batch, head) gains 2 % by it (200 pairs x 100 mini-batches, backward 4.05 -> 3.97 ms); in the others the compiler recognises a pair of
+// the running gradients two stages on, keeps it until then and spills for it (32 x 512 4.97 -> 5.13 ms).
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <bool PAIRS>
+TTT_DEV void put_cvt(bf16x8& o, int j, float a, float b) {
+  if constexpr (PAIRS) {
+    const f32x2 ab = {a, b};
+    const bf16x2 h = __builtin_convertvector(ab, bf16x2);
+    o[j] = h[0];
+    o[j + 1] = h[1];
+  } else {
+    o[j] = (bf16)a;
+    o[j + 1] = (bf16)b;
+  }
+}
+template <bool PAIRS = false>
+TTT_DEV bf16x8 cvt8(const float (&x)[8]) {
+  bf16x8 o;
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) put_cvt<PAIRS>(o, j, x[j], x[j + 1]);
+  return o;
+}
+template <bool PAIRS = false>
 TTT_DEV bf16x8 pack8(const f32x16& x, int t) {
   bf16x8 o;
 #pragma unroll
-  for (int j = 0; j < 8; j++) o[j] = (bf16)x[8 * t + j];
+  for (int j = 0; j < 8; j += 2) put_cvt<PAIRS>(o, j, x[8 * t + j], x[8 * t + j + 1]);
   return o;
 }
 
@@ -49,13 +74,26 @@ TTT_DEV bf16x8 pack8(const f32x16& x, int t) {
 // recurrence's state from one mini-batch to the next near 2^-17 instead of 2^-9.
 // Two values at a time: one packed conversion for the high-order terms, a shift and a mask to read them back as
 // fp32, two subtractions, one packed conversion for the low-order terms (6 instructions per pair).
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 TTT_DEV void split2(float a, float b, bf16x2& hi, bf16x2& lo) {
   const f32x2 ab = {a, b};
   hi = __builtin_convertvector(ab, bf16x2);
   const uint32_t hp = __builtin_bit_cast(uint32_t, hi);
   const f32x2 r = {a - __builtin_bit_cast(float, hp << 16), b - __builtin_bit_cast(float, hp & 0xffff0000u)};
   lo = __builtin_convertvector(r, bf16x2);
+}
+template <bool PAIRS>
+TTT_DEV void put_split(bf16x8& hi, bf16x8& lo, int j, float a, float b) {   // the same, into elements j, j + 1
+  if constexpr (PAIRS) {
+    bf16x2 h2, l2;
+    split2(a, b, h2, l2);
+    hi[j] = h2[0]; hi[j + 1] = h2[1];
+    lo[j] = l2[0]; lo[j + 1] = l2[1];
+  } else {
+    const bf16 h0 = (bf16)a, h1 = (bf16)b;
+    hi[j] = h0; hi[j + 1] = h1;
+    lo[j] = (bf16)(a - (float)h0);
+    lo[j + 1] = (bf16)(b - (float)h1);
+  }
 }
 TTT_DEV void split8(const f32x16& x, int t, bf16x8& hi, bf16x8& lo) {
 #pragma unroll
@@ -493,9 +531,10 @@ TTT_DEV void clear_word(int* w, int n, int i, const int* report) {   // word i o
   const int k = i - (n - STATUS_WORDS);
   if (i < n) w[i] = k == 2 ? static_cast<int>(static_cast<uint32_t>(r)) : k == 3 ? static_cast<int>(static_cast<uint32_t>(r >> 32)) : 0;
 }
-TTT_DEV void raise_status(int* status) {
-  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  int* const report = reinterpret_cast<int*>(__hip_atomic_load(reinterpret_cast<uint64_t*>(status + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+TTT_DEV void raise_status(int* status) { __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// (apart from it, on the way out, where waits are in a hot loop: next to them it cost the recurrence on two CUs 1.5 %)
+TTT_DEV void report_status(const int* status) {
+  int* const report = reinterpret_cast<int*>(__hip_atomic_load(reinterpret_cast<const uint64_t*>(status + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   if (report != nullptr) __hip_atomic_store(report, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 TTT_DEV bool wait_at_least(int* word, int target, int* status, int* s_flag, uint64_t limit) {
@@ -508,6 +547,7 @@ TTT_DEV bool wait_at_least(int* word, int target, int* status, int* s_flag, uint
     while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
         raise_status(status);
+        report_status(status);
         ok = 0;
         break;
       }
@@ -530,6 +570,7 @@ TTT_DEV int wait_for_pace(int* word, int target, int* status, int* s_flag, uint6
     while ((seen = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
         raise_status(status);
+        report_status(status);
         seen = -1;
         break;
       }
@@ -551,6 +592,7 @@ TTT_DEV int wait_for_both(int* a, int* b, int target, int* status, int* s_flag, 
                        __hip_atomic_load(b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < target) {
       if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > limit) {
         raise_status(status);
+        report_status(status);
         seen = -1;
         break;
       }

@@ -366,7 +366,10 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   const bool near = on_one_xcd(words + WDW_XCD, n_wg, lane, w_status, p.wait_limit, alive);
   if (!alive && lane == 0) *s_flag = 1;
   __syncthreads();
-  if (flag() != 0) return;
+  if (flag() != 0) {
+    if (lane == 0) report_status(w_status);
+    return;
+  }
   const gword64_t xch = (gword64_t)(p.xchg + (size_t)bh * FWD_XCHG_WORDS);
   const float* const s_row0 = reinterpret_cast<const float*>(smem + WD_P0) + t_in * LDP + f0;
   const float* const s_row1 = reinterpret_cast<const float*>(smem + WD_P1) + t_in * LDP + f0;
@@ -507,7 +510,10 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     TTT_STAGE(FWH_LN1);
     __syncthreads();   // B3
     TTT_STAGE(FWH_B3);
-    if (flag() != 0) return;
+    if (flag() != 0) {
+      if (lane == 0) report_status(w_status);
+      return;
+    }
     if (u == 0 && lane == 0 && mb > 0) give(mb);   // the stores of the last mini-batch's state were acknowledged before B3
     // b2's step, while the compute waves are busy: the four helper waves wait for each other's shares (all of them come here)
     ln_token_sum_store_product(s_b2p + (4 + u) * FD, gx, scale, lane, f0);

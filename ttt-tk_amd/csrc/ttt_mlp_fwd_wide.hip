@@ -13,11 +13,14 @@
 // One or two more workgroups per pair compute Out from the states left in a ring, as in the two-workgroup launch.
 // Every sum has the order of the one-workgroup kernel: results are the same to the bit.
 //
-// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.57 ms here (6.1 us per
-// mini-batch), 48 x 4,096: 32.5 -> 24.2 ms.  With the stage clocks in, 14.3 k clocks: block 0's products 2.7 k; block 1's 3.7 k
-// while block 0's sums cross (gather and send 1.25 k, 1.1 k under way, LayerNorm 1.8 k) and 0.75 k of waiting for them;
-// block 0's weight step 2.0 k while block 1's sums cross and 2.35 k of waiting for those; block 1's weight step and the
-// split of the new state 2.65 k.
+// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.55 ms here (6.1 us per
+// mini-batch), 24 x 256 1.49 ms.  With the stage clocks in, 13.9 k clocks: block 0's GELU and partial sums 2.4 k; block 1's 3.7 k
+// while block 0's sums cross (gather and send 1.3 k, 0.9 k under way, LayerNorm 1.7 k) and 0.45 k of waiting for them;
+// block 0's weight step 2.1 k while block 1's sums cross and 2.25 k of waiting for those; block 1's weight step, the
+// split of the new state and Z1 of the next block 0 2.9 k.  (Before Z1 was started under that split, and with the token
+// sums for b2 and the wait for a free ring slot between the exchanges, 14.2 k: 24 x 256 1.53 ms, 12 x 64 396 us, now 383.)
+// From 40 pairs on the shorter chain is mostly paid back in clock rate: 48 x 256 1.545 ms before, 1.55 alone, 1.57 -> 1.55
+// in a step.
 #include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
 
@@ -129,6 +132,18 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     bf16x8 xk[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) xk[s] = xpiece_rows(reinterpret_cast<const bf16*>(smem + WD_XK), 0, s, c, h);
+    // Z1 = XK W1 + b1 of the token block in xk; that of a mini-batch's block 0 is formed at the end of the one before, under the split of
+    // the new W1
+    f32x16 z1;
+    auto z1_start = [&]() {
+#pragma unroll
+      for (int i = 0; i < 16; i++) z1[i] = b1L;
+    };
+    z1_start();
+#pragma unroll
+    for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
+#pragma unroll
+    for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
     TTT_STAGES_BEGIN();
     for (int mb = 0; mb < p.NC; mb++) {
       const bf16* const s_xk = reinterpret_cast<const bf16*>(smem + WD_XK + (mb & 1) * SM_TILE);
@@ -155,16 +170,17 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
 #pragma unroll
         for (int s = 0; s < 4; s++) xk[s] = xpiece_rows(x, rb, s, c, h);
       };
-      // Z1 = XK W1 + b1 and X2 = gelu(Z1), gelu'(Z1) of token block rb; X2's high-order term to LDS
+      // X2 = gelu(Z1), gelu'(Z1) of token block rb; X2's high-order term to LDS
       auto z1_block = [&](int rb, bool images) {
         WD_LANE;
-        f32x16 x2;
+        if (rb == 1) {
+          z1_start();
 #pragma unroll
-        for (int i = 0; i < 16; i++) x2[i] = b1L;
+          for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
 #pragma unroll
-        for (int s = 0; s < 4; s++) x2 = MFMA(xk[s], w1l.v[0][s], x2);
-#pragma unroll
-        for (int s = 0; s < 4; s++) x2 = MFMA(xk[s], w1h.v[0][s], x2);
+          for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
+        }
+        f32x16 x2 = z1;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           if (images) {
@@ -329,7 +345,17 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       b1L += half_sum_valu(colsum);
       load_xk(mb + 1, 0);   // (put there before B2)
       cvt_chain_split(W2s, w2h, w2l);
-      cvt_chain_split(W1s, w1h, w1l);
+      __builtin_amdgcn_sched_barrier(0);
+      z1_start();
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        split8(W1s.b[s >> 1][0], s & 1, w1h.v[0][s], w1l.v[0][s]);
+        __builtin_amdgcn_sched_barrier(0);
+        z1 = MFMA(xk[s], w1l.v[0][s], z1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
       TTT_STAGE(FWC_STEP1);
       if (gave_up != 0) return;
     }
@@ -376,7 +402,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   float b2v[8], b2L = s_b2[lane];                     // b2 of this lane's features, and of feature `lane` (wave 4 stores that one)
 #pragma unroll
   for (int e = 0; e < 8; e++) b2v[e] = s_b2[f0 + e];
-  float gx[8], scale = 0.f;                           // G2 of the last block (gx * scale): its token sums are formed while the next block's sums travel
+  float gx[2][8], scale[2] = {0.f, 0.f};               // G2 of the two blocks (gx * scale), whose token sums wait until the compute waves have what they wait for
   __builtin_amdgcn_s_setprio(2);                      // these waves' few instructions are what the other four wait for
   int seen0 = 0, seen1 = 0;                           // mini-batches the output workgroups are known to have finished
   bool gave_up = false;
@@ -434,10 +460,10 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
         z[2 * k + 1] = (wd_hi(wv[k]) + m0[2 * k + 1]) + m1[2 * k + 1];
       }
     }
-    scale = ln_loss_gradient(z, xk, xv, bf2f(eta), s_gam + f0, s_bet + f0, gx);
+    scale[blk] = ln_loss_gradient(z, xk, xv, bf2f(eta), s_gam + f0, s_bet + f0, gx[blk]);
     f32x16 g2;
 #pragma unroll
-    for (int e = 0; e < 8; e++) { g2[e] = gx[e] * scale; g2[8 + e] = 0.f; }
+    for (int e = 0; e < 8; e++) { g2[e] = gx[blk][e] * scale[blk]; g2[8 + e] = 0.f; }
     bf16x8 o, ol;
     split8_plain(g2, 0, o, ol);
     lds_put16(s_g2 + tok * FLD + f0, __builtin_bit_cast(u32x4, o));
@@ -454,6 +480,28 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       b2L += q[lane];
     }
     if (u == 0 && half == 0) p.bias_img[((size_t)bh * FWD_WIDE_RING + m % FWD_WIDE_RING) * FWD_BIAS_FLOATS + HID + lane] = b2L;
+  };
+  // The slot that mini-batch mb's state goes to is free once the output branch is done with mini-batch mb - RING.  Waited for ahead of
+  // the sums, where these waves have time (with one output workgroup, which only just keeps up, behind block 0's: 72 pairs x 256 1.78 ms
+  // so, 1.86 ms ahead of them; 24 x 256 1.51 ms and 1.485).
+  auto ring_slot = [&](int mb) {
+    if (u == 3 && mb >= FWD_WIDE_RING) {
+      const int old = mb - FWD_WIDE_RING, o = old % p.n_out, need = old / p.n_out + 1;
+      int seen = o == 0 ? seen0 : seen1;
+      if (seen < need) {
+        const uint64_t t0 = wall_clock64();
+        while ((seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(words + WDW_TAKEN + 4 * o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < need) {
+          if (__hip_atomic_load(w_status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > p.wait_limit) {
+            raise_status(w_status);
+            gave_up = true;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(4);
+        }
+        if (o == 0) seen0 = seen;
+        else seen1 = seen;
+      }
+    }
   };
   // this half's states of mini-batches 0 .. n - 1 are out
   auto give = [&](int n) {
@@ -474,6 +522,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       eta[k] = g_ldh(gEta, 2 * t_in, mb * (CS * 2) + k * CS);
     }
     load_xk(mb + 1 < p.NC ? mb + 1 : mb);
+    if (p.n_out > 1) ring_slot(mb);
     TTT_STAGE(FWH_ASK);
     __syncthreads();   // B1
     TTT_STAGE(FWH_B1);
@@ -481,29 +530,11 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     put_xk(mb + 1);   // the buffer was last read a mini-batch ago
     TTT_STAGE(FWH_SEND0);
     finish_block(mb, 0, xk[0], xv[0], eta[0]);
-    if (u == 3 && mb >= FWD_WIDE_RING) {
-      // the slot this mini-batch's state goes to is free once the output branch is done with mini-batch mb - RING
-      const int old = mb - FWD_WIDE_RING, o = old % p.n_out, need = old / p.n_out + 1;
-      int seen = o == 0 ? seen0 : seen1;
-      if (seen < need) {
-        const uint64_t t0 = wall_clock64();
-        while ((seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(words + WDW_TAKEN + 4 * o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < need) {
-          if (__hip_atomic_load(w_status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > p.wait_limit) {
-            raise_status(w_status);
-            gave_up = true;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(4);
-        }
-        if (o == 0) seen0 = seen;
-        else seen1 = seen;
-      }
-    }
+    if (p.n_out == 1) ring_slot(mb);
     TTT_STAGE(FWH_LN0);
     __syncthreads();   // B2
     TTT_STAGE(FWH_B2);
     gather_send(mb, 1);
-    ln_token_sum_store_product(s_b2p + u * FD, gx, scale, lane, f0);
     TTT_STAGE(FWH_SEND1);
     finish_block(mb, 1, xk[1], xv[1], eta[1]);
     if (gave_up && lane == 0) *s_flag = 1;
@@ -516,7 +547,8 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     }
     if (u == 0 && lane == 0 && mb > 0) give(mb);   // the stores of the last mini-batch's state were acknowledged before B3
     // b2's step, while the compute waves are busy: the four helper waves wait for each other's shares (all of them come here)
-    ln_token_sum_store_product(s_b2p + (4 + u) * FD, gx, scale, lane, f0);
+    ln_token_sum_store_product(s_b2p + u * FD, gx[0], scale[0], lane, f0);
+    ln_token_sum_store_product(s_b2p + (4 + u) * FD, gx[1], scale[1], lane, f0);
     if (lane == 0) __hip_atomic_fetch_add(s_flag + 1, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     while (__hip_atomic_load(s_flag + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < 4 * (mb + 1)) __builtin_amdgcn_s_sleep(1);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");

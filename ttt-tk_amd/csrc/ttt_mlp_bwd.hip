@@ -376,6 +376,94 @@ TTT_DEV int parts_until(const BwdParams& p, int done) {
   return use + (done - use * p.n_sets < p.n_shared ? p.n_parts : 1);
 }
 
+// ------------------------------------------------------------------ one workgroup per (batch, head), and helpers
+// Between half and all of the CUs' number of pairs a workgroup each leaves CUs idle, and a second workgroup for each does not fit.  The idle ones
+// replay checkpoint groups for whoever has most to do: one is free to take a group as soon as one of the pair's sets
+// beyond the caller's is free, and writes it into that set; the pair's own workgroup, when it comes to a group, walks it from the set
+// if it is taken and replays it itself if it is not.  Who takes what depends on the timing, the results do not.  A
+// workgroup waits only for a group that a running one has taken, so nothing has to be resident at once.
+constexpr int HELP_ONE = 24, HELP_TWO = 44;   // first bits of what is taken into sets 1 and 2
+// The pair's workgroup comes to group number `done`: the set it is (being) replayed into, or 0.  Its sets of the group before
+// are free again: every wave has what it read of them.
+TTT_DEV int take_group(int* word, int done, int* s_flag, bool first_lane) {
+  __syncthreads();
+  if (first_lane) {
+    uint64_t* const w = reinterpret_cast<uint64_t*>(word);
+    uint64_t old = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), to;
+    int set;
+    do {
+      uint64_t one = (old >> HELP_ONE) & 0xfffff, two = old >> HELP_TWO;
+      const uint64_t here = done + 1;
+      set = one == here ? 1 : two == here ? 2 : 0;
+      if (one < here) one = 0;
+      if (two < here) two = 0;
+      to = (two << HELP_TWO) | (one << HELP_ONE) | (2 * (uint64_t)done + (set > 0 ? 1 : 0));
+    } while (!__hip_atomic_compare_exchange_strong(w, &old, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    *s_flag = set;
+  }
+  __syncthreads();
+  return uni(*s_flag);
+}
+// A helper takes a group: job[0] = pair (of the launch), job[1] = number of the group, job[2] = set; false: there is none left to
+// take (or a wait gave up, or nothing came free for as long as one may wait: nobody waits for this workgroup).
+// Taken is the group that the pair will come to next once this one could be ready: the one behind those taken already, else the
+// next one while the pair replays, the one behind that while it walks.
+TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
+  const int lane = threadIdx.x & 63;
+  __syncthreads();   // the last job has been read by every wave
+  if (threadIdx.x < 64) {
+    int* const words = p.sync + (size_t)p.bh0 * BWD_SYNC_STRIDE + BWD_HELP;
+    const uint64_t t0 = wall_clock64();
+    int took = 0;
+    for (bool more = true; more;) {
+      // what is left to do of a pair, in hundredths of a mini-batch of its own workgroup: a group's replay is half of it
+      int most = -1, pair = 0, group = 0, set = 0;
+      uint64_t seen = 0;
+      bool open = false;
+      for (int i = lane; i < p.nbh; i += 64) {
+        const int q = i + me < p.nbh ? i + me : i + me - p.nbh;   // (not all helpers the same one)
+        const uint64_t w = __hip_atomic_load(reinterpret_cast<uint64_t*>(words + (size_t)q * BWD_SYNC_STRIDE), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int at = static_cast<int>(w & 0xffffff), done = at >> 1, walks = at & 1;
+        const int one = static_cast<int>((w >> HELP_ONE) & 0xfffff), two = static_cast<int>(w >> HELP_TWO), last = max(one, two);
+        const int ahead = (one > done + 1) + (two > done + 1);
+        const int next = ahead > 0 ? last : min(done + 1 + walks, max(p.K - 1, done + 1));
+        if (next >= p.K) continue;
+        open = true;
+        const int s = one == 0 ? 1 : two == 0 && p.n_sets > 2 ? 2 : 0;
+        const int left = 2 * (p.K - done) - walks - ahead;
+        if (s > 0 && left > most) { most = left; pair = q; group = next; set = s; seen = w; }
+      }
+      if (!__any(open)) break;
+      int key = most < 0 ? -1 : most * 64 + 63 - lane, best = key;
+#pragma unroll
+      for (int d = 1; d < 64; d *= 2) best = max(best, __shfl_xor(best, d, 64));
+      if (best < 0) {
+        more = __hip_atomic_load(p.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0 && wall_clock64() - t0 <= p.wait_limit;
+        __builtin_amdgcn_s_sleep(64);
+        continue;
+      }
+      bool mine = false;
+      if (key == best) {
+        const uint64_t to = seen | ((uint64_t)(group + 1) << (set == 1 ? HELP_ONE : HELP_TWO));
+        mine = __hip_atomic_compare_exchange_strong(reinterpret_cast<uint64_t*>(words + (size_t)pair * BWD_SYNC_STRIDE), &seen, to,
+                                                    __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (mine) {
+          job[0] = pair;
+          job[1] = group;
+          job[2] = set;
+        }
+      }
+      if (__any(mine)) {
+        took = 1;
+        break;
+      }
+    }
+    if (lane == 0) job[3] = took;
+  }
+  __syncthreads();
+  return uni(job[3]) != 0;
+}
+
 // ------------------------------------------------------------------ several workgroups per (batch, head)
 // The replay of a checkpoint group needs only the checkpoint, so it can run ahead of the reverse walk
 // on other CUs: one or more workgroups replay group after group, in turn, into alternating sets of the per-group
@@ -392,10 +480,11 @@ TTT_DEV int parts_until(const BwdParams& p, int done) {
 // workgroup (bwd_finish_dxk) forms grad_L_XK, grad_L_XV and the norm gradients.
 // WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
 // PARTS: several workgroups at once replay each of the p.n_shared groups walked first, a stretch of its mini-batches each.
-template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false>
+// HELPED: a workgroup that replays and walks (ROLE 0) where others (ROLE 1) replay groups ahead of it.
+template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false, bool HELPED = false>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; ROLE 2: K - 1 .. 0).
 // part (PARTS): which of the p.n_parts stretches of the group's mini-batches this workgroup replays; it takes the state there from
-// the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).
+// the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).  HELPED: the set it is replayed into.
 // False: a wait gave up.
 TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi, const int k_lo, const int part = 0) {
   constexpr bool PAIRS = ROLE == 0;
@@ -417,7 +506,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   float* s_deta = reinterpret_cast<float*>(smem + SB_DETA);
   float* s_red = reinterpret_cast<float*>(smem + SB_RED);
 
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
+  int tid0 = threadIdx.x;
+  if constexpr (HELPED) asm volatile("" : "+v"(tid0));   // (what a helper and a pair's own workgroup derive from it is not to be shared)
+  const int tid = tid0, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int v = __builtin_amdgcn_readfirstlane(tid >> 6);        // wave index, in a scalar register
   const int pp = v & 3, r = v >> 2;                              // pair, index inside the pair
   const int tb[2] = {r, 1 - r};                                  // token block held in column block 0 / 1 of a Q tile
@@ -474,9 +565,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   // through a pointer that is refreshed with the offsets, instead of all fifty living in scalar registers.
   typedef const __attribute__((address_space(4))) BwdParams* KernArgs;
   KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
-#define REFRESH_OFFSETS() asm volatile("" : "+s"(ka), "+s"(ox), "+s"(oe), "+s"(of), "+s"(oh), "+s"(ot), "+s"(opk), "+s"(ock))
+#define REFRESH_OFFSETS()                                                                                                       \
+  asm volatile("" : "+s"(ka), "+s"(ox), "+s"(oe), "+s"(of), "+s"(oh), "+s"(ot), "+s"(opk), "+s"(ock));                          \
+  if constexpr (HELPED) asm volatile("" : "+s"(kg))
   // per-group tensors: the caller's (set 0) or, with several workgroups, one of the alternate sets
-#define GRP(name) (ROLE != 0 && set ? ka->alt_##name[ROLE != 0 ? set - 1 : 0] : ka->name)
+// (with helpers through a pointer to the set's: choosing between the two at every use costs the workgroup that does everything 3 %)
+  typedef const __attribute__((address_space(4))) BwdSet* KernSets;
+  KernSets kg = nullptr;
+#define GRP(name) (HELPED ? kg->name : ROLE != 0 && set ? ka->alt_##name[ROLE != 0 && set ? set - 1 : 0] : ka->name)
 #define bXQ gbuf(ka->XQ + ox)
 #define bXK gbuf(ka->XK + ox)
 #define bXV gbuf(ka->XV + ox)
@@ -573,22 +669,29 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
   }
 
   TTT_STAGES_BEGIN();
-  for (int k = k_hi; k >= k_lo; k--) {
+  for (int kk = k_hi; kk >= k_lo; kk--) {
+    int k = kk;
+    if constexpr (HELPED) asm volatile("" : "+s"(k));   // (no offsets that run with k in vector registers)
     const int n_mb = min(cgs, p.NC - k * cgs);
     const int done = p.K - 1 - k;                    // number of this group, counted from the end of the sequence
-    const int set = ROLE == 0 ? 0 : done % n_sets;
-    int* const w_replayed = w_sync + set;
+    const int in_set = HELPED ? (ROLE == 1 ? part : take_group(w_sync + BWD_HELP, done, s_flag, v == 0 && lane_v == 0)) : ROLE == 0 ? 0 : done % n_sets;
+    int* const w_replayed = w_sync + in_set;
+    if constexpr (HELPED) kg = (KernSets)((const __attribute__((address_space(4))) char*)ka + offsetof(BwdParams, help_sets)) + in_set;
     REFRESH_OFFSETS();
     const size_t slot = (size_t)bh * p.K + k;
     const unsigned ckW = static_cast<unsigned>(k) * (FD * HID * 4u);   // byte offset of this group's checkpoint in bCW1 / bCW2
     // ================================================================= replay
-    if constexpr (ROLE != 2) {
-      if constexpr (ROLE == 1) {   // the set is free once the reverse walk is done with the group that used it last
+    if constexpr (ROLE != 2)
+    if (ROLE == 1 || !HELPED || in_set == 0) {
+      const int set = ROLE == 0 ? 0 : in_set;
+      if constexpr (ROLE == 1 && !HELPED) {   // the set is free once the reverse walk is done with the group that used it last
         if (done >= n_sets && !wait_at_least(w_walked, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
         if (WIDE && done >= n_sets && !wait_at_least(w_walked + 4, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
         if constexpr (FIN) {   // ... and so is the workgroup that reads the before-state images for grad_L_XK
           if (done >= n_sets && !wait_at_least(w_finished, done - n_sets + 1, w_status, s_flag, p.wait_limit)) return false;
         }
+      }
+      if constexpr (ROLE == 1) {
         WAVE_SYNC();
         s_dgw[lane] = 0.f;   // (every lane its own words)
         s_dbw[lane] = 0.f;
@@ -1132,31 +1235,46 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         g_stf(g, o, FD * 4, r1 + a1);
         WAVE_SYNC();
       }
-      if constexpr (ROLE == 1) publish_part(w_replayed);
+      if constexpr (ROLE == 1 && !HELPED) publish_part(w_replayed);
+      if constexpr (ROLE == 1 && HELPED) publish(w_replayed, done + 1);
+      if constexpr (ROLE == 0 && HELPED) {
+        if (v == 0 && lane_v == 0) __hip_atomic_fetch_add(reinterpret_cast<uint64_t*>(w_sync + BWD_HELP), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       TTT_STAGE(BS_PUBLISH);
     }
+    const int set = in_set;
 
     // ================================================================= reverse walk
     // Operands are fetched from HBM right where they are consumed: with two waves per SIMD the other
     // wave covers the latency, while holding requests in registers across stages costs more in spills
     // than it gains (measured).
+    // adds the replay's share of the norm gradients of the group in `set` to the running sum
+    auto add_norm_sums = [&]() {
+      LANE_VARS;
+      float a0 = 0.f, a1 = 0.f;
+      for (int e = 0; e * eighth < n_mb; e++) {
+        const gptr_t gs = group_sums(set, e);
+        a0 = e > 0 ? a0 + g_ldf(gs, 4 * lane, 0) : g_ldf(gs, 4 * lane, 0);
+        a1 = e > 0 ? a1 + g_ldf(gs, 4 * lane, FD * 4) : g_ldf(gs, 4 * lane, FD * 4);
+      }
+      const gptr_t g = park();
+      const unsigned o = (v * 2 * FD + lane) * 4;
+      const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);
+      g_stf(g, o, 0, r0 + a0);
+      g_stf(g, o, FD * 4, r1 + a1);
+    };
+    if constexpr (ROLE == 0 && HELPED) {
+      if (set > 0) {
+        if (uni(wait_at_least(w_replayed, done + 1, w_status, s_flag, p.wait_limit)) == 0) return false;
+        add_norm_sums();
+      }
+    }
     if constexpr (ROLE == 2) {
       if (!wait_at_least(w_replayed, parts_until(p, done), w_status, s_flag, p.wait_limit)) return false;
       if constexpr (FIN) {   // the hand-over set of this group's parity is free once the group before last is finished
         if (done >= 2 && !wait_at_least(w_finished, done - 1, w_status, s_flag, p.wait_limit)) return false;
       } else {
-        LANE_VARS;
-        float a0 = 0.f, a1 = 0.f;
-        for (int e = 0; e * eighth < n_mb; e++) {
-          const gptr_t gs = group_sums(set, e);
-          a0 = e > 0 ? a0 + g_ldf(gs, 4 * lane, 0) : g_ldf(gs, 4 * lane, 0);
-          a1 = e > 0 ? a1 + g_ldf(gs, 4 * lane, FD * 4) : g_ldf(gs, 4 * lane, FD * 4);
-        }
-        const gptr_t g = park();
-        const unsigned o = (v * 2 * FD + lane) * 4;
-        const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);
-        g_stf(g, o, 0, r0 + a0);
-        g_stf(g, o, FD * 4, r1 + a1);
+        add_norm_sums();
       }
     }
     // hand-over buffers of this group for the grad_L_XK workgroup (set = parity of the group)
@@ -1956,6 +2074,22 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_split_kernel(const Bwd
     if (!bwd_body<1, IMG, false>(p, smem, bh, k, k)) return;
 }
 
+// nbh workgroups with a pair each, n_helpers that replay for them.
+__global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_helped_kernel(const BwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b < p.nbh) {
+    bwd_body<0, false, false, false, false, true>(p, smem, p.bh0 + b, p.K - 1, 0);
+    return;
+  }
+  int* const job = reinterpret_cast<int*>(smem + SB_FLAG);
+  const int me = uni((b - p.nbh) * (p.nbh / p.n_helpers));
+  while (help_take(p, me, job)) {
+    const int k = uni(p.K - 1 - job[1]);
+    bwd_body<1, false, false, false, false, true>(p, smem, uni(p.bh0 + job[0]), k, k, uni(job[2]));
+  }
+}
+
 __global__ void ttt_mlp_zero_words(int* w, int n, const int* report) { clear_word(w, n, blockIdx.x * blockDim.x + threadIdx.x, report); }
 
 }  // namespace ttt
@@ -1974,13 +2108,14 @@ hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
   const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
   int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
   hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
-  const dim3 grid((p.n_replay + 1) * p.nbh), block(ttt::BW_THREADS);
+  const dim3 grid(p.n_helpers > 0 ? p.nbh + p.n_helpers : (p.n_replay + 1) * p.nbh), block(ttt::BW_THREADS);
   auto launch = [&](auto kernel) -> hipError_t {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };
+  if (p.n_helpers > 0) return launch(ttt::ttt_mlp_bwd_helped_kernel);
   return p.n_replay == 2 ? launch(ttt::ttt_mlp_bwd_split_kernel<2>) : launch(ttt::ttt_mlp_bwd_split_kernel<1>);
 }
 #else

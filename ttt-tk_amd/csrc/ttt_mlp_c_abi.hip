@@ -163,6 +163,10 @@ struct LaunchPlan {
   int sets = 0;             // backward: sets of the per-group tensors
   int shared = 0;           // backward: groups, the first ones walked, that several workgroups at once replay
   int parts = 1;            // backward: that many, a stretch of the group each
+  int helpers = 0;          // backward, one workgroup per pair: further ones that replay groups for all of them
+  bool waits() const { return rest_split || helpers > 0; }                    // workgroups that wait for each other, in a workspace
+  long long first_waiting() const { return helpers > 0 ? 0 : n_single; }      // of these pairs
+  long long n_waiting() const { return helpers > 0 ? n_single : n_rest; }
 };
 // Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
 // of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others.
@@ -186,6 +190,12 @@ void divide_workers(int pairs, int workers, int walk, int replay, int finish, in
 // Where the stretches of a group begin, in eighths of it.  To the state at its first mini-batch a workgroup takes the half of every
 // replay before that carries the state, about a third of the whole, so the stretches get shorter.
 constexpr int PART_START[ttt::BWD_MAX_PARTS][ttt::BWD_MAX_PARTS + 1] = {{0, 8, 8, 8, 8}, {0, 5, 8, 8, 8}, {0, 4, 6, 8, 8}, {0, 3, 5, 7, 8}};
+// One workgroup for each of 129 to 248 pairs on 256 CUs: the CUs left over replay groups for all of them (ttt_mlp_bwd.hip).  In ms,
+// backward alone -> with helpers (two sets for the groups they take; with one 168 x 128 4.37, 176 x 128 4.92): 136 pairs x 128
+// mini-batches 4.71 -> 3.77, 168 x 128 4.87 -> 4.20, 200 x 100 4.03 -> 3.78, 200 x 256 10.44 -> 9.52, 232 x 512 21.9 -> 21.0, 248 x 512
+// 22.7 -> 22.3.  (In clocks it is twice that: a device with every CU busy runs slower, and the forward after it too, 1.20 -> 1.33 ms for
+// 200 x 100; both together 5.24 -> 5.10 ms.)  Fewer than one helper per XCD gain less than that costs.
+constexpr int MIN_HELPERS = 8;
 LaunchPlan plan_for(long long BH, int cus, bool backward) {
   LaunchPlan pl;
   if (BH <= 0 || cus <= 0) {
@@ -198,6 +208,10 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
   if (!pl.rest_split) {
     pl.n_single = BH;
     pl.n_rest = 0;
+    if (backward && BH <= cus - MIN_HELPERS) {
+      pl.helpers = static_cast<int>(cus - BH);
+      pl.sets = ttt::BWD_HELP_SETS;
+    }
     return pl;
   }
   const long long per_xcd = (pl.n_rest + 7) / 8;
@@ -357,6 +371,11 @@ SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, in
 // Sets of the per-group tensors that carry replayed groups to the walk, used in turn.  Set 0 is the caller's own; a sequence of K
 // groups uses K.
 int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K < pl.sets ? K : pl.sets); }
+// Whether the helpers get to a group of every pair in time: a helper replays 1.75 groups while a pair's own workgroup replays and walks
+// one, and there is nothing to take in the first of a pair.  If they do not, the pairs without help end as late as
+// without helpers, at a lower clock: in ms, alone -> with helpers, 184 pairs x 32 mini-batches in 2 groups 1.349 -> 1.351 and 4 %
+// on the forward after it, 200 x 64 in 2 2.58 -> 2.81, 200 x 48 in 3 2.01 -> 2.00; 160 x 32 in 2 1.28 -> 1.08, 200 x 64 in 4 2.62 -> 2.48.
+bool helpers_pay(const LaunchPlan& pl, long long K) { return pl.helpers > 0 && 7 * pl.helpers * (K - 1) >= 4 * pl.n_waiting(); }
 // The launch with less workspace for the same pairs: two replaying workgroups per pair instead of three or four.
 LaunchPlan bwd_reduced(LaunchPlan pl) {
   if (pl.prefetch) {
@@ -382,7 +401,7 @@ struct BwdWorkspace {
   size_t total;
   int alt_sets;
   BwdWorkspace(const LaunchPlan& pl, long long cgs, long long K) {
-    const long long n = pl.n_rest;
+    const long long n = pl.n_waiting();
     alt_sets = bwd_sets_used(pl, K) - 1;
     const size_t slot = (size_t)n * (size_t)cgs;
     const size_t tile = TTT_MLP_CS * TTT_MLP_F * 2, img = TTT_MLP_CS * TTT_MLP_HID * 2, vec = TTT_MLP_CS * 4;
@@ -457,22 +476,26 @@ extern "C" int ttt_mlp_bwd_export_group0(const ttt_mlp_bwd_args* a, void* stream
 extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_group_size) {
   if (B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16)) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
-  return pl.rest_split ? BwdWorkspace(pl, checkpoint_group_size, ttt::BWD_MAX_SETS).total : 0;
+  return pl.waits() ? BwdWorkspace(pl, checkpoint_group_size, ttt::BWD_MAX_SETS).total : 0;
 }
 
 extern "C" int ttt_mlp_bwd_workspace_range(int B, int NH, int checkpoint_group_size, int K, size_t* least, size_t* most) {
   if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || K <= 0)
     return TTT_MLP_ERR_BAD_ARG;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
-  *least = pl.rest_split ? BwdWorkspace(bwd_reduced(pl), checkpoint_group_size, K).total : 0;
-  *most = pl.rest_split ? BwdWorkspace(pl, checkpoint_group_size, K).total : 0;
+  if (pl.helpers > 0 && !helpers_pay(pl, K)) {
+    *least = *most = 0;
+    return TTT_MLP_OK;
+  }
+  *least = pl.waits() ? BwdWorkspace(bwd_reduced(pl), checkpoint_group_size, K).total : 0;
+  *most = pl.waits() ? BwdWorkspace(pl, checkpoint_group_size, K).total : 0;
   return TTT_MLP_OK;
 }
 
 extern "C" size_t ttt_mlp_bwd_status_offset(int B, int NH) {
   if (B <= 0 || NH <= 0) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, true);
-  return pl.rest_split ? (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE * sizeof(int) : 0;
+  return pl.waits() ? (size_t)pl.n_waiting() * ttt::BWD_SYNC_STRIDE * sizeof(int) : 0;
 }
 
 extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
@@ -480,7 +503,7 @@ extern "C" int ttt_mlp_bwd_launch_overlapped(const ttt_mlp_bwd_args* a, void* wo
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
   const LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
-  if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
+  if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, ttt::BWD_MAX_SETS).total) return TTT_MLP_ERR_WORKSPACE;
   return ttt_mlp_bwd_launch_within(a, workspace, workspace_bytes, stream);
 }
@@ -491,7 +514,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
   LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
-  if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
+  if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
   const BwdWorkspace w(pl, p.cgs, p.K);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
@@ -501,27 +524,34 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
     const long long pairs = (long long)p.B * p.NH;
     const int cus = device_cus();
     const SegmentPlan seg = plan_bwd_segments(pl, pairs, cus, p.NC, p.cgs, true);
-    if (seg.seg_len > 0) {
-      if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_rest)),
+    const bool alone = pl.helpers > 0 && !helpers_pay(pl, p.K);
+    if (seg.seg_len > 0 || alone) {
+      if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_waiting())),
                                                  static_cast<hipStream_t>(stream)))
         return static_cast<int>(e);
+      if (alone) {
+        p.bh0 = 0;
+        p.nbh = p.B * p.NH;
+        return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
+      }
       return launch_bwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
     }
   }
-  if (pl.n_single > 0) {
+  if (pl.first_waiting() > 0) {
     p.bh0 = 0;
     p.nbh = static_cast<int>(pl.n_single);
     if (hipError_t e = ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream))) return static_cast<int>(e);
   }
   // The kernels index the workspace by the global pair number: every pointer is moved back by bh0 entries.
-  const size_t b0 = (size_t)pl.n_single;
+  const size_t b0 = (size_t)pl.first_waiting();
   const size_t tile = (size_t)p.cgs * TTT_MLP_CS * TTT_MLP_F, img = (size_t)p.cgs * TTT_MLP_CS * TTT_MLP_HID, vec = (size_t)p.cgs * TTT_MLP_CS;
   const size_t norm = 8 * 2 * TTT_MLP_F;
-  p.bh0 = static_cast<int>(pl.n_single);
-  p.nbh = static_cast<int>(pl.n_rest);
+  p.bh0 = static_cast<int>(pl.first_waiting());
+  p.nbh = static_cast<int>(pl.n_waiting());
+  p.n_helpers = pl.helpers;
   p.gang_pairs = pl.gang;
   p.n_replay = pl.n_replay;
-  p.n_sets = pl.sets;
+  p.n_sets = pl.helpers > 0 ? w.alt_sets + 1 : pl.sets;
   p.n_shared = pl.shared;
   p.n_parts = pl.parts;
   for (int i = 0; i <= ttt::BWD_MAX_PARTS; i++) p.part_start[i] = PART_START[pl.parts - 1][i];
@@ -536,7 +566,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
     p.fin_park = reinterpret_cast<float*>(base + w.off[7]) - b0 * ttt::FIN_PARK_FLOATS;
   }
   int* words = reinterpret_cast<int*>(base + w.off[0]);
-  p.status = words + (size_t)pl.n_rest * ttt::BWD_SYNC_STRIDE;
+  p.status = words + (size_t)pl.n_waiting() * ttt::BWD_SYNC_STRIDE;
   p.sync = words - b0 * ttt::BWD_SYNC_STRIDE;
   p.norm_partial = reinterpret_cast<float*>(base + w.off[1]) - b0 * ttt::BWD_MAX_SETS * 8 * norm;
   p.norm_park = reinterpret_cast<float*>(base + w.off[2]) - b0 * norm;
@@ -564,6 +594,14 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
     p.alt_grad_output_fused_group[s] = reinterpret_cast<__bf16*>(base + o[8]) - b0 * tile;
     p.alt_std_fused_group[s] = reinterpret_cast<float*>(base + o[9]) - b0 * vec;
     p.alt_W1_init_group[s] = reinterpret_cast<float*>(base + o[10]) - b0 * img;   // [cgs][64][256] floats = 2 images per slot
+  }
+  if (pl.helpers > 0) {
+    p.help_sets[0] = {p.X2_group, p.Z1_group, p.Z1_bar_group, p.X2_bar_group, p.grad_l_wrt_Z2_group, p.grad_l_wrt_Z1_group,
+                      p.x_hat_fused_group, p.grad_x_hat_fused_group, p.grad_output_fused_group, p.std_fused_group, p.W1_init_group};
+    for (int s = 0; s < ttt::BWD_HELP_SETS - 1; s++)
+      p.help_sets[s + 1] = {p.alt_X2_group[s], p.alt_Z1_group[s], p.alt_Z1_bar_group[s], p.alt_X2_bar_group[s], p.alt_grad_l_wrt_Z2_group[s],
+                            p.alt_grad_l_wrt_Z1_group[s], p.alt_x_hat_fused_group[s], p.alt_grad_x_hat_fused_group[s],
+                            p.alt_grad_output_fused_group[s], p.alt_std_fused_group[s], p.alt_W1_init_group[s]};
   }
   if (pl.gang) {
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;

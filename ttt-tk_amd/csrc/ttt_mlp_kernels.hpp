@@ -48,6 +48,13 @@ constexpr int FWD_BIAS_FLOATS = 256 + 64;
 constexpr int BWD_MAX_PARTS = 4;
 constexpr int BWD_MAX_SETS = 6;   // sets of per-group tensors in use at once, at most
 
+// A set of the per-group tensors that carry a replayed group to the walk.
+struct BwdSet {
+  __bf16 *X2_group, *Z1_group, *Z1_bar_group, *X2_bar_group, *grad_l_wrt_Z2_group, *grad_l_wrt_Z1_group;
+  __bf16 *x_hat_fused_group, *grad_x_hat_fused_group, *grad_output_fused_group;
+  float *std_fused_group, *W1_init_group;
+};
+constexpr int BWD_HELP_SETS = 3;
 struct BwdParams {
   const __bf16 *XQ, *XK, *XV, *last_eta;
   const float *ttt_norm_weight, *ttt_norm_bias;
@@ -83,6 +90,10 @@ struct BwdParams {
   // gradient wrt W1 and form G1 = -eta * dl/dZ1 themselves; fin_park: [B*NH][FIN_PARK_FLOATS], that copy and the norm-gradient
   // sums between two groups of a pair (n_finish < gang_pairs only).
   int gang_pairs, n_replay, n_finish;
+  // One workgroup per pair and CUs to spare (n_helpers > 0): these replay groups ahead of the pairs, into sets 1 .. n_sets - 1 of
+  // help_sets (0: the caller's tensors).
+  int n_helpers;
+  BwdSet help_sets[BWD_HELP_SETS];
   // The first n_shared groups (at most n_sets) are replayed in n_parts stretches, by as many workgroups at once: part i its eighths
   // part_start[i] .. part_start[i + 1] - 1.
   int n_shared, n_parts, part_start[BWD_MAX_PARTS + 1];
@@ -120,6 +131,11 @@ struct BwdParams {
 // mini-batches of the last group it walks that it has handed on (that group is handed over in chunks).  Word 24 the groups
 // whose finishing is done - then one status word behind all of them (non-zero: a wait gave up).
 constexpr int BWD_SYNC_STRIDE = 32;
+// One workgroup per pair with helpers: words 1, 2 the group last replayed into that set, + 1; words BWD_HELP, + 1 (one 8-byte word)
+// where the pair is and what is taken: bits 0-23 two times the number of the group it is at, + 1 from its walk on; bits 24-43
+// and 44-63 the number, + 1, of the group taken into set 1 and 2 (0: the set is free).  A sequence has fewer than 2^18 groups
+// (its tensors stay below 2 GiB per pair).
+constexpr int BWD_HELP = 16;
 // With the walk on two workgroups: BWW_WALKED + 0 / 4 groups and BWW_GIVEN + 0 / 4 mini-batches done by its two halves,
 // BWW_XCD .. their XCDs, BWW_WORKERS (two words) the gang's other workgroups by XCD.
 constexpr int BWW_WORDS = 9;                                // per lane: two times 8 fp32 sums and the token's share of d eta

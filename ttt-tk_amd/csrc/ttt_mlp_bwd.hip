@@ -407,9 +407,12 @@ TTT_DEV int take_group(int* word, int done, int* s_flag, bool first_lane) {
 // A helper takes a group: job[0] = pair (of the launch), job[1] = number of the group, job[2] = set; false: there is none left to
 // take (or a wait gave up, or nothing came free for as long as one may wait: nobody waits for this workgroup).
 // Taken is the group that the pair will come to next once this one could be ready: the one behind those taken already, else the
-// next one while the pair replays, the one behind that while it walks.
+// next one while the pair replays, the one behind that while it walks.  With many helpers (up to 146 pairs on 256 CUs) also the next one while it
+// walks: a helper is there as soon as the walk frees a set, and the pair waits for less than it would replay (in ms, 136 pairs x 512
+// 14.77 -> 13.66, 144 x 512 15.1 -> 14.5).
 TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
   const int lane = threadIdx.x & 63;
+  const bool many = 4 * p.n_helpers >= 3 * p.nbh;
   __syncthreads();   // the last job has been read by every wave
   if (threadIdx.x < 64) {
     int* const words = p.sync + (size_t)p.bh0 * BWD_SYNC_STRIDE + BWD_HELP;
@@ -426,7 +429,7 @@ TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
         const int at = static_cast<int>(w & 0xffffff), done = at >> 1, walks = at & 1;
         const int one = static_cast<int>((w >> HELP_ONE) & 0xfffff), two = static_cast<int>(w >> HELP_TWO), last = max(one, two);
         const int ahead = (one > done + 1) + (two > done + 1);
-        const int next = ahead > 0 ? last : min(done + 1 + walks, max(p.K - 1, done + 1));
+        const int next = ahead > 0 ? last : min(done + 1 + (many ? 0 : walks), max(p.K - 1, done + 1));
         if (next >= p.K) continue;
         open = true;
         const int s = one == 0 ? 1 : two == 0 && p.n_sets > 2 ? 2 : 0;

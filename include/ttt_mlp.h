@@ -152,9 +152,12 @@ int ttt_mlp_bwd_launch(const ttt_mlp_bwd_args* args, void* stream);
  * the workgroups of ceil(n/8) pairs fit an eighth of the CUs the walk takes two: eight
  * per pair (four recomputing, one reading ahead), else seven (three), else
  * five (two recomputing, none reading ahead) - up to 32, 32 and 48 pairs on 256 CUs.
- * Otherwise four per pair if 4*n fits the CUs, else three if 3*n fits, else two if 2*n fits.
- * ttt_mlp_bwd_workspace_bytes() returns 0 when none does (n = 0 or 2*n > CUs of
- * the current device); the launcher then returns TTT_MLP_ERR_NO_ROOM and the caller
+ * With less room than that the workgroups of an eighth of the device that recompute, and those for
+ * grad_L_XK, serve all of its pairs (up to 80 on 256 CUs), then three or two per pair if they fit.
+ * Where not even two do, one workgroup does everything for each pair and the CUs left over, if eight or more, recompute
+ * groups ahead for whichever pair has most left (129 to 248 pairs on 256 CUs; with too few groups for every pair to get
+ * one the launch leaves them out).  Then n is all pairs.
+ * ttt_mlp_bwd_workspace_bytes() returns 0 otherwise; the launcher then returns TTT_MLP_ERR_NO_ROOM and the caller
  * uses ttt_mlp_bwd_launch.
  * The caller owns the device workspace (256-byte aligned, contents unspecified
  * before and after; calls that overlap in time need separate workspaces).  The int
@@ -233,7 +236,8 @@ const char* ttt_mlp_error_string(int code);
 
 /* How an overlapped launch of `pairs` = B*NH (batch, head) pairs is laid out on a device with
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
- * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  which = 0
+ * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  Workgroups that only help
+ * pairs that have one are not counted.  which = 0
  * forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk),
  * 3 (two replay), 7 or 8 (walk on two, one for grad_L_XK / grad_L_XV, three, or four to eight, that replay, one that reads ahead), and
  * 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly: the whole ones of a pair's share, at most 5, while

@@ -402,7 +402,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           return (unsigned long long)(f > b ? f : b);
         },
         "Bytes of workspace that let ttt_forward and ttt_backward of this shape use several workgroups per (batch, head) "
-        "(0: the shape runs with one workgroup per pair and needs none).  Serves every sequence length; a backward over fewer "
+        "(0: the shape runs with one workgroup per pair, nothing beside them, and needs none).  Serves every sequence length; a backward over fewer "
         "checkpoint groups takes less of it, and with less than it the backward recomputes with fewer workgroups first.");
   m.def("set_workspace", [](c10::optional<torch::Tensor> ws) {
           if (!ws.has_value()) { delete g_workspace; g_workspace = nullptr; return; }

@@ -7,7 +7,7 @@
 //
 // Mapping: workgroups of 8 wavefronts (two per SIMD, at most 256 registers each); one per (batch,
 // head), or two or three where the device has CUs to spare - then one or two replay the checkpoint groups (taking
-// turns) and one walks them backwards, a group or more behind.  With more room: ttt_mlp_bwd_wide.hip, which takes the
+// turns) and one walks them backwards, a group or more behind; with fewer to spare than pairs those replay for all of them.  With more room: ttt_mlp_bwd_wide.hip, which takes the
 // roles from here (others form grad_L_XK from what the walk hands them).  Wave v owns hidden columns [32v, 32v+32).  All [tokens x hidden] activations live in
 // registers in the "Q" orientation (accumulator rows = hidden, lane = token), so per-token scalars
 // (eta, dEta partial sums) are per-lane values.  An activation that is also needed with tokens as the

@@ -150,7 +150,7 @@ inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE 
 // is built without the macro and contains none of this.  Reading the clock is a scalar-memory operation: every
 // boundary also waits for the wave's outstanding LDS reads, which makes an instrumented kernel some 10 % slower.
 // Role of a workgroup in the buffer: forward 0 = the recurrence (or the one workgroup), 1 / 2 = the output branch, 3 / 4 = the halves
-// of a recurrence on two workgroups; backward 0 .. 3 = the replaying workgroups, 4 = the reverse walk (or the one
+// of a recurrence on two workgroups; backward 0 = the replaying workgroups together, 4 = the reverse walk (or the one
 // workgroup), 5 = the grad_L_XK workgroup, 6 / 7 = the halves of a walk on two workgroups.
 constexpr int STAGE_SLOTS = 24;
 constexpr int STAGE_ROLES = 8;

@@ -176,9 +176,6 @@ def main() -> int:
     def halves(clocks, role):   # both workgroups of every pair, as if they were pairs of their own
         return torch.cat((present(clocks[:, role]), present(clocks[:, role + 1])))
 
-    def mini_batches(turn, n):  # of the groups (counted from the end) that replaying workgroup `turn` of n takes
-        return sum(min(cgs, NC - (K - 1 - g) * cgs) for g in range(turn, K, n))
-
     wide_f, split_f = ran(cf[:, HALF]), ran(cf[:, OUT]) & ~ran(cf[:, HALF])
     one_f = ran(cf[:, 0]) & ~split_f
     if one_f.any():
@@ -192,15 +189,13 @@ def main() -> int:
         out += table(f"forward, recurrence on two workgroups, compute waves ({int(wide_f.sum())} pairs)", both[:, :4], fwd_wide_names, NC) + [""]
         out += table("forward, recurrence on two workgroups, helper waves", both[:, 4:], fwd_wide_names, NC) + [""]
         out += table(f"forward, output-branch workgroup 0 of {n_out}", cf[wide_f, OUT], fwd_names, -(-NC // n_out)) + [""]
-    n_rep = sum(bool(ran(cb[:, r]).any()) for r in range(4))
     wide_b, rep0 = ran(cb[:, WALK_HALF]), ran(cb[:, 0])
     walk_b = ran(cb[:, WALK])
     if (walk_b & ~rep0).any():
         one_b = walk_b & ~rep0
         out += table(f"backward, one workgroup per pair ({int(one_b.sum())} pairs)", cb[one_b, WALK], bwd_names, NC) + [""]
     if rep0.any():
-        mb0 = mini_batches(0, n_rep)
-        out += table(f"backward, replaying workgroup 0 of {n_rep} ({int(rep0.sum())} pairs, {mb0} of the {NC} mini-batches)", cb[rep0, 0], bwd_names, mb0) + [""]
+        out += table(f"backward, replaying workgroups, all that worked for a pair ({int(rep0.sum())} pairs)", cb[rep0, 0], bwd_names, NC) + [""]
     if (walk_b & rep0).any():
         out += table(f"backward, reverse-walk workgroup ({int((walk_b & rep0).sum())} pairs)", cb[walk_b & rep0, WALK], bwd_names, NC) + [""]
     if wide_b.any():

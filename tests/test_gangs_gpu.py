@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("NH,NC,cgs,scatter", [(49, 9, 2, 0), (53, 7, 1, 1), (56, 25, 4, 0), (56, 3, 4, 0), (57, 5, 2, 0), (64, 6, 4, 0),
-                                               (65, 9, 4, 0), (75, 11, 2, 0), (80, 8, 1, 1), (80, 2, 3, 0)])
+                                               (65, 9, 4, 0), (75, 11, 2, 0), (80, 8, 1, 1), (80, 2, 3, 0),
+                                               (53, 13, 4, 1), (55, 31, 10, 0), (65, 93, 8, 0), (72, 95, 24, 0), (80, 91, 10, 1), (80, 99, 30, 0)])
 def test_shared_workgroups_are_bit_identical(NH, NC, cgs, scatter):
     import test_time_training as ext
     import ttt_mlp_host as host
@@ -40,18 +41,18 @@ def test_shared_workgroups_are_bit_identical(NH, NC, cgs, scatter):
         assert torch.equal(t[k], ref[k]), k
 
 
-@pytest.mark.parametrize("NH", [52, 76])
-def test_a_shared_workgroup_that_gives_up_ends_the_launch(NH):
+@pytest.mark.parametrize("NH,NC,cgs", [(52, 12, 2), (76, 12, 2), (52, 12, 4), (76, 92, 10)])
+def test_a_shared_workgroup_that_gives_up_ends_the_launch(NH, NC, cgs):
     import test_time_training as ext
     import ttt_mlp_host as host
-    t = _tensors(host, NH, 12, 2, torch.device("cuda:0"))
-    ref = _reference(host, ext, t, 2)
+    t = _tensors(host, NH, NC, cgs, torch.device("cuda:0"))
+    ref = _reference(host, ext, t, cgs)
     for limit in (1, 1000, 3000, 2_000_000_000):
         print(f"case NH={NH} limit={limit}", flush=True)
         host.zero_accumulating_grads(t)
         ext.set_wait_limit(limit)
         try:
-            host.backward(t, 2)
+            host.backward(t, cgs)
         except RuntimeError as e:
             assert "gave up" in str(e) and limit < 2_000_000_000
             continue

@@ -1254,15 +1254,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
     // adds the replay's share of the norm gradients of the group in `set` to the running sum
     auto add_norm_sums = [&]() {
       LANE_VARS;
+      const gptr_t g = park();
+      const unsigned o = (v * 2 * FD + lane) * 4;
+      const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);   // under way with the sums
       float a0 = 0.f, a1 = 0.f;
       for (int e = 0; e * eighth < n_mb; e++) {
         const gptr_t gs = group_sums(set, e);
         a0 = e > 0 ? a0 + g_ldf(gs, 4 * lane, 0) : g_ldf(gs, 4 * lane, 0);
         a1 = e > 0 ? a1 + g_ldf(gs, 4 * lane, FD * 4) : g_ldf(gs, 4 * lane, FD * 4);
       }
-      const gptr_t g = park();
-      const unsigned o = (v * 2 * FD + lane) * 4;
-      const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);
       g_stf(g, o, 0, r0 + a0);
       g_stf(g, o, FD * 4, r1 + a1);
     };

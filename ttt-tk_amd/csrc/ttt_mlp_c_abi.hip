@@ -388,6 +388,29 @@ LaunchPlan bwd_reduced(LaunchPlan pl) {
   }
   return pl;
 }
+// The launch for groups as short, or as few, as the sequence at hand has.  Finishing workgroups that take groups of several pairs in turn
+// park 72 KiB between two groups and end a whole group after the last walk, and the workgroups that serve a pair meet once a group; with
+// short groups whole workgroups for each pair are faster: with the walk on two CUs, up to 56 pairs, four with the walk on one (gang /
+// whole: groups of 1 1.20, of 2 1.03 - 1.13, of 4 0.93 - 1.00, of 16 0.85 - 0.95); of 65 to 80 pairs three, without finishing ones (80
+// pairs: 6 groups of 1 1.35, 8 of 4 1.10, 3 of 32 1.02, 4 of 16 1.01; 12 of 8 1.00, 8 of 12 0.97, 6 of 16 0.985, 4 of 32 0.98).
+LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K) {
+  if (cgs < 2) {   // no stretches to divide a group into
+    pl.parts = 1;
+    pl.shared = 0;
+  }
+  const bool four = 4 * pl.gang <= cus / 8;
+  if (four && pl.wide && pl.n_finish < pl.gang && cgs < 4) {
+    pl.wide = false;
+    pl.n_finish = pl.gang;
+    pl.n_replay = 2 * pl.gang;
+    pl.per_pair = 4;
+  } else if (!four && !pl.wide && pl.gang && (cgs < 8 || K < 4 || cgs * K < 90)) {
+    pl.gang = pl.n_finish = 0;
+    pl.n_replay = 2;
+    pl.per_pair = 3;
+  }
+  return pl;
+}
 // Workspace of the backward with several workgroups per pair, for n (batch, head) pairs of K groups: the synchronisation
 // words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
 // CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
@@ -482,7 +505,7 @@ extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_grou
 extern "C" int ttt_mlp_bwd_workspace_range(int B, int NH, int checkpoint_group_size, int K, size_t* least, size_t* most) {
   if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || K <= 0)
     return TTT_MLP_ERR_BAD_ARG;
-  const LaunchPlan pl = plan_launches((long long)B * NH, true);
+  const LaunchPlan pl = bwd_for_groups(plan_launches((long long)B * NH, true), device_cus(), checkpoint_group_size, K);
   if (pl.helpers > 0 && !helpers_pay(pl, K)) {
     *least = *most = 0;
     return TTT_MLP_OK;
@@ -515,6 +538,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   if (int rc = check_workspace(workspace)) return rc;
   LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
   if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
+  pl = bwd_for_groups(pl, device_cus(), p.cgs, p.K);
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
   const BwdWorkspace w(pl, p.cgs, p.K);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;

@@ -19,8 +19,8 @@
 // block 0's weight step 2.1 k while block 1's sums cross and 2.25 k of waiting for those; block 1's weight step, the
 // split of the new state and Z1 of the next block 0 2.9 k.  (Before Z1 was started under that split, and with the token
 // sums for b2 and the wait for a free ring slot between the exchanges, 14.2 k: 24 x 256 1.53 ms, 12 x 64 396 us, now 383.)
-// From 40 pairs on the shorter chain is mostly paid back in clock rate: 48 x 256 1.545 ms before, 1.55 alone, 1.57 -> 1.55
-// in a step.
+// From 40 pairs on the shorter chain is paid back in clock rate: 48 x 256 1.59 -> 1.56 ms one call at a time, 1.545 and 1.55 back to back,
+// 64 x 256 (every CU busy) 1.55 -> 1.58 back to back, 64 x 32 and 80 x 256 no change.
 #include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
 

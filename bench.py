@@ -157,6 +157,23 @@ def launched_kernel(which, pairs, NC, cgs, cus, overlapped):
     return f"{one_each} + {several}" if one.value else several
 
 
+def running_kernel(which, pairs, NC, cgs, cus, overlapped):
+    """The same by the name of the kernel in a trace: `launched_kernel` names a backward by the roles of a pair's own workgroups; where the
+    workgroups of an XCD work for all of its pairs, or idle CUs for all pairs, the roles are in one kernel."""
+    name = launched_kernel(which, pairs, NC, cgs, cus, overlapped)
+    if which == 0 or not overlapped or "cut" in name:
+        return name
+    one, rest, K = pairs // cus * cus, pairs % cus, -(-NC // cgs)
+    if 2 * rest > cus:
+        return "ttt_mlp_bwd_helped_kernel"
+    per_xcd, short = -(-rest // 8), cgs < 8 or K < 4 or cgs * K < 90
+    if 3 * per_xcd <= cus // 8 and not (short and 4 * per_xcd > cus // 8):
+        several = "ttt_mlp_bwd_gang_kernel"
+    else:
+        several = f"ttt_mlp_bwd_split_kernel<{2 if 3 * rest <= cus else 1}>"
+    return f"ttt_mlp_bwd_kernel + {several}" if one else several
+
+
 def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibrate_copy=False):
     """Times `steps` forward (+ backward) steps of one workload and returns the figures of its JSON block."""
     import torch
@@ -217,7 +234,7 @@ def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibra
     all_tflops = (FWD_G + (BWD_G if backward else 0)) * G_FLOP * mb_steps / (ms_per_step * 1e-3) / 1e12
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     fwd_kernel = launched_kernel(0, B * NH, NC, cgs, cus, ext.last_forward_mode() == 1)
-    bwd_kernel = launched_kernel(1, B * NH, NC, cgs, cus, ext.last_backward_mode() == 1) if backward else None
+    bwd_kernel = running_kernel(1, B * NH, NC, cgs, cus, ext.last_backward_mode() == 1) if backward else None
     traffic, note = measured_traffic_checked(name, "bwd" if backward else "fwd")
     # the dominant kernel: the backward (the forward where there is no backward)
     roofline = {"bound": "mfma", "kernel": bwd_kernel if backward else fwd_kernel,

@@ -51,3 +51,25 @@ def test_groups_replayed_by_helpers_are_bit_identical(NH, NC, cgs, cus):
         check()
     finally:
         ext.set_compute_units(0)
+
+
+@pytest.mark.parametrize("NH,NC,cgs", [(136, 24, 4), (200, 30, 3)])
+def test_a_pair_that_gives_up_ends_the_launch(NH, NC, cgs):
+    """A pair that stops waiting for a taken group ends the launch with an error; a helper that stops waiting for one to take only leaves."""
+    import test_time_training as ext
+    import ttt_mlp_host as host
+    t = _tensors(host, NH, NC, cgs, torch.device("cuda:0"))
+    ref = _reference(host, ext, t, cgs)
+    for limit in (1, 1000, 2_000_000_000):
+        print(f"case NH={NH} limit={limit}", flush=True)
+        host.zero_accumulating_grads(t)
+        ext.set_wait_limit(limit)
+        try:
+            host.backward(t, cgs)
+        except RuntimeError as e:
+            assert "gave up" in str(e) and limit < 2_000_000_000
+            continue
+        finally:
+            ext.set_wait_limit(2_000_000_000)
+        for k in host.GRAD_NAMES:
+            assert torch.equal(t[k], ref[k]), (limit, k)

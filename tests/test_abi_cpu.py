@@ -264,6 +264,10 @@ def test_segment_plan_cuts_sequences_where_a_last_round_would_idle(lib):
     assert plan(0, 312, 256, 101, 30, 1) == (30, 5)                   # 30, 30, 30 and 11 mini-batches
     assert plan(1, 276, 256, 329, 15, 1) == (45, 9)                   # 44, six of 45, and 15
     assert plan(1, 318, 256, 612, 12, 1) == (156, 5)
+    # the uncut backward is priced with the launch for groups as short or as few as these (three whole workgroups for each of the 65 to 80
+    # pairs left over, four for each of 49 to 56), which is what it is weighed against when it is launched
+    assert plan(1, 305, 256, 45, 1, 1) == (9, 6)
+    assert plan(1, 336, 256, 55, 32, 1) == (32, 3)
     assert plan(0, 400, 256, 18, 1, 1)[0] == 0                        # two launches' gaps are a tenth of the sequence: 0.495 ms uncut, 0.505 cut
     assert lib.ttt_mlp_segment_plan(2, ctypes.c_longlong(8), 8, 8, 8, 0, ctypes.byref(ctypes.c_int()), ctypes.byref(ctypes.c_int())) == 1001
     assert lib.ttt_mlp_segment_plan(0, ctypes.c_longlong(8), 8, 8, 8, 0, None, None) == 1001

@@ -411,6 +411,8 @@ LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K) {
   }
   return pl;
 }
+// The launch of a backward call with a workspace.
+LaunchPlan plan_bwd(long long pairs, int cus, long long cgs, long long K) { return bwd_for_groups(plan_for(pairs, cus, true), cus, cgs, K); }
 // Workspace of the backward with several workgroups per pair, for n (batch, head) pairs of K groups: the synchronisation
 // words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
 // CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
@@ -505,7 +507,7 @@ extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_grou
 extern "C" int ttt_mlp_bwd_workspace_range(int B, int NH, int checkpoint_group_size, int K, size_t* least, size_t* most) {
   if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || K <= 0)
     return TTT_MLP_ERR_BAD_ARG;
-  const LaunchPlan pl = bwd_for_groups(plan_launches((long long)B * NH, true), device_cus(), checkpoint_group_size, K);
+  const LaunchPlan pl = plan_bwd((long long)B * NH, device_cus(), checkpoint_group_size, K);
   if (pl.helpers > 0 && !helpers_pay(pl, K)) {
     *least = *most = 0;
     return TTT_MLP_OK;
@@ -536,9 +538,8 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   ttt::BwdParams p;
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
-  LaunchPlan pl = plan_launches((long long)p.B * p.NH, true);
+  LaunchPlan pl = plan_bwd((long long)p.B * p.NH, device_cus(), p.cgs, p.K);
   if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
-  pl = bwd_for_groups(pl, device_cus(), p.cgs, p.K);
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
   const BwdWorkspace w(pl, p.cgs, p.K);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
@@ -820,7 +821,8 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
   if (segment_minibatches == nullptr || launches == nullptr || pairs <= 0 || compute_units <= 0 || NC <= 0 ||
       checkpoint_group_size <= 0 || (which != 0 && which != 1))
     return TTT_MLP_ERR_BAD_ARG;
-  const LaunchPlan pl = plan_for(pairs, compute_units, which == 1);
+  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size)
+                                   : plan_for(pairs, compute_units, false);
   const SegmentPlan seg = which == 1 ? plan_bwd_segments(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0)
                                      : plan_segments(pairs, compute_units, NC, checkpoint_group_size, false,
                                                      uncut_x1000(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0, false));

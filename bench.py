@@ -137,41 +137,15 @@ def measured_traffic_checked(workload, which):
 
 
 def launched_kernel(which, pairs, NC, cgs, cus, overlapped):
-    """Kernel(s) that a forward (which = 0) or backward (1) of this shape launches; one is compiled per combination of roles."""
+    """Kernel(s) that a forward (which = 0) or backward (1) of this shape launches, by their names in a trace, as the library plans them."""
     import ctypes
     lib = ctypes.CDLL(os.path.join(ROOT, "ttt-tk_amd", "libttt_mlp.so"))
-    one_each = ("ttt_mlp_fwd_kernel", "ttt_mlp_bwd_kernel")[which]
-    seg, launches = ctypes.c_int(), ctypes.c_int()
-    lib.ttt_mlp_segment_plan(which, ctypes.c_longlong(pairs), cus, NC, cgs, 1 if overlapped else 0, ctypes.byref(seg), ctypes.byref(launches))
-    if seg.value > 0:
-        return f"{one_each} x {launches.value} (sequences cut at checkpoints)"
-    if not overlapped:
-        return one_each
-    one, rest, per = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
-    lib.ttt_mlp_launch_plan(which, ctypes.c_longlong(pairs), cus, ctypes.byref(one), ctypes.byref(rest), ctypes.byref(per))
-    if which == 0:   # <mini-batches per hand-over>
-        several = "ttt_mlp_fwd_wide_kernel" if per.value > 2 else f"ttt_mlp_fwd_split_kernel<{32 if NC >= 512 else 8}>"
-    else:            # <replaying workgroups, grad_L_XK workgroup> / <replaying workgroups, workgroup that reads ahead>
-        several = {2: "ttt_mlp_bwd_split_kernel<1, false>", 3: "ttt_mlp_bwd_split_kernel<2, false>", 4: "ttt_mlp_bwd_split_kernel<2, true>",
-                   5: "ttt_mlp_bwd_wide_kernel<2, false>", 7: "ttt_mlp_bwd_wide_kernel<3, true>", 8: "ttt_mlp_bwd_wide_kernel<4, true>"}.get(per.value, "")
-    return f"{one_each} + {several}" if one.value else several
-
-
-def running_kernel(which, pairs, NC, cgs, cus, overlapped):
-    """The same by the name of the kernel in a trace: `launched_kernel` names a backward by the roles of a pair's own workgroups; where the
-    workgroups of an XCD work for all of its pairs, or idle CUs for all pairs, the roles are in one kernel."""
-    name = launched_kernel(which, pairs, NC, cgs, cus, overlapped)
-    if which == 0 or not overlapped or "cut" in name:
-        return name
-    one, rest, K = pairs // cus * cus, pairs % cus, -(-NC // cgs)
-    if 2 * rest > cus:
-        return "ttt_mlp_bwd_helped_kernel"
-    per_xcd, short = -(-rest // 8), cgs < 8 or K < 4 or cgs * K < 90
-    if 3 * per_xcd <= cus // 8 and not (short and 4 * per_xcd > cus // 8):
-        several = "ttt_mlp_bwd_gang_kernel"
-    else:
-        several = f"ttt_mlp_bwd_split_kernel<{2 if 3 * rest <= cus else 1}>"
-    return f"ttt_mlp_bwd_kernel + {several}" if one else several
+    lib.ttt_mlp_launched_kernel.restype = ctypes.c_char_p
+    names, dispatches = [], ctypes.c_int()
+    while (name := lib.ttt_mlp_launched_kernel(which, ctypes.c_longlong(pairs), cus, NC, cgs, 1 if overlapped else 0, len(names), None,
+                                               ctypes.byref(dispatches), None)) is not None:
+        names.append(name.decode() + (f" x {dispatches.value} (sequences cut at checkpoints)" if dispatches.value > 1 else ""))
+    return " + ".join(names)
 
 
 def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibrate_copy=False):
@@ -234,7 +208,7 @@ def run_workload(name, steps, warmup, overwrite=False, no_overlap=False, calibra
     all_tflops = (FWD_G + (BWD_G if backward else 0)) * G_FLOP * mb_steps / (ms_per_step * 1e-3) / 1e12
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     fwd_kernel = launched_kernel(0, B * NH, NC, cgs, cus, ext.last_forward_mode() == 1)
-    bwd_kernel = running_kernel(1, B * NH, NC, cgs, cus, ext.last_backward_mode() == 1) if backward else None
+    bwd_kernel = launched_kernel(1, B * NH, NC, cgs, cus, ext.last_backward_mode() == 1) if backward else None
     traffic, note = measured_traffic_checked(name, "bwd" if backward else "fwd")
     # the dominant kernel: the backward (the forward where there is no backward)
     roofline = {"bound": "mfma", "kernel": bwd_kernel if backward else fwd_kernel,

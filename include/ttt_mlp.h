@@ -136,7 +136,7 @@ int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* args, void* stream);
 /* Same for the remat backward. */
 int ttt_mlp_bwd_launch(const ttt_mlp_bwd_args* args, void* stream);
 
-/* The same backward (bit-identical results) with two to eight workgroups per
+/* The same backward (bit-identical results) with two to twelve workgroups per
  * (batch, head) where the device has CUs to spare: one to four recompute checkpoint
  * group after checkpoint group, one walks each recomputed group backwards - or two,
  * which hold half of the hidden columns each and exchange partial sums - another
@@ -149,9 +149,9 @@ int ttt_mlp_bwd_launch(const ttt_mlp_bwd_args* args, void* stream);
  * Workgroups that wait for each other must be resident together (one per CU),
  * so the pairs are covered by up to two launches in a row: the largest multiple
  * of the CU count with one workgroup per pair, then the remaining n pairs.  Where
- * the workgroups of ceil(n/8) pairs fit an eighth of the CUs the walk takes two: eight
- * per pair (four recomputing, one reading ahead), else seven (three), else
- * five (two recomputing, none reading ahead) - up to 32, 32 and 48 pairs on 256 CUs.
+ * the workgroups of ceil(n/8) pairs fit an eighth of the CUs the walk takes two: twelve, ten or eight
+ * per pair (eight, six or four recomputing, one reading ahead), else seven (three), else six or
+ * five (three or two recomputing, none reading ahead) - up to 16, 24, 32, 32, 40 and 48 pairs on 256 CUs.
  * With less room than that the workgroups of an eighth of the device that recompute, and those for
  * grad_L_XK, serve all of its pairs (up to 80 on 256 CUs), then three or two per pair if they fit.
  * Where not even two do, one workgroup does everything for each pair and the CUs left over, if eight or more, recompute
@@ -236,14 +236,13 @@ const char* ttt_mlp_error_string(int code);
 
 /* How an overlapped launch of `pairs` = B*NH (batch, head) pairs is laid out on a device with
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
- * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none).  Workgroups that only help
- * pairs that have one are not counted.  which = 0
- * forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk),
- * 3 (two replay), 7 or 8 (walk on two, one for grad_L_XK / grad_L_XV, three, or four to eight, that replay, one that reads ahead), and
- * 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly: the whole ones of a pair's share, at most 5, while
- * the workgroups that replay and those for grad_L_XK may serve all of those pairs.  More than 2 forward, and all
- * backward but 2 and the 3 that has no eighth of the device for its pairs: the workgroups of a pair share an XCD, and those of
- * ceil(*other_pairs / 8) pairs fit an eighth of the CUs. */
+ * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none): whole ones of a pair's share where
+ * those of an eighth of the device work for all of its pairs.  Workgroups that only help pairs that have one are not counted.
+ * which = 0 forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk), 3 (two
+ * replay); with the walk on two and one for grad_L_XK / grad_L_XV 12, 10, 8 or 7 (eight, six, four or three that replay, one that reads
+ * ahead), 6 or 5 (three or two that replay); 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly.  More than 2
+ * forward, and all backward but 2 and the 3 that has no eighth of the device for its pairs: the workgroups of a pair share an XCD, and those of
+ * ceil(*other_pairs / 8) pairs fit an eighth of the CUs.  Backward calls whose checkpoint groups are short or few may take fewer. */
 int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long* one_workgroup_pairs,
                         long long* other_pairs, int* workgroups_per_other_pair);
 

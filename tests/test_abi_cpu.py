@@ -180,29 +180,32 @@ def test_host_module_offers_the_autograd_wrapper(lib):
 
 
 def test_launch_plan_keeps_waiting_workgroups_within_the_device(lib):
-    """Workgroups that wait for each other must all be resident: whatever the plan, the launch with several
-    workgroups per pair never exceeds the CU count, and full rounds of the device come first."""
+    """Full rounds of the device come first, then several workgroups for each of the pairs left over, as many as there is room for
+    (test_workgroups_that_wait_for_each_other_fit_the_device looks at the grids themselves)."""
     def plan(which, pairs, cus):
         a, b, c = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
         assert lib.ttt_mlp_launch_plan(which, ctypes.c_longlong(pairs), cus, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c)) == 0
         return a.value, b.value, c.value
     assert plan(1, 48, 256) == (0, 48, 5)          # the metric's configuration: two replay, two walk, one for grad_L_XK
-    assert plan(1, 32, 256) == (0, 32, 8)          # four replay, two walk, one for grad_L_XK, one that reads ahead
-    assert plan(1, 33, 256) == (0, 33, 5)          # five pairs on an XCD: eight each would not fit its 32 CUs
+    assert plan(1, 16, 256) == (0, 16, 12)         # eight replay (four at once the groups walked first), two walk, one for grad_L_XK, one that reads ahead
+    assert plan(1, 24, 256) == (0, 24, 10)         # six replay
+    assert plan(1, 32, 256) == (0, 32, 8)          # four
+    assert plan(1, 33, 256) == (0, 33, 6)          # five pairs on an XCD: eight each would not fit its 32 CUs; three replay
+    assert plan(1, 41, 256) == (0, 41, 5)          # two replay
     assert plan(1, 44, 256) == (0, 44, 5)          # (the grid is padded to a multiple of 8 pairs)
-    assert plan(1, 49, 256) == (0, 49, 4)          # seven pairs on an XCD: the walk stays on one CU
+    assert plan(1, 49, 256) == (0, 49, 4)          # seven pairs on an XCD: the workgroups that do not walk serve all of them
     assert plan(1, 56, 256) == (0, 56, 4)
-    assert plan(1, 64, 256) == (0, 64, 4)          # four per pair fill the device exactly
+    assert plan(1, 64, 256) == (0, 64, 4)          # eight: the walk on one CU
     assert plan(1, 72, 256) == (0, 72, 3)
     assert plan(1, 96, 256) == (0, 96, 2)
     assert plan(1, 128, 256) == (0, 128, 2)
     assert plan(1, 200, 256) == (200, 0, 0)        # two per pair would not fit: one each
     assert plan(1, 384, 256) == (256, 128, 2)      # one full round, the rest with two each
-    assert plan(1, 260, 256) == (256, 4, 8)
-    assert plan(1, 264, 256) == (256, 8, 8)
+    assert plan(1, 260, 256) == (256, 4, 12)
+    assert plan(1, 264, 256) == (256, 8, 12)
     assert plan(1, 512, 256) == (512, 0, 0)
     assert plan(1, 8, 56) == (0, 8, 7)             # seven CUs on an XCD: three replay
-    assert plan(1, 8, 48) == (0, 8, 5)
+    assert plan(1, 8, 48) == (0, 8, 6)             # six: the same without the one that reads ahead
     assert plan(0, 48, 256) == (0, 48, 4)          # forward: the recurrence on two, two for the output
     assert plan(0, 64, 256) == (0, 64, 4)
     assert plan(0, 65, 256) == (0, 65, 3)
@@ -219,12 +222,60 @@ def test_launch_plan_keeps_waiting_workgroups_within_the_device(lib):
                 one, rest, per = plan(which, pairs, cus)
                 assert one + rest == pairs and one % cus == 0 or rest == 0
                 assert rest * per <= cus
-                assert per in ((0, 2, 3, 4) if which == 0 else (0, 2, 3, 4, 5, 7, 8))
+                assert per in ((0, 2, 3, 4) if which == 0 else (0, 2, 3, 4, 5, 6, 7, 8, 10, 12))
                 if per > (2, 4)[which]:            # the workgroups of a pair on one XCD, the grid padded to a multiple of 8 pairs
                     assert -(-rest // 8) * per <= cus // 8
                 if which == 1 and per == 4:        # a fifth workgroup on the walk's XCD never has room beside a walk on one CU
                     assert not (5 * rest <= cus and rest % 8 == 0)
     assert lib.ttt_mlp_launch_plan(2, ctypes.c_longlong(1), 1, None, None, None) == 1001
+
+
+def _launched(lib, which, pairs, cus, NC, cgs, with_workspace=1):
+    """[(kernel, workgroups, dispatches, whether they have to be resident at once)]"""
+    lib.ttt_mlp_launched_kernel.restype = ctypes.c_char_p
+    out = []
+    grid, dispatches, resident = ctypes.c_longlong(), ctypes.c_int(), ctypes.c_int()
+    while (name := lib.ttt_mlp_launched_kernel(which, ctypes.c_longlong(pairs), cus, NC, cgs, with_workspace, len(out), ctypes.byref(grid),
+                                               ctypes.byref(dispatches), ctypes.byref(resident))) is not None:
+        out.append((name.decode(), grid.value, dispatches.value, resident.value))
+    return out
+
+
+def test_workgroups_that_wait_for_each_other_fit_the_device(lib):
+    """The grid that is launched, for every number of pairs, groups of every kind and devices of several sizes: where workgroups wait for
+    others that may not have started, all of them are resident at once; one workgroup per pair, and helpers, need not be."""
+    seen = set()
+    for which in (0, 1):
+        for cus in (8, 17, 56, 104, 256, 304):
+            for pairs in list(range(1, cus + 3)) + [2 * cus - 1, 2 * cus + cus // 3]:
+                for NC, cgs in ((1, 1), (4, 1), (9, 4), (31, 3), (95, 24), (64, 8), (512, 32), (2048, 64)):
+                    calls = _launched(lib, which, pairs, cus, NC, cgs)
+                    assert 1 <= len(calls) <= 2
+                    for name, grid, dispatches, resident in calls:
+                        seen.add(name)
+                        assert grid > 0 and dispatches >= 1
+                        assert resident == 0 or (grid <= cus and dispatches == 1), (which, cus, pairs, NC, cgs, name, grid)
+                    # every pair has a workgroup that carries its state, and what is left over none that waits
+                    one = calls[0][1] if len(calls) == 2 else 0
+                    assert one % cus == 0
+                    name, grid, dispatches, resident = calls[-1]
+                    assert dispatches > 1 or grid >= pairs - one
+                    assert name not in ("ttt_mlp_fwd_kernel", "ttt_mlp_bwd_kernel") or resident == 0
+    sources = "".join(open(os.path.join(PKG, "csrc", f)).read() for f in sorted(os.listdir(os.path.join(PKG, "csrc"))))
+    for name in seen:
+        assert re.search(r"__global__[^;{]*\b" + name.split("<")[0] + r"\(", sources), name
+    declared = set(re.findall(r"X\(\w+, (ttt_mlp_\w+(?:<[^>]*>)?)\)", sources))
+    assert seen == declared, declared - seen   # a kernel that no shape launches
+    # the helpers take the CUs that one workgroup per pair leaves, where the groups go round
+    assert _launched(lib, 1, 200, 256, 100, 16) == [("ttt_mlp_bwd_helped_kernel", 256, 1, 0)]
+    assert _launched(lib, 1, 200, 256, 64, 32) == [("ttt_mlp_bwd_kernel", 200, 1, 0)]
+    # 51 pairs: all 32 CUs of an XCD work for its seven; groups too short for that: four whole workgroups each
+    assert _launched(lib, 1, 51, 256, 77, 10) == [("ttt_mlp_bwd_gang_kernel<true, false, false, false, false>", 256, 1, 1)]
+    assert _launched(lib, 1, 51, 256, 77, 3) == [("ttt_mlp_bwd_gang_kernel<false, true, false, true, false>", 224, 1, 1)]
+    assert _launched(lib, 1, 8, 256, 64, 8) == [("ttt_mlp_bwd_gang_kernel<true, true, true, true, true>", 96, 1, 1)]
+    assert _launched(lib, 1, 384, 256, 512, 32) == [("ttt_mlp_bwd_kernel", 256, 3, 0)]
+    assert _launched(lib, 1, 48, 256, 512, 32, 0) == [("ttt_mlp_bwd_kernel", 48, 1, 0)]
+    assert _launched(lib, 2, 48, 256, 512, 32) == _launched(lib, 0, 0, 256, 512, 32) == _launched(lib, 0, 8, 0, 512, 32) == []
 
 
 def test_export_of_group_zero_validates_like_the_backward(lib):

@@ -2100,26 +2100,22 @@ __global__ void ttt_mlp_zero_words(int* w, int n, const int* report) { clear_wor
 extern "C" int ttt_mlp_bwd_threads() { return ttt::BW_THREADS; }
 extern "C" int ttt_mlp_bwd_lds_bytes() { return ttt::SM_BWD_BYTES; }
 
-hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(ttt::ttt_mlp_bwd_kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
-  if (e != hipSuccess) return e;
-  if (p.sync == nullptr) {
-    hipLaunchKernelGGL(ttt::ttt_mlp_bwd_kernel, dim3(p.nbh), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);
-    return hipGetLastError();
-  }
-  const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
-  int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
-  hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
-  const dim3 grid(p.n_helpers > 0 ? p.nbh + p.n_helpers : (p.n_replay + 1) * p.nbh), block(ttt::BW_THREADS);
-  auto launch = [&](auto kernel) -> hipError_t {
-    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
+hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
+  auto launch = [&](auto k) -> hipError_t {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
+    if (e != hipSuccess) return e;
+    if (p.sync != nullptr) {
+      const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
+      int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
+      hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
+    }
+    hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };
-  if (p.n_helpers > 0) return launch(ttt::ttt_mlp_bwd_helped_kernel);
-  return p.n_replay == 2 ? launch(ttt::ttt_mlp_bwd_split_kernel<2>) : launch(ttt::ttt_mlp_bwd_split_kernel<1>);
+  switch (kernel) {
+    TTT_BWD_KERNELS(TTT_KERNEL_LAUNCH)
+    default: return hipErrorInvalidValue;
+  }
 }
 #else
 }  // namespace ttt

@@ -860,23 +860,20 @@ __global__ void ttt_mlp_bwd_wide_clear(int* w, int n, const int* report, uint4* 
 
 }  // namespace ttt
 
-hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream) {
-  const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
-  int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-  const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
-  hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
-                     reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
-  const int slots = (p.wide ? 2 : 1) * p.gang_pairs + p.n_finish + p.n_replay + (p.n_prefetch ? p.gang_pairs : 0);
-  const dim3 grid(8 * slots), block(ttt::BW_THREADS);
-  auto launch = [&](auto kernel) -> hipError_t {
-    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(kernel, grid, block, ttt::SM_BWD_BYTES, stream, p);
+hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
+  auto launch = [&](auto k) -> hipError_t {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
+    if (e != hipSuccess) return e;
+    const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
+    int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
+    const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
+    hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
+                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };
-  const bool own = p.n_finish == p.gang_pairs;
-  if (p.n_prefetch) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, true, true, true, true>);
-  if (p.wide && p.n_shared > 0) return launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true, true>);
-  if (p.wide) return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, true, false>) : launch(ttt::ttt_mlp_bwd_gang_kernel<true, false, false, false, false>);
-  return own ? launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, true, false>) : launch(ttt::ttt_mlp_bwd_gang_kernel<false, true, false, false, false>);
+  switch (kernel) {
+    TTT_BWD_GANG_KERNELS(TTT_KERNEL_LAUNCH)
+    default: return hipErrorInvalidValue;
+  }
 }

@@ -154,7 +154,6 @@ struct LaunchPlan {
   long long n_rest = 0;     // pairs n_single .. n_single+n_rest-1
   bool rest_split = false;
   bool wide = false;
-  int per_pair = 1;         // workgroups per pair of the rest, in every role (whole ones, at most five, where some are shared)
   int n_out = 0;            // forward, wide: that compute Out
   int gang = 0;             // backward: pairs of an XCD that share workgroups, 0: whole ones, that replay or walk, for each pair
   int n_replay = 0;         // backward: that replay checkpoint groups, of a gang or of a pair
@@ -167,6 +166,31 @@ struct LaunchPlan {
   bool waits() const { return rest_split || helpers > 0; }                    // workgroups that wait for each other, in a workspace
   long long first_waiting() const { return helpers > 0 ? 0 : n_single; }      // of these pairs
   long long n_waiting() const { return helpers > 0 ? n_single : n_rest; }
+  // Workgroups of an XCD: of a gang, or of the pairs that a forward with the recurrence on two CUs deals to it.
+  int slots(bool backward) const {
+    return backward ? (wide ? 2 : 1) * gang + n_finish + n_replay + (prefetch ? gang : 0) : static_cast<int>((n_rest + 7) / 8) * (2 + n_out);
+  }
+  // The launch behind the full rounds of one workgroup per pair: its kernel and its workgroups.
+  TttKernel kernel(bool backward, int NC) const {
+    if (!backward) return wide ? FWD_WIDE : NC >= 512 ? FWD_SPLIT_32 : FWD_SPLIT_8;   // (mini-batches per hand-over)
+    if (helpers > 0) return BWD_HELPED;
+    if (!gang) return n_replay == 2 ? BWD_SPLIT_2 : BWD_SPLIT_1;
+    const bool own = n_finish == gang;
+    if (prefetch) return BWD_GANG_AHEAD;
+    if (wide) return shared > 0 ? BWD_GANG_PARTS : own ? BWD_GANG_WIDE : BWD_GANG_WIDE_SHARED;
+    return own ? BWD_GANG : BWD_GANG_SHARED;
+  }
+  long long grid(bool backward) const {
+    if (helpers > 0) return n_single + helpers;
+    if (wide || gang) return 8LL * slots(backward);
+    return n_rest * (backward ? n_replay + 1 : 2);
+  }
+  // Workgroups per pair of the rest, whole ones where some are shared.
+  int per_pair(bool backward) const {
+    if (!rest_split) return 0;
+    if (backward && gang) return slots(true) / gang;
+    return backward ? n_replay + 1 : 2 + n_out;
+  }
 };
 // Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
 // of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others.
@@ -220,7 +244,6 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     // one output workgroup keeps up with a recurrence on two CUs only just; two where they fit
     pl.n_out = fits_xcd(4) ? 2 : fits_xcd(3) ? 1 : 0;
     pl.wide = pl.n_out > 0;
-    pl.per_pair = 2 + pl.n_out;
     return pl;
   }
   // Four replaying workgroups per pair leave a walk on two CUs to itself, also where they evaluate the GELU family for it (32 pairs x 512:
@@ -238,7 +261,6 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     pl.parts = each >= 8 ? 4 : each >= 6 ? 3 : each >= 4 ? 2 : 1;
     pl.shared = each >= 4 ? 3 : 0;
     pl.n_replay = (each >= 4 ? 2 * pl.parts : 3) * pairs;
-    pl.per_pair = each >= 4 ? 8 : 7;
     pl.sets = each >= 4 ? 6 : 5;
     return pl;
   }
@@ -264,12 +286,10 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     } else {
       divide_workers(pairs, on_xcd - pairs, 330, COST_REPLAY_IMG, COST_FINISH_IMG, &pl.n_replay, &pl.n_finish);
     }
-    pl.per_pair = on_xcd / pairs < 5 ? on_xcd / pairs : 5;
     pl.sets = 4;
     return pl;
   }
   pl.n_replay = 3 * pl.n_rest <= cus ? 2 : 1;
-  pl.per_pair = pl.n_replay + 1;
   pl.sets = 2 * pl.n_replay;
   return pl;
 }
@@ -356,12 +376,12 @@ int launch_segments(Params p, const SegmentPlan& plan, int cus, Enqueue enqueue)
 }
 int launch_fwd_segments(ttt::FwdParams p, const SegmentPlan& plan, int cus, hipStream_t stream) {
   p.seg_len = plan.seg_len;
-  return launch_segments(p, plan, cus, [stream](const ttt::FwdParams& q) { return ttt_mlp_fwd_enqueue(q, stream); });
+  return launch_segments(p, plan, cus, [stream](const ttt::FwdParams& q) { return ttt_mlp_fwd_enqueue(q, FWD_ONE, q.nbh, stream); });
 }
 // Backward: segment 0 = the last groups of every sequence.
 int launch_bwd_segments(ttt::BwdParams p, const SegmentPlan& plan, int cus, hipStream_t stream) {
   p.seg_groups = plan.groups;
-  return launch_segments(p, plan, cus, [stream](const ttt::BwdParams& q) { return ttt_mlp_bwd_enqueue(q, stream); });
+  return launch_segments(p, plan, cus, [stream](const ttt::BwdParams& q) { return ttt_mlp_bwd_enqueue(q, BWD_ONE, q.nbh, stream); });
 }
 SegmentPlan plan_bwd_segments(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace) {
   // (the two norm sums that a segment leaves behind, 4 KiB each, fill one 8 KiB slot of x_hat_ln_group)
@@ -383,7 +403,6 @@ LaunchPlan bwd_reduced(LaunchPlan pl) {
     pl.parts = 1;
     pl.shared = 0;
     pl.prefetch = false;
-    pl.per_pair = 5;
     pl.sets = 4;
   }
   return pl;
@@ -403,16 +422,38 @@ LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K) {
     pl.wide = false;
     pl.n_finish = pl.gang;
     pl.n_replay = 2 * pl.gang;
-    pl.per_pair = 4;
   } else if (!four && !pl.wide && pl.gang && (cgs < 8 || K < 4 || cgs * K < 90)) {
     pl.gang = pl.n_finish = 0;
     pl.n_replay = 2;
-    pl.per_pair = 3;
   }
   return pl;
 }
 // The launch of a backward call with a workspace.
 LaunchPlan plan_bwd(long long pairs, int cus, long long cgs, long long K) { return bwd_for_groups(plan_for(pairs, cus, true), cus, cgs, K); }
+// What a call enqueues to do its work: sequences cut into segments, a device's worth of them at a time, or `n` kernels in a row.
+struct Call {
+  SegmentPlan seg;
+  int n = 1;
+  TttKernel kernel[2];
+  long long grid[2];
+};
+Call plan_call(bool backward, const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace) {
+  Call c;
+  c.kernel[0] = backward ? BWD_ONE : FWD_ONE;
+  c.seg = backward ? plan_bwd_segments(pl, pairs, cus, NC, cgs, with_workspace)
+                   : plan_segments(pairs, cus, NC, cgs, false, uncut_x1000(pl, pairs, cus, NC, cgs, with_workspace, false));
+  if (c.seg.seg_len > 0) {
+    c.grid[0] = cus;
+    return c;
+  }
+  c.grid[0] = pairs;
+  if (!with_workspace || !pl.waits() || (pl.helpers > 0 && !helpers_pay(pl, ((long long)NC + cgs - 1) / cgs))) return c;
+  c.n = 0;
+  if (pl.first_waiting() > 0) c.grid[c.n++] = pl.n_single;
+  c.kernel[c.n] = pl.kernel(backward, NC);
+  c.grid[c.n++] = pl.grid(backward);
+  return c;
+}
 // Workspace of the backward with several workgroups per pair, for n (batch, head) pairs of K groups: the synchronisation
 // words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
 // CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
@@ -479,15 +520,12 @@ int check_workspace(const void* workspace) {
 extern "C" int ttt_mlp_bwd_launch(const ttt_mlp_bwd_args* a, void* stream) {
   ttt::BwdParams p;
   if (int rc = make_bwd_params(a, p)) return rc;
-  {
-    const long long pairs = (long long)p.B * p.NH;
-    const int cus = device_cus();
-    const SegmentPlan seg = plan_bwd_segments(LaunchPlan{}, pairs, cus, p.NC, p.cgs, false);
-    if (seg.seg_len > 0) return launch_bwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
-  }
+  const int cus = device_cus();
+  const Call call = plan_call(true, LaunchPlan{}, (long long)p.B * p.NH, cus, p.NC, p.cgs, false);
+  if (call.seg.seg_len > 0) return launch_bwd_segments(p, call.seg, cus, static_cast<hipStream_t>(stream));
   p.bh0 = 0;
   p.nbh = p.B * p.NH;
-  return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
+  return static_cast<int>(ttt_mlp_bwd_enqueue(p, call.kernel[0], static_cast<int>(call.grid[0]), static_cast<hipStream_t>(stream)));
 }
 
 extern "C" int ttt_mlp_bwd_export_group0(const ttt_mlp_bwd_args* a, void* stream) {
@@ -538,34 +576,30 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   ttt::BwdParams p;
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
-  LaunchPlan pl = plan_bwd((long long)p.B * p.NH, device_cus(), p.cgs, p.K);
+  const int cus = device_cus();
+  LaunchPlan pl = plan_bwd((long long)p.B * p.NH, cus, p.cgs, p.K);
   if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
   const BwdWorkspace w(pl, p.cgs, p.K);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
-  {
-    // cut sequences where they beat a last round on several workgroups per pair (see the forward)
-    const long long pairs = (long long)p.B * p.NH;
-    const int cus = device_cus();
-    const SegmentPlan seg = plan_bwd_segments(pl, pairs, cus, p.NC, p.cgs, true);
-    const bool alone = pl.helpers > 0 && !helpers_pay(pl, p.K);
-    if (seg.seg_len > 0 || alone) {
-      if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_waiting())),
-                                                 static_cast<hipStream_t>(stream)))
-        return static_cast<int>(e);
-      if (alone) {
-        p.bh0 = 0;
-        p.nbh = p.B * p.NH;
-        return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
-      }
-      return launch_bwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
-    }
+  const Call call = plan_call(true, pl, (long long)p.B * p.NH, cus, p.NC, p.cgs, true);
+  const TttKernel kernel = call.kernel[call.n - 1];
+  const int grid = static_cast<int>(call.grid[call.n - 1]);
+  // cut sequences where they beat a last round on several workgroups per pair (see the forward)
+  if (kernel == BWD_ONE) {
+    if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_waiting())),
+                                               static_cast<hipStream_t>(stream)))
+      return static_cast<int>(e);
+    if (call.seg.seg_len > 0) return launch_bwd_segments(p, call.seg, cus, static_cast<hipStream_t>(stream));
+    p.bh0 = 0;
+    p.nbh = p.B * p.NH;
+    return static_cast<int>(ttt_mlp_bwd_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
   }
-  if (pl.first_waiting() > 0) {
+  if (call.n > 1) {
     p.bh0 = 0;
     p.nbh = static_cast<int>(pl.n_single);
-    if (hipError_t e = ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream))) return static_cast<int>(e);
+    if (hipError_t e = ttt_mlp_bwd_enqueue(p, call.kernel[0], p.nbh, static_cast<hipStream_t>(stream))) return static_cast<int>(e);
   }
   // The kernels index the workspace by the global pair number: every pointer is moved back by bh0 entries.
   const size_t b0 = (size_t)pl.first_waiting();
@@ -631,9 +665,9 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   if (pl.gang) {
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
     p.scatter = scatter ? 1 : 0;
-    return static_cast<int>(ttt_mlp_bwd_gang_enqueue(p, static_cast<hipStream_t>(stream)));
+    return static_cast<int>(ttt_mlp_bwd_gang_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
   }
-  return static_cast<int>(ttt_mlp_bwd_enqueue(p, static_cast<hipStream_t>(stream)));
+  return static_cast<int>(ttt_mlp_bwd_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
 }
 }  // namespace
 
@@ -644,13 +678,12 @@ extern "C" int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* a, void* worksp
 extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
   ttt::FwdParams p;
   if (int rc = make_fwd_params(a, p)) return rc;
-  const long long pairs = (long long)p.B * p.NH;
   const int cus = device_cus();
-  const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, false, uncut_x1000(LaunchPlan{}, pairs, cus, p.NC, p.cgs, false, false));
-  if (seg.seg_len > 0) return launch_fwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
+  const Call call = plan_call(false, LaunchPlan{}, (long long)p.B * p.NH, cus, p.NC, p.cgs, false);
+  if (call.seg.seg_len > 0) return launch_fwd_segments(p, call.seg, cus, static_cast<hipStream_t>(stream));
   p.bh0 = 0;
   p.nbh = p.B * p.NH;
-  return static_cast<int>(ttt_mlp_fwd_enqueue(p, static_cast<hipStream_t>(stream)));
+  return static_cast<int>(ttt_mlp_fwd_enqueue(p, call.kernel[0], static_cast<int>(call.grid[0]), static_cast<hipStream_t>(stream)));
 }
 
 extern "C" size_t ttt_mlp_fwd_workspace_bytes(int B, int NH) {
@@ -670,28 +703,27 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
   ttt::FwdParams p;
   if (int rc = make_fwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
-  const LaunchPlan pl = plan_launches((long long)p.B * p.NH, false);
+  const int cus = device_cus();
+  const LaunchPlan pl = plan_for((long long)p.B * p.NH, cus, false);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
   const FwdWorkspace w(pl.n_rest, pl.n_out);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
-  {
+  const Call call = plan_call(false, pl, (long long)p.B * p.NH, cus, p.NC, p.cgs, true);
+  const TttKernel kernel = call.kernel[call.n - 1];
+  const int grid = static_cast<int>(call.grid[call.n - 1]);
+  if (call.seg.seg_len > 0) {
     // cut sequences beat a last round on two workgroups per pair where there are full rounds before it: the
     // workspace then only has its words cleared (callers read the status word behind them)
-    const long long pairs = (long long)p.B * p.NH;
-    const int cus = device_cus();
-    const SegmentPlan seg = plan_segments(pairs, cus, p.NC, p.cgs, false, uncut_x1000(pl, pairs, cus, p.NC, p.cgs, true, false));
-    if (seg.seg_len > 0) {
-      if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_rest)),
-                                                 static_cast<hipStream_t>(stream)))
-        return static_cast<int>(e);
-      return launch_fwd_segments(p, seg, cus, static_cast<hipStream_t>(stream));
-    }
+    if (hipError_t e = ttt_mlp_fwd_clear_words(reinterpret_cast<int*>(base + w.off[0]), static_cast<int>(ttt::bwd_sync_ints(pl.n_rest)),
+                                               static_cast<hipStream_t>(stream)))
+      return static_cast<int>(e);
+    return launch_fwd_segments(p, call.seg, cus, static_cast<hipStream_t>(stream));
   }
-  if (pl.n_single > 0) {
+  if (call.n > 1) {
     p.bh0 = 0;
     p.nbh = static_cast<int>(pl.n_single);
-    if (hipError_t e = ttt_mlp_fwd_enqueue(p, static_cast<hipStream_t>(stream))) return static_cast<int>(e);
+    if (hipError_t e = ttt_mlp_fwd_enqueue(p, call.kernel[0], p.nbh, static_cast<hipStream_t>(stream))) return static_cast<int>(e);
   }
   const size_t b0 = (size_t)pl.n_single;
   p.bh0 = static_cast<int>(pl.n_single);
@@ -707,12 +739,12 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
     p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
     p.scatter = scatter ? 1 : 0;
-    return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, static_cast<hipStream_t>(stream)));
+    return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, grid, static_cast<hipStream_t>(stream)));
   }
-  p.ring_log2 = p.NC >= 512 ? 5 : 3;   // 32 or 8 mini-batches per hand-over
+  p.ring_log2 = kernel == FWD_SPLIT_32 ? 5 : 3;
   p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * 2 * ttt::FWD_RING_MAX * (ttt::FWD_IMG_BYTES / 2);
   p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * 2 * ttt::FWD_RING_MAX * ttt::FWD_BIAS_FLOATS;
-  return static_cast<int>(ttt_mlp_fwd_enqueue(p, static_cast<hipStream_t>(stream)));
+  return static_cast<int>(ttt_mlp_fwd_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
 }
 }  // namespace
 
@@ -811,7 +843,7 @@ extern "C" int ttt_mlp_launch_plan(int which, long long pairs, int compute_units
   const LaunchPlan pl = plan_for(pairs, compute_units, which == 1);
   *one_workgroup_pairs = pl.n_single;
   *other_pairs = pl.n_rest;
-  *workgroups_per_other_pair = pl.n_rest > 0 ? pl.per_pair : 0;
+  *workgroups_per_other_pair = pl.per_pair(which == 1);
   return TTT_MLP_OK;
 }
 
@@ -823,12 +855,29 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
     return TTT_MLP_ERR_BAD_ARG;
   const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size)
                                    : plan_for(pairs, compute_units, false);
-  const SegmentPlan seg = which == 1 ? plan_bwd_segments(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0)
-                                     : plan_segments(pairs, compute_units, NC, checkpoint_group_size, false,
-                                                     uncut_x1000(pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0, false));
-  *segment_minibatches = seg.seg_len;
-  *launches = seg.seg_len > 0 ? seg.launches : (with_workspace != 0 && pl.rest_split && pl.n_single > 0 ? 2 : 1);
+  const Call call = plan_call(which == 1, pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0);
+  *segment_minibatches = call.seg.seg_len;
+  *launches = call.seg.seg_len > 0 ? call.seg.launches : call.n;
   return TTT_MLP_OK;
+}
+
+extern "C" const char* ttt_mlp_launched_kernel(int which, long long pairs, int compute_units, int NC, int checkpoint_group_size, int with_workspace,
+                                               int index, long long* workgroups, int* dispatches, int* resident) {
+  if (pairs <= 0 || compute_units <= 0 || NC <= 0 || checkpoint_group_size <= 0 || (which != 0 && which != 1) || index < 0) return nullptr;
+  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size)
+                                   : plan_for(pairs, compute_units, false);
+  const Call call = plan_call(which == 1, pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0);
+  if (index >= call.n) return nullptr;
+  const TttKernel kernel = call.kernel[index];
+  if (workgroups != nullptr) *workgroups = call.grid[index];
+  if (dispatches != nullptr) *dispatches = call.seg.seg_len > 0 ? call.seg.launches : 1;
+  if (resident != nullptr) *resident = kernel != FWD_ONE && kernel != BWD_ONE && kernel != BWD_HELPED;
+  switch (kernel) {
+#define TTT_KERNEL_NAME(number, ...) case number: return #__VA_ARGS__;
+    TTT_FWD_KERNELS(TTT_KERNEL_NAME) TTT_FWD_WIDE_KERNELS(TTT_KERNEL_NAME) TTT_BWD_KERNELS(TTT_KERNEL_NAME) TTT_BWD_GANG_KERNELS(TTT_KERNEL_NAME)
+#undef TTT_KERNEL_NAME
+  }
+  return nullptr;
 }
 
 extern "C" int ttt_mlp_kernel_info(int which, int* lds_bytes, int* threads_per_workgroup) {

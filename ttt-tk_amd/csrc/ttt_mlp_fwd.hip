@@ -476,25 +476,21 @@ hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, hipStream_t stream) {
-  // Per-device attribute; cheap enough to set on every launch.
-  if (p.sync == nullptr) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(ttt::ttt_mlp_fwd_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_FWD_BYTES);
+hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
+  auto launch = [&](auto k) -> hipError_t {
+    // Per-device attribute; cheap enough to set on every launch.
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_FWD_BYTES);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(ttt::ttt_mlp_fwd_kernel, dim3(p.nbh), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
+    if (p.sync != nullptr) {
+      const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
+      int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
+      hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
+    }
+    hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
     return hipGetLastError();
+  };
+  switch (kernel) {
+    TTT_FWD_KERNELS(TTT_KERNEL_LAUNCH)
+    default: return hipErrorInvalidValue;
   }
-  const void* kernel = p.ring_log2 == 5 ? reinterpret_cast<const void*>(ttt::ttt_mlp_fwd_split_kernel<32>)
-                                        : reinterpret_cast<const void*>(ttt::ttt_mlp_fwd_split_kernel<8>);
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_FWD_BYTES);
-  if (e != hipSuccess) return e;
-  const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
-  int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
-  if (p.ring_log2 == 5)
-    hipLaunchKernelGGL(ttt::ttt_mlp_fwd_split_kernel<32>, dim3(2 * p.nbh), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
-  else
-    hipLaunchKernelGGL(ttt::ttt_mlp_fwd_split_kernel<8>, dim3(2 * p.nbh), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
-  return hipGetLastError();
 }

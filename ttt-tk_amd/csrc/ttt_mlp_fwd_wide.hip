@@ -589,7 +589,7 @@ __global__ void ttt_mlp_fwd_wide_clear(int* w, int n, const int* report, uint4* 
 
 }  // namespace ttt
 
-hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream) {
+hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, int grid, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(ttt::ttt_mlp_fwd_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      ttt::SM_FWD_BYTES);
   if (e != hipSuccess) return e;
@@ -599,6 +599,6 @@ hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream)
   const int need = nx > n ? nx : n;
   hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n, p.report,
                      reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::FWD_XCHG_WORDS), nx);
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_kernel, dim3((p.nbh + 7) / 8 * 8 * (2 + p.n_out)), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
+  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_kernel, dim3(grid), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
   return hipGetLastError();
 }

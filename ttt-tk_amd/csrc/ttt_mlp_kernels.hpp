@@ -253,15 +253,39 @@ static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <=
 extern "C" void ttt_mlp_set_stage_clocks(unsigned* forward, unsigned* backward);
 #endif
 
-// p.sync == nullptr: one workgroup per (batch, head); otherwise two (state recurrence / output branch).
-hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, hipStream_t stream);
-// The recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
-hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, hipStream_t stream);
+// The kernels that do a call's work: one is compiled per combination of roles.  X(number, kernel); the kernel's text is also its name
+// in a trace.
+#define TTT_FWD_KERNELS(X) \
+  X(FWD_ONE, ttt_mlp_fwd_kernel) X(FWD_SPLIT_8, ttt_mlp_fwd_split_kernel<8>) X(FWD_SPLIT_32, ttt_mlp_fwd_split_kernel<32>)
+#define TTT_FWD_WIDE_KERNELS(X) X(FWD_WIDE, ttt_mlp_fwd_wide_kernel)
+#define TTT_BWD_KERNELS(X) \
+  X(BWD_ONE, ttt_mlp_bwd_kernel) X(BWD_HELPED, ttt_mlp_bwd_helped_kernel) \
+  X(BWD_SPLIT_1, ttt_mlp_bwd_split_kernel<1>) X(BWD_SPLIT_2, ttt_mlp_bwd_split_kernel<2>)
+#define TTT_BWD_GANG_KERNELS(X)                                                                                                    \
+  X(BWD_GANG_AHEAD, ttt_mlp_bwd_gang_kernel<true, true, true, true, true>)                                                         \
+  X(BWD_GANG_PARTS, ttt_mlp_bwd_gang_kernel<true, false, false, true, true>)                                                       \
+  X(BWD_GANG_WIDE, ttt_mlp_bwd_gang_kernel<true, false, false, true, false>)                                                       \
+  X(BWD_GANG_WIDE_SHARED, ttt_mlp_bwd_gang_kernel<true, false, false, false, false>)                                               \
+  X(BWD_GANG, ttt_mlp_bwd_gang_kernel<false, true, false, true, false>)                                                            \
+  X(BWD_GANG_SHARED, ttt_mlp_bwd_gang_kernel<false, true, false, false, false>)
+#define TTT_KERNEL_NUMBER(number, ...) number,
+enum TttKernel {
+  TTT_FWD_KERNELS(TTT_KERNEL_NUMBER) TTT_FWD_WIDE_KERNELS(TTT_KERNEL_NUMBER)
+  TTT_BWD_KERNELS(TTT_KERNEL_NUMBER) TTT_BWD_GANG_KERNELS(TTT_KERNEL_NUMBER)
+};
+#undef TTT_KERNEL_NUMBER
+// A case of a switch over TttKernel.
+#define TTT_KERNEL_LAUNCH(number, ...) case number: return launch(ttt::__VA_ARGS__);
+// `grid` workgroups of `kernel`, behind a small kernel that clears the synchronisation words where p.sync is set.  FWD_ONE, FWD_SPLIT_*: one
+// workgroup per (batch, head), or two (state recurrence / output branch).
+hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
+// FWD_WIDE: the recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
+hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, int grid, hipStream_t stream);
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
-// p.sync == nullptr: one workgroup per (batch, head); otherwise two (replay / reverse walk).
-hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, hipStream_t stream);
-// Gangs: p.gang_pairs pairs per XCD, walked by one or two workgroups each (p.wide), and workgroups that serve all of them.
-hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, hipStream_t stream);
+// BWD_ONE, BWD_HELPED, BWD_SPLIT_*: one workgroup per (batch, head), with helpers, or two or three (replays / reverse walk).
+hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
+// BWD_GANG*: p.gang_pairs pairs per XCD, walked by one or two workgroups each (p.wide), and workgroups that serve all of them.
+hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
 // Replays checkpoint group 0 and writes the sixteen per-group tensors row-major (side path, one workgroup per pair).
 hipError_t ttt_mlp_export_group0_enqueue(const ttt::BwdParams& p, hipStream_t stream);
 extern "C" int ttt_mlp_fwd_lds_bytes();

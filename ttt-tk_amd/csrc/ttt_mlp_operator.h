@@ -30,6 +30,14 @@ int ttt_mlp_launch_reporting(int which, const void* args, void* workspace, size_
  * one.  For tests: same results, slower. */
 int ttt_mlp_launch_scattered(int which, const void* args, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The kernels that a forward (which = 0) or backward (1) of this shape enqueues on a device with `compute_units` CUs, in order and
+ * without the small ones that clear words: the name of number `index` as a trace has it, NULL from the first one on that there is not.  *workgroups:
+ * the most of one dispatch; *dispatches: how many of it in a row (more than one: sequences cut at checkpoints); *resident: 1 if its workgroups
+ * wait for others that may not have started, so that all of them have to fit the device at once.  with_workspace as in ttt_mlp_segment_plan, 1: of
+ * the size that ttt_mlp_*_workspace_bytes() say.  Any of the pointers may be NULL.  No device needed. */
+const char* ttt_mlp_launched_kernel(int which, long long pairs, int compute_units, int NC, int checkpoint_group_size, int with_workspace,
+                                    int index, long long* workgroups, int* dispatches, int* resident);
+
 #ifdef __cplusplus
 }
 #endif

@@ -53,6 +53,16 @@ def test_groups_replayed_by_helpers_are_bit_identical(NH, NC, cgs, cus):
         ext.set_compute_units(0)
 
 
+@pytest.mark.parametrize("NH", [129, 200])
+def test_sets_of_helpers_hold_what_a_helper_writes(NH):
+    """Two further sets of five images, four tiles and a vector per mini-batch of a group: the GELU images of the other launches have no
+    place in them."""
+    from test_overlapped_abi_gpu import _lib
+    lib = _lib()
+    for cgs in (4, 16, 64):
+        assert lib.ttt_mlp_bwd_workspace_bytes(1, NH, 2 * cgs) - lib.ttt_mlp_bwd_workspace_bytes(1, NH, cgs) == NH * cgs * 2 * (5 * 32768 + 4 * 8192 + 256)
+
+
 @pytest.mark.parametrize("NH,NC,cgs", [(136, 24, 4), (200, 30, 3)])
 def test_a_pair_that_gives_up_ends_the_launch(NH, NC, cgs):
     """A pair that stops waiting for a taken group ends the launch with an error; a helper that stops waiting for one to take only leaves."""

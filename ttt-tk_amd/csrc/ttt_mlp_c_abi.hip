@@ -473,9 +473,10 @@ struct BwdWorkspace {
     const size_t tile = TTT_MLP_CS * TTT_MLP_F * 2, img = TTT_MLP_CS * TTT_MLP_HID * 2, vec = TTT_MLP_CS * 4;
     const size_t norm = (size_t)n * 8 * 2 * TTT_MLP_F * sizeof(float);
     // per set: X2, Z1, Z1_bar, X2_bar (images), gZ2 (tile), gZ1 (image), x_hat_fused, g_x_hat_fused, g_out_fused
-    // (tiles), std_fused, W1_init (two images per slot)
+    // (tiles), std_fused, W1_init (two images per slot: GELU' and GELU'', which helpers leave to the walk: 200 pairs in groups
+    // of 64 without it 4.7 instead of 6.3 GiB)
     const size_t per_set[PER_SET] = {slot * img, slot * img, slot * img, slot * img, slot * tile, slot * img,
-                                     slot * tile, slot * tile, slot * tile, slot * vec, slot * 2 * img};
+                                     slot * tile, slot * tile, slot * tile, slot * vec, pl.helpers > 0 ? 0 : slot * 2 * img};
     size_t o = 0;
     auto put = [&](int i, size_t bytes) { off[i] = o; o += (bytes + 255) & ~(size_t)255; };
     put(0, ttt::bwd_sync_ints(n) * sizeof(int));
@@ -652,7 +653,8 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
     p.alt_grad_x_hat_fused_group[s] = reinterpret_cast<__bf16*>(base + o[7]) - b0 * tile;
     p.alt_grad_output_fused_group[s] = reinterpret_cast<__bf16*>(base + o[8]) - b0 * tile;
     p.alt_std_fused_group[s] = reinterpret_cast<float*>(base + o[9]) - b0 * vec;
-    p.alt_W1_init_group[s] = reinterpret_cast<float*>(base + o[10]) - b0 * img;   // [cgs][64][256] floats = 2 images per slot
+    // [cgs][64][256] floats = 2 images per slot; not in the sets of helpers, and not touched by them
+    p.alt_W1_init_group[s] = pl.helpers > 0 ? p.W1_init_group : reinterpret_cast<float*>(base + o[10]) - b0 * img;
   }
   if (pl.helpers > 0) {
     p.help_sets[0] = {p.X2_group, p.Z1_group, p.Z1_bar_group, p.X2_bar_group, p.grad_l_wrt_Z2_group, p.grad_l_wrt_Z1_group,

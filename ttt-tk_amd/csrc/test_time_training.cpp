@@ -8,10 +8,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
-#include <mutex>
-#include <vector>
-
 #include "ttt_mlp_operator.h"
+#include "ttt_mlp_report.hpp"
 
 namespace {
 
@@ -52,50 +50,6 @@ std::string gave_up_text() {
          "compute units available to this launch?); the outputs are invalid - set_overlap(False) avoids the mode";
 }
 
-// Ints in host memory that the device writes when a wait gives up, so that after its own wait for the stream the host knows without
-// a copy from the device (a second wait: forward of 2 pairs x 4 mini-batches 75.3 us with it, 62.8 us so).  One block, allocated at the first
-// launch that needs one and kept for the process; word 0 collects the launches that nobody waits for, the others serve one
-// waiting call each.
-struct ReportWords {
-  static constexpr int WORDS = 64, STRIDE = 16;   // ints; a cache line each
-  std::mutex mutex;
-  int* block = nullptr;
-  bool asked = false;
-  std::vector<int> unused;
-  bool ready() {   // (mutex held)
-    if (!asked) {
-      asked = true;
-      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // the caller may be recording a graph
-      (void)hipThreadExchangeStreamCaptureMode(&mode);
-      void* p = nullptr;
-      if (hipHostMalloc(&p, WORDS * STRIDE * sizeof(int), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
-        block = static_cast<int*>(p);
-        for (int i = 0; i < WORDS * STRIDE; i++) block[i] = 0;
-        for (int i = 1; i < WORDS; i++) unused.push_back(i);
-      } else {
-        (void)hipGetLastError();
-      }
-      (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-    return block != nullptr;
-  }
-  int* collecting() {
-    const std::lock_guard<std::mutex> lock(mutex);
-    return ready() ? block : nullptr;
-  }
-  int* take() {   // nullptr: none left
-    const std::lock_guard<std::mutex> lock(mutex);
-    if (!ready() || unused.empty()) return nullptr;
-    int* const w = block + unused.back() * STRIDE;
-    unused.pop_back();
-    __atomic_store_n(w, 0, __ATOMIC_RELAXED);
-    return w;
-  }
-  void give(int* w) {
-    const std::lock_guard<std::mutex> lock(mutex);
-    unused.push_back(static_cast<int>(w - block) / STRIDE);
-  }
-};
 ReportWords& report_words() {
   static ReportWords* const words = new ReportWords;   // (not destroyed: launches may outlive the end of main)
   return *words;
@@ -103,18 +57,16 @@ ReportWords& report_words() {
 int g_unwaited_device = -1;   // of the last launch with several workgroups per pair that nobody waited for
 
 // A launch with several workgroups per (batch, head): enqueued by `launch(report word)`, waited for and checked unless the host
-// does not wait.  `status`: device address of the launch's status word.
+// does not wait (`waits`, and then report_words().serves(waits) holds).  `status`: device address of the launch's status word.
 template <class Launch>
-void run_overlapped(Launch launch, hipStream_t stream, const char* what, const torch::Device& dev, const void* status) {
+void run_overlapped(Launch launch, bool waits, hipStream_t stream, const char* what, const torch::Device& dev, const void* status) {
   struct Word {
     int* w;
     ~Word() { if (w != nullptr) report_words().give(w); }
-  } word{g_synchronize ? report_words().take() : nullptr};
-  int* const collecting = g_synchronize ? nullptr : report_words().collecting();
-  TORCH_CHECK(g_synchronize || collecting != nullptr, what, ": no host memory for the status of a launch that is not waited for");
-  const int rc = launch(g_synchronize ? word.w : collecting);
+  } word{waits ? report_words().take() : nullptr};
+  const int rc = launch(waits ? word.w : report_words().collecting());
   TORCH_CHECK(rc == TTT_MLP_OK, what, " launch failed: ", ttt_mlp_error_string(rc));
-  if (!g_synchronize) {
+  if (!waits) {
     g_unwaited_device = dev.index();
     return;
   }
@@ -137,7 +89,7 @@ void finish(int rc, hipStream_t stream, const char* what) {
 // blocks) for.  They are used only if their workspace fits comfortably into what the device has free
 // (memory held by torch's caching allocator counts as free for torch, so this is conservative).  A small one (a thousandth of
 // 288 GB) is not worth the question (the same forward 62.8 us with it, 52.6 us without): it is there, or the allocator says
-// that it is not.
+// that it is not (after giving back blocks that nothing uses).
 constexpr size_t SMALL_WORKSPACE = (size_t)256 << 20;
 bool workspace_is_affordable(size_t bytes) {
   if (bytes <= SMALL_WORKSPACE) return bytes > 0;
@@ -220,16 +172,17 @@ torch::Tensor ttt_forward(const torch::Tensor XQ, const torch::Tensor XK, const 
   a.B = (int32_t)B; a.NH = (int32_t)NH; a.NC = (int32_t)NC; a.K = (int32_t)K;
   const c10::DeviceGuard guard(XQ.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(XQ.device().index()).stream();
+  const bool waits = g_synchronize;
   // With few (batch, head) pairs most CUs would idle: then further workgroups per pair compute Out behind
   // the state recurrence.  Its workspace: the caller's (set_workspace) or torch's caching allocator's.
   // (more pairs than CUs and sequences that the launcher cuts at checkpoints: one workgroup each, no workspace)
-  const size_t ws_bytes = (g_overlap && NC >= 2 && !sequences_cut(0, B * NH, NC, checkpoint_group_size))
+  const size_t ws_bytes = (g_overlap && NC >= 2 && !sequences_cut(0, B * NH, NC, checkpoint_group_size) && report_words().serves(waits))
                               ? ttt_mlp_fwd_workspace_bytes((int32_t)B, (int32_t)NH) : 0;
   const Workspace ws = take_workspace(ws_bytes, XQ.device());
   if (ws.ptr != nullptr) {
     g_last_forward_mode = 1;
     const char* status = static_cast<const char*>(ws.ptr) + ttt_mlp_fwd_status_offset((int32_t)B, (int32_t)NH);
-    run_overlapped([&](int* report) { return ttt_mlp_launch_reporting(0, &a, ws.ptr, ws_bytes, report, stream); }, stream, "ttt_forward",
+    run_overlapped([&](int* report) { return ttt_mlp_launch_reporting(0, &a, ws.ptr, ws_bytes, report, stream); }, waits, stream, "ttt_forward",
                    XQ.device(), status);
   } else {
     g_last_forward_mode = 0;
@@ -335,11 +288,12 @@ torch::Tensor ttt_backward(
   a.overwrite = g_accumulate ? 0 : 1;
   const c10::DeviceGuard guard(XQ.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(XQ.device().index()).stream();
+  const bool waits = g_synchronize;
   // With few (batch, head) pairs most CUs would idle: then further workgroups per pair recompute the
   // checkpoint groups ahead of the reverse walk.  Its workspace (further sets of the per-group tensors): the
   // caller's (set_workspace) or torch's caching allocator's.
   size_t least = 0, ws_bytes = 0;
-  if (g_overlap && K >= 2 && !sequences_cut(1, B * NH, NC, checkpoint_group_size))
+  if (g_overlap && K >= 2 && !sequences_cut(1, B * NH, NC, checkpoint_group_size) && report_words().serves(waits))
     (void)ttt_mlp_bwd_workspace_range((int32_t)B, (int32_t)NH, checkpoint_group_size, (int32_t)K, &least, &ws_bytes);
   Workspace ws = take_workspace(ws_bytes, XQ.device());
   if (ws.ptr == nullptr && least < ws_bytes) ws = take_workspace(ws_bytes = least, XQ.device());   // fewer sets before one workgroup per pair
@@ -349,7 +303,7 @@ torch::Tensor ttt_backward(
     run_overlapped([&](int* report) {
       const int rc = ttt_mlp_launch_reporting(1, &a, ws.ptr, ws_bytes, report, stream);
       return rc == 0 && g_fill_group_tensors ? ttt_mlp_bwd_export_group0(&a, stream) : rc;
-    }, stream, "ttt_backward", XQ.device(), status);
+    }, waits, stream, "ttt_backward", XQ.device(), status);
   } else {
     g_last_backward_mode = 0;
     int rc = ttt_mlp_bwd_launch(&a, stream);

@@ -484,7 +484,8 @@ TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
 // WIDE: the walk runs on two workgroups (ttt_mlp_bwd_wide.hip), which say separately how far they are.
 // PARTS: several workgroups at once replay each of the p.n_shared groups walked first, a stretch of its mini-batches each.
 // HELPED: a workgroup that replays and walks (ROLE 0) where others (ROLE 1) replay groups ahead of it.
-template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false, bool HELPED = false>
+// EIGHTHS: a replay hands over its norm-gradient sums by eighths of the group (eighth_done); needed with PARTS.
+template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false, bool HELPED = false, bool EIGHTHS = PARTS>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; ROLE 2: K - 1 .. 0).
 // part (PARTS): which of the p.n_parts stretches of the group's mini-batches this workgroup replays; it takes the state there from
 // the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).  HELPED: the set it is replayed into.
@@ -988,15 +989,24 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier
         }
       }
-      // The norm-gradient sums of an eighth of the group go out on their own, at the top of the next one, where their stores have a
-      // whole mini-batch to arrive (of one workgroup per (batch, head) the last eighth's stay in LDS).
-      auto eighth_out = [&](int e) {
+      // The norm-gradient sums of an eighth of the group end at the top of the next one.  Where a group may be replayed in parts they go
+      // out on their own, otherwise they are added up here, in the same order, and one sum goes out with the group: two registers (which
+      // spill) instead of two stores an eighth and of as many trips to HBM for whoever adds them (ms: 96 x 64 in groups of 8 1.443 ->
+      // 1.427, 72 x 64 in 4 1.417 -> 1.366, 51 x 77 in 10 1.205 -> 1.183, 128 x 128 in 16 3.207 -> 3.179).  Of one workgroup per (batch, head)
+      // they go out, and the last eighth's stay in LDS.
+      float sum0 = 0.f, sum1 = 0.f;
+      auto eighth_done = [&](int e) {
         WAVE_SYNC();
         LANE_VARS;
-        const gptr_t g = ROLE == 1 ? group_sums(set, e) : park();
-        const unsigned o = ROLE == 1 ? 4 * lane : np_off(), so = ROLE == 1 ? 0 : (2 + e) * PARK_BYTES;
-        g_stf(g, o, so, s_dgw[lane]);
-        g_stf(g, o, so + FD * 4, s_dbw[lane]);
+        if constexpr (ROLE == 1 && !EIGHTHS) {
+          sum0 = e > 0 ? sum0 + s_dgw[lane] : s_dgw[lane];
+          sum1 = e > 0 ? sum1 + s_dbw[lane] : s_dbw[lane];
+        } else {
+          const gptr_t g = ROLE == 1 ? group_sums(set, e) : park();
+          const unsigned o = ROLE == 1 ? 4 * lane : np_off(), so = ROLE == 1 ? 0 : (2 + e) * PARK_BYTES;
+          g_stf(g, o, so, s_dgw[lane]);
+          g_stf(g, o, so + FD * 4, s_dbw[lane]);
+        }
         s_dgw[lane] = 0.f;
         s_dbw[lane] = 0.f;
         WAVE_SYNC();
@@ -1009,7 +1019,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         __syncthreads();   // the staged inputs (and, for j = 0, the biases) are visible
         TTT_STAGE(BS_R_TOP);
         if (j == e_end) {
-          eighth_out(e++);
+          eighth_done(e++);
           e_end += eighth;
         }
         if (PARTS && j == j_first && j > 0) tile_to_lds<CPOL_NT>(bXQ, mb * TILE_BYTES, smem + SB_XQ, v, lane);   // XK was there until now
@@ -1204,7 +1214,13 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier at the loop's top
         TTT_STAGE(BS_R_OUT_BACKWARD);
       }
-      if constexpr (ROLE == 1) eighth_out(e);
+      if constexpr (ROLE == 1) eighth_done(e);
+      if constexpr (ROLE == 1 && !EIGHTHS) {
+        LANE_VARS;
+        const gptr_t g = group_sums(set, 0);
+        g_stf(g, 4 * lane, 0, sum0);
+        g_stf(g, 4 * lane, FD * 4, sum1);
+      }
       // running gradients back into registers
       if constexpr (ROLE == 0) {
         LANE_VARS;
@@ -1256,13 +1272,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       LANE_VARS;
       const gptr_t g = park();
       const unsigned o = (v * 2 * FD + lane) * 4;
-      const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4);   // under way with the sums
-      float a0 = 0.f, a1 = 0.f;
-      for (int e = 0; e * eighth < n_mb; e++) {
-        const gptr_t gs = group_sums(set, e);
-        a0 = e > 0 ? a0 + g_ldf(gs, 4 * lane, 0) : g_ldf(gs, 4 * lane, 0);
-        a1 = e > 0 ? a1 + g_ldf(gs, 4 * lane, FD * 4) : g_ldf(gs, 4 * lane, FD * 4);
-      }
+      const gptr_t gs = group_sums(set, 0);
+      const float r0 = g_ldf(g, o, 0), r1 = g_ldf(g, o, FD * 4), a0 = g_ldf(gs, 4 * lane, 0), a1 = g_ldf(gs, 4 * lane, FD * 4);
       g_stf(g, o, 0, r0 + a0);
       g_stf(g, o, FD * 4, r1 + a1);
     };
@@ -1765,8 +1776,8 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_kernel(const BwdParams
 // the hidden dimension, + g_y, accumulated into grad_L_XK.  Same wave / lane roles and the same order of every
 // sum as in the walk, so the result is the same to the bit.  OWN: the whole sequence (k_hi = K - 1); otherwise fewer such
 // workgroups than pairs take the groups in turn and this is group k_hi, with what is carried from group to group (the copy of
-// the gradient wrt W1 and the norm-gradient sums) parked in between.  False: a wait gave up.
-template <bool IMG, bool WIDE, bool OWN>
+// the gradient wrt W1 and the norm-gradient sums) parked in between.  EIGHTHS: as in the replay.  False: a wait gave up.
+template <bool IMG, bool WIDE, bool OWN, bool EIGHTHS>
 TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int bh, const int k_hi) {
   float* s_P = reinterpret_cast<float*>(smem + SB_P);
   int tid = threadIdx.x;
@@ -1914,11 +1925,11 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
         if (!wait_at_least(w_sync + 12, n_mb - (j & ~(FIN_CHUNK - 1)), p.status, s_flag, p.wait_limit)) return false;
         TTT_STAGE(BS_X_GROUP);
       }
-      if (j == n_mb - 1) {   // the group's norm-gradient sums, by eighths: published with it, and the walk has acquired it
+      if (j == n_mb - 1) {   // the group's norm-gradient sum, or its eighths': published with it, and the walk has acquired it
         const float* np = p.norm_partial + ((size_t)bh * BWD_MAX_SETS + set) * (8 * BW_NWAVE * 2 * FD) + v * 2 * FD + lane;
         const int eighth = (cgs + 7) / 8;
         float a0 = np[0], a1 = np[FD];
-        for (int e = 1; e * eighth < n_mb; e++) {
+        for (int e = 1; EIGHTHS && e * eighth < n_mb; e++) {
           a0 += np[e * (BW_NWAVE * 2 * FD)];
           a1 += np[e * (BW_NWAVE * 2 * FD) + FD];
         }

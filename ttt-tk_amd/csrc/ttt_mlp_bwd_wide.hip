@@ -793,6 +793,8 @@ TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const in
 template <bool WIDE, bool IMG, bool PREFETCH, bool OWN, bool PARTS>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  // (57 to 64 pairs wait for their walks: the stores of the eighths cost them nothing, registers for the sum do: 64 x 128 2.231 ms so, 2.245 with them)
+  constexpr bool EIGHTHS = PARTS || (!WIDE && OWN);
   const int b = blockIdx.x, walkers = (WIDE ? 2 : 1) * p.gang_pairs;
   const int slots = walkers + p.n_finish + p.n_replay + (PREFETCH ? p.gang_pairs : 0);
   const int gang = uni(p.scatter ? b / slots : b & 7);   // (a division leaves its result in a vector register)
@@ -836,17 +838,17 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
         before = shared;
       }
       const int q = uni(n / pairs), k = uni(p.K - 1 - (before + q));
-      if (!bwd_body<1, IMG, true, WIDE, PARTS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
+      if (!bwd_body<1, IMG, true, WIDE, PARTS, false, EIGHTHS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
     }
   }
   if constexpr (OWN) {
-    if (!replays && slot < pairs) bwd_finish_dxk<IMG, WIDE, true>(p, smem, bh0 + 8 * slot, p.K - 1);
+    if (!replays && slot < pairs) bwd_finish_dxk<IMG, WIDE, true, EIGHTHS>(p, smem, bh0 + 8 * slot, p.K - 1);
   } else {
     // (n_replay >= pairs: one of the last groups each)
     const int last = (p.K - 1) * pairs, end = replays ? last + pairs : last;
     for (int job = replays ? last + r : slot; job < end; job += replays ? p.n_replay : p.n_finish) {
       const int done = uni(job / pairs);
-      if (!bwd_finish_dxk<IMG, WIDE, false>(p, smem, bh0 + 8 * (job - done * pairs), p.K - 1 - done)) return;
+      if (!bwd_finish_dxk<IMG, WIDE, false, EIGHTHS>(p, smem, bh0 + 8 * (job - done * pairs), p.K - 1 - done)) return;
     }
   }
 }

@@ -80,7 +80,9 @@ struct BwdParams {
   __bf16 *alt_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_x_hat_fused_group[BWD_MAX_SETS - 1], *alt_grad_output_fused_group[BWD_MAX_SETS - 1];
   float* alt_std_fused_group[BWD_MAX_SETS - 1];
   float* alt_W1_init_group[BWD_MAX_SETS - 1];
-  float* norm_partial;   // [B*NH][BWD_MAX_SETS][8][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set, by eighths of it
+  // [B*NH][BWD_MAX_SETS][8][8 waves][2][64]: the replay's share of the norm-weight / norm-bias gradients of the group in a set, by eighths
+  // of it (bwd_body's EIGHTHS), else their sum in the place of the first
+  float* norm_partial;
   float* norm_park;      // [B*NH][8 waves][2][64]: their sum over the groups walked so far (without a grad_L_XK workgroup)
   __bf16* walk_park;     // [B*NH][64][256]: one register image the walking workgroup parks across its LayerNorm stage
   // Gang (gang_pairs > 0: pairs per XCD, gang g = pairs g, g + 8, ..; ttt_mlp_bwd_wide.hip): n_replay workgroups replay for all of

@@ -269,9 +269,17 @@ def test_workgroups_that_wait_for_each_other_fit_the_device(lib):
     # the helpers take the CUs that one workgroup per pair leaves, where the groups go round
     assert _launched(lib, 1, 200, 256, 100, 16) == [("ttt_mlp_bwd_helped_kernel", 256, 1, 0)]
     assert _launched(lib, 1, 200, 256, 64, 32) == [("ttt_mlp_bwd_kernel", 200, 1, 0)]
-    # 51 pairs: all 32 CUs of an XCD work for its seven; groups too short for that: four whole workgroups each
+    # 51 pairs: all 32 CUs of an XCD work for its seven; groups too short for that: four whole workgroups each; so do two groups that 12
+    # replaying workgroups would take in two rounds
     assert _launched(lib, 1, 51, 256, 77, 10) == [("ttt_mlp_bwd_gang_kernel<true, false, false, false, false>", 256, 1, 1)]
-    assert _launched(lib, 1, 51, 256, 77, 3) == [("ttt_mlp_bwd_gang_kernel<false, true, false, true, false>", 224, 1, 1)]
+    whole = [("ttt_mlp_bwd_gang_kernel<false, true, false, true, false>", 224, 1, 1)]
+    assert _launched(lib, 1, 51, 256, 9, 1) == _launched(lib, 1, 56, 256, 107, 64) == _launched(lib, 1, 56, 256, 83, 48) == whole
+    # 65 to 80 pairs by what measures faster: a ragged group in four makes three and a half
+    gang, three = "ttt_mlp_bwd_gang_kernel<false, true, false, false, false>", "ttt_mlp_bwd_split_kernel<2>"
+    assert _launched(lib, 1, 80, 256, 256, 32) == [(gang, 256, 1, 1)] and _launched(lib, 1, 80, 256, 112, 32) == [(three, 240, 1, 1)]
+    assert _launched(lib, 1, 76, 256, 113, 32) == [(three, 228, 1, 1)]
+    assert _launched(lib, 1, 72, 256, 96, 6)[0][0] == "ttt_mlp_bwd_gang_kernel<false, true, false, true, false>"
+    assert _launched(lib, 1, 72, 256, 128, 64) == [(three, 216, 1, 1)]
     assert _launched(lib, 1, 8, 256, 64, 8) == [("ttt_mlp_bwd_gang_kernel<true, true, true, true, true>", 96, 1, 1)]
     assert _launched(lib, 1, 384, 256, 512, 32) == [("ttt_mlp_bwd_kernel", 256, 3, 0)]
     assert _launched(lib, 1, 48, 256, 512, 32, 0) == [("ttt_mlp_bwd_kernel", 48, 1, 0)]

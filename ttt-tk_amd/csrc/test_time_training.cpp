@@ -294,7 +294,7 @@ torch::Tensor ttt_backward(
   // caller's (set_workspace) or torch's caching allocator's.
   size_t least = 0, ws_bytes = 0;
   if (g_overlap && K >= 2 && !sequences_cut(1, B * NH, NC, checkpoint_group_size) && report_words().serves(waits))
-    (void)ttt_mlp_bwd_workspace_range((int32_t)B, (int32_t)NH, checkpoint_group_size, (int32_t)K, &least, &ws_bytes);
+    (void)ttt_mlp_bwd_workspace_for((int32_t)B, (int32_t)NH, checkpoint_group_size, (int32_t)NC, &least, &ws_bytes);
   Workspace ws = take_workspace(ws_bytes, XQ.device());
   if (ws.ptr == nullptr && least < ws_bytes) ws = take_workspace(ws_bytes = least, XQ.device());   // fewer sets before one workgroup per pair
   if (ws.ptr != nullptr) {

@@ -193,8 +193,12 @@ struct LaunchPlan {
   }
 };
 // Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
-// of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others.
+// of a mini-batch and its finishing; with the GELU family evaluated by the replay, and so not by the others; the walk of one on two CUs, on
+// one, and on one that does the finishing too.  Then what a group costs each role whatever its length (fitted, with the last of the walks, to
+// 273 calls of 49 to 80 pairs, groups of 1 to 64 and 2 to 16 of them).
 constexpr int COST_REPLAY = 443, COST_FINISH = 200, COST_REPLAY_IMG = 488, COST_FINISH_IMG = 185;
+constexpr int COST_WALK_WIDE = 215, COST_WALK = 330, COST_WALK_ALL = 400;
+constexpr int COST_GROUP_REPLAY = 550, COST_GROUP_WALK = 250, COST_GROUP_FINISH = 450;
 // `workers` of an XCD divided between replaying and finishing for its `pairs`, so that the slower of the two is as fast as can be;
 // a finishing workgroup for each pair, which then follows its walk closely, where the replay still keeps up with `walk`.
 void divide_workers(int pairs, int workers, int walk, int replay, int finish, int* n_replay, int* n_finish) {
@@ -282,9 +286,9 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
         pl.shared = 1;
       }
     } else if (pl.wide) {
-      divide_workers(pairs, on_xcd - 2 * pairs, 215, COST_REPLAY, COST_FINISH, &pl.n_replay, &pl.n_finish);
+      divide_workers(pairs, on_xcd - 2 * pairs, COST_WALK_WIDE, COST_REPLAY, COST_FINISH, &pl.n_replay, &pl.n_finish);
     } else {
-      divide_workers(pairs, on_xcd - pairs, 330, COST_REPLAY_IMG, COST_FINISH_IMG, &pl.n_replay, &pl.n_finish);
+      divide_workers(pairs, on_xcd - pairs, COST_WALK, COST_REPLAY_IMG, COST_FINISH_IMG, &pl.n_replay, &pl.n_finish);
     }
     pl.sets = 4;
     return pl;
@@ -407,29 +411,74 @@ LaunchPlan bwd_reduced(LaunchPlan pl) {
   }
   return pl;
 }
-// The launch for groups as short, or as few, as the sequence at hand has.  Finishing workgroups that take groups of several pairs in turn
-// park 72 KiB between two groups and end a whole group after the last walk, and the workgroups that serve a pair meet once a group; with
-// short groups whole workgroups for each pair are faster: with the walk on two CUs, up to 56 pairs, four with the walk on one (gang /
-// whole: groups of 1 1.20, of 2 1.03 - 1.13, of 4 0.93 - 1.00, of 16 0.85 - 0.95); of 65 to 80 pairs three, without finishing ones (80
-// pairs: 6 groups of 1 1.35, 8 of 4 1.10, 3 of 32 1.02, 4 of 16 1.01; 12 of 8 1.00, 8 of 12 0.97, 6 of 16 0.985, 4 of 32 0.98).
-LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K) {
+// Clocks, in hundreds, until a gang, or two replaying workgroups, one that walks and (`finish` > 0) one that finishes for one pair, is through
+// with a sequence: its jobs in their order, each as early as its workgroup and what it waits for allow.
+int backward_span(int pairs, int n_replay, int n_finish, bool wide, int walk, int replay, int finish, int NC, int cgs, int K) {
+  constexpr int SETS = 4;
+  int replaying[64] = {}, finishing[64] = {}, walked[64] = {}, walk_end[SETS][64] = {}, finished[SETS][64] = {}, span = 0;
+  const int groups = K < 16 ? K : 16;   // (longer: nothing new)
+  for (int g = 0; g < groups; g++) {
+    const int n = g == 0 ? NC - (K - 1) * cgs : cgs, now = g % SETS, last = (g + SETS - 1) % SETS, set = (g + SETS - 2) % SETS;
+    const bool own = n_finish == pairs, end = g == groups - 1;
+    int start[64];
+    for (int i = 0; i < pairs; i++) {   // (the set of `now` is free once the group that used it last is walked and finished)
+      int& w = replaying[(g * pairs + i) % n_replay];
+      const int free = walk_end[now][i] > finished[now][i] ? walk_end[now][i] : finished[now][i];
+      w = (w > free ? w : free) + COST_GROUP_REPLAY + n * replay;
+      start[i] = w > walked[i] ? w : walked[i];
+      if (finish > 0 && g >= 2 && finished[set][i] > start[i]) start[i] = finished[set][i];   // (two sets of what is handed over)
+      walked[i] = start[i] + COST_GROUP_WALK + n * walk;
+    }
+    for (int i = 0; i < pairs; i++) {
+      walk_end[now][i] = walked[i];
+      if (finish > 0) {   // behind the walk mini-batch by mini-batch where it says so each (on two CUs, and in the last group), else behind the group
+        int& w = own ? finishing[i] : end ? replaying[i % n_replay] : finishing[(g * pairs + i) % n_finish];
+        int t = g > 0 && finished[last][i] > w ? finished[last][i] : w;
+        const int from = wide || end ? start[i] : walked[i];
+        t = (t > from ? t : from) + n * finish;
+        if (t < walked[i] + finish) t = walked[i] + finish;
+        finished[now][i] = w = t + COST_GROUP_FINISH;
+      } else {
+        finished[now][i] = walked[i];
+      }
+      if (finished[now][i] > span) span = finished[now][i];
+    }
+  }
+  return span;
+}
+// The launch for groups as short, or as few, as the sequence at hand has.  Where workgroups that serve several pairs have to take another
+// round for what does not divide among them, or spend themselves on what a group costs whatever its length, whole ones for each pair are
+// faster: with the walk on two CUs and finishing workgroups that take turns (49 to 56 pairs) four with the walk on one, with the walk on
+// one CU and less than four per pair (65 to 80) three, without finishing ones.  (gang / whole, 56 pairs: groups of 1 1.16 - 1.21, 16 of 2 1.08, 6 of
+// 3 0.96, two of 64 and one of them half 1.05, five of 12 0.84; 72: 8 of 3 1.02, 16 of 6 0.93, two of 64 1.05, 12 of 16 0.95; 80: 16 of 6 1.04, three and
+// a half of 24 to 48 1.05 - 1.07, 5 of 16 0.99, 8 of 32 0.97.)  Of 273 such calls timed both ways the spans take the slower launch for 3 by
+// more than 1 %; with thresholds in group size and number it was 39, up to 7 %.
+LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K, long long NC) {
   if (cgs < 2) {   // no stretches to divide a group into
     pl.parts = 1;
     pl.shared = 0;
   }
-  const bool four = 4 * pl.gang <= cus / 8;
-  if (four && pl.wide && pl.n_finish < pl.gang && cgs < 4) {
+  const bool four = 4 * pl.gang <= cus / 8, shared = four ? pl.wide && pl.n_finish < pl.gang : pl.gang && !pl.wide;
+  if (!shared || cus / 8 > 64) return pl;
+  const int n = static_cast<int>(NC), c = static_cast<int>(cgs), k = static_cast<int>(K);
+  const int gang = pl.wide ? backward_span(pl.gang, pl.n_replay, pl.n_finish, true, COST_WALK_WIDE, COST_REPLAY, COST_FINISH, n, c, k)
+                           : backward_span(pl.gang, pl.n_replay, pl.n_finish, false, COST_WALK, COST_REPLAY_IMG, COST_FINISH_IMG, n, c, k);
+  const int whole = backward_span(1, 2, 1, false, four ? COST_WALK : COST_WALK_ALL, COST_REPLAY_IMG, four ? COST_FINISH_IMG : 0, n, c, k);
+  if (gang < whole) return pl;
+  if (four) {
     pl.wide = false;
     pl.n_finish = pl.gang;
     pl.n_replay = 2 * pl.gang;
-  } else if (!four && !pl.wide && pl.gang && (cgs < 8 || K < 4 || cgs * K < 90)) {
+  } else {
     pl.gang = pl.n_finish = 0;
     pl.n_replay = 2;
   }
   return pl;
 }
 // The launch of a backward call with a workspace.
-LaunchPlan plan_bwd(long long pairs, int cus, long long cgs, long long K) { return bwd_for_groups(plan_for(pairs, cus, true), cus, cgs, K); }
+LaunchPlan plan_bwd(long long pairs, int cus, long long cgs, long long NC) {
+  return bwd_for_groups(plan_for(pairs, cus, true), cus, cgs, (NC + cgs - 1) / cgs, NC);
+}
 // What a call enqueues to do its work: sequences cut into segments, a device's worth of them at a time, or `n` kernels in a row.
 struct Call {
   SegmentPlan seg;
@@ -543,16 +592,27 @@ extern "C" size_t ttt_mlp_bwd_workspace_bytes(int B, int NH, int checkpoint_grou
   return pl.waits() ? BwdWorkspace(pl, checkpoint_group_size, ttt::BWD_MAX_SETS).total : 0;
 }
 
+namespace {
+void bwd_range(const LaunchPlan& pl, long long cgs, long long K, size_t* least, size_t* most) {
+  *least = *most = 0;
+  if (!pl.waits() || (pl.helpers > 0 && !helpers_pay(pl, K))) return;
+  *least = BwdWorkspace(bwd_reduced(pl), cgs, K).total;
+  *most = BwdWorkspace(pl, cgs, K).total;
+}
+}  // namespace
+
 extern "C" int ttt_mlp_bwd_workspace_range(int B, int NH, int checkpoint_group_size, int K, size_t* least, size_t* most) {
   if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || K <= 0)
     return TTT_MLP_ERR_BAD_ARG;
-  const LaunchPlan pl = plan_bwd((long long)B * NH, device_cus(), checkpoint_group_size, K);
-  if (pl.helpers > 0 && !helpers_pay(pl, K)) {
-    *least = *most = 0;
-    return TTT_MLP_OK;
-  }
-  *least = pl.waits() ? BwdWorkspace(bwd_reduced(pl), checkpoint_group_size, K).total : 0;
-  *most = pl.waits() ? BwdWorkspace(pl, checkpoint_group_size, K).total : 0;
+  bwd_range(plan_launches((long long)B * NH, true), checkpoint_group_size, K, least, most);
+  return TTT_MLP_OK;
+}
+
+extern "C" int ttt_mlp_bwd_workspace_for(int B, int NH, int checkpoint_group_size, int NC, size_t* least, size_t* most) {
+  if (least == nullptr || most == nullptr || B <= 0 || NH <= 0 || checkpoint_group_size <= 0 || checkpoint_group_size > (1 << 16) || NC <= 0)
+    return TTT_MLP_ERR_BAD_ARG;
+  bwd_range(plan_bwd((long long)B * NH, device_cus(), checkpoint_group_size, NC), checkpoint_group_size,
+            ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size, least, most);
   return TTT_MLP_OK;
 }
 
@@ -578,7 +638,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   if (int rc = make_bwd_params(a, p)) return rc;
   if (int rc = check_workspace(workspace)) return rc;
   const int cus = device_cus();
-  LaunchPlan pl = plan_bwd((long long)p.B * p.NH, cus, p.cgs, p.K);
+  LaunchPlan pl = plan_bwd((long long)p.B * p.NH, cus, p.cgs, p.NC);
   if (!pl.waits()) return TTT_MLP_ERR_NO_ROOM;
   if (workspace_bytes < BwdWorkspace(pl, p.cgs, p.K).total) pl = bwd_reduced(pl);
   const BwdWorkspace w(pl, p.cgs, p.K);
@@ -855,7 +915,10 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
   if (segment_minibatches == nullptr || launches == nullptr || pairs <= 0 || compute_units <= 0 || NC <= 0 ||
       checkpoint_group_size <= 0 || (which != 0 && which != 1))
     return TTT_MLP_ERR_BAD_ARG;
-  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size)
+  *segment_minibatches = 0;
+  *launches = 1;
+  if (pairs <= compute_units) return TTT_MLP_OK;   // (asked ahead of every call of the operators)
+  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, NC)
                                    : plan_for(pairs, compute_units, false);
   const Call call = plan_call(which == 1, pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0);
   *segment_minibatches = call.seg.seg_len;
@@ -866,7 +929,7 @@ extern "C" int ttt_mlp_segment_plan(int which, long long pairs, int compute_unit
 extern "C" const char* ttt_mlp_launched_kernel(int which, long long pairs, int compute_units, int NC, int checkpoint_group_size, int with_workspace,
                                                int index, long long* workgroups, int* dispatches, int* resident) {
   if (pairs <= 0 || compute_units <= 0 || NC <= 0 || checkpoint_group_size <= 0 || (which != 0 && which != 1) || index < 0) return nullptr;
-  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, ((long long)NC + checkpoint_group_size - 1) / checkpoint_group_size)
+  const LaunchPlan pl = which == 1 ? plan_bwd(pairs, compute_units, checkpoint_group_size, NC)
                                    : plan_for(pairs, compute_units, false);
   const Call call = plan_call(which == 1, pl, pairs, compute_units, NC, checkpoint_group_size, with_workspace != 0);
   if (index >= call.n) return nullptr;

@@ -1,5 +1,5 @@
 /* Entry points of libttt_mlp.so for the operator module in this folder and for the tests; not part of the C ABI in
- * include/ttt_mlp.h.  The first three let the operator take a workspace that fits the call at hand instead of one that fits
+ * include/ttt_mlp.h.  The first four let the operator take a workspace that fits the call at hand instead of one that fits
  * every call of its B, NH and checkpoint_group_size, and learn without a copy whether a wait gave up. */
 #ifndef TTT_MLP_OPERATOR_H_
 #define TTT_MLP_OPERATOR_H_
@@ -13,10 +13,12 @@ extern "C" {
 /* Workspace of the backward over a sequence of K checkpoint groups.  ttt_mlp_bwd_workspace_bytes() serves every length, with a set of
  * per-group tensors for each group that may be under way at once; a short sequence has fewer groups than that.  *most: the
  * launch of the plan; *least: the launch with the fewest sets (two workgroups that recompute instead of three or four;
- * the same as *most where the plan has no more than two).  Both 0 when the mode does not apply. */
+ * the same as *most where the plan has no more than two).  Both 0 when the mode does not apply.  _for: over one of NC mini-batches, whose launch may
+ * be one that takes less. */
 int ttt_mlp_bwd_workspace_range(int32_t B, int32_t NH, int32_t checkpoint_group_size, int32_t K, size_t* least, size_t* most);
+int ttt_mlp_bwd_workspace_for(int32_t B, int32_t NH, int32_t checkpoint_group_size, int32_t NC, size_t* least, size_t* most);
 
-/* As ttt_mlp_bwd_launch_overlapped, with any workspace of at least *least bytes (ttt_mlp_bwd_workspace_range): the launch
+/* As ttt_mlp_bwd_launch_overlapped, with any workspace of at least *least bytes (ttt_mlp_bwd_workspace_range, _for): the launch
  * of the plan from *most bytes on, the one with fewer sets below.  Same results, bit for bit. */
 int ttt_mlp_bwd_launch_within(const ttt_mlp_bwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -1,6 +1,7 @@
 """The backward whose replaying and finishing workgroups serve several (batch, head) pairs, against the one-workgroup launch, bit
 for bit: gangs of unequal size, more and fewer groups than sets and workgroups, groups of one mini-batch, ragged and single
-groups, the pair counts at both ends of the walk on two CUs (49 to 56 pairs) and on one (57 to 80), and a wait that gives up."""
+groups, the pair counts at both ends of the walk on two CUs (49 to 56 pairs) and on one (57 to 80), and a wait that gives up.  Groups too
+short or few for that have whole workgroups for each pair, which are among the cases."""
 import ctypes
 
 import pytest
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("NH,NC,cgs,scatter", [(49, 9, 2, 0), (53, 7, 1, 1), (56, 25, 4, 0), (56, 3, 4, 0), (57, 5, 2, 0), (64, 6, 4, 0),
                                                (65, 9, 4, 0), (75, 11, 2, 0), (80, 8, 1, 1), (80, 2, 3, 0),
-                                               (53, 13, 4, 1), (55, 31, 10, 0), (65, 93, 8, 0), (72, 95, 24, 0), (80, 91, 10, 1), (80, 99, 30, 0)])
+                                               (53, 13, 4, 1), (55, 31, 10, 0), (65, 93, 8, 0), (72, 95, 24, 0), (80, 91, 10, 1), (80, 99, 30, 0),
+                                               (65, 36, 4, 1), (73, 97, 7, 1), (79, 130, 9, 0), (80, 160, 32, 0)])
 def test_shared_workgroups_are_bit_identical(NH, NC, cgs, scatter):
     import test_time_training as ext
     import ttt_mlp_host as host

@@ -174,14 +174,15 @@ def test_bench_names_the_kernels_that_run():
         (48, 4096, 64): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<true, false, false, true, false>"),
         (32, 512, 32): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<true, true, true, true, true>"),
         (40, 512, 32): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<true, false, false, true, true>"),
-        (51, 77, 10): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<true, false, false, false, false>"),
+        (51, 77, 10): ("ttt_mlp_fwd_wide_early_kernel", "ttt_mlp_bwd_gang_kernel<true, false, false, false, false>"),
         (64, 256, 16): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<false, true, false, true, false>"),
         (80, 256, 16): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_gang_kernel<false, true, false, false, false>"),
+        (24, 256, 16): ("ttt_mlp_fwd_wide_early_kernel", "ttt_mlp_bwd_gang_kernel<true, true, true, true, true>"),
         (80, 32, 4): ("ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_split_kernel<2>"),
         (96, 128, 16): ("ttt_mlp_fwd_split_kernel<8>", "ttt_mlp_bwd_split_kernel<1>"),
         (128, 512, 32): ("ttt_mlp_fwd_split_kernel<32>", "ttt_mlp_bwd_split_kernel<1>"),
         (200, 100, 16): ("ttt_mlp_fwd_kernel", "ttt_mlp_bwd_helped_kernel"),
-        (260, 64, 64): ("ttt_mlp_fwd_kernel + ttt_mlp_fwd_wide_kernel", "ttt_mlp_bwd_kernel + ttt_mlp_bwd_gang_kernel<true, true, true, true, true>"),
+        (260, 64, 64): ("ttt_mlp_fwd_kernel + ttt_mlp_fwd_wide_early_kernel", "ttt_mlp_bwd_kernel + ttt_mlp_bwd_gang_kernel<true, true, true, true, true>"),
         (384, 512, 32): ("ttt_mlp_fwd_kernel x 3 (sequences cut at checkpoints)", "ttt_mlp_bwd_kernel x 3 (sequences cut at checkpoints)")}
     for (pairs, NC, cgs), names in shapes.items():
         assert tuple(bench.launched_kernel(which, pairs, NC, cgs, 256, True) for which in (0, 1)) == names

@@ -172,7 +172,8 @@ struct LaunchPlan {
   }
   // The launch behind the full rounds of one workgroup per pair: its kernel and its workgroups.
   TttKernel kernel(bool backward, int NC) const {
-    if (!backward) return wide ? FWD_WIDE : NC >= 512 ? FWD_SPLIT_32 : FWD_SPLIT_8;   // (mini-batches per hand-over)
+    if (!backward && wide) return n_out == 2 && NC <= 256 && n_rest * NC <= 6144 ? FWD_WIDE_EARLY : FWD_WIDE;   // (ttt_mlp_fwd_wide.hip)
+    if (!backward) return NC >= 512 ? FWD_SPLIT_32 : FWD_SPLIT_8;   // (mini-batches per hand-over)
     if (helpers > 0) return BWD_HELPED;
     if (!gang) return n_replay == 2 ? BWD_SPLIT_2 : BWD_SPLIT_1;
     const bool own = n_finish == gang;
@@ -801,7 +802,7 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
     p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
     p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
     p.scatter = scatter ? 1 : 0;
-    return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, grid, static_cast<hipStream_t>(stream)));
+    return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
   }
   p.ring_log2 = kernel == FWD_SPLIT_32 ? 5 : 3;
   p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * 2 * ttt::FWD_RING_MAX * (ttt::FWD_IMG_BYTES / 2);

@@ -17,10 +17,12 @@
 // mini-batch), 24 x 256 1.49 ms.  With the stage clocks in, 13.9 k clocks: block 0's GELU and partial sums 2.4 k; block 1's 3.7 k
 // while block 0's sums cross (gather and send 1.3 k, 0.9 k under way, LayerNorm 1.7 k) and 0.45 k of waiting for them;
 // block 0's weight step 2.1 k while block 1's sums cross and 2.25 k of waiting for those; block 1's weight step, the
-// split of the new state and Z1 of the next block 0 2.9 k.  (Before Z1 was started under that split, and with the token
-// sums for b2 and the wait for a free ring slot between the exchanges, 14.2 k: 24 x 256 1.53 ms, 12 x 64 396 us, now 383.)
-// From 40 pairs on the shorter chain is paid back in clock rate: 48 x 256 1.59 -> 1.56 ms one call at a time, 1.545 and 1.55 back to back,
-// 64 x 256 (every CU busy) 1.55 -> 1.58 back to back, 64 x 32 and 80 x 256 no change.
+// split of the new state and Z1 of the next block 0 2.9 k.  With the token sums for b2 and the wait for a free ring slot between the
+// exchanges it was 12 x 64 399 us, now 379, 48 x 256 1.576 ms, now 1.517, 64 x 256 1.589, now 1.538.  The Z1 of a mini-batch's block 0 started under
+// the split of the state before (EARLY) shortens the chain of short calls; longer ones, and those of more pairs, run at a clock that falls by
+// more: us or ms without / with it, back to back: 12 x 64 383 / 379, 8 x 128 751 / 743, 24 x 256 1.500 / 1.480, 32 x 192 1.133 / 1.119, 64 x 32 no
+// difference, but 26 x 256 1.500 / 1.511, 36 x 256 1.508 / 1.528, 48 x 256 1.517 / 1.551, 64 x 256 1.538 / 1.593, 64 x 1024 6.006 / 6.217, 24 x 512 2.97 /
+// 3.00, 12 x 2048 11.72 / 11.84, 80 x 64 480 / 486.  The launcher draws the line at 256 mini-batches and 24 x 256 in all (LaunchPlan::kernel).
 #include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
 
@@ -51,6 +53,7 @@ static_assert(WD_BYTES <= SM_FWD_BYTES, "the launch asks for SM_FWD_BYTES (the o
 // output workgroups, 24 .. the XCD each workgroup of the pair runs on (+ 1).
 constexpr int WDW_GIVEN = 0, WDW_TAKEN = 16, WDW_XCD = 24;
 
+template <bool EARLY>
 TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const int bh, const int half) {
   bf16* const s_g2 = reinterpret_cast<bf16*>(smem + WD_G2);
   bf16* const s_g2l = reinterpret_cast<bf16*>(smem + WD_G2L);
@@ -132,18 +135,21 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     bf16x8 xk[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) xk[s] = xpiece_rows(reinterpret_cast<const bf16*>(smem + WD_XK), 0, s, c, h);
-    // Z1 = XK W1 + b1 of the token block in xk; that of a mini-batch's block 0 is formed at the end of the one before, under the split of
-    // the new W1
+    // Z1 = XK W1 + b1 of the token block in xk; EARLY: that of a mini-batch's block 0 is formed at the end of the one before, under the
+    // split of the new W1
     f32x16 z1;
     auto z1_start = [&]() {
 #pragma unroll
       for (int i = 0; i < 16; i++) z1[i] = b1L;
     };
-    z1_start();
+    auto z1_whole = [&]() {
+      z1_start();
 #pragma unroll
-    for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
+      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
 #pragma unroll
-    for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
+      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
+    };
+    if constexpr (EARLY) z1_whole();
     TTT_STAGES_BEGIN();
     for (int mb = 0; mb < p.NC; mb++) {
       const bf16* const s_xk = reinterpret_cast<const bf16*>(smem + WD_XK + (mb & 1) * SM_TILE);
@@ -173,13 +179,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       // X2 = gelu(Z1), gelu'(Z1) of token block rb; X2's high-order term to LDS
       auto z1_block = [&](int rb, bool images) {
         WD_LANE;
-        if (rb == 1) {
-          z1_start();
-#pragma unroll
-          for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
-#pragma unroll
-          for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
-        }
+        if (!EARLY || rb == 1) z1_whole();
         f32x16 x2 = z1;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -345,17 +345,21 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       b1L += half_sum_valu(colsum);
       load_xk(mb + 1, 0);   // (put there before B2)
       cvt_chain_split(W2s, w2h, w2l);
-      __builtin_amdgcn_sched_barrier(0);
-      z1_start();
+      if constexpr (EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        z1_start();
 #pragma unroll
-      for (int s = 0; s < 4; s++) {
-        split8(W1s.b[s >> 1][0], s & 1, w1h.v[0][s], w1l.v[0][s]);
-        __builtin_amdgcn_sched_barrier(0);
-        z1 = MFMA(xk[s], w1l.v[0][s], z1);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < 4; s++) {
+          split8(W1s.b[s >> 1][0], s & 1, w1h.v[0][s], w1l.v[0][s]);
+          __builtin_amdgcn_sched_barrier(0);
+          z1 = MFMA(xk[s], w1l.v[0][s], z1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
+      } else {
+        cvt_chain_split(W1s, w1h, w1l);
       }
-#pragma unroll
-      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
       TTT_STAGE(FWC_STEP1);
       if (gave_up != 0) return;
     }
@@ -564,7 +568,8 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
 // 2 + n_out workgroups per (batch, head): the two halves of the recurrence, then the output workgroups, which take the
 // mini-batches in turn.  Workgroups are dealt to the 8 XCDs in turn, so the grid is laid out for a multiple of 8 pairs
 // (workgroups of pairs that do not exist leave at once) and the workgroups of a pair are 8 apart: same XCD, same L2.
-__global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_kernel(const FwdParams p) {
+template <bool EARLY>
+TTT_DEV void fwd_wide(const FwdParams& p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x, per = 2 + p.n_out;
   int bh = p.scatter ? b / per : (b / (8 * per)) * 8 + (b & 7);
@@ -572,12 +577,16 @@ __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
   if (bh >= p.nbh) return;
   bh += p.bh0;
   if (role < 2) {
-    fwd_wide_recurrence(p, smem, bh, role);
+    fwd_wide_recurrence<EARLY>(p, smem, bh, role);
     return;
   }
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   if (threadIdx.x == 0) say_xcd(words + WDW_XCD + role);
   fwd_output_branch<1, true>(p, smem, bh, role - 2);
+}
+__global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_kernel(const FwdParams p) { fwd_wide<false>(p); }
+__global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_early_kernel(const FwdParams p) {
+  fwd_wide<true>(p);
 }
 
 // Clears the synchronisation words and marks every word of the exchange empty.
@@ -589,16 +598,21 @@ __global__ void ttt_mlp_fwd_wide_clear(int* w, int n, const int* report, uint4* 
 
 }  // namespace ttt
 
-hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, int grid, hipStream_t stream) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(ttt::ttt_mlp_fwd_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     ttt::SM_FWD_BYTES);
-  if (e != hipSuccess) return e;
-  const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
-  int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-  const int nx = p.nbh * (ttt::FWD_XCHG_WORDS / 2);
-  const int need = nx > n ? nx : n;
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n, p.report,
-                     reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::FWD_XCHG_WORDS), nx);
-  hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_kernel, dim3(grid), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
-  return hipGetLastError();
+hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
+  auto launch = [&](auto k) -> hipError_t {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_FWD_BYTES);
+    if (e != hipSuccess) return e;
+    const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
+    int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
+    const int nx = p.nbh * (ttt::FWD_XCHG_WORDS / 2);
+    const int need = nx > n ? nx : n;
+    hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n, p.report,
+                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::FWD_XCHG_WORDS), nx);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
+    return hipGetLastError();
+  };
+  switch (kernel) {
+    TTT_FWD_WIDE_KERNELS(TTT_KERNEL_LAUNCH)
+    default: return hipErrorInvalidValue;
+  }
 }

@@ -259,7 +259,7 @@ extern "C" void ttt_mlp_set_stage_clocks(unsigned* forward, unsigned* backward);
 // in a trace.
 #define TTT_FWD_KERNELS(X) \
   X(FWD_ONE, ttt_mlp_fwd_kernel) X(FWD_SPLIT_8, ttt_mlp_fwd_split_kernel<8>) X(FWD_SPLIT_32, ttt_mlp_fwd_split_kernel<32>)
-#define TTT_FWD_WIDE_KERNELS(X) X(FWD_WIDE, ttt_mlp_fwd_wide_kernel)
+#define TTT_FWD_WIDE_KERNELS(X) X(FWD_WIDE, ttt_mlp_fwd_wide_kernel) X(FWD_WIDE_EARLY, ttt_mlp_fwd_wide_early_kernel)
 #define TTT_BWD_KERNELS(X) \
   X(BWD_ONE, ttt_mlp_bwd_kernel) X(BWD_HELPED, ttt_mlp_bwd_helped_kernel) \
   X(BWD_SPLIT_1, ttt_mlp_bwd_split_kernel<1>) X(BWD_SPLIT_2, ttt_mlp_bwd_split_kernel<2>)
@@ -281,8 +281,8 @@ enum TttKernel {
 // `grid` workgroups of `kernel`, behind a small kernel that clears the synchronisation words where p.sync is set.  FWD_ONE, FWD_SPLIT_*: one
 // workgroup per (batch, head), or two (state recurrence / output branch).
 hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
-// FWD_WIDE: the recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
-hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, int grid, hipStream_t stream);
+// FWD_WIDE*: the recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
+hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
 // BWD_ONE, BWD_HELPED, BWD_SPLIT_*: one workgroup per (batch, head), with helpers, or two or three (replays / reverse walk).
 hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream);

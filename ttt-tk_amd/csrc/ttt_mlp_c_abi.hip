@@ -335,8 +335,9 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backwa
     const long long left = (long long)(K - (segs - 1) * groups) * cgs, missing = (long long)K * cgs - NC;
     const long long len0 = backward ? len - missing : len, len_last = backward ? left : left - missing;
     const long long n0 = pairs / cus, n_last = launches - ((segs - 1) * pairs + cus - 1) / cus;
-    // + a mini-batch's worth per launch: gaps, state in and out (measured 0.7 to 2 forward, about 1 backward)
-    const long long t = 1000 * (n0 * len0 + n_last * len_last + (launches - n0 - n_last) * len + launches);
+    // + a mini-batch's worth per launch forward, a tenth backward: gaps, state in and out (measured 0.7 to 2 forward; backward what a launch costs
+    // and what a device gains that is not full all the time cancel)
+    const long long t = 1000 * (n0 * len0 + n_last * len_last + (launches - n0 - n_last) * len) + (backward ? 100 : 1000) * launches;
     if (t < best_t) {
       best_t = t;
       best.seg_len = static_cast<int>(len);
@@ -353,14 +354,17 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backwa
 // (6.5 ms forward, 23.1 ms backward for 512 mini-batches), at the most pairs of a shape.  Forward: 530 per mini-batch (4 pairs; 430
 // for 64), 545 (80 pairs) and 650 (128 pairs), and the mini-batches by which Out trails.  The backward's walk waits for the
 // first group's replay, hence the term in 1 / K: 4 to 32 pairs 240 at K = 16, 320 at 4; 48 pairs 265 and 335, 56 pairs 290 at
-// K = 16, 64 pairs 350 and 435, 80 pairs 410 at K = 16, 85 pairs 435 and 515 at 4, 128 pairs 500 and 605.
+// K = 16, 64 pairs 350 and 435, 80 pairs 410 at K = 16, 85 pairs 435 and 515 at 4, 128 pairs 500 and 605; and a twentieth, behind a device
+// that has been full.
 // A last round that is not full is 5 % shorter than a full one (400 to 456 pairs).
 // What the estimate decides: 312 pairs x 101 mini-batches in 4 groups, forward 1.70 ms cut, 1.93 uncut; 384 x 31 in 16, 0.65 and
-// 0.78; 276 x 329 in 22, backward 17.5 and 18.7; 330 x 395 in 18, 24.3 and 27.3; 384 x 512 in 16, 35.1 and 34.8.
+// 0.78; 276 x 329 in 22, backward 17.5 and 18.7; 330 x 395 in 18, 24.3 and 27.3; 384 x 512 in 16, 35.1 and 34.8.  Of 144 backward calls of
+// 260 to 384 pairs and 20 to 300 mini-batches timed both ways it takes the slower one for 2 by more than 2 % (with a mini-batch per launch and no
+// twentieth for 40, by up to 11 %: 305 x 45 in groups of 5 2.75 cut, 3.03 uncut).
 long long rest_x1000(const LaunchPlan& pl, int NC, int K, bool backward) {
   if (!backward) return pl.n_out == 2 ? 525LL * NC + 3000 : pl.n_out == 1 ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
   const int walk = pl.prefetch ? 210 : pl.wide ? (pl.gang > 6 ? 290 : 235) : pl.gang > 8 ? 380 : pl.gang ? 325 : pl.n_replay == 2 ? 405 : 485;
-  return (long long)(walk + 470 / K) * NC;
+  return (long long)(walk + 470 / K) * NC * 21 / 20;
 }
 long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace, bool backward) {
   if (cus <= 0) return (long long)NC * 1000;

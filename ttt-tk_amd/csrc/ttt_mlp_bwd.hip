@@ -419,7 +419,7 @@ TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
     const uint64_t t0 = wall_clock64();
     int took = 0;
     for (bool more = true; more;) {
-      // what is left to do of a pair, in hundredths of a mini-batch of its own workgroup: a group's replay is half of it
+      // what is left to do of a pair, in halves of a group: its replay is one, its walk the other
       int most = -1, pair = 0, group = 0, set = 0;
       uint64_t seen = 0;
       bool open = false;

@@ -13,13 +13,13 @@
 // One or two more workgroups per pair compute Out from the states left in a ring, as in the two-workgroup launch.
 // Every sum has the order of the one-workgroup kernel: results are the same to the bit.
 //
-// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.55 ms here (6.1 us per
-// mini-batch), 24 x 256 1.49 ms.  With the stage clocks in, 13.9 k clocks: block 0's GELU and partial sums 2.4 k; block 1's 3.7 k
-// while block 0's sums cross (gather and send 1.3 k, 0.9 k under way, LayerNorm 1.7 k) and 0.45 k of waiting for them;
-// block 0's weight step 2.1 k while block 1's sums cross and 2.25 k of waiting for those; block 1's weight step, the
-// split of the new state and Z1 of the next block 0 2.9 k.  With the token sums for b2 and the wait for a free ring slot between the
+// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.52 ms here (5.9 us per
+// mini-batch), 24 x 256 1.48 ms.  With the stage clocks in, 14.2 k clocks: block 0's Z1, GELU and partial sums 2.7 k; block 1's 3.5 k
+// while block 0's sums cross (gather and send 1.3 k, 1.0 k under way, LayerNorm 1.7 k) and 0.7 k of waiting for them;
+// block 0's weight step 1.9 k while block 1's sums cross and 2.5 k of waiting for those; block 1's weight step and the
+// split of the new state 2.65 k.  With the token sums for b2 and the wait for a free ring slot between the
 // exchanges it was 12 x 64 399 us, now 379, 48 x 256 1.576 ms, now 1.517, 64 x 256 1.589, now 1.538.  The Z1 of a mini-batch's block 0 started under
-// the split of the state before (EARLY) shortens the chain of short calls; longer ones, and those of more pairs, run at a clock that falls by
+// the split of the state before (EARLY) shortens the chain of short calls (13.9 k clocks); longer ones, and those of more pairs, run at a clock that falls by
 // more: us or ms without / with it, back to back: 12 x 64 383 / 379, 8 x 128 751 / 743, 24 x 256 1.500 / 1.480, 32 x 192 1.133 / 1.119, 64 x 32 no
 // difference, but 26 x 256 1.500 / 1.511, 36 x 256 1.508 / 1.528, 48 x 256 1.517 / 1.551, 64 x 256 1.538 / 1.593, 64 x 1024 6.006 / 6.217, 24 x 512 2.97 /
 // 3.00, 12 x 2048 11.72 / 11.84, 80 x 64 480 / 486.  The launcher draws the line at 256 mini-batches and 24 x 256 in all (LaunchPlan::kernel).

@@ -202,7 +202,7 @@ enum BwdStage {
 };
 // The recurrence and the walk on two workgroups: their waves 0-3 (compute) and 4-7 (helpers) go through stages of their own.
 enum FwdWideStage {
-  FWC_BLOCK0,        // compute: checkpoint store, Z1, GELU and partial Z2 of token block 0
+  FWC_BLOCK0,        // compute: checkpoint store, Z1 (unless it was started early), GELU and partial Z2 of token block 0
   FWC_B1,            // compute: barrier behind it
   FWC_BLOCK1,        // compute: the same for block 1, W2's terms transposed, the last state's images stored
   FWC_B2,            // compute: barrier behind it (block 0's sums have crossed and been normalised)

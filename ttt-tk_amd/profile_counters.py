@@ -89,7 +89,7 @@ def find_csv(out_dir: str, suffix: str) -> str:
 
 
 def short_name(kernel_name: str) -> str:
-    """ttt::ttt_mlp_bwd_split_kernel<2, true>(ttt::BwdParams) -> ttt_mlp_bwd_split_kernel<2, true>"""
+    """void ttt::ttt_mlp_bwd_split_kernel<2>(ttt::BwdParams) -> ttt_mlp_bwd_split_kernel<2>"""
     n = kernel_name.split("(")[0]
     return n.split("::")[-1].replace("void ", "").strip()
 

@@ -2113,13 +2113,13 @@ extern "C" int ttt_mlp_bwd_lds_bytes() { return ttt::SM_BWD_BYTES; }
 
 hipError_t ttt_mlp_bwd_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
   auto launch = [&](auto k) -> hipError_t {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
-    if (e != hipSuccess) return e;
     if (p.sync != nullptr) {
       const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
       int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync itself is moved back by bh0 entries
       hipLaunchKernelGGL(ttt::ttt_mlp_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, words, n, p.report);
     }
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);   // (while that runs)
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };

@@ -864,13 +864,13 @@ __global__ void ttt_mlp_bwd_wide_clear(int* w, int n, const int* report, uint4* 
 
 hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, TttKernel kernel, int grid, hipStream_t stream) {
   auto launch = [&](auto k) -> hipError_t {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);
-    if (e != hipSuccess) return e;
     const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
     int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
     const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
     hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
                        reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);   // (while that runs)
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);
     return hipGetLastError();
   };

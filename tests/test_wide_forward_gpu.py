@@ -1,6 +1,7 @@
 """The forward with the recurrence of a pair on two workgroups, against the one-workgroup launch, bit for bit: where the ring
 of states wraps, at the smallest sequences, and at the pair counts where the launch changes shape (two output workgroups
-per pair up to 64 pairs, one up to 80, the older two-workgroup launch beyond)."""
+per pair up to 64 pairs, one up to 80, the older two-workgroup launch beyond), and on both sides of the lengths up to which the products
+of a mini-batch are started in the one before."""
 import pytest
 import torch
 
@@ -12,7 +13,8 @@ FWD_KEYS = ("XQ", "XK", "XV", "last_eta", "ttt_norm_weight", "ttt_norm_bias", "W
 
 
 @pytest.mark.parametrize("B,NH,NC,cgs", [(1, 1, 2, 1), (1, 7, 3, 2), (1, 9, 8, 8), (1, 5, 9, 4), (2, 4, 17, 5), (1, 3, 70, 16),
-                                         (1, 64, 11, 4), (5, 13, 11, 4), (1, 80, 10, 4), (1, 81, 3, 2)])
+                                         (1, 64, 11, 4), (5, 13, 11, 4), (1, 80, 10, 4), (1, 81, 3, 2),
+                                         (1, 3, 256, 50), (1, 3, 257, 50), (1, 64, 96, 16), (1, 64, 97, 97)])
 def test_recurrence_on_two_workgroups_is_bit_identical(B, NH, NC, cgs):
     import ttt_mlp_host as host
     import test_time_training as ext

@@ -33,8 +33,9 @@ def _reference(host, ext, t, cgs):
     return {k: t[k].clone() for k in OUT_KEYS + host.GRAD_NAMES}
 
 
-# forward / backward: two output and four replaying workgroups per pair, two and two, one and two replaying with the walk on one CU
-@pytest.mark.parametrize("NH,NC,cgs", [(3, 21, 4), (8, 30, 3), (41, 19, 2), (70, 12, 4)])
+# forward / backward: two output and eight replaying workgroups per pair, two and two, one and two replaying with the walk on one CU; and a
+# forward too long for an early start of the next mini-batch
+@pytest.mark.parametrize("NH,NC,cgs", [(3, 21, 4), (8, 30, 3), (41, 19, 2), (70, 12, 4), (2, 259, 64)])
 def test_workgroups_of_a_pair_on_different_xcds(NH, NC, cgs):
     import test_time_training as ext
     import ttt_mlp_host as host

@@ -154,7 +154,7 @@ struct LaunchPlan {
   long long n_rest = 0;     // pairs n_single .. n_single+n_rest-1
   bool rest_split = false;
   bool wide = false;
-  int n_out = 0;            // forward, wide: that compute Out
+  bool quad = false;        // forward, wide: the recurrence of a pair, and Out, on four CUs; else on two, and Out on a third
   int gang = 0;             // backward: pairs of an XCD that share workgroups, 0: whole ones, that replay or walk, for each pair
   int n_replay = 0;         // backward: that replay checkpoint groups, of a gang or of a pair
   int n_finish = 0;         // backward, of a gang: for grad_L_XK / grad_L_XV
@@ -168,11 +168,11 @@ struct LaunchPlan {
   long long n_waiting() const { return helpers > 0 ? n_single : n_rest; }
   // Workgroups of an XCD: of a gang, or of the pairs that a forward with the recurrence on two CUs deals to it.
   int slots(bool backward) const {
-    return backward ? (wide ? 2 : 1) * gang + n_finish + n_replay + (prefetch ? gang : 0) : static_cast<int>((n_rest + 7) / 8) * (2 + n_out);
+    return backward ? (wide ? 2 : 1) * gang + n_finish + n_replay + (prefetch ? gang : 0) : static_cast<int>((n_rest + 7) / 8) * per_pair(false);
   }
   // The launch behind the full rounds of one workgroup per pair: its kernel and its workgroups.
   TttKernel kernel(bool backward, int NC) const {
-    if (!backward && wide) return n_out == 2 && NC <= 256 && n_rest * NC <= 6144 ? FWD_WIDE_EARLY : FWD_WIDE;   // (ttt_mlp_fwd_wide.hip)
+    if (!backward && wide) return quad && NC <= 256 && n_rest * NC <= 6144 ? FWD_WIDE_EARLY : FWD_WIDE;   // (ttt_mlp_fwd_wide.hip)
     if (!backward) return NC >= 512 ? FWD_SPLIT_32 : FWD_SPLIT_8;   // (mini-batches per hand-over)
     if (helpers > 0) return BWD_HELPED;
     if (!gang) return n_replay == 2 ? BWD_SPLIT_2 : BWD_SPLIT_1;
@@ -190,7 +190,7 @@ struct LaunchPlan {
   int per_pair(bool backward) const {
     if (!rest_split) return 0;
     if (backward && gang) return slots(true) / gang;
-    return backward ? n_replay + 1 : 2 + n_out;
+    return backward ? n_replay + 1 : !wide ? 2 : quad ? 4 : 3;
   }
 };
 // Clocks per mini-batch, in hundreds, that the roles of a backward gang are busy for (stage clocks, 56 and 96 pairs x 512): the replay
@@ -246,9 +246,8 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
   const long long per_xcd = (pl.n_rest + 7) / 8;
   const auto fits_xcd = [&](int per) { return per * per_xcd <= cus / 8; };
   if (!backward) {
-    // one output workgroup keeps up with a recurrence on two CUs only just; two where they fit
-    pl.n_out = fits_xcd(4) ? 2 : fits_xcd(3) ? 1 : 0;
-    pl.wide = pl.n_out > 0;
+    pl.quad = fits_xcd(4);
+    pl.wide = fits_xcd(3);
     return pl;
   }
   // Four replaying workgroups per pair leave a walk on two CUs to itself, also where they evaluate the GELU family for it (32 pairs x 512:
@@ -362,7 +361,7 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backwa
 // 260 to 384 pairs and 20 to 300 mini-batches timed both ways it takes the slower one for 2 by more than 2 % (with a mini-batch per launch and no
 // twentieth for 40, by up to 11 %: 305 x 45 in groups of 5 2.75 cut, 3.03 uncut).
 long long rest_x1000(const LaunchPlan& pl, int NC, int K, bool backward) {
-  if (!backward) return pl.n_out == 2 ? 525LL * NC + 3000 : pl.n_out == 1 ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
+  if (!backward) return pl.quad ? 525LL * NC + 3000 : pl.wide ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
   const int walk = pl.prefetch ? 210 : pl.wide ? (pl.gang > 6 ? 290 : 235) : pl.gang > 8 ? 380 : pl.gang ? 325 : pl.n_replay == 2 ? 405 : 485;
   return (long long)(walk + 470 / K) * NC * 21 / 20;
 }
@@ -549,15 +548,16 @@ struct BwdWorkspace {
 
 // Workspace of the forward with several workgroups per pair: synchronisation words, then per (batch, head) a ring of
 // 2 * FWD_RING_MAX slots of state images and of bias vectors.
-// With the recurrence on two workgroups (n_out > 0) the ring has FWD_WIDE_RING slots, and the exchange follows.
+// With the recurrence on two workgroups the ring has FWD_WIDE_RING slots, and the exchange follows.
 struct FwdWorkspace {
   size_t off[4];
   size_t total;
-  FwdWorkspace(long long n, int n_out) {
-    const size_t slots = (size_t)n * (n_out > 0 ? ttt::FWD_WIDE_RING : 2 * ttt::FWD_RING_MAX);
+  explicit FwdWorkspace(const LaunchPlan& pl) {
+    const long long n = pl.n_rest;
+    const size_t slots = (size_t)n * (pl.quad ? 0 : pl.wide ? ttt::FWD_WIDE_RING : 2 * ttt::FWD_RING_MAX);
     const size_t bytes[4] = {ttt::bwd_sync_ints(n) * sizeof(int), slots * ttt::FWD_IMG_BYTES,
                              slots * ttt::FWD_BIAS_FLOATS * sizeof(float),
-                             n_out > 0 ? (size_t)n * ttt::FWD_XCHG_WORDS * 8 : 0};
+                             pl.wide ? (size_t)n * (pl.quad ? ttt::FWD_QUAD_XCHG_WORDS : ttt::FWD_XCHG_WORDS) * 8 : 0};
     size_t o = 0;
     for (int i = 0; i < 4; i++) { off[i] = o; o += (bytes[i] + 255) & ~(size_t)255; }
     total = o;
@@ -756,7 +756,7 @@ extern "C" int ttt_mlp_fwd_launch(const ttt_mlp_fwd_args* a, void* stream) {
 extern "C" size_t ttt_mlp_fwd_workspace_bytes(int B, int NH) {
   if (B <= 0 || NH <= 0) return 0;
   const LaunchPlan pl = plan_launches((long long)B * NH, false);
-  return pl.rest_split ? FwdWorkspace(pl.n_rest, pl.n_out).total : 0;
+  return pl.rest_split ? FwdWorkspace(pl).total : 0;
 }
 
 extern "C" size_t ttt_mlp_fwd_status_offset(int B, int NH) {
@@ -773,7 +773,7 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
   const int cus = device_cus();
   const LaunchPlan pl = plan_for((long long)p.B * p.NH, cus, false);
   if (!pl.rest_split) return TTT_MLP_ERR_NO_ROOM;
-  const FwdWorkspace w(pl.n_rest, pl.n_out);
+  const FwdWorkspace w(pl);
   if (workspace_bytes < w.total) return TTT_MLP_ERR_WORKSPACE;
   char* base = static_cast<char*>(workspace);
   const Call call = plan_call(false, pl, (long long)p.B * p.NH, cus, p.NC, p.cgs, true);
@@ -801,10 +801,10 @@ int fwd_launch(const ttt_mlp_fwd_args* a, void* workspace, size_t workspace_byte
   p.wait_limit = g_wait_limit;
   p.report = report;
   if (pl.wide) {
-    p.n_out = pl.n_out;
+    p.quad = pl.quad ? 1 : 0;
     p.state_img = reinterpret_cast<__bf16*>(base + w.off[1]) - b0 * ttt::FWD_WIDE_RING * (ttt::FWD_IMG_BYTES / 2);
     p.bias_img = reinterpret_cast<float*>(base + w.off[2]) - b0 * ttt::FWD_WIDE_RING * ttt::FWD_BIAS_FLOATS;
-    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * ttt::FWD_XCHG_WORDS;
+    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[3]) - b0 * (pl.quad ? ttt::FWD_QUAD_XCHG_WORDS : ttt::FWD_XCHG_WORDS);
     p.scatter = scatter ? 1 : 0;
     return static_cast<int>(ttt_mlp_fwd_wide_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
   }
@@ -887,7 +887,7 @@ extern "C" int ttt_mlp_fwd_launch_static(const ttt_mlp_fwd_args* a, int* sticky_
   if (pairs > STATIC_MAX_PAIRS) return TTT_MLP_ERR_SCRATCH;
   const LaunchPlan pl = plan_launches(pairs, false);
   if (!pl.rest_split || pl.n_single != 0) return TTT_MLP_ERR_NO_ROOM;
-  const FwdWorkspace w(pl.n_rest, pl.n_out);
+  const FwdWorkspace w(pl);
   static_assert(static_scratch_bytes() % 256 == 0, "scratch parts are 256-byte aligned");
   if (w.total > static_scratch_bytes()) return TTT_MLP_ERR_SCRATCH;
   void* ws = nullptr;

@@ -461,7 +461,7 @@ __global__ __launch_bounds__(FW_THREADS) void ttt_mlp_fwd_split_kernel(const Fwd
   }
   bh += p.bh0;
   if (role == 0) fwd_body<1, RING>(p, smem, bh, 0, p.NC);
-  else fwd_output_branch<RING, false>(p, smem, bh, 0);
+  else fwd_output_branch<RING, false>(p, smem, bh);
 }
 
 __global__ void ttt_mlp_fwd_zero_words(int* w, int n, const int* report) { clear_word(w, n, blockIdx.x * blockDim.x + threadIdx.x, report); }

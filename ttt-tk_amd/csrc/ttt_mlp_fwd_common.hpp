@@ -146,8 +146,31 @@ TTT_DEV void pair_sum_halves(float* tile, HALF0 half0, HALF1 half1, int r, int c
   else pair_sum_halves_r<1>(tile, [&](int rb) { return rb == 0 ? half0() : half1(); }, c, h);
 }
 
-// Output LayerNorm + residual for the 8 features [f0, f0+8) of token `tok`: Out = XQ + LN(sum of the four
-// pair sums + b2).  8 lanes per token, 8 tokens per wave.
+// Output LayerNorm + residual for 8 features of a token: XQ + LN(z).  8 lanes per token.
+TTT_DEV bf16x8 output_layernorm_row(float (&z)[8], const float* s_gam, const float* s_bet, const bf16x8 qv) {
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) sum += z[e];
+  const float mu = oct_sum(sum) * (1.f / FD);
+  float var = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) { z[e] -= mu; var = __builtin_fmaf(z[e], z[e], var); }
+  const float rstd = __builtin_amdgcn_rsqf(oct_sum(var) * (1.f / FD) + LN_EPS);
+  float gam[8], bet[8];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const f32x4 gq = *reinterpret_cast<const f32x4*>(s_gam + 4 * q);
+    const f32x4 bq = *reinterpret_cast<const f32x4*>(s_bet + 4 * q);
+#pragma unroll
+    for (int e = 0; e < 4; e++) { gam[4 * q + e] = gq[e]; bet[4 * q + e] = bq[e]; }
+  }
+  bf16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; e++) o[e] = (bf16)(bf2f(qv[e]) + __builtin_fmaf(gam[e], z[e] * rstd, bet[e]));
+  return o;
+}
+
+// Out = XQ + LN(sum of the four pair sums + b2) for the features [f0, f0+8) of token `tok`; 8 tokens per wave.
 TTT_DEV void output_layernorm(const float* s_P, const float* s_b2, const float* s_gam, const float* s_bet,
                               const bf16* s_xq, gptr_t gOut, int mb, int tok, int f0) {
   float z[8];
@@ -162,32 +185,13 @@ TTT_DEV void output_layernorm(const float* s_P, const float* s_b2, const float* 
 #pragma unroll
     for (int e = 0; e < 4; e++) { z[e] = a0[e]; z[4 + e] = a1[e]; }
   }
-  float sum = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; e++) sum += z[e];
-  const float mu = oct_sum(sum) * (1.f / FD);
-  float var = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; e++) { z[e] -= mu; var = __builtin_fmaf(z[e], z[e], var); }
-  const float rstd = __builtin_amdgcn_rsqf(oct_sum(var) * (1.f / FD) + LN_EPS);
-  const bf16x8 qv = lds_get8h(s_xq + xrow(tok) + f0);
-  float gam[8], bet[8];
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const f32x4 gq = *reinterpret_cast<const f32x4*>(s_gam + f0 + 4 * q);
-    const f32x4 bq = *reinterpret_cast<const f32x4*>(s_bet + f0 + 4 * q);
-#pragma unroll
-    for (int e = 0; e < 4; e++) { gam[4 * q + e] = gq[e]; bet[4 * q + e] = bq[e]; }
-  }
-  bf16x8 o;
-#pragma unroll
-  for (int e = 0; e < 8; e++) o[e] = (bf16)(bf2f(qv[e]) + __builtin_fmaf(gam[e], z[e] * rstd, bet[e]));
+  const bf16x8 o = output_layernorm_row(z, s_gam + f0, s_bet + f0, lds_get8h(s_xq + xrow(tok) + f0));
   g_st8h(gOut, (tok * FD + f0) * 2, mb * TILE_BYTES, o);
 }
 
 // LayerNorm-fused gradient of the reconstruction loss for the 8 features of this lane's token (8 lanes per token):
-// z = Z2 in; gx times the returned scale is G2 = -eta * dl/dZ2.
-TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, const float eta, const float* s_gam, const float* s_bet,
+// z = Z2 in, target = XV - XK; gx times the returned scale is G2 = -eta * dl/dZ2.
+TTT_DEV float ln_loss_gradient(float (&z)[8], const float (&target)[8], const float eta, const float* s_gam, const float* s_bet,
                               float (&gx)[8]) {
   float sum = 0.f;
 #pragma unroll
@@ -209,7 +213,7 @@ TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, 
 #pragma unroll
   for (int e = 0; e < 8; e++) {
     const float xh = z[e] * rstd;
-    const float go = __builtin_fmaf(gam[e], xh, bet[e]) - (bf2f(vv[e]) - bf2f(kv[e]));
+    const float go = __builtin_fmaf(gam[e], xh, bet[e]) - target[e];
     z[e] = xh;
     gx[e] = go * gam[e];
     s1 += gx[e];
@@ -221,6 +225,14 @@ TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, 
 #pragma unroll
   for (int e = 0; e < 8; e++) gx[e] = FD * gx[e] - s1 - z[e] * s2;
   return scale;
+}
+
+TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, const float eta, const float* s_gam, const float* s_bet,
+                              float (&gx)[8]) {
+  float target[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) target[e] = bf2f(vv[e]) - bf2f(kv[e]);
+  return ln_loss_gradient(z, target, eta, s_gam, s_bet, gx);
 }
 
 // Everything derived from the lane index is cheap to recompute and expensive to keep in a register
@@ -235,10 +247,9 @@ TTT_DEV float ln_loss_gradient(float (&z)[8], const bf16x8 kv, const bf16x8 vv, 
 // The output branch of the forward on its own workgroup: Out[mb] = XQ + LN(gelu(XQ W1' + b1') W2' + b2')
 // with the state after mini-batch mb, taken from the operand images the recurrence leaves behind.  Nothing
 // is carried from one mini-batch to the next here.
-// WIDE: the recurrence runs on two workgroups, which hand over every mini-batch (RING = 1), and the n_out output workgroups
-// take the mini-batches in turn, this one number `turn` first.
+// WIDE: the recurrence runs on two workgroups, which hand over every mini-batch (RING = 1).
 template <int RING, bool WIDE>
-TTT_DEV void fwd_output_branch(const FwdParams& p, unsigned char* smem, const int bh, const int turn) {
+TTT_DEV void fwd_output_branch(const FwdParams& p, unsigned char* smem, const int bh) {
   float* s_P = reinterpret_cast<float*>(smem + SM_P);
   float* s_b1 = reinterpret_cast<float*>(smem + SM_B1);
   float* s_b2 = reinterpret_cast<float*>(smem + SM_B2);   // two buffers: the second takes the place of the eta vector
@@ -264,11 +275,10 @@ TTT_DEV void fwd_output_branch(const FwdParams& p, unsigned char* smem, const in
   int* const s_flag = reinterpret_cast<int*>(smem + SM_FLAG);
 
   TTT_STAGES_BEGIN();
-  const int step = WIDE ? p.n_out : 1;
-  for (int mb = WIDE ? turn : 0; mb < p.NC; mb += step) {
+  for (int mb = 0; mb < p.NC; mb++) {
     LANE_VARS;
     constexpr int ring = RING; const int grp = mb / ring, at = mb % ring, slot = WIDE ? mb % FWD_WIDE_RING : (grp & 1) * ring + at;
-    const int buf = WIDE ? (mb / step) & 1 : mb & 1;
+    const int buf = mb & 1;
     if (at == 0) {
       if (!wait_at_least(w_given, grp + 1, w_status, s_flag, p.wait_limit)) return;
       if (WIDE && !wait_at_least(w_given + 8, grp + 1, w_status, s_flag, p.wait_limit)) return;
@@ -328,11 +338,11 @@ TTT_DEV void fwd_output_branch(const FwdParams& p, unsigned char* smem, const in
     }
     TTT_STAGE(FS_OUT_LN);
     if constexpr (WIDE) {   // every wave has read its operands (the pair sum's barriers are behind it); nothing else is ordered by this count
-      if (threadIdx.x == 0) __hip_atomic_store(w_taken + 4 * turn, mb / step + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (threadIdx.x == 0) __hip_atomic_store(w_taken, mb + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else if (at == ring - 1 || mb == p.NC - 1) publish(w_taken, grp + 1);
     TTT_STAGE(FS_PUBLISH);
   }
-  TTT_STAGES_END(bh, STAGE_ROLE_OUT + turn);
+  TTT_STAGES_END(bh, STAGE_ROLE_OUT);
 }
 
 }  // namespace ttt

@@ -1,4 +1,5 @@
-// Forward scan with the recurrence of one (batch, head) spread over two CUs (few pairs: the chain is the bound).
+// Forward scan with the recurrence of one (batch, head) spread over two CUs, where four each (ttt_mlp_fwd_quad.hpp) do not fit:
+// 65 to 80 pairs on 256 CUs.
 //
 // The recurrence of a pair is sequential and one CU spends 19.4 k clocks on a mini-batch of it, close to the sum of
 // what the two waves of each SIMD issue.  Here two workgroups of the same XCD hold 128 hidden columns each, and inside a
@@ -10,21 +11,16 @@
 // What crosses the CUs is one or two fp32 tiles per mini-batch and direction (16 / 32 KiB; both CUs form the LayerNorm of
 // all tokens, from the same sums in the same order).  No flags: a word is sent as it is and its slot holds an impossible
 // value (a NaN that is never sent) before and after; the receiver polls the data itself and puts the mark back.
-// One or two more workgroups per pair compute Out from the states left in a ring, as in the two-workgroup launch.
+// One more workgroup per pair computes Out from the states left in a ring, as in the two-workgroup launch.
 // Every sum has the order of the one-workgroup kernel: results are the same to the bit.
 //
-// What bounds it: the chain.  48 pairs x 256 mini-batches: 2.21 ms with the recurrence on one CU, 1.52 ms here (5.9 us per
-// mini-batch), 24 x 256 1.48 ms.  With the stage clocks in, 14.2 k clocks: block 0's Z1, GELU and partial sums 2.7 k; block 1's 3.5 k
-// while block 0's sums cross (gather and send 1.3 k, 1.0 k under way, LayerNorm 1.7 k) and 0.7 k of waiting for them;
+// What bounds it: the chain, 14.2 k clocks per mini-batch (with a second workgroup for Out beside it): block 0's Z1, GELU and partial sums
+// 2.7 k; block 1's 3.5 k while block 0's sums cross (gather and send 1.3 k, 1.0 k under way, LayerNorm 1.7 k) and 0.7 k of waiting for them;
 // block 0's weight step 1.9 k while block 1's sums cross and 2.5 k of waiting for those; block 1's weight step and the
-// split of the new state 2.65 k.  With the token sums for b2 and the wait for a free ring slot between the
-// exchanges it was 12 x 64 399 us, now 379, 48 x 256 1.576 ms, now 1.517, 64 x 256 1.589, now 1.538.  The Z1 of a mini-batch's block 0 started under
-// the split of the state before (EARLY) shortens the chain of short calls (13.9 k clocks); longer ones, and those of more pairs, run at a clock that falls by
-// more: us or ms without / with it, back to back: 12 x 64 383 / 379, 8 x 128 751 / 743, 24 x 256 1.500 / 1.480, 32 x 192 1.133 / 1.119, 64 x 32 no
-// difference, but 26 x 256 1.500 / 1.511, 36 x 256 1.508 / 1.528, 48 x 256 1.517 / 1.551, 64 x 256 1.538 / 1.593, 64 x 1024 6.006 / 6.217, 24 x 512 2.97 /
-// 3.00, 12 x 2048 11.72 / 11.84, 80 x 64 480 / 486.  The launcher draws the line at 256 mini-batches and 24 x 256 in all (LaunchPlan::kernel).
+// split of the new state 2.65 k.  80 pairs x 512 mini-batches 3.72 ms; the recurrence on one CU 4.4.
 #include "ttt_mlp_exchange.hpp"
 #include "ttt_mlp_fwd_common.hpp"
+#include "ttt_mlp_fwd_quad.hpp"
 
 namespace ttt {
 
@@ -49,11 +45,10 @@ constexpr int WD_FLAG = WD_B2P + 8 * FD * 4;             // [0] non-zero: a wait
 constexpr int WD_BYTES = WD_FLAG + 16;
 static_assert(WD_BYTES <= SM_FWD_BYTES, "the launch asks for SM_FWD_BYTES (the output branch's carve-up)");
 
-// Synchronisation words of a pair: 0 / 8 mini-batches handed over by the two halves, 16 / 20 mini-batches finished by the
-// output workgroups, 24 .. the XCD each workgroup of the pair runs on (+ 1).
+// Synchronisation words of a pair: 0 / 8 mini-batches handed over by the two halves, 16 mini-batches finished by the
+// output workgroup, 24 .. the XCD each workgroup of the pair runs on (+ 1).
 constexpr int WDW_GIVEN = 0, WDW_TAKEN = 16, WDW_XCD = 24;
 
-template <bool EARLY>
 TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const int bh, const int half) {
   bf16* const s_g2 = reinterpret_cast<bf16*>(smem + WD_G2);
   bf16* const s_g2l = reinterpret_cast<bf16*>(smem + WD_G2L);
@@ -75,7 +70,6 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
 
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   int* const w_status = p.status;
-  const int n_wg = 2 + p.n_out;
   if (tid == 0) say_xcd(words + WDW_XCD + half);
   if (tid < FD) {
     s_b2[tid] = p.b2[(size_t)bh * FD + tid];
@@ -135,21 +129,6 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     bf16x8 xk[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) xk[s] = xpiece_rows(reinterpret_cast<const bf16*>(smem + WD_XK), 0, s, c, h);
-    // Z1 = XK W1 + b1 of the token block in xk; EARLY: that of a mini-batch's block 0 is formed at the end of the one before, under the
-    // split of the new W1
-    f32x16 z1;
-    auto z1_start = [&]() {
-#pragma unroll
-      for (int i = 0; i < 16; i++) z1[i] = b1L;
-    };
-    auto z1_whole = [&]() {
-      z1_start();
-#pragma unroll
-      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1l.v[0][s], z1);
-#pragma unroll
-      for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
-    };
-    if constexpr (EARLY) z1_whole();
     TTT_STAGES_BEGIN();
     for (int mb = 0; mb < p.NC; mb++) {
       const bf16* const s_xk = reinterpret_cast<const bf16*>(smem + WD_XK + (mb & 1) * SM_TILE);
@@ -179,8 +158,13 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       // X2 = gelu(Z1), gelu'(Z1) of token block rb; X2's high-order term to LDS
       auto z1_block = [&](int rb, bool images) {
         WD_LANE;
-        if (!EARLY || rb == 1) z1_whole();
-        f32x16 x2 = z1;
+        f32x16 x2;   // Z1 = XK W1 + b1
+#pragma unroll
+        for (int i = 0; i < 16; i++) x2[i] = b1L;
+#pragma unroll
+        for (int s = 0; s < 4; s++) x2 = MFMA(xk[s], w1l.v[0][s], x2);
+#pragma unroll
+        for (int s = 0; s < 4; s++) x2 = MFMA(xk[s], w1h.v[0][s], x2);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           if (images) {
@@ -345,21 +329,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       b1L += half_sum_valu(colsum);
       load_xk(mb + 1, 0);   // (put there before B2)
       cvt_chain_split(W2s, w2h, w2l);
-      if constexpr (EARLY) {
-        __builtin_amdgcn_sched_barrier(0);
-        z1_start();
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-          split8(W1s.b[s >> 1][0], s & 1, w1h.v[0][s], w1l.v[0][s]);
-          __builtin_amdgcn_sched_barrier(0);
-          z1 = MFMA(xk[s], w1l.v[0][s], z1);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; s++) z1 = MFMA(xk[s], w1h.v[0][s], z1);
-      } else {
-        cvt_chain_split(W1s, w1h, w1l);
-      }
+      cvt_chain_split(W1s, w1h, w1l);
       TTT_STAGE(FWC_STEP1);
       if (gave_up != 0) return;
     }
@@ -393,7 +363,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   put_xk(0);
   __syncthreads();   // the flag is clear
   bool alive = true;
-  const bool near = on_one_xcd(words + WDW_XCD, n_wg, lane, w_status, p.wait_limit, alive);
+  const bool near = on_one_xcd(words + WDW_XCD, 3, lane, w_status, p.wait_limit, alive);
   if (!alive && lane == 0) *s_flag = 1;
   __syncthreads();
   if (flag() != 0) {
@@ -408,7 +378,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   for (int e = 0; e < 8; e++) b2v[e] = s_b2[f0 + e];
   float gx[2][8], scale[2] = {0.f, 0.f};               // G2 of the two blocks (gx * scale), whose token sums wait until the compute waves have what they wait for
   __builtin_amdgcn_s_setprio(2);                      // these waves' few instructions are what the other four wait for
-  int seen0 = 0, seen1 = 0;                           // mini-batches the output workgroups are known to have finished
+  int seen = 0;                                       // mini-batches the output workgroup is known to have finished
   bool gave_up = false;
   TTT_STAGES_BEGIN();
 
@@ -485,16 +455,14 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     }
     if (u == 0 && half == 0) p.bias_img[((size_t)bh * FWD_WIDE_RING + m % FWD_WIDE_RING) * FWD_BIAS_FLOATS + HID + lane] = b2L;
   };
-  // The slot that mini-batch mb's state goes to is free once the output branch is done with mini-batch mb - RING.  Waited for ahead of
-  // the sums, where these waves have time (with one output workgroup, which only just keeps up, behind block 0's: 72 pairs x 256 1.78 ms
-  // so, 1.86 ms ahead of them; 24 x 256 1.51 ms and 1.485).
+  // The slot that mini-batch mb's state goes to is free once the output branch, which only just keeps up, is done with mini-batch mb - RING:
+  // waited for behind block 0's sums (72 pairs x 256 1.78 ms so, 1.86 ms ahead of them).
   auto ring_slot = [&](int mb) {
     if (u == 3 && mb >= FWD_WIDE_RING) {
-      const int old = mb - FWD_WIDE_RING, o = old % p.n_out, need = old / p.n_out + 1;
-      int seen = o == 0 ? seen0 : seen1;
+      const int need = mb - FWD_WIDE_RING + 1;
       if (seen < need) {
         const uint64_t t0 = wall_clock64();
-        while ((seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(words + WDW_TAKEN + 4 * o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < need) {
+        while ((seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(words + WDW_TAKEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) < need) {
           if (__hip_atomic_load(w_status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || wall_clock64() - t0 > p.wait_limit) {
             raise_status(w_status);
             gave_up = true;
@@ -502,8 +470,6 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
           }
           __builtin_amdgcn_s_sleep(4);
         }
-        if (o == 0) seen0 = seen;
-        else seen1 = seen;
       }
     }
   };
@@ -526,7 +492,6 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
       eta[k] = g_ldh(gEta, 2 * t_in, mb * (CS * 2) + k * CS);
     }
     load_xk(mb + 1 < p.NC ? mb + 1 : mb);
-    if (p.n_out > 1) ring_slot(mb);
     TTT_STAGE(FWH_ASK);
     __syncthreads();   // B1
     TTT_STAGE(FWH_B1);
@@ -534,7 +499,7 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
     put_xk(mb + 1);   // the buffer was last read a mini-batch ago
     TTT_STAGE(FWH_SEND0);
     finish_block(mb, 0, xk[0], xv[0], eta[0]);
-    if (p.n_out == 1) ring_slot(mb);
+    ring_slot(mb);
     TTT_STAGE(FWH_LN0);
     __syncthreads();   // B2
     TTT_STAGE(FWH_B2);
@@ -565,26 +530,33 @@ TTT_DEV void fwd_wide_recurrence(const FwdParams& p, unsigned char* smem, const 
   if (u == 0 && lane == 0) give(p.NC);
 }
 
-// 2 + n_out workgroups per (batch, head): the two halves of the recurrence, then the output workgroups, which take the
-// mini-batches in turn.  Workgroups are dealt to the 8 XCDs in turn, so the grid is laid out for a multiple of 8 pairs
+// Four workgroups per (batch, head) that share its recurrence and compute Out, or three: the two halves of the recurrence and one that
+// computes Out.  Workgroups are dealt to the 8 XCDs in turn, so the grid is laid out for a multiple of 8 pairs
 // (workgroups of pairs that do not exist leave at once) and the workgroups of a pair are 8 apart: same XCD, same L2.
-template <bool EARLY>
+template <bool QUAD>
 TTT_DEV void fwd_wide(const FwdParams& p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int b = blockIdx.x, per = 2 + p.n_out;
+  const bool quad = QUAD || p.quad != 0;
+  const int b = blockIdx.x, per = quad ? QD_CUS : 3;
   int bh = p.scatter ? b / per : (b / (8 * per)) * 8 + (b & 7);
   const int role = (p.scatter ? b : b >> 3) % per;
   if (bh >= p.nbh) return;
   bh += p.bh0;
+  if (quad) {
+    fwd_quad_recurrence(p, smem, bh, role);
+    return;
+  }
   if (role < 2) {
-    fwd_wide_recurrence<EARLY>(p, smem, bh, role);
+    fwd_wide_recurrence(p, smem, bh, role);
     return;
   }
   int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
   if (threadIdx.x == 0) say_xcd(words + WDW_XCD + role);
-  fwd_output_branch<1, true>(p, smem, bh, role - 2);
+  fwd_output_branch<1, true>(p, smem, bh);
 }
 __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_kernel(const FwdParams p) { fwd_wide<false>(p); }
+// Four workgroups per pair and nothing else: 1 % shorter than the kernel that holds both launches in calls of a few hundred mini-batches (12 pairs x 32
+// 163.3 -> 161.5 us, 24 x 256 1.228 -> 1.213 ms, 64 x 96 0.492 -> 0.486).
 __global__ __launch_bounds__(FW_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void ttt_mlp_fwd_wide_early_kernel(const FwdParams p) {
   fwd_wide<true>(p);
 }
@@ -604,10 +576,10 @@ hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, TttKernel kernel, i
     if (e != hipSuccess) return e;
     const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
     int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-    const int nx = p.nbh * (ttt::FWD_XCHG_WORDS / 2);
+    const int per = p.quad ? ttt::FWD_QUAD_XCHG_WORDS : ttt::FWD_XCHG_WORDS, nx = p.nbh * (per / 2);
     const int need = nx > n ? nx : n;
     hipLaunchKernelGGL(ttt::ttt_mlp_fwd_wide_clear, dim3((need + 255) / 256), dim3(256), 0, stream, words, n, p.report,
-                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::FWD_XCHG_WORDS), nx);
+                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * per), nx);
     hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::FW_THREADS), ttt::SM_FWD_BYTES, stream, p);
     return hipGetLastError();
   };

@@ -25,11 +25,11 @@ struct FwdParams {
   int* status;    // the status word behind the synchronisation words
   int* report;    // one more int, in host memory, that a wait that gives up is told to (or nullptr)
   unsigned long long wait_limit;   // ticks of the 100 MHz clock a workgroup waits for another before it gives up
-  // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2 x 2048 fp32],
-  // and the output workgroups per pair (1 or 2); the ring then has FWD_WIDE_RING slots.
+  // Recurrence on two workgroups (ttt_mlp_fwd_wide.hip): what they exchange, [B*NH][2 parities][2 halves][2 token blocks][2 x 2048 fp32];
+  // the ring then has FWD_WIDE_RING slots.  On four (quad != 0, ttt_mlp_fwd_quad.hpp): FWD_QUAD_XCHG_WORDS per pair, and no ring.
   // scatter: the workgroups of a pair on consecutive XCDs instead of on one, for tests.
   unsigned long long* xchg;
-  int n_out, scatter;
+  int quad, scatter;
   int bh0, nbh;   // this launch covers (batch, head) pairs bh0 .. bh0 + nbh - 1
   // One workgroup per pair, sequence cut into segments (seg_len > 0, a multiple of cgs): workgroup i of the launch
   // runs job job0 + i, job q = segment q / (B*NH) of pair q % (B*NH); a segment starts from the checkpoint that the
@@ -42,6 +42,7 @@ struct FwdParams {
 constexpr int FWD_RING_MAX = 32;               // most mini-batches per hand-over (8 or 32 are compiled)
 constexpr int FWD_WIDE_RING = 8;               // ring slots with the recurrence on two workgroups
 constexpr int FWD_XCHG_WORDS = 2 * 2 * 2 * 2048;  // 8-byte words of a pair's exchange: 128 KiB
+constexpr int FWD_QUAD_XCHG_WORDS = 48640;      // with the recurrence on four workgroups (ttt_mlp_fwd_quad.hpp): 380 KiB
 constexpr int FWD_IMG_BYTES = 64 * 256 * 2 * 2;  // W1 and W2 as bf16 operands
 constexpr int FWD_BIAS_FLOATS = 256 + 64;
 
@@ -222,6 +223,30 @@ enum FwdWideStage {
   FWH_B2STEP,        // helpers: state announced, step of b2
   FWX_COUNT
 };
+// The recurrence on four workgroups.
+enum FwdQuadStage {
+  FQC_SUMS,          // compute: Z1, GELU and partial Z2
+  FQC_B1,            // compute: barrier behind it
+  FQC_OUTPUT,        // compute: the output branch of the mini-batch before, operands of the step, checkpoint
+  FQC_B2,            // compute: barrier behind it (the sums have crossed and been normalised)
+  FQC_G1,            // compute: G1, W2's step, G1 split
+  FQC_B3,            // compute: barrier behind it
+  FQC_STEP,          // compute: W1's step and the split of the new state
+  FQC_B4,            // compute: barrier behind it
+  FQH_TOP,           // helpers: marks of the last mini-batch waited for
+  FQH_B1,            // helpers: wait for the partial sums
+  FQH_SEND,          // helpers: sum over this CU's hidden columns, sent to the CUs that normalise it
+  FQH_TAKE,          // helpers, two of the four: wait for the other CUs' shares
+  FQH_LN,            // helpers, two of the four: LayerNorm and loss gradient of 8 tokens, G2 sent
+  FQH_OUTPUT,        // helpers, the other two: Out of the mini-batch before the last
+  FQH_TAKE2,         // helpers: marks, share of the step of b2; wait for the other CUs' G2
+  FQH_B2,            // helpers: barrier behind it
+  FQH_GIVE,          // helpers: Out's partial sums gathered, step of b2
+  FQH_B3,            // helpers: wait for G1
+  FQH_NEXT,          // helpers: Out's partial sums sent, the next inputs asked for
+  FQH_B4,            // helpers: wait for the new state
+  FQX_COUNT
+};
 enum BwdWideStage {
   BWC_BAR_TERMS,     // compute: what the output branch adds to the running gradients
   BWC_STEP0,         // compute: weight step backwards, partial sums of token block 0
@@ -245,7 +270,7 @@ enum BwdWideStage {
   BWH_STORE1,        // helpers: block 1's outputs stored, gradient wrt b2
   BWX_COUNT
 };
-static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <= STAGE_SLOTS && BWX_COUNT <= STAGE_SLOTS, "stage slots");
+static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <= STAGE_SLOTS && FQX_COUNT <= STAGE_SLOTS && BWX_COUNT <= STAGE_SLOTS, "stage slots");
 
 }  // namespace ttt
 
@@ -281,7 +306,7 @@ enum TttKernel {
 // `grid` workgroups of `kernel`, behind a small kernel that clears the synchronisation words where p.sync is set.  FWD_ONE, FWD_SPLIT_*: one
 // workgroup per (batch, head), or two (state recurrence / output branch).
 hipError_t ttt_mlp_fwd_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
-// FWD_WIDE*: the recurrence of every pair on two workgroups, 1 or 2 output workgroups per pair (p.n_out).
+// FWD_WIDE: the recurrence of every pair on four workgroups, or (p.quad == 0) on two beside one that computes Out; FWD_WIDE_EARLY: on four.
 hipError_t ttt_mlp_fwd_wide_enqueue(const ttt::FwdParams& p, TttKernel kernel, int grid, hipStream_t stream);
 hipError_t ttt_mlp_fwd_clear_words(int* words, int n, hipStream_t stream);   // zeroes n ints with a small kernel
 // BWD_ONE, BWD_HELPED, BWD_SPLIT_*: one workgroup per (batch, head), with helpers, or two or three (replays / reverse walk).

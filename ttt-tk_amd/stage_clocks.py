@@ -86,6 +86,7 @@ def main() -> int:
     header = open(os.path.join(HERE, "csrc", "ttt_mlp_kernels.hpp")).read()
     fwd_names, bwd_names = stage_names(header, "FwdStage"), stage_names(header, "BwdStage")
     fwd_wide_names, bwd_wide_names = stage_names(header, "FwdWideStage"), stage_names(header, "BwdWideStage")
+    fwd_quad_names = stage_names(header, "FwdQuadStage")
     if a.shape:
         B, NH, NC, cgs, eta_std = *(int(x) for x in a.shape.split(",")), 1.0
         label, option = "custom", f"--shape {a.shape}"
@@ -183,7 +184,11 @@ def main() -> int:
     if split_f.any():
         out += table(f"forward, recurrence workgroup ({int(split_f.sum())} pairs)", cf[split_f, 0], fwd_names, NC) + [""]
         out += table(f"forward, output-branch workgroup ({int(split_f.sum())} pairs)", cf[split_f, OUT], fwd_names, NC) + [""]
-    if wide_f.any():
+    if wide_f.any() and not ran(cf[:, OUT]).any():   # (of the four workgroups the first two keep clocks)
+        both = halves(cf, HALF)
+        out += table(f"forward, recurrence on four workgroups, compute waves ({int(wide_f.sum())} pairs)", both[:, :4], fwd_quad_names, NC) + [""]
+        out += table("forward, recurrence on four workgroups, helper waves", both[:, 4:], fwd_quad_names, NC) + [""]
+    elif wide_f.any():
         both = halves(cf, HALF)
         n_out = 2 if ran(cf[:, OUT + 1]).any() else 1
         out += table(f"forward, recurrence on two workgroups, compute waves ({int(wide_f.sum())} pairs)", both[:, :4], fwd_wide_names, NC) + [""]

@@ -1,6 +1,6 @@
-// Remat backward with the reverse walk of one (batch, head) spread over two CUs (few pairs: the walk's chain is the bound).
+// Remat backward with the reverse walk of one (batch, head) spread over several CUs (few pairs: the walk's chain is the bound).
 //
-// The walk on one CU spends 28 k clocks on a mini-batch.  Here two workgroups of one XCD hold 128 hidden columns each
+// The walk on one CU spends 28 k clocks on a mini-batch.  In bwd_wide_walk two workgroups of one XCD hold 128 hidden columns each
 // (two of the four wave pairs of ttt_mlp_bwd.hip), with two kinds of waves as in ttt_mlp_fwd_wide.hip:
 //   waves 0-3 (one per SIMD)  32 hidden columns each: every matrix product and the running gradients
 //   waves 4-7                 sums over the hidden dimension, their exchange with the other CU, the LayerNorm lanes, the
@@ -11,11 +11,10 @@
 // (bwd_finish_dxk), whole ones for each pair or shared by the pairs of an XCD; that launch also runs with the walk on one CU
 // (ttt_mlp_bwd_gang_kernel).  Every sum has the order of the one-workgroup kernel: same results to the bit.
 //
-// 48 pairs x 256 mini-batches 3.60 ms with the walk on one CU, 3.03 ms here; 48 x 4,096 49.8 -> 41.2 ms; 32 x 512 6.73 -> 5.10 ms.
-// With the stage clocks in, 21.8 k clocks per mini-batch at 48 pairs, 19.2 k at 32.  At 48 the two replaying workgroups bound
-// it (42.9 k clocks per mini-batch each, hardly any of it waiting).  At 32 the chain does: what the output branch adds 2.2 k,
-// the weight step backwards 2.5 k + 2.8 k, the exchange of block 0's sums 2.3 k of waiting beyond that, the products that need
-// no sums 3.2 k, the inner MLP backwards 1.7 k + 3.1 k, the exchange of block 1's sums 0.9 k of waiting.
+// 48 pairs x 256 mini-batches 3.60 ms with the walk on one CU, 3.03 ms here; 48 x 4,096 49.8 -> 41.2 ms.
+// With the stage clocks in, 21.8 k clocks per mini-batch at 48 pairs, where the two replaying workgroups bound it (42.9 k clocks
+// per mini-batch each, hardly any of it waiting).  Up to 32 pairs, where this chain would be the bound (19.2 k), the walk has
+// four CUs (ttt_mlp_bwd_quad.hpp).
 #define TTT_BWD_ROLES_ONLY
 #include "ttt_mlp_bwd.hip"
 #include "ttt_mlp_exchange.hpp"
@@ -82,7 +81,6 @@ TTT_DEV float walk_layernorm(float (&gg)[8], const float (&gb)[8], float neg_eta
   return eta_bias;
 }
 
-template <bool IMG>
 TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh, const int half) {
   typedef __attribute__((address_space(3))) int* lint_t;
   const lint_t s_flag = (lint_t)reinterpret_cast<int*>(smem + BWW_FLAG);
@@ -142,29 +140,23 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
     bf16x8 x2b[4], g1b[4];   // what the output branch adds (lane = hid, contraction = tok), asked for a mini-batch ahead
     bf16x8 w2bf[4];          // W2 before the step, and gelu, gelu', gelu'' of Z1 by token block
     bf16x8 gq[2][2], aq[2][2], bq[2][2];
-    gptr_t gX2B, gGZ1B, gI2, gZ, gD;
+    gptr_t gX2B, gGZ1B, gI2, gZ;
     auto group_images = [&](int set) {
       gX2B = gbuf(WGRP(X2_bar_group) + oh);
       gGZ1B = gbuf(WGRP(Z1_bar_group) + oh);
       gI2 = gbuf(WGRP(grad_l_wrt_Z1_group) + oh);
       gZ = gbuf(WGRP(Z1_group) + oh);
-      gD = gbuf(WGRP(W1_init_group) + oh);
     };
     const gptr_t gCk = gbuf(ka->W2_ck + ock);
     auto ask_gelu = [&](int i, int j) {
       WW_LANE;
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        gq[i][t] = image_load<IMG>(gZ, j * IMG_BYTES, 2 * i + t, t16);
-        if constexpr (IMG) {
-          aq[i][t] = image_load<false>(gD, 2 * j * IMG_BYTES, 2 * i + t, t16);
-          bq[i][t] = image_load<true>(gD, 2 * j * IMG_BYTES + IMG_BYTES, 2 * i + t, t16);
-        }
+        gq[i][t] = image_load<false>(gZ, j * IMG_BYTES, 2 * i + t, t16);
       }
     };
-    // Operands are asked for one to two stages ahead.  One CU cannot keep enough requests in flight to hide the way to HBM (80 KiB
-    // asked for in a row take 9 k clocks to issue), so another workgroup brings the lines into the L2 before (bwd_wide_prefetch, with three or four replaying ones);
-    // what the grad_L_XK workgroup reads next is left there.
+    // Operands are asked for one to two stages ahead (one CU cannot keep enough requests in flight to hide the way to HBM: 80 KiB
+    // asked for in a row take 9 k clocks to issue); what the grad_L_XK workgroup reads next is left in the L2.
     auto ask_bar = [&](int j) {
       WW_LANE;
 #pragma unroll
@@ -288,20 +280,16 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
           bf16x8 x2c[2], uc[2];
 #pragma unroll
           for (int t = 0; t < 2; t++) {
-            if constexpr (!IMG) {
-              const bf16x8 zc = gq[i][t];
+            const bf16x8 zc = gq[i][t];
 #pragma unroll
-              for (int jj = 0; jj < 8; jj++) {
-                float g, a, b;
-                gelu_fdd((float)zc[jj], g, a, b);
-                x2c[t][jj] = (bf16)g;
-                aq[i][t][jj] = (bf16)a;
-                bq[i][t][jj] = (bf16)b;
-              }
-              asm volatile("" : "+v"(x2c[t]), "+v"(aq[i][t]), "+v"(bq[i][t]));   // finished here (see the replay's gelu')
-            } else {
-              x2c[t] = gq[i][t];
+            for (int jj = 0; jj < 8; jj++) {
+              float g, a, b;
+              gelu_fdd((float)zc[jj], g, a, b);
+              x2c[t][jj] = (bf16)g;
+              aq[i][t][jj] = (bf16)a;
+              bq[i][t][jj] = (bf16)b;
             }
+            asm volatile("" : "+v"(x2c[t]), "+v"(aq[i][t]), "+v"(bq[i][t]));   // finished here (see the replay's gelu')
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) {
               const float a = (float)aq[i][t][jj], b = (float)bq[i][t][jj];
@@ -726,103 +714,46 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
 #undef WW_LANE
 }
 
-// The workgroup that reads ahead of the walk.  The walk asks per mini-batch for 240 KiB that a replaying workgroup wrote a
-// checkpoint group earlier or that the caller passed in: none of it is in the L2 by then, and a CU whose registers and LDS are
-// full cannot keep enough requests in flight to hide the way to HBM.  This one computes nothing: it reads one dword of every
-// 128-byte line that the walk and the grad_L_XK workgroup will ask for, two mini-batches ahead of the walk, which asks for
-// most of it one ahead.  On the walk's XCD it leaves the lines in the L2 that the walk's requests go to.  Purely a hint: the
-// values are dropped, nothing is written except the status word of a wait that gives up, and the results do not depend on
-// whether, when or where this workgroup runs.
-constexpr int BWW_AHEAD = 2;
-TTT_DEV void bwd_wide_prefetch(const BwdParams& p, unsigned char* smem, const int bh) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int v = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cgs = p.cgs, n_sets = p.n_sets;
-  int* const words = p.sync + (size_t)bh * BWD_SYNC_STRIDE;
-  int* const s_flag = reinterpret_cast<int*>(smem + BWW_FLAG);
-  const size_t ox = uni64((size_t)bh * p.NC * (CS * FD)), of = uni64((size_t)bh * cgs * (CS * FD)), oh = uni64((size_t)bh * cgs * (CS * HID));
-  const unsigned line_t = 128u * lane, line_i = 128u * (tid & 255);   // this thread's line of a tile / of an image
-  const bool up = v >= 4;
-  int n = 0, seen = 0;
-  for (int k = p.K - 1; k >= 0; k--) {
-    const int n_mb = min(cgs, p.NC - k * cgs);
-    const int done = p.K - 1 - k, set = done % n_sets;
-    if (!wait_at_least(words + set, parts_until(p, done), p.status, s_flag, p.wait_limit)) return;
-#define PGRP(name) (set ? p.alt_##name[set - 1] : p.name)
-    // wave v: tile v (two inputs, four of the set); waves 0-3 / 4-7: one image each of a pair
-    gptr_t tile = gbuf(p.XQ + ox);
-    unsigned tile0 = k * cgs * TILE_BYTES;
-    if (v == 1) tile = gbuf(p.XK + ox);
-    if (v >= 2) tile0 = 0;
-    if (v == 2) tile = gbuf(PGRP(grad_l_wrt_Z2_group) + of);
-    if (v == 3) tile = gbuf(PGRP(grad_x_hat_fused_group) + of);
-    if (v == 4) tile = gbuf(PGRP(x_hat_fused_group) + of);
-    if (v >= 5) tile = gbuf(PGRP(grad_output_fused_group) + of);
-    const gptr_t img0 = up ? gbuf(PGRP(Z1_bar_group) + oh) : gbuf(PGRP(X2_bar_group) + oh);
-    const gptr_t img1 = up ? gbuf(PGRP(grad_l_wrt_Z1_group) + oh) : gbuf(PGRP(Z1_group) + oh);
-    const gptr_t img2 = gbuf(PGRP(W1_init_group) + oh), img3 = gbuf(PGRP(X2_group) + oh);
-#undef PGRP
-    for (int j = n_mb - 1; j >= 0; j--, n++) {
-      if (seen < n + 1 - BWW_AHEAD) {
-        const int s = wait_for_pace(words + BWW_GIVEN, n + 1 - BWW_AHEAD, p.status, s_flag, p.wait_limit);
-        if (s == 0) return;
-        seen = s - 1;
-      }
-      if (seen > n) continue;   // the walk is past this mini-batch already
-      const unsigned ho = j * IMG_BYTES, before = (j > 0 ? j - 1 : 0) * IMG_BYTES;
-      unsigned got[5] = {0, 0, 0, 0, 0};
-      got[1] = g_ld<unsigned>(img0, line_i, ho);
-      got[2] = g_ld<unsigned>(img1, line_i, up ? before : ho);
-      got[3] = g_ld<unsigned>(img2, line_i, 2 * ho + (up ? IMG_BYTES : 0));
-      if (v < 6) got[0] = g_ld<unsigned>(tile, line_t, tile0 + j * TILE_BYTES);
-      if (up) got[4] = g_ld<unsigned>(img3, line_i, before);   // W1 before the step, for the grad_L_XK workgroup
-#pragma unroll
-      for (int i = 0; i < 5; i++) asm volatile("" ::"v"(got[i]));   // landed; nothing is done with them
-    }
-  }
-}
+}  // namespace ttt
+#include "ttt_mlp_bwd_quad.hpp"
+namespace ttt {
 
 // The workgroups of a gang: gang g has pairs g, g + 8, .. and, as workgroups are dealt to the 8 XCDs in turn, one XCD.  WALKERS of
 // them walk each pair, the others work for all of its pairs: n_replay take the replays in turn, ordered by group, then by pair (all
 // walks go at one pace) and then by part of the group, n_finish the finishing of the groups (grad_L_XK and the norm gradients) in the same
-// order, PREFETCH: one per pair reads ahead of its walk.  With a finishing workgroup for each pair it stays with that
-// pair; with fewer, the last group of each pair is finished by a replaying workgroup, all of them together.
+// order.  With a finishing workgroup for each pair it stays with that
+// pair; with none (QUAD) the walkers finish what they walk; with fewer, the last group of each pair is finished by a replaying workgroup, all of them together.
 // Nobody waits for a later job than his own: a replay waits for the set of n_sets groups ago to be walked and finished, the
 // finishing of a group for its walk and the group before, a walk for its replay and the finishing of two groups ago; so of
 // the jobs not yet done the first can always go on.
-template <bool WIDE, bool IMG, bool PREFETCH, bool OWN, bool PARTS>
+template <bool WIDE, bool IMG, bool QUAD, bool OWN, bool PARTS>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // (57 to 64 pairs wait for their walks: the stores of the eighths cost them nothing, registers for the sum do: 64 x 128 2.231 ms so, 2.245 with them)
   constexpr bool EIGHTHS = PARTS || (!WIDE && OWN);
-  const int b = blockIdx.x, walkers = (WIDE ? 2 : 1) * p.gang_pairs;
-  const int slots = walkers + p.n_finish + p.n_replay + (PREFETCH ? p.gang_pairs : 0);
+  constexpr int WALKERS = QUAD ? BWQ_CUS : WIDE ? 2 : 1;   // per pair
+  const int b = blockIdx.x, walkers = WALKERS * p.gang_pairs;
+  const int slots = walkers + p.n_finish + p.n_replay;
   const int gang = uni(p.scatter ? b / slots : b & 7);   // (a division leaves its result in a vector register)
   int slot = uni(p.scatter ? b % slots : b >> 3);
   const int pairs = (p.nbh - gang + 7) / 8;   // of this gang
   // Where every pair has as many replaying workgroups, what belongs to a pair is placed side by side (24 pairs x 512 4.66 ms, 4.70 by
   // kind; the CUs that share an instruction cache are a few workgroups apart).
   if (OWN && slots % p.gang_pairs == 0) {
-    const int per = uni(slots / p.gang_pairs), n = WIDE ? 2 : 1, i = uni(slot / per), role = slot - i * per;
-    slot = role < n ? n * i + role : role == n ? walkers + i : PREFETCH && role == per - 1 ? slots - p.gang_pairs + i : walkers + p.gang_pairs + (role - n - 1) * p.gang_pairs + i;
+    const int per = uni(slots / p.gang_pairs), i = uni(slot / per), role = slot - i * per;
+    slot = role < WALKERS ? WALKERS * i + role : walkers + (role - WALKERS) * p.gang_pairs + i;
   }
   if (pairs <= 0) return;
   const int bh0 = p.bh0 + gang;
   if (slot < walkers) {
-    const int i = WIDE ? slot >> 1 : slot;
+    const int i = slot / WALKERS;
     if (i >= pairs) return;
-    if constexpr (WIDE) bwd_wide_walk<IMG>(p, smem, bh0 + 8 * i, slot & 1);
+    if constexpr (QUAD) bwd_quad_walk(p, smem, bh0 + 8 * i, slot & 3);
+    else if constexpr (WIDE) bwd_wide_walk(p, smem, bh0 + 8 * i, slot & 1);
     else bwd_body<2, IMG, true>(p, smem, bh0 + 8 * i, p.K - 1, 0);
     return;
   }
   slot -= walkers;
-  if constexpr (PREFETCH) {
-    if (slot >= p.n_finish + p.n_replay) {
-      const int i = slot - (p.n_finish + p.n_replay);
-      if (i < pairs) bwd_wide_prefetch(p, smem, bh0 + 8 * i);
-      return;
-    }
-  }
   if (WIDE && threadIdx.x < pairs) say_worker(p.sync + (size_t)(bh0 + 8 * (int)threadIdx.x) * BWD_SYNC_STRIDE + BWW_WORKERS);
   const bool replays = slot >= p.n_finish;
   const int r = slot - p.n_finish;
@@ -841,6 +772,7 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
       if (!bwd_body<1, IMG, true, WIDE, PARTS, false, EIGHTHS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
     }
   }
+  if constexpr (QUAD) return;
   if constexpr (OWN) {
     if (!replays && slot < pairs) bwd_finish_dxk<IMG, WIDE, true, EIGHTHS>(p, smem, bh0 + 8 * slot, p.K - 1);
   } else {
@@ -866,9 +798,9 @@ hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, TttKernel kernel, i
   auto launch = [&](auto k) -> hipError_t {
     const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
     int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-    const int nx = p.wide ? p.nbh * (ttt::BWW_XCHG_WORDS / 2) : 0;
+    const int per = kernel == BWD_GANG_AHEAD ? ttt::BWQ_XCHG_WORDS : ttt::BWW_XCHG_WORDS, nx = p.wide ? p.nbh * (per / 2) : 0;
     hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
-                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * ttt::BWW_XCHG_WORDS), nx);
+                       reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * per), nx);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);   // (while that runs)
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(grid), dim3(ttt::BW_THREADS), ttt::SM_BWD_BYTES, stream, p);

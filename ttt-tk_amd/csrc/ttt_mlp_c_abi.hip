@@ -154,11 +154,10 @@ struct LaunchPlan {
   long long n_rest = 0;     // pairs n_single .. n_single+n_rest-1
   bool rest_split = false;
   bool wide = false;
-  bool quad = false;        // forward, wide: the recurrence of a pair, and Out, on four CUs; else on two, and Out on a third
+  bool quad = false;        // wide: the recurrence (walk) of a pair, and what hangs on it, on four CUs; else on two
   int gang = 0;             // backward: pairs of an XCD that share workgroups, 0: whole ones, that replay or walk, for each pair
   int n_replay = 0;         // backward: that replay checkpoint groups, of a gang or of a pair
   int n_finish = 0;         // backward, of a gang: for grad_L_XK / grad_L_XV
-  bool prefetch = false;    // backward, wide: and one per pair that fetches ahead of the walk
   int sets = 0;             // backward: sets of the per-group tensors
   int shared = 0;           // backward: groups, the first ones walked, that several workgroups at once replay
   int parts = 1;            // backward: that many, a stretch of the group each
@@ -168,7 +167,7 @@ struct LaunchPlan {
   long long n_waiting() const { return helpers > 0 ? n_single : n_rest; }
   // Workgroups of an XCD: of a gang, or of the pairs that a forward with the recurrence on two CUs deals to it.
   int slots(bool backward) const {
-    return backward ? (wide ? 2 : 1) * gang + n_finish + n_replay + (prefetch ? gang : 0) : static_cast<int>((n_rest + 7) / 8) * per_pair(false);
+    return backward ? (quad ? 4 : wide ? 2 : 1) * gang + n_finish + n_replay : static_cast<int>((n_rest + 7) / 8) * per_pair(false);
   }
   // The launch behind the full rounds of one workgroup per pair: its kernel and its workgroups.
   TttKernel kernel(bool backward, int NC) const {
@@ -177,7 +176,7 @@ struct LaunchPlan {
     if (helpers > 0) return BWD_HELPED;
     if (!gang) return n_replay == 2 ? BWD_SPLIT_2 : BWD_SPLIT_1;
     const bool own = n_finish == gang;
-    if (prefetch) return BWD_GANG_AHEAD;
+    if (quad) return BWD_GANG_AHEAD;
     if (wide) return shared > 0 ? BWD_GANG_PARTS : own ? BWD_GANG_WIDE : BWD_GANG_WIDE_SHARED;
     return own ? BWD_GANG : BWD_GANG_SHARED;
   }
@@ -250,18 +249,19 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     pl.wide = fits_xcd(3);
     return pl;
   }
-  // Four replaying workgroups per pair leave a walk on two CUs to itself, also where they evaluate the GELU family for it (32 pairs x 512:
-  // 25 us per replayed mini-batch, 9.9 us per walked one, with a workgroup that fetches ahead).  What is left then is the walk's wait
-  // for the first group's replay: the first groups are replayed by two to four workgroups at once, and as many groups
+  // Three replaying workgroups per pair or more leave the walk to itself, also where they evaluate the GELU family for it, and it has four CUs
+  // (against two, one that fetches ahead for them and one that finishes, in ms: 2 pairs x 4 0.093 -> 0.064, 12 x 64 0.628 -> 0.541, 24 x 64
+  // 0.695 -> 0.592, 16 x 256 2.22 -> 1.88, 24 x 512 4.59 -> 3.94, 32 x 512 4.88 -> 4.28).  With two replaying ones (40 pairs) they would bound it:
+  // 54 k clocks a mini-batch, and the walk on four CUs takes 16 k.  What is left is the walk's wait for the first group's replay: the first groups are replayed by two to four workgroups at once, and as many groups
   // that way as it takes for a group replayed by one workgroup to be ready in time (three: replay of a group 57 k clocks a
-  // mini-batch, in two parts 35 k, in four 27 k; walk 19 k).  In ms, four replaying workgroups and whole groups -> so: 8 pairs x 64 in groups of 8
+  // mini-batch, in two parts 35 k, in four 27 k).  In ms, walk on two CUs, four replaying workgroups and whole groups -> so: 8 pairs x 64 in groups of 8
   // 0.683 -> 0.617 (four parts, eight workgroups), 24 x 64 0.733 -> 0.691 and 24 x 512 in groups of 32 4.88 -> 4.64 (three, six),
   // 32 x 512 5.12 -> 5.06 (two, four; all groups in parts: 5.25, the work done twice takes clock from the walk).
   const int on_xcd = cus / 8, pairs = static_cast<int>(per_xcd);
   if (fits_xcd(7)) {
     const int each = on_xcd / pairs - 4;
-    pl.wide = pl.prefetch = true;
-    pl.gang = pl.n_finish = pairs;
+    pl.wide = pl.quad = true;
+    pl.gang = pairs;
     pl.parts = each >= 8 ? 4 : each >= 6 ? 3 : each >= 4 ? 2 : 1;
     pl.shared = each >= 4 ? 3 : 0;
     pl.n_replay = (each >= 4 ? 2 * pl.parts : 3) * pairs;
@@ -362,7 +362,7 @@ SegmentPlan plan_segments(long long pairs, int cus, int NC, int cgs, bool backwa
 // twentieth for 40, by up to 11 %: 305 x 45 in groups of 5 2.75 cut, 3.03 uncut).
 long long rest_x1000(const LaunchPlan& pl, int NC, int K, bool backward) {
   if (!backward) return pl.quad ? 525LL * NC + 3000 : pl.wide ? 545LL * NC + 8000 : 650LL * NC + (NC >= 512 ? 32000 : 8000);
-  const int walk = pl.prefetch ? 210 : pl.wide ? (pl.gang > 6 ? 290 : 235) : pl.gang > 8 ? 380 : pl.gang ? 325 : pl.n_replay == 2 ? 405 : 485;
+  const int walk = pl.quad ? 210 : pl.wide ? (pl.gang > 6 ? 290 : 235) : pl.gang > 8 ? 380 : pl.gang ? 325 : pl.n_replay == 2 ? 405 : 485;
   return (long long)(walk + 470 / K) * NC * 21 / 20;
 }
 long long uncut_x1000(const LaunchPlan& pl, long long pairs, int cus, int NC, int cgs, bool with_workspace, bool backward) {
@@ -406,11 +406,12 @@ int bwd_sets_used(const LaunchPlan& pl, long long K) { return static_cast<int>(K
 bool helpers_pay(const LaunchPlan& pl, long long K) { return pl.helpers > 0 && 7 * pl.helpers * (K - 1) >= 4 * pl.n_waiting(); }
 // The launch with less workspace for the same pairs: two replaying workgroups per pair instead of three or four.
 LaunchPlan bwd_reduced(LaunchPlan pl) {
-  if (pl.prefetch) {
+  if (pl.quad) {
+    pl.n_finish = pl.gang;
     pl.n_replay = 2 * pl.gang;
     pl.parts = 1;
     pl.shared = 0;
-    pl.prefetch = false;
+    pl.quad = false;
     pl.sets = 4;
   }
   return pl;
@@ -462,7 +463,7 @@ LaunchPlan bwd_for_groups(LaunchPlan pl, int cus, long long cgs, long long K, lo
     pl.parts = 1;
     pl.shared = 0;
   }
-  const bool four = 4 * pl.gang <= cus / 8, shared = four ? pl.wide && pl.n_finish < pl.gang : pl.gang && !pl.wide;
+  const bool four = 4 * pl.gang <= cus / 8, shared = four ? pl.wide && !pl.quad && pl.n_finish < pl.gang : pl.gang && !pl.wide;
   if (!shared || cus / 8 > 64) return pl;
   const int n = static_cast<int>(NC), c = static_cast<int>(cgs), k = static_cast<int>(K);
   const int gang = pl.wide ? backward_span(pl.gang, pl.n_replay, pl.n_finish, true, COST_WALK_WIDE, COST_REPLAY, COST_FINISH, n, c, k)
@@ -511,6 +512,7 @@ Call plan_call(bool backward, const LaunchPlan& pl, long long pairs, int cus, in
 // words, the replay's shares of the norm gradients (one sum per set + a running sum), a parked image, what a walk on two
 // CUs exchanges, what the walk hands to the grad_L_XK workgroup (one image, dZ1, and two fp32 tiles, g_y and the norm-weight
 // gradient terms, per slot, two sets), what fewer of those than pairs park between two groups, then the sets of per-group tensors beyond the caller's; each part 256-byte aligned.
+static_assert(ttt::BWQ_XCHG_WORDS <= ttt::BWW_XCHG_WORDS + 2 * (TTT_MLP_CS * TTT_MLP_HID * 2 + 4 * TTT_MLP_CS * TTT_MLP_F * 2) / 8, "exchange of four CUs");
 struct BwdWorkspace {
   static constexpr int PER_SET = 11;
   static constexpr int ALT_SETS = ttt::BWD_MAX_SETS - 1;
@@ -536,10 +538,10 @@ struct BwdWorkspace {
     put(1, ttt::BWD_MAX_SETS * 8 * norm);
     put(2, norm);
     put(3, (size_t)n * img);
-    put(4, pl.wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);
+    put(4, pl.wide ? (size_t)n * ttt::BWW_XCHG_WORDS * 8 : 0);   // (a walk on four CUs exchanges through this and the next two, which it has no other use for)
     put(5, pl.gang ? 2 * slot * img : 0);
     put(6, pl.gang ? 2 * slot * 4 * tile : 0);
-    put(7, pl.n_finish < pl.gang ? (size_t)n * ttt::FIN_PARK_FLOATS * sizeof(float) : 0);
+    put(7, !pl.quad && pl.n_finish < pl.gang ? (size_t)n * ttt::FIN_PARK_FLOATS * sizeof(float) : 0);
     for (int s = 0; s < ALT_SETS; s++)
       for (int t = 0; t < PER_SET; t++) put(FIRST_SET + PER_SET * s + t, s < alt_sets ? per_set[t] : 0);
     total = o;
@@ -681,7 +683,6 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
   p.n_parts = pl.parts;
   for (int i = 0; i <= ttt::BWD_MAX_PARTS; i++) p.part_start[i] = PART_START[pl.parts - 1][i];
   p.n_finish = pl.n_finish;
-  p.n_prefetch = pl.prefetch ? 1 : 0;
   p.wide = pl.wide ? 1 : 0;
   p.wait_limit = g_wait_limit;
   p.report = report;
@@ -730,7 +731,7 @@ int bwd_launch(const ttt_mlp_bwd_args* a, void* workspace, size_t workspace_byte
                             p.alt_grad_output_fused_group[s], p.alt_std_fused_group[s], p.alt_W1_init_group[s]};
   }
   if (pl.gang) {
-    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * ttt::BWW_XCHG_WORDS;
+    p.xchg = reinterpret_cast<unsigned long long*>(base + w.off[4]) - b0 * (pl.quad ? ttt::BWQ_XCHG_WORDS : ttt::BWW_XCHG_WORDS);
     p.scatter = scatter ? 1 : 0;
     return static_cast<int>(ttt_mlp_bwd_gang_enqueue(p, kernel, grid, static_cast<hipStream_t>(stream)));
   }

@@ -104,15 +104,13 @@ struct BwdParams {
   float* fin_gy;
   float* fin_park;
   // wide: the walk on two workgroups, which exchange through xchg, [B*NH][2 parities][2 halves][2 token blocks][BWW_WORDS *
-  // 256 8-byte words].
-  // n_prefetch = 1 (with three or four replaying workgroups per pair): one more per pair reads nothing for itself; it touches every
-  // cache line that the walk is about to ask for, ahead of it, so that the walk's own requests are answered by the L2 the
-  // two share instead of by HBM.
+  // 256 8-byte words]; or on four, which form grad_L_XK, grad_L_XV and the norm gradients as well (n_finish = 0), and exchange through
+  // [B*NH][BWQ_XCHG_WORDS], which reaches into what fin_dz and fin_gy are otherwise.
   // scatter: the workgroups of a gang on consecutive XCDs instead of on one, for tests.
   int wide;
   unsigned long long* xchg;
   int n_sets;
-  int n_prefetch, scatter;
+  int scatter;
   int* sync;
   int* status;    // the status word behind the synchronisation words
   int* report;    // one more int, in host memory, that a wait that gives up is told to (or nullptr)
@@ -143,6 +141,8 @@ constexpr int BWD_HELP = 16;
 // BWW_XCD .. their XCDs, BWW_WORKERS (two words) the gang's other workgroups by XCD.
 constexpr int BWW_WORDS = 9;                                // per lane: two times 8 fp32 sums and the token's share of d eta
 constexpr int BWW_XCHG_WORDS = 2 * 2 * 2 * BWW_WORDS * 256;  // 8-byte words of a pair's exchange: 144 KiB
+// With the walk on four (ttt_mlp_bwd_quad.hpp, which names its own words): those that count groups done, words 8, 12 and 24, alike.
+constexpr int BWQ_XCHG_WORDS = 31744;                       // 248 KiB
 constexpr int BWW_WALKED = 8, BWW_GIVEN = 16, BWW_XCD = 26, BWW_WORKERS = 28;
 constexpr int FIN_PARK_FLOATS = 64 * 256 + 8 * 4 * 64;
 inline size_t bwd_sync_ints(long long BH) { return (size_t)BH * BWD_SYNC_STRIDE + 32; }   // 32: STATUS_WORDS (ttt_mlp_common.hpp)
@@ -270,7 +270,35 @@ enum BwdWideStage {
   BWH_STORE1,        // helpers: block 1's outputs stored, gradient wrt b2
   BWX_COUNT
 };
-static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <= STAGE_SLOTS && FQX_COUNT <= STAGE_SLOTS && BWX_COUNT <= STAGE_SLOTS, "stage slots");
+// The walk on four workgroups.
+enum BwdQuadStage {
+  BQC_BAR,           // compute: what the output branch adds to the running gradients
+  BQC_BX,            // compute: barrier behind it
+  BQC_STEP,          // compute: weight step backwards, shares of the sums
+  BQC_B1,            // compute: barrier behind it
+  BQC_PRODUCTS,      // compute: products that do not need the sums
+  BQC_B2,            // compute: barrier behind it (the sums have crossed, dZ2 is there)
+  BQC_MLP,           // compute: inner MLP backwards, the next mini-batch's output-branch images asked for
+  BQC_B3,            // compute: barrier behind it
+  BQC_UPDATE,        // compute: gradient wrt W1, shares of grad_L_XK, the next mini-batch's other images asked for
+  BQC_BE,            // compute: barrier behind it
+  BQH_GATHER,        // helpers: grad_L_XK's shares of the mini-batch before summed, XK and dl/dZ2 to LDS
+  BQH_BX,            // helpers: barrier behind it
+  BQH_ASK,           // helpers: those sums sent, marks, own tokens' inputs asked for, gradient wrt b2, next group waited for
+  BQH_B1,            // helpers: wait for the shares of the sums
+  BQH_SEND,          // helpers: sum over this CU's hidden columns, sent to the CUs that take it through the LayerNorm
+  BQH_TAKE,          // helpers, two of the four: wait for the other CUs' shares
+  BQH_LN,            // helpers, two of the four: second-order LayerNorm pass of 8 tokens, dZ2 sent
+  BQH_DXK,           // helpers, the other two: grad_L_XK of the mini-batch before
+  BQH_TAKE2,         // helpers: norm gradients; wait for the other CUs' dZ2
+  BQH_B2,            // helpers: barrier behind it
+  BQH_PUT,           // helpers: the next mini-batch's tiles asked for, gradient wrt b2
+  BQH_B3,            // helpers: wait for dZ1
+  BQH_NORM,          // helpers: per checkpoint group, the replays' norm-gradient sums; XQ and gZ2_bar to LDS, outputs
+  BQH_BE,            // helpers: wait for the end of the mini-batch
+  BQX_COUNT
+};
+static_assert(FS_COUNT <= STAGE_SLOTS && BS_COUNT <= STAGE_SLOTS && FWX_COUNT <= STAGE_SLOTS && FQX_COUNT <= STAGE_SLOTS && BWX_COUNT <= STAGE_SLOTS && BQX_COUNT <= STAGE_SLOTS, "stage slots");
 
 }  // namespace ttt
 

@@ -86,7 +86,7 @@ def main() -> int:
     header = open(os.path.join(HERE, "csrc", "ttt_mlp_kernels.hpp")).read()
     fwd_names, bwd_names = stage_names(header, "FwdStage"), stage_names(header, "BwdStage")
     fwd_wide_names, bwd_wide_names = stage_names(header, "FwdWideStage"), stage_names(header, "BwdWideStage")
-    fwd_quad_names = stage_names(header, "FwdQuadStage")
+    fwd_quad_names, bwd_quad_names = stage_names(header, "FwdQuadStage"), stage_names(header, "BwdQuadStage")
     if a.shape:
         B, NH, NC, cgs, eta_std = *(int(x) for x in a.shape.split(",")), 1.0
         label, option = "custom", f"--shape {a.shape}"
@@ -203,7 +203,11 @@ def main() -> int:
         out += table(f"backward, replaying workgroups, all that worked for a pair ({int(rep0.sum())} pairs)", cb[rep0, 0], bwd_names, NC) + [""]
     if (walk_b & rep0).any():
         out += table(f"backward, reverse-walk workgroup ({int((walk_b & rep0).sum())} pairs)", cb[walk_b & rep0, WALK], bwd_names, NC) + [""]
-    if wide_b.any():
+    if wide_b.any() and not ran(cb[:, DXK]).any():   # (of the four workgroups the first two keep clocks)
+        both = halves(cb, WALK_HALF)
+        out += table(f"backward, walk on four workgroups, compute waves ({int(wide_b.sum())} pairs)", both[:, :4], bwd_quad_names, NC) + [""]
+        out += table("backward, walk on four workgroups, helper waves", both[:, 4:], bwd_quad_names, NC) + [""]
+    elif wide_b.any():
         both = halves(cb, WALK_HALF)
         out += table(f"backward, walk on two workgroups, compute waves ({int(wide_b.sum())} pairs)", both[:, :4], bwd_wide_names, NC) + [""]
         out += table("backward, walk on two workgroups, helper waves", both[:, 4:], bwd_wide_names, NC) + [""]

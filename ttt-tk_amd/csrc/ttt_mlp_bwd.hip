@@ -475,7 +475,7 @@ TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
 // when the grid fits the CUs of the device.  A wait that sees no progress for p.wait_limit ticks of the
 // 100 MHz clock raises the status word and all of them leave, so every wave always exits.
 // ROLE 0: replay and reverse walk of every group in one workgroup; 1: one replay (k_hi = k_lo); 2: the reverse walks only.
-// IMG (two replaying workgroups per pair and the walk on one CU, three or four and the walk on two): the replay has time to spare and evaluates gelu,
+// IMG (two replaying workgroups per pair and the walk on one CU): the replay has time to spare and evaluates gelu,
 // gelu', gelu'' of the rounded Z1 for the walk, which gets them as three images instead of the image of Z1.  Same values
 // either way.
 // FIN: grad_L_XK is a leaf of the walk - it needs the running gradients, but nothing needs it.  Where one more workgroup

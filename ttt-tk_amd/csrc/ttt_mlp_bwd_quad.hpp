@@ -1,4 +1,4 @@
-// Reverse walk of one (batch, head) spread over four CUs, which form grad_L_XK, grad_L_XV and the norm gradients as well (up to 32
+// Reverse walk of one (batch, head) spread over four CUs, which form grad_L_XK, grad_L_XV and the norm gradients as well (up to 40
 // pairs on 256 CUs: the walk's chain is the bound there).
 //
 // CU `part` of a pair holds the hidden columns part and part + 4 of the eight of 32 (a wave of the one-workgroup kernel each), so its
@@ -20,13 +20,14 @@
 //
 // What bounds it: per-CU memory latency and issue, and then the chain.  A CU gets some 16 bytes per clock out of HBM (its requests in flight over the
 // latency), a wave that asks for more waits to issue, and the words an exchange waits for queue behind what was asked for before them.  A mini-batch
-// takes 90 KiB, so nothing is asked for between B1 and B2, where sums and dZ2 cross, except W1 (needed behind B2); images go
+// takes 74 KiB, so little is asked for between B1 and B2, where sums and dZ2 cross: W1 (needed behind B2) and the next Z1, whose GELU family the
+// compute waves evaluate in that wait (as images from the replays it was 16 KiB more, and 11 k clocks more of each replay); images go
 // straight to LDS where two waves need them (read twice by registers: 24 KiB more), and each stage's operands are asked for one or two
 // stages ahead.  24 pairs x 512, clocks per mini-batch with the stage clocks in: all operands asked for in a row behind B1 18.5 k, that
 // with tiles straight to LDS as well 20.9 k (4 bytes per lane and request; and behind such a request the compiler waits for all
 // of them before it reads LDS), spread as here 17.4 k, the helper waves' own sums out of scratch memory 16.2 k: what the output branch
-// adds 1.7 k, weight step backwards 3.0 k, sums out 0.9 k, their wait 2.2 k, LayerNorm 1.5 k, dZ2 crossing 1.3 k, inner MLP backwards 1.3 k, update
-// 1.7 k, the rest barriers.  Times of launches are at the rule that chooses it (ttt_mlp_c_abi.hip).
+// adds 1.7 k, weight step backwards 2.8 k, sums out 0.9 k, their wait 2.7 k, LayerNorm 1.5 k, dZ2 crossing 1.3 k, inner MLP backwards 1.3 k, update
+// 1.4 k, the rest barriers.  Times of launches are at the rule that chooses it (ttt_mlp_c_abi.hip).
 #pragma once
 #include "ttt_mlp_exchange.hpp"
 
@@ -151,15 +152,14 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
     if (flag(0) != 0) return;
     // Operands of a mini-batch, asked for during the one before it (its state is half of a wave's registers elsewhere).
     bf16x8 w2bf[2];                   // this wave's half of W2 before the step (lane = hid, contraction = F)
-    bf16x8 gq[2], aq[2], bq[2];       // gelu, gelu', gelu'' of Z1 of this wave's tokens
-    gptr_t gX2B, gGZ1B, gI1, gI2, gZ, gD;
+    bf16x8 gq[2], aq[2], bq[2];       // gelu, gelu', gelu'' of Z1 of this wave's tokens, evaluated a mini-batch ahead (gq: Z1 until then)
+    gptr_t gX2B, gGZ1B, gI1, gI2, gZ;
     auto group_images = [&](int set) {
       gX2B = gbuf(QGRP(X2_bar_group) + oh);
       gGZ1B = gbuf(QGRP(Z1_bar_group) + oh);
       gI1 = gbuf(QGRP(X2_group) + oh);
       gI2 = gbuf(QGRP(grad_l_wrt_Z1_group) + oh);
       gZ = gbuf(QGRP(Z1_group) + oh);
-      gD = gbuf(QGRP(W1_init_group) + oh);
     };
     const gptr_t gCk1 = gbuf(ka->W1_ck + ock), gCk2 = gbuf(ka->W2_ck + ock);
     auto ask_bar = [&](int j) {
@@ -179,11 +179,18 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
 #pragma unroll
         for (int t = 0; t < 2; t++) w2bf[t] = piece_from_f32(gCk2, static_cast<unsigned>(k) * (FD * HID * 4u), FD, hid0, 0, 2 * tb + t, c, h);
       }
+    };
+    auto ask_z = [&](int j) {
+      WQ_LANE;
+#pragma unroll
+      for (int t = 0; t < 2; t++) gq[t] = image_load<true>(gZ, j * IMG_BYTES, 2 * tb + t, t16);
+    };
+    auto gelu = [&]() {
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        gq[t] = image_load<true>(gZ, j * IMG_BYTES, 2 * tb + t, t16);
-        aq[t] = image_load<true>(gD, 2 * j * IMG_BYTES, 2 * tb + t, t16);
-        bq[t] = image_load<true>(gD, 2 * j * IMG_BYTES + IMG_BYTES, 2 * tb + t, t16);
+        const bf16x8 z = gq[t];
+        gelu_images<false>(z, gq[t], aq[t], bq[t]);
+        asm volatile("" : "+v"(gq[t]), "+v"(aq[t]), "+v"(bq[t]));   // finished here
       }
     };
     // gb1 += row sums of a 32-row operand of four pieces, formed on the matrix cores (as lds_rowsum_add_jit)
@@ -225,6 +232,8 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
       const int j0 = min(cgs, p.NC - (p.K - 1) * cgs) - 1;
       ask_bar(j0);
       ask_step(p.K - 1, j0);
+      ask_z(j0);
+      gelu();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();   // the first tiles
@@ -360,9 +369,10 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
             image_to_lds(gI1, (j - 1) * IMG_BYTES, 2 * tb + t, t16, s_w1);
         }
         QSCHED();
-        if (j == 0) group_images((done + 1) % n_sets);
+        if (j == 0) group_images((done + 1) % n_sets);   // (the helpers made sure of it before B1)
         const int kn = j > 0 || k == 0 ? k : k - 1, jn = j > 0 ? j - 1 : k == 0 ? 0 : cgs - 1;   // (behind the last mini-batch: dropped)
-        // ---- while they cross: the products that do not need them
+        ask_z(jn);
+        // ---- while they cross: the products that do not need them, and the next mini-batch's GELU family
         f32x16 q, dk[2];
         {
           WQ_LANE;
@@ -392,6 +402,7 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
             for (int t = 0; t < 2; t++) s_w1[64 * (2 * tb + t) + lane] = piece_from_f32(gCk1, static_cast<unsigned>(k) * (FD * HID * 4u), HID, 32 * tb, hid0, t, c, h);
           }
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // W1 is there
+          gelu();
         }
         QSCHED();
         TTT_STAGE(BQC_PRODUCTS);
@@ -456,7 +467,7 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
           if (tb == 1) add_gb1(rowsum(dz1));
           store_share(dk);
         }
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // the next mini-batch's images are there (all but the at least eight loads of ask_step)
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");   // the next mini-batch's images are there (what ask_step asked for is two loads at least)
         QSCHED();
         TTT_STAGE(BQC_UPDATE);
         __syncthreads();                                    // BE: grad_L_XK's shares; the next mini-batch's tiles

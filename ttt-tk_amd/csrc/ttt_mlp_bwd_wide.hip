@@ -13,7 +13,7 @@
 //
 // 48 pairs x 256 mini-batches 3.60 ms with the walk on one CU, 3.03 ms here; 48 x 4,096 49.8 -> 41.2 ms.
 // With the stage clocks in, 21.8 k clocks per mini-batch at 48 pairs, where the two replaying workgroups bound it (42.9 k clocks
-// per mini-batch each, hardly any of it waiting).  Up to 32 pairs, where this chain would be the bound (19.2 k), the walk has
+// per mini-batch each, hardly any of it waiting).  Up to 40 pairs, where this chain would be the bound (19.2 k), the walk has
 // four CUs (ttt_mlp_bwd_quad.hpp).
 #define TTT_BWD_ROLES_ONLY
 #include "ttt_mlp_bwd.hip"
@@ -726,11 +726,15 @@ namespace ttt {
 // Nobody waits for a later job than his own: a replay waits for the set of n_sets groups ago to be walked and finished, the
 // finishing of a group for its walk and the group before, a walk for its replay and the finishing of two groups ago; so of
 // the jobs not yet done the first can always go on.
-template <bool WIDE, bool IMG, bool QUAD, bool OWN, bool PARTS>
+// WIDE: the walk on several CUs, two, or with PARTS (groups replayed in parts) four.  IMG: the replays evaluate the GELU family for a walk on one CU
+// (on two or four its waves have the time).  EVEN: a walk on four, and as many replaying workgroups for every pair.  OWN: a
+// finishing workgroup, if any, for every pair.
+template <bool WIDE, bool IMG, bool EVEN, bool OWN, bool PARTS>
 __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // (57 to 64 pairs wait for their walks: the stores of the eighths cost them nothing, registers for the sum do: 64 x 128 2.231 ms so, 2.245 with them)
   constexpr bool EIGHTHS = PARTS || (!WIDE && OWN);
+  constexpr bool QUAD = WIDE && PARTS, IMAGES = IMG && !WIDE;
   constexpr int WALKERS = QUAD ? BWQ_CUS : WIDE ? 2 : 1;   // per pair
   const int b = blockIdx.x, walkers = WALKERS * p.gang_pairs;
   const int slots = walkers + p.n_finish + p.n_replay;
@@ -739,7 +743,7 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
   const int pairs = (p.nbh - gang + 7) / 8;   // of this gang
   // Where every pair has as many replaying workgroups, what belongs to a pair is placed side by side (24 pairs x 512 4.66 ms, 4.70 by
   // kind; the CUs that share an instruction cache are a few workgroups apart).
-  if (OWN && slots % p.gang_pairs == 0) {
+  if (QUAD ? EVEN : OWN && slots % p.gang_pairs == 0) {
     const int per = uni(slots / p.gang_pairs), i = uni(slot / per), role = slot - i * per;
     slot = role < WALKERS ? WALKERS * i + role : walkers + (role - WALKERS) * p.gang_pairs + i;
   }
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
     if (i >= pairs) return;
     if constexpr (QUAD) bwd_quad_walk(p, smem, bh0 + 8 * i, slot & 3);
     else if constexpr (WIDE) bwd_wide_walk(p, smem, bh0 + 8 * i, slot & 1);
-    else bwd_body<2, IMG, true>(p, smem, bh0 + 8 * i, p.K - 1, 0);
+    else bwd_body<2, IMAGES, true>(p, smem, bh0 + 8 * i, p.K - 1, 0);
     return;
   }
   slot -= walkers;
@@ -769,18 +773,18 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_gang_kernel(const BwdP
         before = shared;
       }
       const int q = uni(n / pairs), k = uni(p.K - 1 - (before + q));
-      if (!bwd_body<1, IMG, true, WIDE, PARTS, false, EIGHTHS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
+      if (!bwd_body<1, IMAGES, true, WIDE, PARTS, false, EIGHTHS>(p, smem, uni(bh0 + 8 * (n - q * pairs)), k, k, uni(part))) return;
     }
   }
   if constexpr (QUAD) return;
   if constexpr (OWN) {
-    if (!replays && slot < pairs) bwd_finish_dxk<IMG, WIDE, true, EIGHTHS>(p, smem, bh0 + 8 * slot, p.K - 1);
+    if (!replays && slot < pairs) bwd_finish_dxk<IMAGES, WIDE, true, EIGHTHS>(p, smem, bh0 + 8 * slot, p.K - 1);
   } else {
     // (n_replay >= pairs: one of the last groups each)
     const int last = (p.K - 1) * pairs, end = replays ? last + pairs : last;
     for (int job = replays ? last + r : slot; job < end; job += replays ? p.n_replay : p.n_finish) {
       const int done = uni(job / pairs);
-      if (!bwd_finish_dxk<IMG, WIDE, false, EIGHTHS>(p, smem, bh0 + 8 * (job - done * pairs), p.K - 1 - done)) return;
+      if (!bwd_finish_dxk<IMAGES, WIDE, false, EIGHTHS>(p, smem, bh0 + 8 * (job - done * pairs), p.K - 1 - done)) return;
     }
   }
 }
@@ -798,7 +802,7 @@ hipError_t ttt_mlp_bwd_gang_enqueue(const ttt::BwdParams& p, TttKernel kernel, i
   auto launch = [&](auto k) -> hipError_t {
     const int n = static_cast<int>(ttt::bwd_sync_ints(p.nbh));
     int* const words = p.status - (size_t)p.nbh * ttt::BWD_SYNC_STRIDE;   // p.sync and p.xchg are moved back by bh0 entries
-    const int per = kernel == BWD_GANG_AHEAD ? ttt::BWQ_XCHG_WORDS : ttt::BWW_XCHG_WORDS, nx = p.wide ? p.nbh * (per / 2) : 0;
+    const int per = kernel == BWD_GANG_AHEAD || kernel == BWD_GANG_PARTS ? ttt::BWQ_XCHG_WORDS : ttt::BWW_XCHG_WORDS, nx = p.wide ? p.nbh * (per / 2) : 0;
     hipLaunchKernelGGL(ttt::ttt_mlp_bwd_wide_clear, dim3(((nx > n ? nx : n) + 255) / 256), dim3(256), 0, stream, words, n, p.report,
                        reinterpret_cast<uint4*>(p.xchg + (size_t)p.bh0 * per), nx);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, ttt::SM_BWD_BYTES);   // (while that runs)

@@ -176,8 +176,8 @@ struct LaunchPlan {
     if (helpers > 0) return BWD_HELPED;
     if (!gang) return n_replay == 2 ? BWD_SPLIT_2 : BWD_SPLIT_1;
     const bool own = n_finish == gang;
-    if (quad) return BWD_GANG_AHEAD;
-    if (wide) return shared > 0 ? BWD_GANG_PARTS : own ? BWD_GANG_WIDE : BWD_GANG_WIDE_SHARED;
+    if (quad) return n_replay % gang == 0 ? BWD_GANG_AHEAD : BWD_GANG_PARTS;
+    if (wide) return own ? BWD_GANG_WIDE : BWD_GANG_WIDE_SHARED;
     return own ? BWD_GANG : BWD_GANG_SHARED;
   }
   long long grid(bool backward) const {
@@ -249,10 +249,12 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
     pl.wide = fits_xcd(3);
     return pl;
   }
-  // Three replaying workgroups per pair or more leave the walk to itself, also where they evaluate the GELU family for it, and it has four CUs
-  // (against two, one that fetches ahead for them and one that finishes, in ms: 2 pairs x 4 0.093 -> 0.064, 12 x 64 0.628 -> 0.541, 24 x 64
-  // 0.695 -> 0.592, 16 x 256 2.22 -> 1.88, 24 x 512 4.59 -> 3.94, 32 x 512 4.88 -> 4.28).  With two replaying ones (40 pairs) they would bound it:
-  // 54 k clocks a mini-batch, and the walk on four CUs takes 16 k.  What is left is the walk's wait for the first group's replay: the first groups are replayed by two to four workgroups at once, and as many groups
+  // Three replaying workgroups per pair or more leave the walk to itself, and it has four CUs (against two, with one more that fetched ahead for
+  // them and one that finished, in ms: 2 pairs x 4 0.093 -> 0.063, 12 x 64 0.627 -> 0.540, 24 x 64 0.695 -> 0.584, 16 x 256 2.22 -> 1.87,
+  // 24 x 512 4.59 -> 3.79, 32 x 512 4.87 -> 4.03; with the GELU family evaluated by the replays, three images instead of one, 24 x 512 3.94, 32 x 512
+  // 4.28).  The same with 2.4 of them (against three, two walking and one finishing: 33 x 128 1.44 -> 1.35, 40 x 64 0.817 -> 0.743, 40 x 256
+  // 2.79 -> 2.46): a replay takes 43 k clocks a mini-batch, the walk 16 k; with 1.3 (48 pairs) they would bound it by far.
+  // What is left is the walk's wait for the first group's replay: the first groups are replayed by two to four workgroups at once, and as many groups
   // that way as it takes for a group replayed by one workgroup to be ready in time (three: replay of a group 57 k clocks a
   // mini-batch, in two parts 35 k, in four 27 k).  In ms, walk on two CUs, four replaying workgroups and whole groups -> so: 8 pairs x 64 in groups of 8
   // 0.683 -> 0.617 (four parts, eight workgroups), 24 x 64 0.733 -> 0.691 and 24 x 512 in groups of 32 4.88 -> 4.64 (three, six),
@@ -277,14 +279,14 @@ LaunchPlan plan_for(long long BH, int cus, bool backward) {
   if (3 * pairs <= on_xcd) {
     pl.wide = 9 * pairs <= 2 * on_xcd;
     pl.gang = pairs;
-    if (fits_xcd(5)) {
+    if (fits_xcd(6)) {   // (33 to 40 pairs: twelve of an XCD replay for its five)
+      pl.quad = true;
+      pl.n_replay = on_xcd - 4 * pairs;
+      pl.parts = 2;
+      pl.shared = 1;
+    } else if (fits_xcd(5)) {
       pl.n_finish = pairs;
       pl.n_replay = 2 * pairs;
-      if (fits_xcd(6)) {   // (a third per pair pays once the first group is replayed in two parts: 40 x 512 5.67 -> 5.36 ms; five pairs on 32 CUs)
-        pl.n_replay = 3 * pairs;
-        pl.parts = 2;
-        pl.shared = 1;
-      }
     } else if (pl.wide) {
       divide_workers(pairs, on_xcd - 2 * pairs, COST_WALK_WIDE, COST_REPLAY, COST_FINISH, &pl.n_replay, &pl.n_finish);
     } else {

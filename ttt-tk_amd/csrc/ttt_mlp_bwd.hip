@@ -593,7 +593,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #define bGZ2 gbuf(GRP(grad_l_wrt_Z2_group) + of)
 #define bSDF gbuf(GRP(std_fused_group) + ot)
   // While a group is replayed the running gradients are parked in W*_init_group; during the reverse
-  // walk the same two 64 KiB slots park what must survive the LayerNorm stage (three 32 KiB images).
+  // walk the same two 64 KiB slots park what must survive the LayerNorm stage (block 0's half of three 32 KiB images).
   // Several workgroups per (batch, head): slot j of W1_init_group (of the set) carries gelu'(Z1) and gelu''(Z1)
   // of mini-batch j as two register images, and Z1_group carries gelu(Z1) instead of Z1.
 #define bDD gbuf(GRP(W1_init_group) + opk)
@@ -1383,12 +1383,16 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 
       TTT_STAGE(BS_W_BAR_TERMS);
       // ---- the weight step, backwards (uses the state BEFORE this mini-batch).
-      //      Parked across the LayerNorm stage: X2 in T0; packed d1 = gelu'(Z1), g1 = -eta * dl/dZ1 and
+      //      Kept across the LayerNorm stage: X2 in T0; packed d1 = gelu'(Z1), g1 = -eta * dl/dZ1 and
       //      t2 = -eta * (gZ2 W2^T) * (XK gW1 + gb1) * gelu''(Z1).
       bf16x8 dxv_old;            // LayerNorm lanes: the two outputs the stage accumulates into
       bf16 deta_old;
       bf16x8 xhf_n, gof_n;       // and the saved x_hat, grad_output, std of the fused LayerNorm
       float sdf_n;
+      // Block 1's of what block 0 parks across the LayerNorm stage (below).  With the GELU images, twelve of which are held while the
+      // blocks are computed, both blocks' are parked.
+      constexpr bool KEEP = !IMG;
+      bf16x8 k_uh[2], k_d1[2], k_t2[2], k_g1[2];
       {
         LANE_VARS;
         // T1 = W2 before the step, rows [hid][F]; T2 = gW1, rows [hid][F]
@@ -1446,13 +1450,26 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
               put_cvt<PAIRS>(g1c, jj, g[0], g[1]);
               put_cvt<PAIRS>(t2c, jj, t2[0], t2[1]);
             }
-            chunk_store(bPUH, 0, 2 * tb[i] + t, t16, uhc);
-            // nothing stays in registers across the LayerNorm stage: g1 and t2 (and, without the images,
-            // gelu'(Z1)) go to their parks at once (L2-resident, rewritten every mini-batch)
-            if constexpr (!IMG) chunk_store(bPW1, PARK_D1, 2 * tb[i] + t, t16, ac[t]);
-            chunk_store(bPW2, PARK_T2, 2 * tb[i] + t, t16, t2c);
-            // only grad_L_XK needs G1: its workgroup, where there is one, forms G1 itself
-            if constexpr (!FIN) chunk_store(bPW2, PARK_G1, 2 * tb[i] + t, t16, g1c);
+            // Block 0's go to their parks across the LayerNorm stage (rewritten every mini-batch): held as well, they are more than
+            // there are registers for while block 1 is computed (two of the four held: 14 registers spilled for 16).  Block 1's take the
+            // place of its R and S and stay, half of 256 KiB per mini-batch that 32 workgroups an L2 mostly sent through HBM (ms,
+            // forward + backward: 384 x 512 45.6 -> 43.2, 200 x 100 5.20 -> 5.01).
+            // Only grad_L_XK needs G1: its workgroup, where there is one, forms G1 itself.
+            if (KEEP && i == 1) {
+              k_uh[t] = uhc;
+              k_d1[t] = ac[t];
+              k_t2[t] = t2c;
+              asm volatile("" : "+v"(k_uh[t]), "+v"(k_d1[t]), "+v"(k_t2[t]));   // finished here, not where they are used
+              if constexpr (!FIN) {
+                k_g1[t] = g1c;
+                asm volatile("" : "+v"(k_g1[t]));
+              }
+            } else {
+              chunk_store(bPUH, 0, 2 * tb[i] + t, t16, uhc);
+              if constexpr (!IMG) chunk_store(bPW1, PARK_D1, 2 * tb[i] + t, t16, ac[t]);
+              chunk_store(bPW2, PARK_T2, 2 * tb[i] + t, t16, t2c);
+              if constexpr (!FIN) chunk_store(bPW2, PARK_G1, 2 * tb[i] + t, t16, g1c);
+            }
             store_piece_rows<LDH>(T0, tb[i], t, c, h, x2c[t]);             // X2 rows [tok][hid]
           }
           // pz[:, i] = gW2^T X2^T ; dEta partial ; + W2^T u^T
@@ -1580,6 +1597,10 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         bf16x8 w2b[4];   // W2 before the step: lane = hid, contraction = F
 #pragma unroll
         for (int s = 0; s < 4; s++) w2b[s] = w2_before<ROLE == 2>(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);   // second and last read
+        // converted anew: kept from the weight step backwards, the bf16 gradients are 32 registers (and spilled) for 32 instructions
+        if constexpr (KEEP)
+#pragma unroll
+          for (int fb = 0; fb < 2; fb++) asm volatile("" : "+v"(gW1s.b[fb][0]), "+v"(gW2s.b[0][fb]));
         // T2 = gW1 rows [hid][F] (for gW1 G1^T), T1 = gW2 rows [F][hid] (transposed read gives lane = hid)
         if constexpr (!FIN) store_state_rows<LDF>(T2, gW1s, c, h);
         store_state_rows<LDH>(T1, gW2s, c, h);
@@ -1588,7 +1609,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         acc_zero(dk);
         bf16x8 dzp[2][2], uhp[2][2];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int ib = 0; ib < 2; ib++) {
+          const int i = KEEP ? 1 - ib : ib;   // block 1 first, which has what it needs
           AccT<1, 1> dx2;
           acc_zero(dx2);
           mma_jit<4>(dx2, [&](int, int s) { return piece_tr<LDH>(T1, 0, s, lane); },           // gW2: lane = hid, contraction = F
@@ -1598,20 +1620,21 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           mma_jit<4>(dx2, [&](int, int s) { return w2b[s]; },                                  // + dZ2 W2^T
                      [&](int, int s) { return piece_rows<LDX>(s_a, tb[i], s, c, h); });
           // dk[:, i] = gW1 G1^T  (gW1: lane = F, contraction = hid)
-          bf16x8 g1c[2];
-          if constexpr (!FIN) {
-            g1c[0] = chunk_load(bPW2, PARK_G1, 2 * tb[i], t16);
-            g1c[1] = chunk_load(bPW2, PARK_G1, 2 * tb[i] + 1, t16);
+          bf16x8 g1c[2], d1c[2], t2c[2];
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            const int n = 2 * tb[i] + t;
+            if (KEEP && i == 1) {
+              if constexpr (!FIN) g1c[t] = k_g1[t];
+              d1c[t] = k_d1[t];
+              t2c[t] = k_t2[t];
+            } else {
+              if constexpr (!FIN) g1c[t] = chunk_load(bPW2, PARK_G1, n, t16);
+              if constexpr (!IMG) d1c[t] = chunk_load(bPW1, PARK_D1, n, t16);
+              else d1c[t] = image_load<true>(bDD, j * (2 * IMG_BYTES), n, t16);   // its last reader on this XCD
+              t2c[t] = chunk_load(bPW2, PARK_T2, n, t16);
+            }
           }
-          bf16x8 d1c[2];
-          if constexpr (!IMG) {
-            d1c[0] = chunk_load(bPW1, PARK_D1, 2 * tb[i], t16);
-            d1c[1] = chunk_load(bPW1, PARK_D1, 2 * tb[i] + 1, t16);
-          } else {
-            d1c[0] = image_load<true>(bDD, j * (2 * IMG_BYTES), 2 * tb[i], t16);   // its last reader on this XCD
-            d1c[1] = image_load<true>(bDD, j * (2 * IMG_BYTES), 2 * tb[i] + 1, t16);
-          }
-          const bf16x8 t2c[2] = {chunk_load(bPW2, PARK_T2, 2 * tb[i], t16), chunk_load(bPW2, PARK_T2, 2 * tb[i] + 1, t16)};
           if constexpr (!FIN) {
 #pragma unroll
             for (int t = 0; t < 2; t++)
@@ -1625,8 +1648,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             for (int jj = 0; jj < 8; jj += 2)
               put_cvt<PAIRS>(dzp[i][t], jj, __builtin_fmaf(dx2.b[0][0][8 * t + jj], (float)d1c[t][jj], (float)t2c[t][jj]),
                                        __builtin_fmaf(dx2.b[0][0][8 * t + jj + 1], (float)d1c[t][jj + 1], (float)t2c[t][jj + 1]));
-          uhp[i][0] = chunk_load(bPUH, 0, 2 * tb[i], t16);       // -eta * S * gelu', formed with S two stages back
-          uhp[i][1] = chunk_load(bPUH, 0, 2 * tb[i] + 1, t16);
+#pragma unroll
+          for (int t = 0; t < 2; t++) uhp[i][t] = KEEP && i == 1 ? k_uh[t] : chunk_load(bPUH, 0, 2 * tb[i] + t, t16);   // -eta * S * gelu', formed with S two stages back
         }
         bf16x8 w1bf[2][2];   // W1^T before the step (lane = F, contraction = hid), for the product after the next fence
         if constexpr (!FIN) {

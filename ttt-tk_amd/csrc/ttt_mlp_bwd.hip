@@ -353,7 +353,7 @@ TTT_DEV void stage3_store(const Staged3& s, bf16* sa, bf16* sb, bf16* sc, bf16* 
 
 // Piece s of W2[shard] before mini-batch j of the group as an operand (lane = hid row, contraction =
 // F): the image the replay stored after mini-batch j-1, or straight from the fp32 checkpoint.
-// STREAM: the second and last read of the image on this CU, so it need not stay in the L2.
+// STREAM: the only read of the image on this CU, so it need not stay in the L2.
 template <bool STREAM = false>
 TTT_DEV bf16x8 w2_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int s, int hid0, int c, int h, unsigned t16) {
   // the image offset is clamped so that the load stays inside the buffer even if it is hoisted above the branch
@@ -1356,7 +1356,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       {
         LANE_VARS;
 #pragma unroll
-        for (int s = 0; s < 4; s++) w2bf[s] = w2_before(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);
+        for (int s = 0; s < 4; s++) w2bf[s] = w2_before<ROLE == 2>(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);
         if constexpr (IMG) {   // the three GELU images of the next stage, under way during this one
 #pragma unroll
           for (int i = 0; i < 2; i++)
@@ -1389,6 +1389,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       bf16 deta_old;
       bf16x8 xhf_n, gof_n;       // and the saved x_hat, grad_output, std of the fused LayerNorm
       float sdf_n;
+      bf16x8 w2b[4];             // W2 before the step: lane = hid, contraction = F
       // Block 1's of what block 0 parks across the LayerNorm stage (below).  With the GELU images, twelve of which are held while the
       // blocks are computed, both blocks' are parked.
       constexpr bool KEEP = !IMG;
@@ -1493,6 +1494,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           const float a = half_sum_valu(de[i]);   // (a shuffle keeps a lane index over the loop, and reloads it here)
           if (h == 0) s_deta[v * CS + 32 * tb[i] + c] = a;
         }
+        // W2 is needed once more, behind the LayerNorm stage.  With several workgroups per pair it comes from T1, which is about to go:
+        // its image, read 25 k clocks ago, has left the L2 (backward, ms, 96 x 512 10.28 -> 9.91, 128 x 128 2.99 -> 2.89).  One workgroup
+        // per pair has no registers for it here (sixteen spilled, read twice) and asks for the image again.
+        if constexpr (ROLE == 2)
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            w2b[s] = piece_rows<LDF>(T1, 0, s, c, h);
+            asm volatile("" : "+v"(w2b[s]));
+          }
         WAVE_SYNC();   // this wave's readers of T1 / T2 are done
         TTT_STAGE(BS_W_STEP_BACK);
         {   // what the LayerNorm stage reads from HBM is under way during the pair sum
@@ -1594,9 +1604,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
       bf16x8 dxk_old;
       {
         LANE_VARS;
-        bf16x8 w2b[4];   // W2 before the step: lane = hid, contraction = F
+        if constexpr (ROLE == 0)
 #pragma unroll
-        for (int s = 0; s < 4; s++) w2b[s] = w2_before<ROLE == 2>(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);   // second and last read
+          for (int s = 0; s < 4; s++) w2b[s] = w2_before(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);   // second and last read
         // converted anew: kept from the weight step backwards, the bf16 gradients are 32 registers (and spilled) for 32 instructions
         if constexpr (KEEP)
 #pragma unroll

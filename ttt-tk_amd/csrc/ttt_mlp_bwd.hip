@@ -1142,11 +1142,16 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         TTT_STAGE(BS_R_OUT_LN);
         {
           LANE_VARS;
-          bf16x8 w1a[2][2];   // W1 after the step (lane = F, contraction = hid): the image stored above, fetched ahead of its use
+          // W1 after the step (lane = F, contraction = hid).  Beside a walk it is the image stored above, fetched ahead of its use; where
+          // the same workgroup walks, and every CU is busy, that is a trip to HBM, and it goes through T2 once more (backward,
+          // ms, 384 x 512 33.5 -> 33.3, 200 x 100 3.68 -> 3.65 or the same; 96 x 128, with 64 CUs idle, 2.65 -> 2.67).
+          constexpr bool W1_AGAIN = ROLE == 0;
+          bf16x8 w1a[2][2];
+          if constexpr (!W1_AGAIN)
 #pragma unroll
-          for (int rb = 0; rb < 2; rb++)
+            for (int rb = 0; rb < 2; rb++)
 #pragma unroll
-            for (int s = 0; s < 2; s++) w1a[rb][s] = chunk_load(bIMG1, j * IMG_BYTES, 2 * rb + s, t16);
+              for (int s = 0; s < 2; s++) w1a[rb][s] = chunk_load(bIMG1, j * IMG_BYTES, 2 * rb + s, t16);
           {
             LANE_VARS;
             AccT<1, 2> gz1b;   // (gZ2_bar W2^T) * gelu'(Z1_bar): rows hid, lane = tok
@@ -1185,10 +1190,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
                 store_piece_rows<LDH>(T1, tb[i], t, c, h, gzb);    // gZ1_bar rows [tok][hid]
               }
           }
-          WAVE_SYNC();
+          WAVE_SYNC();   // (W2's low-order term is read)
+          if constexpr (W1_AGAIN) {
+            store_state_rows<LDF>(T2, W1s, c, h);   // rows [hid][F]
+            WAVE_SYNC();
+          }
           AccT<2, 2> dq;
           acc_zero(dq);
-          mma_jit<2>(dq, [&](int rb, int s) { return w1a[rb][s]; },                                // W1 after: lane = F
+          mma_jit<2>(dq, [&](int rb, int s) { return W1_AGAIN ? piece_tr<LDF>(T2, rb, s, lane) : w1a[rb][s]; },
                      [&](int i, int s) { return piece_rows<LDH>(T1, tb[i], s, c, h); });                   // gZ1_bar: lane = tok
           // what the reverse walk adds to the running gradients, as ready-made operands (lane = hid, contraction = tok)
 #pragma unroll

@@ -95,19 +95,12 @@ constexpr unsigned IMG_BYTES = CS * HID * 2;          // 32 KiB
 constexpr unsigned CHUNK_BYTES = BW_THREADS * 16;     // 8 KiB
 constexpr unsigned TILE_BYTES = CS * FD * 2;          // one [64][64] bf16 tile in HBM: 8 KiB
 TTT_DEV void chunk_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) { g_st8h(b, t16, img + n * CHUNK_BYTES, v); }
-// The replay's images: written once and read a checkpoint group later.  When another workgroup reads them
-// (STREAM) they bypass the cache hierarchy as far as the hardware lets them, so that they do not push out
-// lines that are re-used; with one workgroup per (batch, head) keeping them cached measured faster.
-template <bool STREAM>
-TTT_DEV void image_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) {
-  if constexpr (STREAM) g_st_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES, v);
-  else g_st8h(b, t16, img + n * CHUNK_BYTES, v);
-}
-template <bool STREAM>
-TTT_DEV bf16x8 image_load(gptr_t b, unsigned img, int n, unsigned t16) {
-  if constexpr (STREAM) return g_ld_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES);
-  else return g_ld8h(b, t16, img + n * CHUNK_BYTES);
-}
+// The replay's images: written once and read a checkpoint group later, with streaming stores and loads, so that they do not push out
+// lines that are re-used.  With one workgroup per (batch, head) those are the walk's parks: since they take 64 KiB instead of 128,
+// 2 MiB of an XCD's 4 MiB L2 with every CU busy, streaming everything else keeps them there (backward, ms, 384 x 512 33.5 -> 32.0,
+// 200 x 100 3.68 -> 3.51; it gave nothing while they took the whole of it).
+TTT_DEV void image_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) { g_st_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES, v); }
+TTT_DEV bf16x8 image_load(gptr_t b, unsigned img, int n, unsigned t16) { return g_ld_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES); }
 TTT_DEV bf16x8 chunk_load(gptr_t b, unsigned img, int n, unsigned t16) { return g_ld8h(b, t16, img + n * CHUNK_BYTES); }
 
 // fp32 accumulator tile <-> HBM in the caller's row-major layout.  `ld` = row length, (r0, c0) =
@@ -147,13 +140,9 @@ TTT_DEV void ln_store_h(bf16* p, bf16x8 v) {
 }
 template <bool PAIRS = false>
 TTT_DEV void ln_store(bf16* p, const float (&x)[8]) { ln_store_h(p, cvt8<PAIRS>(x)); }
-// 8 features of this lane's token to / from a [tok][F] bf16 tile in HBM (16 bytes per lane).
-template <bool STREAM = false, bool PAIRS = false>
-TTT_DEV void ln_store_g(gptr_t b, unsigned voff, unsigned soff, const float (&x)[8]) {
-  const bf16x8 v = cvt8<PAIRS>(x);
-  if constexpr (STREAM) g_st_stream<bf16x8>(b, voff, soff, v);
-  else g_st8h(b, voff, soff, v);
-}
+// 8 features of this lane's token to a [tok][F] bf16 tile in HBM (16 bytes per lane), which is read a checkpoint group later.
+template <bool PAIRS = false>
+TTT_DEV void ln_store_g(gptr_t b, unsigned voff, unsigned soff, const float (&x)[8]) { g_st_stream<bf16x8>(b, voff, soff, cvt8<PAIRS>(x)); }
 TTT_DEV void ln_cvt8(float (&x)[8], bf16x8 v) {
 #pragma unroll
   for (int e = 0; e < 8; e++) x[e] = (float)v[e];
@@ -357,13 +346,13 @@ TTT_DEV void stage3_store(const Staged3& s, bf16* sa, bf16* sb, bf16* sc, bf16* 
 template <bool STREAM = false>
 TTT_DEV bf16x8 w2_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int s, int hid0, int c, int h, unsigned t16) {
   // the image offset is clamped so that the load stays inside the buffer even if it is hoisted above the branch
-  bf16x8 r = image_load<STREAM>(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, s, t16);
+  bf16x8 r = STREAM ? image_load(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, s, t16) : chunk_load(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, s, t16);
   if (j == 0) r = piece_from_f32(ck, ck_off, FD, hid0, 0, s, c, h);
   return r;
 }
 // Piece (row block rb, k-step s) of W1[:, shard]^T before mini-batch j (lane = F row, contraction = hid).
 TTT_DEV bf16x8 w1_before(gptr_t img, gptr_t ck, unsigned ck_off, int j, int rb, int s, int hid0, int c, int h, unsigned t16) {
-  bf16x8 r = image_load<false>(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, 2 * rb + s, t16);
+  bf16x8 r = image_load(img, (j > 0 ? j - 1 : 0) * IMG_BYTES, 2 * rb + s, t16);
   if (j == 0) r = piece_from_f32(ck, ck_off, HID, 32 * rb, hid0, s, c, h);
   return r;
 }
@@ -771,15 +760,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             for (int t = 0; t < 2; t++) {
               const bf16x8 zr = pack8<PAIRS>(x2.b[0][i], t);
               if constexpr (FULL && !IMG) {
-                image_store<ROLE != 0>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
+                image_store(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
               } else if constexpr (FULL) {
                 // The walk needs gelu, gelu' and gelu'' of the ROUNDED Z1 (what it would compute from the image
                 // of Z1); a replaying workgroup has the time to do that for it.
                 bf16x8 gv, av, bv;
                 gelu_images<PAIRS>(zr, gv, av, bv);
-                image_store<ROLE != 0>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, gv);
-                image_store<ROLE != 0>(bDD, j * (2 * IMG_BYTES), 2 * tb[i] + t, t16, av);
-                image_store<ROLE != 0>(bDD, j * (2 * IMG_BYTES) + IMG_BYTES, 2 * tb[i] + t, t16, bv);
+                image_store(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, gv);
+                image_store(bDD, j * (2 * IMG_BYTES), 2 * tb[i] + t, t16, av);
+                image_store(bDD, j * (2 * IMG_BYTES) + IMG_BYTES, 2 * tb[i] + t, t16, bv);
               }
               bf16x8 xv;
 #pragma unroll
@@ -850,14 +839,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             }
           }
           if constexpr (FULL) {
-            ln_store_g<ROLE != 0, PAIRS>(bXHF, vln, j * TILE_BYTES, z);
-            ln_store_g<ROLE != 0, PAIRS>(bGOF, vln, j * TILE_BYTES, go);
+            ln_store_g<PAIRS>(bXHF, vln, j * TILE_BYTES, z);
+            ln_store_g<PAIRS>(bGOF, vln, j * TILE_BYTES, go);
           }
           const float s1 = oct_sum(sum8(gx)), s2 = oct_sum(dot8(gx, z));
           const float sc = rstd * (1.f / FD), neg_eta = -bf2f(s_etah[tok]);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;   // dl/dZ2
-          if constexpr (FULL) ln_store_g<ROLE != 0, PAIRS>(bGZ2, vln, j * TILE_BYTES, gx);
+          if constexpr (FULL) ln_store_g<PAIRS>(bGZ2, vln, j * TILE_BYTES, gx);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] *= neg_eta;                             // G2, in two terms (the second in
           ln_token_sum_store(s_deta + v * CS, gx, lane, f0);   // b2's step: this wave's share (s_deta is the walk's otherwise)
@@ -1036,12 +1025,12 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int s = 0; s < 4; s++) {
             w2a[s] = piece_tr<LDH>(T1, 0, s, lane);
-            image_store<ROLE != 0>(bIMG2, j * IMG_BYTES, s, t16, w2a[s]);
+            image_store(bIMG2, j * IMG_BYTES, s, t16, w2a[s]);
           }
 #pragma unroll
           for (int fb = 0; fb < 2; fb++)
 #pragma unroll
-            for (int s = 0; s < 2; s++) image_store<ROLE != 0>(bIMG1, j * IMG_BYTES, 2 * fb + s, t16, piece_tr<LDF>(T2, fb, s, lane));
+            for (int s = 0; s < 2; s++) image_store(bIMG1, j * IMG_BYTES, 2 * fb + s, t16, piece_tr<LDF>(T2, fb, s, lane));
         }
         TTT_STAGE(BS_R_IMAGES);
         // post-update forward on XQ; X2_bar rows [tok][hid] -> T0, gelu'(Z1_bar) packed
@@ -1136,7 +1125,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;
           ln_store<PAIRS>(s_a + tok * LDX + f0, gx);            // gZ2_bar
-          ln_store_g<ROLE != 0, PAIRS>(bGZB, vln, j * TILE_BYTES, gx);
+          ln_store_g<PAIRS>(bGZB, vln, j * TILE_BYTES, gx);
         }
         __syncthreads();
         TTT_STAGE(BS_R_OUT_LN);
@@ -1202,8 +1191,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           // what the reverse walk adds to the running gradients, as ready-made operands (lane = hid, contraction = tok)
 #pragma unroll
           for (int s = 0; s < 4; s++) {
-            image_store<ROLE != 0>(bX2B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T0, 0, s, lane));
-            image_store<ROLE != 0>(bGZ1B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T1, 0, s, lane));
+            image_store(bX2B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T0, 0, s, lane));
+            image_store(bGZ1B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T1, 0, s, lane));
           }
           WAVE_SYNC();   // every reader of T1 / T2 is done before the pair sum takes their place
           {
@@ -1317,15 +1306,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #define WALK_FETCH(jn)                                                                                   \
     {                                                                                                    \
       LANE_VARS;                                                                                         \
-      constexpr bool ST = ROLE != 0;   /* tiles another workgroup left here are read once */             \
       const int jf = __builtin_amdgcn_readfirstlane(jn), mbf = k * cgs + jf;                             \
       const unsigned xo = mbf * TILE_BYTES, so = jf * TILE_BYTES;                                        \
       n_etai[0] = g_ldh(bETA, 2 * c, mbf * (CS * 2) + 64 * tb[0]);                                       \
       n_etai[1] = g_ldh(bETA, 2 * c, mbf * (CS * 2) + 64 * tb[1]);                                       \
-      n_xq = ST ? g_ld_stream<u32x4>(bXQ, t16, xo) : g_ld16(bXQ, t16, xo);                               \
-      n_xk = ST ? g_ld_stream<u32x4>(bXK, t16, xo) : g_ld16(bXK, t16, xo);                               \
-      n_gz = ST ? g_ld_stream<u32x4>(bGZ2, t16, so) : g_ld16(bGZ2, t16, so);                             \
-      n_gzb = ST ? g_ld_stream<u32x4>(bGZB, t16, so) : g_ld16(bGZB, t16, so);                            \
+      n_xq = g_ld_stream<u32x4>(bXQ, t16, xo);                                                           \
+      n_xk = g_ld_stream<u32x4>(bXK, t16, xo);                                                           \
+      n_gz = g_ld_stream<u32x4>(bGZ2, t16, so);                                                          \
+      n_gzb = g_ld_stream<u32x4>(bGZB, t16, so);                                                         \
       n_eta = g_ldh(bETA, 2 * (tid & (CS - 1)), mbf * (CS * 2));                                         \
     }
     if constexpr (ROLE != 1) WALK_FETCH(n_mb - 1);
@@ -1347,8 +1335,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         // the two operand images of the next stage are asked for here: on their way across both barriers
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-          x2b[s] = image_load<ROLE != 0>(bX2B, ho, s, t16);
-          g1b[s] = image_load<ROLE != 0>(bGZ1B, ho, s, t16);
+          x2b[s] = image_load(bX2B, ho, s, t16);
+          g1b[s] = image_load(bGZ1B, ho, s, t16);
         }
         __syncthreads();   // the previous mini-batch's readers of these tiles are done
         lds_put16x(s_xq, tid, n_xq);
@@ -1371,15 +1359,15 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-              gq[i][t] = image_load<true>(bZ1, ho, 2 * tb[i] + t, t16);
+              gq[i][t] = image_load(bZ1, ho, 2 * tb[i] + t, t16);
               aq[i][t] = chunk_load(bDD, j * (2 * IMG_BYTES), 2 * tb[i] + t, t16);   // read again two stages on
-              bq[i][t] = image_load<true>(bDD, j * (2 * IMG_BYTES) + IMG_BYTES, 2 * tb[i] + t, t16);
+              bq[i][t] = image_load(bDD, j * (2 * IMG_BYTES) + IMG_BYTES, 2 * tb[i] + t, t16);
             }
         } else {               // the image of Z1 (gq takes it), from which the next stage evaluates the three
 #pragma unroll
           for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int t = 0; t < 2; t++) gq[i][t] = image_load<ROLE != 0>(bZ1, ho, 2 * tb[i] + t, t16);
+            for (int t = 0; t < 2; t++) gq[i][t] = image_load(bZ1, ho, 2 * tb[i] + t, t16);
         }
         mma_jit<4>(gW2s, [&](int, int s) { return x2b[s]; },                                   // X2_bar^T: lane = hid
                    [&](int fb, int s) { return piece_tr<LDX>(s_a, fb, s, lane); });            // gZ2_bar: lane = F
@@ -1518,8 +1506,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           LANE_VARS;
           if constexpr (!FIN) dxv_old = g_ld_stream<bf16x8>(OLD_VALUE(bDXV, xo));
           deta_old = g_ldh(ka->overwrite ? gbuf(zero_tile) : bDETA, 2 * tok, ka->overwrite ? 0u : mb * (CS * 2));
-          xhf_n = ROLE != 0 ? g_ld_stream<bf16x8>(bXHF, vln, so) : g_ld8h(bXHF, vln, so);
-          gof_n = ROLE != 0 ? g_ld_stream<bf16x8>(bGOF, vln, so) : g_ld8h(bGOF, vln, so);
+          xhf_n = g_ld_stream<bf16x8>(bXHF, vln, so);
+          gof_n = g_ld_stream<bf16x8>(bGOF, vln, so);
           sdf_n = g_ldf(bSDF, vtok, j * (CS * 4));
         }
         pair_sum(s_own, s_partner, pz, c, h);
@@ -1615,7 +1603,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         LANE_VARS;
         if constexpr (ROLE == 0)
 #pragma unroll
-          for (int s = 0; s < 4; s++) w2b[s] = w2_before(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);   // second and last read
+          for (int s = 0; s < 4; s++) w2b[s] = w2_before<true>(bIMG2, bCW2, ckW, j, s, hid0, c, h, t16);   // second and last read
         // converted anew: kept from the weight step backwards, the bf16 gradients are 32 registers (and spilled) for 32 instructions
         if constexpr (KEEP)
 #pragma unroll
@@ -1650,7 +1638,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             } else {
               if constexpr (!FIN) g1c[t] = chunk_load(bPW2, PARK_G1, n, t16);
               if constexpr (!IMG) d1c[t] = chunk_load(bPW1, PARK_D1, n, t16);
-              else d1c[t] = image_load<true>(bDD, j * (2 * IMG_BYTES), n, t16);   // its last reader on this XCD
+              else d1c[t] = image_load(bDD, j * (2 * IMG_BYTES), n, t16);   // its last reader on this XCD
               t2c[t] = chunk_load(bPW2, PARK_T2, n, t16);
             }
           }
@@ -1680,7 +1668,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int t = 0; t < 2; t++) image_store<true>(bFDZ, ho, 2 * tb[i] + t, t16, dzp[i][t]);
+            for (int t = 0; t < 2; t++) image_store(bFDZ, ho, 2 * tb[i] + t, t16, dzp[i][t]);
         }
         TTT_STAGE(BS_W_MLP_BACK);
         WAVE_SYNC();   // S, P2 and gW1 G1^T have consumed T2 / T1
@@ -1921,13 +1909,13 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
     auto ask_g1b = [&](int jn) {
       FIN_LANE;
 #pragma unroll
-      for (int s = 0; s < 4; s++) g1b[s] = image_load<true>(gGZ1B, jn * IMG_BYTES, s, t16);
+      for (int s = 0; s < 4; s++) g1b[s] = image_load(gGZ1B, jn * IMG_BYTES, s, t16);
     };
     auto ask_w2 = [&](int jn) {
       FIN_LANE;
       if (jn > 0) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) w2bf[s] = image_load<true>(gIMG2, (jn - 1) * IMG_BYTES, s, t16);
+        for (int s = 0; s < 4; s++) w2bf[s] = image_load(gIMG2, (jn - 1) * IMG_BYTES, s, t16);
       } else {
 #pragma unroll
         for (int s = 0; s < 4; s++) w2bf[s] = piece_from_f32(gCW2, ckW, FD, hid0, 0, s, c, h);
@@ -1938,7 +1926,7 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
 #pragma unroll
       for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int t = 0; t < 2; t++) d1[a][t] = image_load<true>(gDD, jn * (IMG ? 2 * IMG_BYTES : IMG_BYTES), 2 * tb[a] + t, t16);
+        for (int t = 0; t < 2; t++) d1[a][t] = image_load(gDD, jn * (IMG ? 2 * IMG_BYTES : IMG_BYTES), 2 * tb[a] + t, t16);
     };
     auto ask_w1 = [&](int jn) {   // W1 before the step
       FIN_LANE;
@@ -1946,7 +1934,7 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
-          for (int t = 0; t < 2; t++) w1b[a][t] = image_load<true>(gIMG1, (jn - 1) * IMG_BYTES, 2 * a + t, t16);
+          for (int t = 0; t < 2; t++) w1b[a][t] = image_load(gIMG1, (jn - 1) * IMG_BYTES, 2 * a + t, t16);
       } else {
 #pragma unroll
         for (int a = 0; a < 2; a++)
@@ -1993,7 +1981,7 @@ TTT_DEV bool bwd_finish_dxk(const BwdParams& p, unsigned char* smem, const int b
 #pragma unroll
       for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int t = 0; t < 2; t++) dz[a][t] = image_load<true>(gDZ, ho, 2 * tb[a] + t, t16);
+        for (int t = 0; t < 2; t++) dz[a][t] = image_load(gDZ, ho, 2 * tb[a] + t, t16);
       const float eta_i[2] = {bf2f(eta_n[0]), bf2f(eta_n[1])};
       lds_put16x(s_xq, tid, xq);
       lds_put16x(s_xk, tid, xk);

@@ -174,7 +174,7 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
       WQ_LANE;
       if (j > 0) {
 #pragma unroll
-        for (int t = 0; t < 2; t++) w2bf[t] = image_load<false>(gI2, (j - 1) * IMG_BYTES, 2 * tb + t, t16);
+        for (int t = 0; t < 2; t++) w2bf[t] = chunk_load(gI2, (j - 1) * IMG_BYTES, 2 * tb + t, t16);
       } else {
 #pragma unroll
         for (int t = 0; t < 2; t++) w2bf[t] = piece_from_f32(gCk2, static_cast<unsigned>(k) * (FD * HID * 4u), FD, hid0, 0, 2 * tb + t, c, h);
@@ -183,7 +183,7 @@ TTT_DEV void bwd_quad_walk(const BwdParams& p, unsigned char* smem, const int bh
     auto ask_z = [&](int j) {
       WQ_LANE;
 #pragma unroll
-      for (int t = 0; t < 2; t++) gq[t] = image_load<true>(gZ, j * IMG_BYTES, 2 * tb + t, t16);
+      for (int t = 0; t < 2; t++) gq[t] = image_load(gZ, j * IMG_BYTES, 2 * tb + t, t16);
     };
     auto gelu = [&]() {
 #pragma unroll

@@ -152,7 +152,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       WW_LANE;
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        gq[i][t] = image_load<false>(gZ, j * IMG_BYTES, 2 * i + t, t16);
+        gq[i][t] = chunk_load(gZ, j * IMG_BYTES, 2 * i + t, t16);
       }
     };
     // Operands are asked for one to two stages ahead (one CU cannot keep enough requests in flight to hide the way to HBM: 80 KiB
@@ -161,15 +161,15 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
       WW_LANE;
 #pragma unroll
       for (int s = 0; s < 4; s++) {
-        x2b[s] = image_load<true>(gX2B, j * IMG_BYTES, s, t16);
-        g1b[s] = image_load<false>(gGZ1B, j * IMG_BYTES, s, t16);
+        x2b[s] = image_load(gX2B, j * IMG_BYTES, s, t16);
+        g1b[s] = chunk_load(gGZ1B, j * IMG_BYTES, s, t16);
       }
     };
     auto ask_step = [&](int k, int j) {
       WW_LANE;
       if (j > 0) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) w2bf[s] = image_load<false>(gI2, (j - 1) * IMG_BYTES, s, t16);
+        for (int s = 0; s < 4; s++) w2bf[s] = chunk_load(gI2, (j - 1) * IMG_BYTES, s, t16);
       } else {
 #pragma unroll
         for (int s = 0; s < 4; s++) w2bf[s] = piece_from_f32(gCk, static_cast<unsigned>(k) * (FD * HID * 4u), FD, hid0, 0, s, c, h);
@@ -383,7 +383,7 @@ TTT_DEV void bwd_wide_walk(const BwdParams& p, unsigned char* smem, const int bh
             bf16x8 dz;
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) dz[jj] = (bf16)__builtin_fmaf(q[8 * t + jj], (float)d1p[i][t][jj], (float)t2p[i][t][jj]);   // dZ1
-            image_store<true>(gDZ, ho, 2 * i + t, t16, dz);                                    // for the grad_L_XK workgroup
+            image_store(gDZ, ho, 2 * i + t, t16, dz);                                    // for the grad_L_XK workgroup
             store_piece_rows<LDH>(T2, i, t, c, h, dz);                                         // rows [tok][hid]
           }
 #pragma unroll

@@ -99,7 +99,12 @@ TTT_DEV void chunk_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) 
 // lines that are re-used.  With one workgroup per (batch, head) those are the walk's parks: since they take 64 KiB instead of 128,
 // 2 MiB of an XCD's 4 MiB L2 with every CU busy, streaming everything else keeps them there (backward, ms, 384 x 512 33.5 -> 32.0,
 // 200 x 100 3.68 -> 3.51; it gave nothing while they took the whole of it).
-TTT_DEV void image_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) { g_st_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES, v); }
+// CACHED: few pairs with one workgroup each, whose groups the memory-side cache holds until they are walked (below).
+template <bool CACHED = false>
+TTT_DEV void image_store(gptr_t b, unsigned img, int n, unsigned t16, bf16x8 v) {
+  if constexpr (CACHED) chunk_store(b, img, n, t16, v);
+  else g_st_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES, v);
+}
 TTT_DEV bf16x8 image_load(gptr_t b, unsigned img, int n, unsigned t16) { return g_ld_stream<bf16x8>(b, t16, img + n * CHUNK_BYTES); }
 TTT_DEV bf16x8 chunk_load(gptr_t b, unsigned img, int n, unsigned t16) { return g_ld8h(b, t16, img + n * CHUNK_BYTES); }
 
@@ -141,8 +146,12 @@ TTT_DEV void ln_store_h(bf16* p, bf16x8 v) {
 template <bool PAIRS = false>
 TTT_DEV void ln_store(bf16* p, const float (&x)[8]) { ln_store_h(p, cvt8<PAIRS>(x)); }
 // 8 features of this lane's token to a [tok][F] bf16 tile in HBM (16 bytes per lane), which is read a checkpoint group later.
-template <bool PAIRS = false>
-TTT_DEV void ln_store_g(gptr_t b, unsigned voff, unsigned soff, const float (&x)[8]) { g_st_stream<bf16x8>(b, voff, soff, cvt8<PAIRS>(x)); }
+template <bool CACHED, bool PAIRS>
+TTT_DEV void ln_store_g(gptr_t b, unsigned voff, unsigned soff, const float (&x)[8]) {
+  const bf16x8 v = cvt8<PAIRS>(x);
+  if constexpr (CACHED) g_st8h(b, voff, soff, v);
+  else g_st_stream<bf16x8>(b, voff, soff, v);
+}
 TTT_DEV void ln_cvt8(float (&x)[8], bf16x8 v) {
 #pragma unroll
   for (int e = 0; e < 8; e++) x[e] = (float)v[e];
@@ -474,7 +483,7 @@ TTT_DEV bool help_take(const BwdParams& p, int me, int* job) {
 // PARTS: several workgroups at once replay each of the p.n_shared groups walked first, a stretch of its mini-batches each.
 // HELPED: a workgroup that replays and walks (ROLE 0) where others (ROLE 1) replay groups ahead of it.
 // EIGHTHS: a replay hands over its norm-gradient sums by eighths of the group (eighth_done); needed with PARTS.
-template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false, bool HELPED = false, bool EIGHTHS = PARTS>
+template <int ROLE, bool IMG, bool FIN, bool WIDE = false, bool PARTS = false, bool HELPED = false, bool EIGHTHS = PARTS, bool CACHED = false>
 // k_hi, k_lo: the checkpoint groups k_hi, k_hi - 1, .. k_lo of the sequence (ROLE 0: a segment; ROLE 2: K - 1 .. 0).
 // part (PARTS): which of the p.n_parts stretches of the group's mini-batches this workgroup replays; it takes the state there from
 // the checkpoint itself, through the state-carrying half of the mini-batches before (`light`).  HELPED: the set it is replayed into.
@@ -760,7 +769,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             for (int t = 0; t < 2; t++) {
               const bf16x8 zr = pack8<PAIRS>(x2.b[0][i], t);
               if constexpr (FULL && !IMG) {
-                image_store(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
+                image_store<CACHED>(bZ1, j * IMG_BYTES, 2 * tb[i] + t, t16, zr);
               } else if constexpr (FULL) {
                 // The walk needs gelu, gelu' and gelu'' of the ROUNDED Z1 (what it would compute from the image
                 // of Z1); a replaying workgroup has the time to do that for it.
@@ -839,14 +848,14 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             }
           }
           if constexpr (FULL) {
-            ln_store_g<PAIRS>(bXHF, vln, j * TILE_BYTES, z);
-            ln_store_g<PAIRS>(bGOF, vln, j * TILE_BYTES, go);
+            ln_store_g<CACHED, PAIRS>(bXHF, vln, j * TILE_BYTES, z);
+            ln_store_g<CACHED, PAIRS>(bGOF, vln, j * TILE_BYTES, go);
           }
           const float s1 = oct_sum(sum8(gx)), s2 = oct_sum(dot8(gx, z));
           const float sc = rstd * (1.f / FD), neg_eta = -bf2f(s_etah[tok]);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;   // dl/dZ2
-          if constexpr (FULL) ln_store_g<PAIRS>(bGZ2, vln, j * TILE_BYTES, gx);
+          if constexpr (FULL) ln_store_g<CACHED, PAIRS>(bGZ2, vln, j * TILE_BYTES, gx);
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] *= neg_eta;                             // G2, in two terms (the second in
           ln_token_sum_store(s_deta + v * CS, gx, lane, f0);   // b2's step: this wave's share (s_deta is the walk's otherwise)
@@ -1025,12 +1034,12 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int s = 0; s < 4; s++) {
             w2a[s] = piece_tr<LDH>(T1, 0, s, lane);
-            image_store(bIMG2, j * IMG_BYTES, s, t16, w2a[s]);
+            image_store<CACHED>(bIMG2, j * IMG_BYTES, s, t16, w2a[s]);
           }
 #pragma unroll
           for (int fb = 0; fb < 2; fb++)
 #pragma unroll
-            for (int s = 0; s < 2; s++) image_store(bIMG1, j * IMG_BYTES, 2 * fb + s, t16, piece_tr<LDF>(T2, fb, s, lane));
+            for (int s = 0; s < 2; s++) image_store<CACHED>(bIMG1, j * IMG_BYTES, 2 * fb + s, t16, piece_tr<LDF>(T2, fb, s, lane));
         }
         TTT_STAGE(BS_R_IMAGES);
         // post-update forward on XQ; X2_bar rows [tok][hid] -> T0, gelu'(Z1_bar) packed
@@ -1125,7 +1134,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
           for (int e = 0; e < 8; e++) gx[e] = (FD * gx[e] - s1 - z[e] * s2) * sc;
           ln_store<PAIRS>(s_a + tok * LDX + f0, gx);            // gZ2_bar
-          ln_store_g<PAIRS>(bGZB, vln, j * TILE_BYTES, gx);
+          ln_store_g<CACHED, PAIRS>(bGZB, vln, j * TILE_BYTES, gx);
         }
         __syncthreads();
         TTT_STAGE(BS_R_OUT_LN);
@@ -1134,7 +1143,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           // W1 after the step (lane = F, contraction = hid).  Beside a walk it is the image stored above, fetched ahead of its use; where
           // the same workgroup walks, and every CU is busy, that is a trip to HBM, and it goes through T2 once more (backward,
           // ms, 384 x 512 33.5 -> 33.3, 200 x 100 3.68 -> 3.65 or the same; 96 x 128, with 64 CUs idle, 2.65 -> 2.67).
-          constexpr bool W1_AGAIN = ROLE == 0;
+          constexpr bool W1_AGAIN = ROLE == 0 && !CACHED;
           bf16x8 w1a[2][2];
           if constexpr (!W1_AGAIN)
 #pragma unroll
@@ -1191,8 +1200,8 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           // what the reverse walk adds to the running gradients, as ready-made operands (lane = hid, contraction = tok)
 #pragma unroll
           for (int s = 0; s < 4; s++) {
-            image_store(bX2B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T0, 0, s, lane));
-            image_store(bGZ1B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T1, 0, s, lane));
+            image_store<CACHED>(bX2B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T0, 0, s, lane));
+            image_store<CACHED>(bGZ1B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T1, 0, s, lane));
           }
           WAVE_SYNC();   // every reader of T1 / T2 is done before the pair sum takes their place
           {
@@ -1797,7 +1806,11 @@ __global__ __launch_bounds__(BW_THREADS) void ttt_mlp_bwd_kernel(const BwdParams
     k_hi = p.K - 1 - seg * p.seg_groups;
     k_lo = k_hi - p.seg_groups + 1 > 0 ? k_hi - p.seg_groups + 1 : 0;
   }
-  bwd_body<0, false, false>(p, smem, bh, k_hi, k_lo);
+  // With few pairs a group's images stay in the memory-side cache until they are walked unless they are streamed there; with many they
+  // do not, and streamed they leave the L2 to the parks.  The line lies between 64 pairs (x 64 mini-batches in groups of 16: 2.24 ms
+  // streamed, 2.19 cached; 48 x 256 8.85, 8.65) and 96 (2.26, 2.29).
+  if (p.nbh < 80) bwd_body<0, false, false, false, false, false, false, true>(p, smem, bh, k_hi, k_lo);
+  else bwd_body<0, false, false>(p, smem, bh, k_hi, k_lo);
 }
 #endif
 

@@ -238,9 +238,9 @@ const char* ttt_mlp_error_string(int code);
  * `compute_units` CUs (no device needed): the first *one_workgroup_pairs pairs run with one workgroup each,
  * the remaining *other_pairs with *workgroups_per_other_pair each (0 if there are none): whole ones of a pair's share where
  * those of an eighth of the device work for all of its pairs.  Workgroups that only help pairs that have one are not counted.
- * which = 0 forward: 2 (recurrence, output), 3 or 4 (recurrence on two, one or two for the output).  1 backward: 2 (replay, walk), 3 (two
- * replay); with the walk on two and one for grad_L_XK / grad_L_XV 12, 10, 8 or 7 (eight, six, four or three that replay, one that reads
- * ahead), 6 or 5 (three or two that replay); 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly.  More than 2
+ * which = 0 forward: 2 (recurrence, output), 3 (recurrence on two, output), 4 (both on all four).  1 backward: 2 (replay, walk), 3 (two
+ * replay); with the walk, grad_L_XK and grad_L_XV on four 12, 10, 8 or 7 (eight, six, four or three that replay) or 6 (2.4); with the walk
+ * on two, one for grad_L_XK / grad_L_XV and two that replay 5; 5, 4 or 3 where the CUs of an eighth of the device do not go round evenly.  More than 2
  * forward, and all backward but 2 and the 3 that has no eighth of the device for its pairs: the workgroups of a pair share an XCD, and those of
  * ceil(*other_pairs / 8) pairs fit an eighth of the CUs.  Backward calls whose checkpoint groups are short or few may take fewer. */
 int ttt_mlp_launch_plan(int which, long long pairs, int compute_units, long long* one_workgroup_pairs,

@@ -337,9 +337,9 @@ struct Staged3 {
 };
 // `mb` = mini-batch index inside this (batch, head); t16 = 16 * tid.
 TTT_DEV void stage3_load(Staged3& s, gptr_t ga, gptr_t gb, gptr_t gc, gptr_t geta, int mb, int tid, unsigned t16) {
-  s.a = g_ld16(ga, t16, mb * TILE_BYTES);
-  s.b = g_ld16(gb, t16, mb * TILE_BYTES);
-  s.c = g_ld16(gc, t16, mb * TILE_BYTES);
+  s.a = g_ld_stream<u32x4>(ga, t16, mb * TILE_BYTES);
+  s.b = g_ld_stream<u32x4>(gb, t16, mb * TILE_BYTES);
+  s.c = g_ld_stream<u32x4>(gc, t16, mb * TILE_BYTES);
   s.eta = g_ldh(geta, 2 * (tid & (CS - 1)), mb * (CS * 2));   // in bounds for every thread; threads >= CS drop it
 }
 TTT_DEV void stage3_store(const Staged3& s, bf16* sa, bf16* sb, bf16* sc, bf16* s_eta, int tid) {
@@ -1025,8 +1025,10 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         // operand images of the state after this step, for the reverse walk; the image of W2 (lane = hid,
         // contraction = F) also serves the output branch below
         bf16x8 w2a[4];
+        bf16x8 gO_n;   // LayerNorm lanes: the upstream gradient of their 8 features, asked for two stages ahead
         {
           LANE_VARS;
+          gO_n = g_ld_stream<bf16x8>(bGO, vln, mb * TILE_BYTES);
           // bIMG2: W2, lane = hid, contraction = F;  bIMG1: W1^T, lane = F, contraction = hid
           store_state_rows<LDF>(T2, W1s, c, h);                                 // rows [hid][F]
           store_state_rows<LDH>(T1, W2s, c, h);                                 // rows [F][hid]
@@ -1044,7 +1046,6 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         TTT_STAGE(BS_R_IMAGES);
         // post-update forward on XQ; X2_bar rows [tok][hid] -> T0, gelu'(Z1_bar) packed
         bf16x8 d1b[2][2];
-        bf16x8 gO_n;   // LayerNorm lanes: the upstream gradient of their 8 features, asked for a stage ahead
         {
           LANE_VARS;
           AccT<1, 2> z1b;
@@ -1085,10 +1086,6 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
           mma_jit<2>(z2, [&](int rb, int s) { return piece_state(W2s, rb, s); },
                      [&](int i, int s) { return x2bQ[i][s]; });
           WAVE_SYNC();   // this wave's readers of T1 / T2 are done
-          {
-            LANE_VARS;
-            gO_n = g_ld_stream<bf16x8>(bGO, vln, mb * TILE_BYTES);   // under way during the pair sum
-          }
           pair_sum(s_own, s_partner, z2, c, h);
         }
         TTT_STAGE(BS_R_OUT_FORWARD);
@@ -1096,22 +1093,9 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         //      right now, and nothing of the running gradients.  Output LayerNorm forward and backward:
         float gO[8];
         bf16x8 dxq_old;
+        Staged3 next;
         {
           LANE_VARS;
-          // The upstream gradient is taken out of its load registers before the loads below are issued: they are
-          // issued under a condition, so a wait for an older load placed after them has to be a wait for all of them.
-          ln_cvt8(gO, gO_n);
-#pragma unroll
-          for (int e = 0; e < 8; e++) asm volatile("" : "+v"(gO[e]));
-          // Every reader of this mini-batch's XQ / XK / XV / eta is past the barriers of the pair sum: the next
-          // mini-batch's leave HBM now - straight to LDS, no registers involved - and have the rest of this
-          // mini-batch to arrive.
-          if (j + 1 < j_end) {
-            tile_to_lds<CPOL_NT>(bXQ, (mb + 1) * TILE_BYTES, smem + SB_XQ, v, lane);
-            tile_to_lds<CPOL_NT>(bXK, (mb + 1) * TILE_BYTES, smem + SB_XK, v, lane);
-            tile_to_lds<CPOL_NT>(bXV, (mb + 1) * TILE_BYTES, smem + SB_E2, v, lane);
-            eta_to_lds(bETA, (mb + 1) * (CS * 2), smem + SB_ETA, v, lane);
-          }
           float z[8], gx[8], gam[8];
           {
             float b2v[8];
@@ -1120,6 +1104,11 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
 #pragma unroll
             for (int e = 0; e < 8; e++) z[e] += b2v[e];
           }
+          asm volatile("" : "+v"(gO_n));   // not converted, and waited for, as soon as it is asked for
+          ln_cvt8(gO, gO_n);
+          // The next mini-batch's tiles: in registers until every reader of this one's is done, at the end (the last one's come again,
+          // unread).  Straight to LDS they were waited for at this stage's barrier, together with every store of images before them.
+          stage3_load(next, bXQ, bXK, bXV, bETA, j + 1 < j_end ? mb + 1 : mb, tid, t16);
           float sd;
           ln_normalize(z, &sd);   // z = x_hat
           ln_load_f32(gam, s_gam + f0);
@@ -1140,6 +1129,7 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
         TTT_STAGE(BS_R_OUT_LN);
         {
           LANE_VARS;
+          dxq_old = g_ld_stream<bf16x8>(OLD_VALUE(bDXQ, mb * TILE_BYTES));   // ahead of the images' stores, which it would have to wait for
           // W1 after the step (lane = F, contraction = hid).  Beside a walk it is the image stored above, fetched ahead of its use; where
           // the same workgroup walks, and every CU is busy, that is a trip to HBM, and it goes through T2 once more (backward,
           // ms, 384 x 512 33.5 -> 33.3, 200 x 100 3.68 -> 3.65 or the same; 96 x 128, with 64 CUs idle, 2.65 -> 2.67).
@@ -1204,23 +1194,21 @@ TTT_DEV bool bwd_body(const BwdParams& p, unsigned char* smem, const int bh, con
             image_store<CACHED>(bGZ1B, j * IMG_BYTES, s, t16, piece_tr<LDH>(T1, 0, s, lane));
           }
           WAVE_SYNC();   // every reader of T1 / T2 is done before the pair sum takes their place
-          {
-            LANE_VARS;
-            dxq_old = g_ld_stream<bf16x8>(OLD_VALUE(bDXQ, mb * TILE_BYTES));   // under way during the pair sum
-          }
           pair_sum(s_own, s_partner, dq, c, h);
         }
         {
           LANE_VARS;
           float z[8];
           ln_gather(z, s_lnrow);
+          asm volatile("" : "+v"(dxq_old));
 #pragma unroll
           for (int e = 0; e < 8; e++) z[e] = (float)dxq_old[e] + (z[e] + gO[e]);
           g_st_stream<bf16x8>(bDXQ, vln, mb * TILE_BYTES, cvt8<PAIRS>(z));
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next mini-batch's inputs are in LDS before the barrier at the loop's top
+        stage3_store(next, s_xq, s_xk, s_e2, s_etah, tid);   // (read last ahead of the output branch's pair sum)
         TTT_STAGE(BS_R_OUT_BACKWARD);
       }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if constexpr (ROLE == 1) eighth_done(e);
       if constexpr (ROLE == 1 && !EIGHTHS) {
         LANE_VARS;
